@@ -28,8 +28,7 @@
 //                      step, and the launch is a single read-modify-write of the matrix; otherwise it
 //                      makes the pass for the maximum first (on registers where the matrix fits the
 //                      register file of the machine, by streaming the rows twice where it does not).
-//                      As separate launches (4a max, 5 update, 6 slot update) on request or while the
-//                      process holds more than one trainer.
+//                      As separate launches (4a max, 5 update, 6 slot update) on request.
 //
 // The device code is in fv_train_gather.h (1), fv_train_group.h (2), fv_train_sparse.h (3),
 // fv_train_dense.h (4 to 6) and fv_train_top2.h (the carried largest weights); fv_train_state.h holds
@@ -108,13 +107,27 @@ static void fv_trainer_free_corpus(fv_trainer *t) {
   t->ahead_valid = false;
 }
 
-// Trainers alive in this process. The single dense launch, where it has to make the pass for max|ds|, exchanges
-// the blocks' maxima inside the launch and so needs every compute unit for itself: two of them in flight at
-// once, from two trainers' streams, could each hold half the machine and wait for the other half. While more
-// than one trainer exists a step therefore enqueues the launch twice, in the form that waits for nobody
-// (fv_dense_args.phase): the first does the whole step whenever max|ds| is known beforehand, the second then
-// ends at once.
-static std::atomic<int> fv_trainers_alive{0};
+// Trainers of this process with steps enqueued that nobody has waited for yet. The single dense launch, where it has
+// to make the pass for max|ds|, exchanges the blocks' maxima inside the launch and so needs every compute unit for
+// itself: two of them in flight at once, from two trainers' streams, could each hold half the machine and wait for
+// the other half. A step that finds another trainer's steps in flight therefore enqueues the launch twice, in the
+// form that waits for nobody (fv_dense_args.phase): the first does the whole step whenever max|ds| is known
+// beforehand, the second then ends at once. Of two trainers that begin together the later one to count itself sees
+// the other, and a trainer leaves the count only when its stream has drained, so launches that wait are in flight
+// from one trainer at most. (Counting the trainers that merely exist, as this did, cost an idle second trainer's
+// owner 3.4 us of 57 us per step at K = 400, V = 20000, B = 10000: the second launch.)
+static std::atomic<int> fv_trainers_in_flight{0};
+
+static void fv_trainer_enters_flight(fv_trainer *t) {
+  if (!t->in_flight) fv_trainers_in_flight.fetch_add(1);
+  t->in_flight = true;
+}
+
+// The trainer's stream has drained (a synchronisation of it has returned).
+static void fv_trainer_leaves_flight(fv_trainer *t) {
+  if (t->in_flight) fv_trainers_in_flight.fetch_sub(1);
+  t->in_flight = false;
+}
 
 // After a single dense launch has given up: the trainer goes on with two launches per step, and the marks
 // the launch left (status word, "dead" flag for the launches behind it) are cleared. Returns the tag.
@@ -134,6 +147,7 @@ static int fv_trainer_take_giveup(fv_trainer *t, uint32_t *out_tag) {
 // Waits for the trainer's stream; reports a single dense launch that gave up waiting for its other blocks.
 static int fv_trainer_wait(fv_trainer *t) {
   FV_HIP(hipStreamSynchronize(t->stream));
+  fv_trainer_leaves_flight(t);
   uint32_t tag = 0;
   FV_TRY(fv_trainer_take_giveup(t, &tag));
   if (tag)
@@ -171,7 +185,7 @@ extern "C" int fv_trainer_destroy(fv_trainer *t) {
   (void)hipFree(t->path_count);
   if (t->onepass_status) (void)hipHostFree(t->onepass_status);
   if (t->stream) (void)hipStreamDestroy(t->stream);
-  fv_trainers_alive.fetch_sub(1);
+  fv_trainer_leaves_flight(t);
   delete t;
   return FV_OK;
 }
@@ -358,7 +372,6 @@ extern "C" int fv_trainer_create(const fv_train_config *cfg, fv_trainer **out_tr
              "batch x window = %llu is out of range", (unsigned long long)cfg->batch * cfg->window);
   fv_trainer *t = new fv_trainer();
   memset(t, 0, sizeof *t);
-  fv_trainers_alive.fetch_add(1);
   t->cfg = *cfg;
   t->K = cfg->hid;
   t->ldk = ldk;
@@ -739,7 +752,8 @@ static int fv_enqueue_step(fv_trainer *t, uint64_t first, uint32_t n, float eps,
   const uint32_t slot_region = grouping_in_sparse && !t->no_block_regions ? t->slot_region : 0u;
   if (slot_region) n_slots = slot_region;
   const bool onepass = t->onepass && n_slots + 1 < FV_SENTINEL_MAX;
-  const bool alone = fv_trainers_alive.load() == 1;
+  fv_trainer_enters_flight(t);
+  const bool alone = fv_trainers_in_flight.load() == 1;
   g.won = nullptr;
   g.won2 = nullptr;
   g.won_words = t->won_words;
@@ -956,7 +970,7 @@ static int fv_enqueue_step(fv_trainer *t, uint64_t first, uint32_t n, float eps,
 #define FV_CASE(U)                                                                     \
   if (anti) fv_launch_onepass<U, true>(d, t->onepass_blocks, smem1, t->stream);        \
   else fv_launch_onepass<U, false>(d, t->onepass_blocks, smem1, t->stream);
-      // alone on the device: one launch that exchanges the blocks' maxima itself where it needs them; else the
+      // no other trainer in flight: one launch that exchanges the blocks' maxima itself where it needs them; else the
       // launch twice, in the form that waits for nobody (both with this step's launch number)
       for (uint32_t phase = alone ? 0u : 1u; phase <= (alone ? 0u : 2u); ++phase) {
         d.phase = phase;
@@ -1092,6 +1106,7 @@ extern "C" int fv_trainer_run_epoch(fv_trainer *t, uint64_t epoch_id, uint64_t n
     t->step_tag = 0;
     FV_TRY(rc);
     FV_HIP(hipStreamSynchronize(t->stream));
+    fv_trainer_leaves_flight(t);
     uint32_t tag = 0;
     FV_TRY(fv_trainer_take_giveup(t, &tag));
     if (!tag) return FV_OK;
@@ -1341,6 +1356,7 @@ extern "C" int fv_trainer_time_kernel(fv_trainer *t, uint32_t kernel_index, uint
   if (kernel_index == 0 && rc == FV_OK)
     rc = fv_enqueue_step(t, t->last_first, t->last_n, t->last_eps, t->last_delta, nullptr, 1u);
   FV_HIP(hipStreamSynchronize(t->stream));
+  fv_trainer_leaves_flight(t);
   float ms = 0.0f;
   FV_HIP(hipEventElapsedTime(&ms, e0, e1));
   *out_mean_ms = ms / (float)reps;

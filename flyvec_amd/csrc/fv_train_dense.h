@@ -50,8 +50,8 @@ struct fv_dense_args {
   float2 *top2_part;     // out: the same of the matrix this launch leaves, over each block's share: [block][ldk]
   uint32_t part_base;    // separate launches: the update launch's blocks come first, then the slot launch's four
   uint32_t *path_count;  // [0] launches that knew max|ds| when they started, [1] launches that made the pass for it
-  // Single-launch form without any wait between blocks, for a device the launch may have to share (a process with
-  // more than one trainer): the step enqueues the kernel twice with the same launch number. phase 1 does the
+  // Single-launch form without any wait between blocks, for a device the launch may have to share (another trainer's
+  // steps are in flight): the step enqueues the kernel twice with the same launch number. phase 1 does the
   // whole step when max|ds| is known beforehand; otherwise it only makes the pass for the maximum and leaves
   // every block's maximum in its arrival word. phase 2 ends at once in the first case (every block evaluates the
   // same rule on the same inputs) and in the second reads the words, all written when it starts, and makes the

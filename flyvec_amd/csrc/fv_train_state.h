@@ -99,6 +99,7 @@ struct fv_trainer {
   float last_eps;
   uint64_t shuffle_calls;
   bool have_corpus, have_weights;
+  bool in_flight;  // steps have been enqueued since the stream was last known to have drained
   unsigned dense_blocks;   // blocks of the absmax launch
   unsigned update_blocks;  // blocks of the dense update launch
   // one launch for both dense passes (a matrix that fits the machine's registers): blocks, 16-byte

@@ -216,8 +216,8 @@ int fv_trainer_get_giveups_recovered(fv_trainer *t, uint64_t *out_count);
  * there is none), 3 for its streaming form whatever the matrix size, 2 for separate launches (maximum, update,
  * sparse elements), 0 returns to the choice made at creation. Results are bit-identical in all forms. Where the
  * single launch has to make the pass for max|ds| its blocks exchange their maxima inside the launch and need the
- * whole device for themselves; while a process holds more than one trainer a step therefore enqueues the launch
- * twice in a form that waits for nobody: the first does the whole step when max|ds| is known beforehand (the
+ * whole device for themselves; a step that finds steps of another trainer of the process in flight (enqueued and
+ * not yet waited for) therefore enqueues the launch twice in a form that waits for nobody: the first does the whole step when max|ds| is known beforehand (the
  * usual case) and the second ends at once, else the first makes the pass and the second the update. */
 int fv_trainer_set_dense_launches(fv_trainer *t, uint32_t launches);
 /* The single launch carries the two largest |W| of every row from step to step; from them and from what

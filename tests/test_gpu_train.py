@@ -465,6 +465,45 @@ def test_second_trainer_alive_while_the_pass_for_the_maximum_is_needed(gpu, orac
     other.close()
 
 
+@pytest.mark.parametrize("launches", [1, 3])
+def test_steps_while_another_trainer_is_in_flight(gpu, oracle_lib, launches):
+    """A step that finds another trainer's steps enqueued and not yet waited for takes the form that waits for nobody;
+    once they have been waited for it returns to the one launch. The same weights as above, so that nearly every
+    step makes the pass for max|ds|, in both situations in turn."""
+    from flyvec_amd import Trainer, synthetic
+    to = oracle_lib
+    V, K, w, B = 800, 96, 9, 2000
+    tokens, offsets = small_corpus(80000, V, seed=2)
+    starts, invf = oracle_inputs(to, tokens, offsets, V, w)
+    perm = np.random.default_rng(3).permutation(len(starts)).astype(np.uint64)
+    hot = np.argsort(-np.bincount(tokens[tokens >= 0], minlength=V))[:6]
+    planted = synthetic.synapses(K, V, seed=9)
+    planted[:, hot[:3]] = np.float32(7.0)
+    other = Trainer(V, 8, w, 16)
+    other.set_corpus(tokens, offsets)
+    other.set_weights(synthetic.synapses(8, V, seed=1))
+    t = Trainer(V, K, w, B, initial_learning_rate=1e-3)
+    t.set_dense_launches(launches)
+    t.set_corpus(tokens, offsets)
+    t.set_permutation(perm)
+    t.set_weights(planted)
+    Wo = planted.copy()
+    for s in range(9):
+        if s % 3 == 0:
+            other.step(0, 16, 1e-4)                  # in flight, whatever the device has finished
+        if s % 3 == 2:
+            other.sync()
+        t.step(s * B, B, 1e-3)
+        ref = to.train_step(Wo, to.inflate(tokens, starts, perm, s * B, B, w, V), invf, 1e-3)
+        xx, nc = t.step_stats()
+        assert np.array_equal(t.winners(B), ref["winners"]) and np.array_equal(xx, ref["xx"]) and nc == ref["nc"], s
+        t.sync()                                     # out of flight: the next step of `other` may be the only one
+    assert np.array_equal(t.get_weights().view(np.uint32), Wo.view(np.uint32))
+    assert sum(t.dense_path_counts) == 9 and t.dense_path_counts[1] >= 4
+    t.close()
+    other.close()
+
+
 def test_device_shuffle_is_a_cumulative_bijection(gpu):
     from flyvec_amd import Trainer
     V, w = 300, 11

@@ -180,10 +180,33 @@ int fv_upload_weights(const float *W_host, float *Wt_dev, uint32_t K, uint64_t N
   return rc;
 }
 
+// The device's address of `bytes` of page-locked host memory at p (hipHostMalloc), or null where the range is anything
+// else: pageable, or not inside one allocation.
+void *fv_device_view(const void *p, size_t bytes) {
+  hipPointerAttribute_t at;
+  void *base = nullptr;
+  size_t size = 0;
+  if (hipPointerGetAttributes(&at, p) != hipSuccess || at.type != hipMemoryTypeHost || !at.devicePointer ||
+      hipMemGetAddressRange((hipDeviceptr_t *)&base, &size, (hipDeviceptr_t)at.devicePointer) != hipSuccess) {
+    (void)hipGetLastError();
+    return nullptr;
+  }
+  const size_t before = (size_t)((char *)at.devicePointer - (char *)base);
+  return before <= size && bytes <= size - before ? at.devicePointer : nullptr;
+}
+
+// To page-locked memory the layout change writes over the link itself: no staging matrix on the device (its allocation
+// and its release, which waits for the device, cost more than the copy of a small matrix), no second pass.
 int fv_download_weights(const float *Wt_dev, float *W_host, uint32_t K, uint64_t N, uint32_t ldk,
                         hipStream_t stream) {
-  float *stage = nullptr;
   size_t bytes = (size_t)K * N * sizeof(float);
+  if (float *view = (float *)fv_device_view(W_host, bytes)) {
+    int rc = fv_launch_to_row_major(Wt_dev, view, K, N, ldk, stream);
+    const hipError_t e = hipStreamSynchronize(stream);
+    if (rc == FV_OK && e != hipSuccess) rc = fv_fail(FV_ERR_HIP, "weight download failed: %s", hipGetErrorString(e));
+    return rc;
+  }
+  float *stage = nullptr;
   FV_HIP(hipMalloc((void **)&stage, bytes));
   int rc = fv_launch_to_row_major(Wt_dev, stage, K, N, ldk, stream);
   hipError_t e = hipSuccess;

@@ -46,19 +46,46 @@
 
 // ---- row norms (log line of flyvec/src/cuda_funcs.cu:1234-1242) -------------------------------
 
-__global__ __launch_bounds__(256) void fv_row_norm_kernel(const float *__restrict__ Wt, uint64_t N,
-                                                          uint32_t ldk, double *__restrict__ out) {
-  __shared__ double part[4];
-  const uint32_t h = blockIdx.x;
+// Sixteen neurons and sixteen tokens per block and turn: of the token-major matrix a wave reads four tokens' 64 bytes.
+// Every block leaves the sum over its tokens, and the second launch adds the blocks' sums in block order. (One block
+// per row, as before, read 4 bytes of every line it fetched, with ten blocks on the whole device: 59 us at N = 40000,
+// 225 us at N = 100000 with K = 1000.)
+#define FV_NORM_BLOCKS 256u
+__global__ __launch_bounds__(256) void fv_row_squares_kernel(const float *__restrict__ Wt, uint64_t N, uint32_t ldk,
+                                                             uint32_t n_rows, double *__restrict__ part) {
+  __shared__ double sum[256];
+  const uint32_t h = blockIdx.y * 16 + (threadIdx.x & 15u);
+  const uint64_t step = (uint64_t)gridDim.x * 16;
   double acc = 0.0;
-  for (uint64_t i = threadIdx.x; i < N; i += 256) {
-    const double v = (double)Wt[i * ldk + h];
-    acc += v * v;
+  if (h < n_rows) {
+    const float *col = Wt + h;
+    uint64_t i = (uint64_t)blockIdx.x * 16 + (threadIdx.x >> 4);
+    for (; i + 3 * step < N; i += 4 * step) {
+      float v[4];
+#pragma unroll
+      for (int k = 0; k < 4; ++k) v[k] = col[(i + k * step) * ldk];
+#pragma unroll
+      for (int k = 0; k < 4; ++k) acc += (double)v[k] * (double)v[k];
+    }
+    for (; i < N; i += step) {
+      const double v = (double)col[i * ldk];
+      acc += v * v;
+    }
   }
+  sum[threadIdx.x] = acc;
+  for (uint32_t d = 128; d >= 16; d >>= 1) {
+    __syncthreads();
+    if (threadIdx.x < d) sum[threadIdx.x] += sum[threadIdx.x + d];
+  }
+  if (threadIdx.x < 16 && h < n_rows) part[(uint64_t)h * gridDim.x + blockIdx.x] = sum[threadIdx.x];
+}
+
+__global__ __launch_bounds__(64) void fv_row_norm_kernel(const double *__restrict__ part, uint32_t n_part,
+                                                         double *__restrict__ out) {
+  double acc = 0.0;
+  for (uint32_t i = threadIdx.x; i < n_part; i += 64) acc += part[(uint64_t)blockIdx.x * n_part + i];
   for (int d = 32; d >= 1; d >>= 1) acc += __shfl_down(acc, d, 64);
-  if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = acc;
-  __syncthreads();
-  if (threadIdx.x == 0) out[h] = sqrt(part[0] + part[1] + part[2] + part[3]);
+  if (threadIdx.x == 0) out[blockIdx.x] = sqrt(acc);
 }
 
 // ---- window order ------------------------------------------------------------------------------
@@ -183,6 +210,8 @@ extern "C" int fv_trainer_destroy(fv_trainer *t) {
   (void)hipFree(t->top2_part);
   (void)hipFree(t->row_hits);
   (void)hipFree(t->path_count);
+  (void)hipFree(t->norm_part);
+  if (t->norms) (void)hipHostFree(t->norms);
   if (t->onepass_status) (void)hipHostFree(t->onepass_status);
   if (t->stream) (void)hipStreamDestroy(t->stream);
   fv_trainer_leaves_flight(t);
@@ -1234,14 +1263,25 @@ extern "C" int fv_trainer_row_norms(fv_trainer *t, uint32_t n_rows, double *out_
   FV_REQUIRE(t->have_weights, FV_ERR_STATE, "no weights set");
   if (n_rows > t->K) n_rows = t->K;
   if (n_rows == 0) return FV_OK;
-  double *d = nullptr;
-  FV_HIP(hipMalloc((void **)&d, n_rows * sizeof(double)));
-  hipLaunchKernelGGL(fv_row_norm_kernel, dim3(n_rows), dim3(256), 0, t->stream, t->Wt, t->N, t->ldk, d);
-  hipError_t e = hipGetLastError();
-  if (e == hipSuccess) e = hipMemcpyAsync(out_norms, d, n_rows * sizeof(double), hipMemcpyDeviceToHost, t->stream);
-  if (e == hipSuccess) e = hipStreamSynchronize(t->stream);
-  (void)hipFree(d);
-  if (e != hipSuccess) return fv_fail(FV_ERR_HIP, "row norms failed: %s", hipGetErrorString(e));
+  // the blocks' sums, and the norms in page-locked memory: kept for as many rows as have been asked for
+  if (t->norm_rows < n_rows) {
+    FV_HIP(hipStreamSynchronize(t->stream));
+    (void)hipFree(t->norm_part);
+    if (t->norms) (void)hipHostFree(t->norms);
+    t->norm_part = t->norms = nullptr;
+    t->norm_rows = 0;
+    FV_HIP(hipMalloc((void **)&t->norm_part, (size_t)n_rows * FV_NORM_BLOCKS * sizeof(double)));
+    FV_HIP(hipHostMalloc((void **)&t->norms, n_rows * sizeof(double), hipHostMallocDefault));
+    t->norm_rows = n_rows;
+  }
+  const uint64_t want = (t->N + 15) / 16;
+  const uint32_t blocks = (uint32_t)(want < FV_NORM_BLOCKS ? want : FV_NORM_BLOCKS);
+  hipLaunchKernelGGL(fv_row_squares_kernel, dim3(blocks, (n_rows + 15) / 16), dim3(256), 0, t->stream, t->Wt, t->N, t->ldk,
+                     n_rows, t->norm_part);
+  hipLaunchKernelGGL(fv_row_norm_kernel, dim3(n_rows), dim3(64), 0, t->stream, t->norm_part, blocks, t->norms);
+  FV_HIP(hipGetLastError());
+  FV_HIP(hipStreamSynchronize(t->stream));
+  memcpy(out_norms, t->norms, n_rows * sizeof(double));
   return FV_OK;
 }
 

@@ -134,5 +134,7 @@ struct fv_trainer {
   uint32_t *onepass_status;  // pinned host word: 0, or the tag of the first launch that gave up
   uint32_t step_tag;         // tag of the step being enqueued: run_epoch numbers its steps from 1, else 0
   uint64_t giveups_recovered;  // epochs in which run_epoch took up again behind a launch that gave up
+  double *norm_part, *norms;   // workspace of fv_trainer_row_norms: FV_NORM_BLOCKS sums per row; page-locked results
+  uint32_t norm_rows;          // rows they hold
   float update_cut;  // largest fp32 <= 1e-10
 };

@@ -504,6 +504,26 @@ def test_steps_while_another_trainer_is_in_flight(gpu, oracle_lib, launches):
     other.close()
 
 
+@pytest.mark.parametrize("K,V", [(1, 1), (17, 3), (64, 505), (130, 2049), (400, 1)])
+def test_row_norms_and_page_locked_checkpoints(gpu, K, V):
+    """Row norms over fewer and more columns than a turn of the launch's blocks takes, for numbers of rows around the
+    sixteen of a block, more rows than before asked for included; and the matrix written straight to page-locked
+    memory (also to a piece of a larger array, and beside one), equal to the copy in ordinary memory."""
+    from flyvec_amd import Trainer, _lib, synthetic
+    W = synthetic.synapses(K, V, seed=K)
+    t = Trainer(V, K, 3, 16)
+    t.set_weights(W)
+    want = np.sqrt((W.astype(np.float64) ** 2).sum(1))
+    for n in (1, 2, 15, 16, 17, 10, K):
+        assert np.allclose(t.row_norms(n), want[:min(n, K)], rtol=1e-13)  # N fp64 roundings of terms of one sign
+    assert np.array_equal(t.get_weights(), W)
+    block = _lib.pinned_empty(3 * W.size, np.float32)
+    block[:] = 7.0
+    assert np.array_equal(t.get_weights(block[W.size:2 * W.size].reshape(W.shape)), W)
+    assert (block[:W.size] == 7.0).all() and (block[2 * W.size:] == 7.0).all()
+    t.close()
+
+
 def test_device_shuffle_is_a_cumulative_bijection(gpu):
     from flyvec_amd import Trainer
     V, w = 300, 11

@@ -15,18 +15,23 @@
 #include <math.h>
 #include <string.h>
 
-#include <atomic>
 #include <memory>
-#include <thread>
 #include <vector>
 
-#include "fv_internal.h"
+#include "fv_host_copy.h"
 
 // Host-buffer batches go through the device in chunks on two streams of equal priority, so that one
 // chunk's copies run while the other's kernel does: per stream a device buffer for the chunk's indices and
 // one for each kind of output, kept from call to call (grown when a call needs more).
 #define FV_HASH_LANES 2
-#define FV_HASH_CHUNK (1u << 17)  // windows per chunk
+#define FV_HASH_CHUNK (1u << 17)  // most windows per chunk
+// A batch is cut into about this many chunks, of output that takes the link some 30 us or more: one call's copies in,
+// kernel, copies out and host copies then overlap also for batches that fit one chunk.
+#define FV_HASH_CHUNKS 8
+#define FV_HASH_CHUNK_MIN_BYTES ((uint64_t)3 << 19)
+// Batches whose indices and codes take no more than this go through one page-locked buffer that the kernel itself
+// reads and writes: a launch and a wait, where two copies and their waits took 30 us of 44.
+#define FV_HASH_DIRECT_BYTES ((uint64_t)1 << 18)
 
 struct fv_hash_lane {
   hipStream_t stream;
@@ -34,9 +39,9 @@ struct fv_hash_lane {
   uint64_t *bits;
   int8_t *codes;
   size_t idx_cap, bits_cap, codes_cap;  // bytes
-  // page-locked staging for outputs that go to pageable host memory, and the event behind a chunk's copies
-  char *stage_bits, *stage_codes;
-  size_t stage_bits_cap, stage_codes_cap;
+  // page-locked staging for indices and outputs in pageable host memory, and the event behind a chunk's copies
+  char *stage_idx, *stage_bits, *stage_codes;
+  size_t stage_idx_cap, stage_bits_cap, stage_codes_cap;
   hipEvent_t done;
 };
 
@@ -45,7 +50,8 @@ struct fv_hasher {
   uint64_t N;
   hipStream_t stream;
   float *Wt;
-  uint32_t *err;  // device flag: a column index outside [-1, N) was met
+  uint32_t *err;  // flag in page-locked memory: a column index outside [-1, N) was met
+  char *direct;   // page-locked, FV_HASH_DIRECT_BYTES (null until the first small batch)
   unsigned max_blocks;
   fv_hash_lane lane[FV_HASH_LANES];  // lane 0 runs on `stream`
 };
@@ -80,7 +86,7 @@ __global__ __launch_bounds__(256) void fv_hash_kernel(fv_hash_args a) {
         if (raw >= 0 && col < (int64_t)a.n_cols)
           idx = (int32_t)col;
         else
-          atomicOr(a.err, 1u);
+          *a.err = 1u;  // (in host memory; every store writes the same value)
       }
     }
 
@@ -220,12 +226,14 @@ extern "C" int fv_hasher_destroy(fv_hasher *h) {
     (void)hipFree(ln.idx);
     (void)hipFree(ln.bits);
     (void)hipFree(ln.codes);
+    if (ln.stage_idx) (void)hipHostFree(ln.stage_idx);
     if (ln.stage_bits) (void)hipHostFree(ln.stage_bits);
     if (ln.stage_codes) (void)hipHostFree(ln.stage_codes);
     if (ln.done) (void)hipEventDestroy(ln.done);
   }
   (void)hipFree(h->Wt);
-  (void)hipFree(h->err);
+  if (h->err) (void)hipHostFree(h->err);
+  if (h->direct) (void)hipHostFree(h->direct);
   if (h->stream) (void)hipStreamDestroy(h->stream);
   delete h;
   return FV_OK;
@@ -257,8 +265,8 @@ extern "C" int fv_hasher_create(const float *W, uint32_t hid, uint64_t n_columns
     if (e == hipSuccess) e = hipMalloc((void **)&h->Wt, (size_t)fv_matrix_alloc_elems(h->K, h->N) * sizeof(float));
     if (e == hipSuccess)
       e = hipMemsetAsync(h->Wt + (size_t)h->N * h->ldk, 0, (size_t)fv_matrix_pad_elems(h->K) * sizeof(float), h->stream);
-    if (e == hipSuccess) e = hipMalloc((void **)&h->err, sizeof(uint32_t));
-    if (e == hipSuccess) e = hipMemsetAsync(h->err, 0, sizeof(uint32_t), h->stream);
+    if (e == hipSuccess) e = hipHostMalloc((void **)&h->err, sizeof(uint32_t), hipHostMallocCoherent);
+    if (e == hipSuccess) *h->err = 0;
     if (e != hipSuccess) rc = fv_fail(FV_ERR_HIP, "hasher allocation failed: %s", hipGetErrorString(e));
   }
   if (rc == FV_OK) rc = fv_upload_weights(W, h->Wt, h->K, h->N, h->ldk, h->stream);
@@ -278,10 +286,8 @@ extern "C" int fv_hasher_get_weights(fv_hasher *h, float *out_W) {
 extern "C" int fv_hasher_sync(fv_hasher *h) {
   FV_REQUIRE(h, FV_ERR_INVALID, "null hasher");
   FV_HIP(hipStreamSynchronize(h->stream));
-  uint32_t err = 0;
-  FV_HIP(hipMemcpy(&err, h->err, sizeof err, hipMemcpyDeviceToHost));
-  if (err) {
-    FV_HIP(hipMemset(h->err, 0, sizeof err));
+  if (*(volatile uint32_t *)h->err) {
+    *(volatile uint32_t *)h->err = 0;
     return fv_fail(FV_ERR_DATA, "a column index outside [-1, %llu) was met; its position was skipped",
                    (unsigned long long)h->N);
   }
@@ -317,79 +323,48 @@ static int fv_hash_reserve_pinned(char **buf, size_t *cap, size_t bytes) {
   return FV_OK;
 }
 
-// Ordinary (pageable) host memory, which the device cannot write by DMA?
-static bool fv_is_pageable(const void *p) {
-  hipPointerAttribute_t at;
-  if (hipPointerGetAttributes(&at, p) != hipSuccess) {
-    (void)hipGetLastError();
-    return true;
-  }
-  return at.type == hipMemoryTypeUnregistered;
+// A small batch: the kernel reads the indices from, and writes its results to, one page-locked buffer.
+static int fv_hash_direct(fv_hasher *h, const int32_t *idx, uint64_t n, uint32_t w, uint32_t k, int32_t shift,
+                          uint64_t *out_bits, int8_t *out_codes) {
+  if (!h->direct) FV_HIP(hipHostMalloc((void **)&h->direct, FV_HASH_DIRECT_BYTES, hipHostMallocCoherent));
+  const size_t bits_bytes = out_bits ? n * ((h->K + 63) / 64) * sizeof(uint64_t) : 0;
+  const size_t idx_bytes = n * w * sizeof(int32_t), codes_bytes = out_codes ? n * h->K : 0;
+  uint64_t *bits = (uint64_t *)h->direct;
+  int32_t *ids = (int32_t *)(h->direct + bits_bytes);
+  int8_t *codes = (int8_t *)(h->direct + bits_bytes + idx_bytes);
+  FV_HIP(hipStreamSynchronize(h->stream));  // an earlier call that failed may have left its kernel behind
+  memcpy(ids, idx, idx_bytes);
+  FV_TRY(fv_enqueue_hash(h, ids, n, w, k, shift, out_bits ? bits : nullptr, out_codes ? codes : nullptr));
+  const int rc = fv_hasher_sync(h);
+  if (rc != FV_OK && rc != FV_ERR_DATA) return rc;  // (with a bad index the codes are those without its position)
+  if (out_bits) memcpy(out_bits, bits, bits_bytes);
+  if (out_codes) memcpy(out_codes, codes, codes_bytes);
+  return rc;
 }
 
-// Copies from page-locked staging to the caller's pageable buffers, done by a few host threads while the
-// device works on the next chunks: one thread copies ~10 GB/s, less than the link delivers. Items are
-// published in order; every worker copies its slice of every item.
-#define FV_HASH_COPY_THREADS 4
-struct fv_copy_ring {
-  struct item {
-    const char *src;
-    char *dst;
-    size_t bytes;
-  };
-  std::vector<item> items;
-  std::unique_ptr<std::atomic<uint32_t>[]> finished;  // workers done with item i
-  std::atomic<uint32_t> published{0};
-  std::atomic<bool> quit{false};
-  std::vector<std::thread> workers;
-
-  explicit fv_copy_ring(size_t max_items) : items(max_items), finished(new std::atomic<uint32_t>[max_items]) {
-    for (size_t i = 0; i < max_items; ++i) finished[i].store(0);
-    for (int p = 0; p < FV_HASH_COPY_THREADS; ++p) workers.emplace_back([this, p] { run(p); });
-  }
-  void run(int p) {
-    for (uint32_t i = 0;; ++i) {
-      while (published.load(std::memory_order_acquire) <= i) {
-        if (quit.load(std::memory_order_acquire)) return;
-        std::this_thread::yield();
-      }
-      const item &it = items[i];
-      const size_t per = (it.bytes + FV_HASH_COPY_THREADS - 1) / FV_HASH_COPY_THREADS;
-      const size_t lo = per * p < it.bytes ? per * p : it.bytes, hi = lo + per < it.bytes ? lo + per : it.bytes;
-      if (hi > lo) memcpy(it.dst + lo, it.src + lo, hi - lo);
-      finished[i].fetch_add(1, std::memory_order_release);
-    }
-  }
-  uint32_t publish(const char *src, char *dst, size_t bytes) {
-    const uint32_t i = published.load(std::memory_order_relaxed);
-    items[i] = {src, dst, bytes};
-    published.store(i + 1, std::memory_order_release);
-    return i;
-  }
-  void wait(uint32_t i) {
-    while (finished[i].load(std::memory_order_acquire) < FV_HASH_COPY_THREADS) std::this_thread::yield();
-  }
-  ~fv_copy_ring() {
-    for (uint32_t i = 0; i < published.load(); ++i) wait(i);
-    quit.store(true, std::memory_order_release);
-    for (auto &t : workers) t.join();
-  }
-};
-
-// A batch in host memory: chunks of FV_HASH_CHUNK windows alternate between the lanes; on its lane a
+// A batch in host memory: chunks of up to FV_HASH_CHUNK windows alternate between the lanes; on its lane a
 // chunk is copied in, hashed and copied out in stream order, so the copies of one chunk overlap the kernel
 // of the other. Host buffers from fv_host_alloc_pinned are copied by DMA as they are. Outputs that go to
 // pageable memory are copied by DMA into the lane's page-locked staging and from there by host threads
-// (fv_copy_ring) while the device goes on; pageable inputs go through the runtime's staging. Nothing is
-// allocated once the lanes' buffers have reached the chunk size.
+// (fv_copy_ring) while the device goes on; pageable inputs are copied into the lane's staging by the calling thread.
+// Nothing is allocated once the lanes' buffers have reached the chunk size. (100003 windows, K = 400, pageable: 4.0 ms
+// as one chunk through the runtime's copies.)
 static int fv_hash_host(fv_hasher *h, const int32_t *idx, uint64_t n, uint32_t w, uint32_t k, int32_t shift,
                         uint64_t *out_bits, int8_t *out_codes) {
   if (n == 0) return FV_OK;
   FV_REQUIRE(idx, FV_ERR_INVALID, "null index buffer");
   const uint32_t words = (h->K + 63) / 64;
-  const uint64_t chunk = n < FV_HASH_CHUNK ? n : FV_HASH_CHUNK;
-  const int lanes = n > chunk ? FV_HASH_LANES : 1;
   const size_t bits_row = words * sizeof(uint64_t), codes_row = h->K;
+  const uint64_t out_row = (out_bits ? bits_row : 0) + (out_codes ? codes_row : 0);
+  if (n <= FV_HASH_DIRECT_BYTES && n * (w * sizeof(int32_t) + out_row) <= FV_HASH_DIRECT_BYTES)
+    return fv_hash_direct(h, idx, n, w, k, shift, out_bits, out_codes);
+  uint64_t chunk = (n + FV_HASH_CHUNKS - 1) / FV_HASH_CHUNKS;
+  const uint64_t least = FV_HASH_CHUNK_MIN_BYTES / (out_row ? out_row : 1) + 1;
+  chunk = chunk < least ? least : chunk;
+  chunk = chunk < FV_HASH_CHUNK ? chunk : FV_HASH_CHUNK;
+  chunk = chunk < n ? chunk : n;
+  const int lanes = n > chunk ? FV_HASH_LANES : 1;
+  const bool stage_idx = fv_is_pageable(idx);
   // staging pays off for outputs of some size that the device cannot reach by DMA
   const bool stage_bits = out_bits && lanes > 1 && fv_is_pageable(out_bits);
   const bool stage_codes = out_codes && lanes > 1 && fv_is_pageable(out_codes);
@@ -404,6 +379,7 @@ static int fv_hash_host(fv_hasher *h, const int32_t *idx, uint64_t n, uint32_t w
     }
     if (!ln.done) FV_HIP(hipEventCreateWithFlags(&ln.done, hipEventDisableTiming));
     FV_TRY(fv_hash_reserve(&ln.idx, &ln.idx_cap, chunk * w * sizeof(int32_t)));
+    if (stage_idx) FV_TRY(fv_hash_reserve_pinned(&ln.stage_idx, &ln.stage_idx_cap, chunk * w * sizeof(int32_t)));
     if (out_bits) FV_TRY(fv_hash_reserve(&ln.bits, &ln.bits_cap, chunk * bits_row));
     if (out_codes) FV_TRY(fv_hash_reserve(&ln.codes, &ln.codes_cap, chunk * codes_row));
     if (stage_bits) FV_TRY(fv_hash_reserve_pinned(&ln.stage_bits, &ln.stage_bits_cap, chunk * bits_row));
@@ -428,7 +404,14 @@ static int fv_hash_host(fv_hasher *h, const int32_t *idx, uint64_t n, uint32_t w
     fv_hash_lane &ln = h->lane[c % lanes];
     const uint64_t first = c * chunk, m = n - first < chunk ? n - first : chunk;
     if (ring && c >= (uint64_t)lanes && last_item[c - lanes] != 0xffffffffu) ring->wait(last_item[c - lanes]);
-    hipError_t e = hipMemcpyAsync(ln.idx, idx + first * w, m * w * sizeof(int32_t), hipMemcpyHostToDevice, ln.stream);
+    const int32_t *from = idx + first * w;
+    hipError_t e = hipSuccess;
+    if (stage_idx) {
+      // the lane's chunk before this one has been copied in
+      if (c >= (uint64_t)lanes) e = hipEventSynchronize(ln.done);
+      if (e == hipSuccess) from = (const int32_t *)memcpy(ln.stage_idx, from, m * w * sizeof(int32_t));
+    }
+    if (e == hipSuccess) e = hipMemcpyAsync(ln.idx, from, m * w * sizeof(int32_t), hipMemcpyHostToDevice, ln.stream);
     if (e != hipSuccess) {
       rc = fv_fail(FV_ERR_HIP, "hash upload failed: %s", hipGetErrorString(e));
       break;
@@ -445,10 +428,10 @@ static int fv_hash_host(fv_hasher *h, const int32_t *idx, uint64_t n, uint32_t w
       e = hipMemcpyAsync(dst, ln.codes, m * codes_row, hipMemcpyDeviceToHost, ln.stream);
       if (e != hipSuccess) rc = fv_fail(FV_ERR_HIP, "download failed: %s", hipGetErrorString(e));
     }
-    if (rc == FV_OK && ring) {
+    if (rc == FV_OK) {
       e = hipEventRecord(ln.done, ln.stream);
       if (e != hipSuccess) rc = fv_fail(FV_ERR_HIP, "event record failed: %s", hipGetErrorString(e));
-      if (rc == FV_OK && c >= 1) rc = hand_over(c - 1);
+      if (rc == FV_OK && ring && c >= 1) rc = hand_over(c - 1);
     }
   }
   if (rc == FV_OK && ring) rc = hand_over(n_chunks - 1);

@@ -41,12 +41,7 @@ void fv_clear_error();
 // Wt[i * ldk .. i * ldk + K), ldk = K rounded up to a multiple of 4 floats (fv_ldk) so every
 // row starts 16-byte aligned; the pad is kept at zero. fv_layout.h sizes the allocation.
 
-// K x N row-major (staging, device) <-> token-major N x ldk (device). Asynchronous.
-int fv_launch_to_token_major(const float *W_rowmajor_dev, float *Wt_dev, uint32_t K, uint64_t N,
-                             uint32_t ldk, hipStream_t stream);
-int fv_launch_to_row_major(const float *Wt_dev, float *W_rowmajor_dev, uint32_t K, uint64_t N,
-                           uint32_t ldk, hipStream_t stream);
-// Upload / download a K x N host matrix through a temporary device staging buffer.
+// Upload / download a K x N row-major host matrix (token-major on the device). The stream has drained on return.
 int fv_upload_weights(const float *W_host, float *Wt_dev, uint32_t K, uint64_t N, uint32_t ldk,
                       hipStream_t stream);
 int fv_download_weights(const float *Wt_dev, float *W_host, uint32_t K, uint64_t N, uint32_t ldk,

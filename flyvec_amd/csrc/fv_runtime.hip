@@ -3,9 +3,11 @@
 // the token-major matrix the kernels read.
 #include <string.h>
 
+#include <condition_variable>
+#include <mutex>
 #include <string>
 
-#include "fv_internal.h"
+#include "fv_host_copy.h"
 
 static thread_local std::string g_last_error;
 
@@ -108,9 +110,11 @@ extern "C" int fv_dev_download(void *dst_host, const void *src_dev, size_t bytes
 
 #define FV_TT 64
 
-__global__ __launch_bounds__(256) void fv_to_token_major_kernel(const float *__restrict__ W,
+// W: K x N of a row-major matrix of `pitch` columns; Wt: where its first column's first row goes. Of Wt's rows the
+// elements from K up to `last` are written as zeros.
+__global__ __launch_bounds__(256) void fv_to_token_major_kernel(const float *__restrict__ W, uint64_t pitch,
                                                                 float *__restrict__ Wt, uint32_t K,
-                                                                uint64_t N, uint32_t ldk) {
+                                                                uint64_t N, uint32_t ldk, uint32_t last) {
   __shared__ float tile[FV_TT][FV_TT + 1];
   const uint64_t i0 = (uint64_t)blockIdx.x * FV_TT;  // token (column of W)
   const uint32_t h0 = blockIdx.y * FV_TT;            // neuron (row of W)
@@ -118,18 +122,18 @@ __global__ __launch_bounds__(256) void fv_to_token_major_kernel(const float *__r
   for (int r = ty; r < FV_TT; r += 4) {
     uint32_t h = h0 + r;
     uint64_t i = i0 + tx;
-    tile[r][tx] = (h < K && i < N) ? W[(uint64_t)h * N + i] : 0.0f;
+    tile[r][tx] = (h < K && i < N) ? W[(uint64_t)h * pitch + i] : 0.0f;
   }
   __syncthreads();
   for (int r = ty; r < FV_TT; r += 4) {
     uint64_t i = i0 + r;
     uint32_t h = h0 + tx;
-    if (i < N && h < ldk) Wt[i * ldk + h] = tile[tx][r];  // pad columns (h >= K) receive 0
+    if (i < N && h < last) Wt[i * ldk + h] = tile[tx][r];
   }
 }
 
 __global__ __launch_bounds__(256) void fv_to_row_major_kernel(const float *__restrict__ Wt,
-                                                              float *__restrict__ W, uint32_t K,
+                                                              float *__restrict__ W, uint64_t pitch, uint32_t K,
                                                               uint64_t N, uint32_t ldk) {
   __shared__ float tile[FV_TT][FV_TT + 1];
   const uint64_t i0 = (uint64_t)blockIdx.x * FV_TT;
@@ -144,41 +148,27 @@ __global__ __launch_bounds__(256) void fv_to_row_major_kernel(const float *__res
   for (int r = ty; r < FV_TT; r += 4) {
     uint32_t h = h0 + r;
     uint64_t i = i0 + tx;
-    if (h < K && i < N) W[(uint64_t)h * N + i] = tile[tx][r];
+    if (h < K && i < N) W[(uint64_t)h * pitch + i] = tile[tx][r];
   }
 }
 
-int fv_launch_to_token_major(const float *W, float *Wt, uint32_t K, uint64_t N, uint32_t ldk,
-                             hipStream_t stream) {
-  dim3 grid((unsigned)((N + FV_TT - 1) / FV_TT), (ldk + FV_TT - 1) / FV_TT);
-  hipLaunchKernelGGL(fv_to_token_major_kernel, grid, dim3(256), 0, stream, W, Wt, K, N, ldk);
+static int fv_launch_to_token_major(const float *W, uint64_t pitch, float *Wt, uint32_t K, uint64_t N, uint32_t ldk,
+                                    uint32_t last, hipStream_t stream) {
+  dim3 grid((unsigned)((N + FV_TT - 1) / FV_TT), (last + FV_TT - 1) / FV_TT);
+  hipLaunchKernelGGL(fv_to_token_major_kernel, grid, dim3(256), 0, stream, W, pitch, Wt, K, N, ldk, last);
   FV_HIP(hipGetLastError());
   return FV_OK;
 }
 
-int fv_launch_to_row_major(const float *Wt, float *W, uint32_t K, uint64_t N, uint32_t ldk,
-                           hipStream_t stream) {
+static int fv_launch_to_row_major(const float *Wt, float *W, uint64_t pitch, uint32_t K, uint64_t N, uint32_t ldk,
+                                  hipStream_t stream) {
   dim3 grid((unsigned)((N + FV_TT - 1) / FV_TT), (K + FV_TT - 1) / FV_TT);
-  hipLaunchKernelGGL(fv_to_row_major_kernel, grid, dim3(256), 0, stream, Wt, W, K, N, ldk);
+  hipLaunchKernelGGL(fv_to_row_major_kernel, grid, dim3(256), 0, stream, Wt, W, pitch, K, N, ldk);
   FV_HIP(hipGetLastError());
   return FV_OK;
 }
 
-int fv_upload_weights(const float *W_host, float *Wt_dev, uint32_t K, uint64_t N, uint32_t ldk,
-                      hipStream_t stream) {
-  float *stage = nullptr;
-  size_t bytes = (size_t)K * N * sizeof(float);
-  FV_HIP(hipMalloc((void **)&stage, bytes));
-  hipError_t e = hipMemcpyAsync(stage, W_host, bytes, hipMemcpyHostToDevice, stream);
-  int rc = FV_OK;
-  if (e != hipSuccess) rc = fv_fail(FV_ERR_HIP, "weight upload failed: %s", hipGetErrorString(e));
-  if (rc == FV_OK) rc = fv_launch_to_token_major(stage, Wt_dev, K, N, ldk, stream);
-  e = hipStreamSynchronize(stream);
-  if (rc == FV_OK && e != hipSuccess)
-    rc = fv_fail(FV_ERR_HIP, "weight upload failed: %s", hipGetErrorString(e));
-  (void)hipFree(stage);
-  return rc;
-}
+// ---- transfers to and from host memory -----------------------------------------------------------------------
 
 // The device's address of `bytes` of page-locked host memory at p (hipHostMalloc), or null where the range is anything
 // else: pageable, or not inside one allocation.
@@ -195,29 +185,200 @@ void *fv_device_view(const void *p, size_t bytes) {
   return before <= size && bytes <= size - before ? at.devicePointer : nullptr;
 }
 
-// To page-locked memory the layout change writes over the link itself: no staging matrix on the device (its allocation
-// and its release, which waits for the device, cost more than the copy of a small matrix), no second pass.
+bool fv_is_pageable(const void *p) {
+  hipPointerAttribute_t at;
+  if (hipPointerGetAttributes(&at, p) != hipSuccess) {
+    (void)hipGetLastError();
+    return true;
+  }
+  return at.type == hipMemoryTypeUnregistered;
+}
+
+// The process's page-locked slots: made when first needed, up to FV_STAGE_SLOTS_MAX, kept for the transfers that follow
+// (page-locking 4 MB takes as long as moving 20) until fv_host_staging_release.
+static std::mutex fv_stage_mutex;
+static std::condition_variable fv_stage_returned;
+static std::vector<char *> fv_stage_idle;
+static unsigned fv_stage_made = 0;
+
+fv_stage_lease::fv_stage_lease(unsigned want) : rc(FV_OK) {
+  {
+    std::unique_lock<std::mutex> lock(fv_stage_mutex);
+    while (slots.size() < want) {
+      if (!fv_stage_idle.empty()) {
+        slots.push_back(fv_stage_idle.back());
+        fv_stage_idle.pop_back();
+      } else if (fv_stage_made < FV_STAGE_SLOTS_MAX) {
+        char *p = nullptr;
+        const hipError_t e = hipHostMalloc((void **)&p, FV_STAGE_SLOT_BYTES, hipHostMallocPortable | hipHostMallocCoherent);
+        if (e != hipSuccess) {
+          (void)hipGetLastError();
+          if (slots.empty()) rc = fv_fail(FV_ERR_HIP, "page-locked staging memory: %s", hipGetErrorString(e));
+          break;  // with fewer than wanted
+        }
+        fv_stage_made++;
+        slots.push_back(p);
+      } else if (slots.empty()) {
+        fv_stage_returned.wait(lock);
+      } else {
+        break;
+      }
+    }
+  }
+  for (size_t i = 0; i < slots.size() && rc == FV_OK; ++i) {
+    hipEvent_t ev = nullptr;
+    const hipError_t e = hipEventCreateWithFlags(&ev, hipEventDisableTiming);
+    if (e != hipSuccess)
+      rc = fv_fail(FV_ERR_HIP, "staging event: %s", hipGetErrorString(e));
+    else
+      events.push_back(ev);
+  }
+}
+
+fv_stage_lease::~fv_stage_lease() {
+  for (hipEvent_t ev : events) (void)hipEventDestroy(ev);
+  {
+    std::lock_guard<std::mutex> lock(fv_stage_mutex);
+    for (char *p : slots) fv_stage_idle.push_back(p);
+  }
+  fv_stage_returned.notify_all();
+}
+
+extern "C" int fv_host_staging_release(void) {
+  std::lock_guard<std::mutex> lock(fv_stage_mutex);
+  for (char *p : fv_stage_idle) (void)hipHostFree(p);
+  fv_stage_made -= (unsigned)fv_stage_idle.size();
+  fv_stage_idle.clear();
+  return FV_OK;
+}
+
+static bool fv_stages(const void *host, size_t bytes) {
+  // both ends: the range may begin or end inside page-locked memory of the caller's
+  return bytes >= FV_STAGE_MIN_BYTES && fv_is_pageable(host) && fv_is_pageable((const char *)host + bytes - 1);
+}
+
+int fv_copy_up(void *dst_dev, const void *src_host, size_t bytes, hipStream_t stream) {
+  if (bytes == 0) return FV_OK;
+  if (!fv_stages(src_host, bytes)) {
+    FV_HIP(hipMemcpyAsync(dst_dev, src_host, bytes, hipMemcpyHostToDevice, stream));
+    FV_HIP(hipStreamSynchronize(stream));
+    return FV_OK;
+  }
+  const size_t slot = bytes >= 4 * FV_STAGE_SLOT_BYTES ? FV_STAGE_SLOT_BYTES : FV_STAGE_SLOT_BYTES / 8;
+  const auto length = [&](uint64_t t) { return bytes - t * slot < slot ? bytes - t * slot : slot; };
+  return fv_pipe_up(
+      (bytes + slot - 1) / slot, stream,
+      [&](uint64_t t, char *p) {
+        return fv_copy_ring::item{(const char *)src_host + t * slot, p, length(t), 0, 0, 1};
+      },
+      [&](uint64_t t, char *p) -> int {
+        FV_HIP(hipMemcpyAsync((char *)dst_dev + t * slot, p, length(t), hipMemcpyHostToDevice, stream));
+        return FV_OK;
+      });
+}
+
+int fv_copy_down(void *dst_host, const void *src_dev, size_t bytes, hipStream_t stream) {
+  if (bytes == 0) return FV_OK;
+  if (!fv_stages(dst_host, bytes)) {
+    FV_HIP(hipMemcpyAsync(dst_host, src_dev, bytes, hipMemcpyDeviceToHost, stream));
+    FV_HIP(hipStreamSynchronize(stream));
+    return FV_OK;
+  }
+  const size_t slot = bytes >= 4 * FV_STAGE_SLOT_BYTES ? FV_STAGE_SLOT_BYTES : FV_STAGE_SLOT_BYTES / 8;
+  const auto length = [&](uint64_t t) { return bytes - t * slot < slot ? bytes - t * slot : slot; };
+  return fv_pipe_down(
+      (bytes + slot - 1) / slot, stream,
+      [&](uint64_t t, char *p) -> int {
+        FV_HIP(hipMemcpyAsync(p, (const char *)src_dev + t * slot, length(t), hipMemcpyDeviceToHost, stream));
+        return FV_OK;
+      },
+      [&](uint64_t t, char *p) { return fv_copy_ring::item{p, (char *)dst_host + t * slot, length(t), 0, 0, 1}; });
+}
+
+// A K x N host matrix goes through the slots in tiles of FV_TT rows by as many columns as a slot holds; the layout
+// change reads and writes the slots over the link. Tile t: rows from h, columns from i.
+struct fv_weight_tiles {
+  uint32_t K;
+  uint64_t N, columns, across, n;
+  fv_weight_tiles(uint32_t K_, uint64_t N_) : K(K_), N(N_) {
+    columns = FV_STAGE_SLOT_BYTES / (FV_TT * sizeof(float));
+    across = (N + columns - 1) / columns;
+    n = across * ((K + FV_TT - 1) / FV_TT);
+  }
+  uint32_t h(uint64_t t) const { return (uint32_t)(t / across) * FV_TT; }
+  uint64_t i(uint64_t t) const { return t % across * columns; }
+  uint32_t rows(uint64_t t) const { return K - h(t) < FV_TT ? K - h(t) : FV_TT; }
+  uint64_t cols(uint64_t t) const { return N - i(t) < columns ? N - i(t) : columns; }
+  uint64_t pitch(uint64_t t) const { return (cols(t) + FV_TT - 1) / FV_TT * FV_TT; }  // of the slot's rows
+};
+
+// Page-locked matrices are read and written in place by the layout change, and pageable ones through page-locked slots:
+// there is no staging matrix on the device, whose allocation and release (which waits for the device) cost more than
+// the copy of a small matrix, and no second pass over it. Memory of any other kind takes the runtime's copies.
+int fv_upload_weights(const float *W_host, float *Wt_dev, uint32_t K, uint64_t N, uint32_t ldk,
+                      hipStream_t stream) {
+  const size_t bytes = (size_t)K * N * sizeof(float);
+  int rc = FV_OK;
+  if (const float *view = (const float *)fv_device_view(W_host, bytes)) {
+    rc = fv_launch_to_token_major(view, N, Wt_dev, K, N, ldk, ldk, stream);
+  } else if (fv_is_pageable(W_host) && fv_is_pageable((const char *)W_host + bytes - 1)) {
+    const fv_weight_tiles tiles(K, N);
+    return fv_pipe_up(
+        tiles.n, stream,
+        [&](uint64_t t, char *p) {
+          return fv_copy_ring::item{(const char *)(W_host + tiles.h(t) * N + tiles.i(t)), p, tiles.cols(t) * sizeof(float),
+                                    N * sizeof(float), tiles.pitch(t) * sizeof(float), tiles.rows(t)};
+        },
+        [&](uint64_t t, char *p) {
+          const uint32_t h = tiles.h(t), rows = tiles.rows(t);
+          return fv_launch_to_token_major((const float *)p, tiles.pitch(t), Wt_dev + tiles.i(t) * ldk + h, rows,
+                                          tiles.cols(t), ldk, h + rows == K ? ldk - h : rows, stream);
+        });
+  } else {
+    float *stage = nullptr;
+    FV_HIP(hipMalloc((void **)&stage, bytes));
+    const hipError_t e = hipMemcpyAsync(stage, W_host, bytes, hipMemcpyHostToDevice, stream);
+    if (e != hipSuccess) rc = fv_fail(FV_ERR_HIP, "weight upload failed: %s", hipGetErrorString(e));
+    if (rc == FV_OK) rc = fv_launch_to_token_major(stage, N, Wt_dev, K, N, ldk, ldk, stream);
+    (void)hipStreamSynchronize(stream);
+    (void)hipFree(stage);
+  }
+  const hipError_t e = hipStreamSynchronize(stream);
+  if (rc == FV_OK && e != hipSuccess) rc = fv_fail(FV_ERR_HIP, "weight upload failed: %s", hipGetErrorString(e));
+  return rc;
+}
+
 int fv_download_weights(const float *Wt_dev, float *W_host, uint32_t K, uint64_t N, uint32_t ldk,
                         hipStream_t stream) {
-  size_t bytes = (size_t)K * N * sizeof(float);
+  const size_t bytes = (size_t)K * N * sizeof(float);
+  int rc = FV_OK;
   if (float *view = (float *)fv_device_view(W_host, bytes)) {
-    int rc = fv_launch_to_row_major(Wt_dev, view, K, N, ldk, stream);
-    const hipError_t e = hipStreamSynchronize(stream);
-    if (rc == FV_OK && e != hipSuccess) rc = fv_fail(FV_ERR_HIP, "weight download failed: %s", hipGetErrorString(e));
-    return rc;
+    rc = fv_launch_to_row_major(Wt_dev, view, N, K, N, ldk, stream);
+  } else if (fv_is_pageable(W_host) && fv_is_pageable((const char *)W_host + bytes - 1)) {
+    const fv_weight_tiles tiles(K, N);
+    return fv_pipe_down(
+        tiles.n, stream,
+        [&](uint64_t t, char *p) {
+          return fv_launch_to_row_major(Wt_dev + tiles.i(t) * ldk + tiles.h(t), (float *)p, tiles.pitch(t), tiles.rows(t),
+                                        tiles.cols(t), ldk, stream);
+        },
+        [&](uint64_t t, char *p) {
+          return fv_copy_ring::item{p, (char *)(W_host + tiles.h(t) * N + tiles.i(t)), tiles.cols(t) * sizeof(float),
+                                    tiles.pitch(t) * sizeof(float), N * sizeof(float), tiles.rows(t)};
+        });
+  } else {
+    float *stage = nullptr;
+    FV_HIP(hipMalloc((void **)&stage, bytes));
+    rc = fv_launch_to_row_major(Wt_dev, stage, N, K, N, ldk, stream);
+    if (rc == FV_OK) {
+      const hipError_t e = hipMemcpyAsync(W_host, stage, bytes, hipMemcpyDeviceToHost, stream);
+      if (e != hipSuccess) rc = fv_fail(FV_ERR_HIP, "weight download failed: %s", hipGetErrorString(e));
+    }
+    (void)hipStreamSynchronize(stream);
+    (void)hipFree(stage);
   }
-  float *stage = nullptr;
-  FV_HIP(hipMalloc((void **)&stage, bytes));
-  int rc = fv_launch_to_row_major(Wt_dev, stage, K, N, ldk, stream);
-  hipError_t e = hipSuccess;
-  if (rc == FV_OK) {
-    e = hipMemcpyAsync(W_host, stage, bytes, hipMemcpyDeviceToHost, stream);
-    if (e != hipSuccess) rc = fv_fail(FV_ERR_HIP, "weight download failed: %s", hipGetErrorString(e));
-  }
-  e = hipStreamSynchronize(stream);
-  if (rc == FV_OK && e != hipSuccess)
-    rc = fv_fail(FV_ERR_HIP, "weight download failed: %s", hipGetErrorString(e));
-  (void)hipFree(stage);
+  const hipError_t e = hipStreamSynchronize(stream);
+  if (rc == FV_OK && e != hipSuccess) rc = fv_fail(FV_ERR_HIP, "weight download failed: %s", hipGetErrorString(e));
   return rc;
 }
 

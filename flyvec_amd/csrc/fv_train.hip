@@ -37,6 +37,7 @@
 // Every one of the n additions of 1/f onto ds[h][i] adds the same value, so the reference's
 // result for that element depends only on n; replaying n sequential fp32 adds reproduces it
 // exactly whatever order its atomics ran in.
+#include "fv_host_copy.h"
 #include "fv_train_state.h"
 #include "fv_train_top2.h"
 #include "fv_train_gather.h"
@@ -129,9 +130,44 @@ static void fv_trainer_free_corpus(fv_trainer *t) {
   t->corpus = nullptr;
   t->starts = t->perm = t->perm_alt = t->pstart = nullptr;
   t->invf = nullptr;
+  t->corpus_cap = t->windows_cap = 0;
+}
+
+// The trainer has no corpus from here on; the buffers of the last one wait for the next.
+static void fv_trainer_forget_corpus(fv_trainer *t) {
   t->n_tokens = t->n_windows = 0;
   t->have_corpus = false;
   t->ahead_valid = false;
+}
+
+// Room for a corpus, and for its window tables. Buffers of an earlier corpus are used again (releasing and allocating
+// them took 1.3 of 3.3 ms at 4 M tokens: a release waits for the device and unmaps), unless they are more than a quarter
+// larger than needed.
+static bool fv_fits_kept(uint64_t need, uint64_t cap) { return need <= cap && cap - need <= need / 4; }
+
+static int fv_trainer_reserve_corpus(fv_trainer *t, uint64_t n_tokens) {
+  if (!fv_fits_kept(n_tokens, t->corpus_cap)) {
+    fv_trainer_free_corpus(t);  // the window tables too: the new corpus finds the memory it would find in a new trainer
+    FV_HIP(hipMalloc((void **)&t->corpus, n_tokens * sizeof(int32_t)));
+    t->corpus_cap = n_tokens;
+  }
+  if (!t->invf) FV_HIP(hipMalloc((void **)&t->invf, t->V * sizeof(float)));
+  return FV_OK;
+}
+
+static int fv_trainer_reserve_windows(fv_trainer *t, uint64_t n_windows) {
+  if (fv_fits_kept(n_windows, t->windows_cap)) return FV_OK;
+  (void)hipFree(t->starts);
+  (void)hipFree(t->perm);
+  (void)hipFree(t->perm_alt);
+  (void)hipFree(t->pstart);
+  t->starts = t->perm = t->perm_alt = t->pstart = nullptr;
+  t->windows_cap = 0;
+  FV_HIP(hipMalloc((void **)&t->starts, n_windows * sizeof(uint64_t)));
+  FV_HIP(hipMalloc((void **)&t->perm, n_windows * sizeof(uint64_t)));
+  FV_HIP(hipMalloc((void **)&t->pstart, n_windows * sizeof(uint64_t)));
+  t->windows_cap = n_windows;
+  return FV_OK;
 }
 
 // Trainers of this process with steps enqueued that nobody has waited for yet. The single dense launch, where it has
@@ -445,18 +481,17 @@ extern "C" int fv_trainer_set_corpus(fv_trainer *t, const int32_t *tokens, uint6
   FV_REQUIRE(tokens && n_tokens > 0, FV_ERR_INVALID, "empty corpus");
   FV_REQUIRE(offsets && n_offsets >= 1, FV_ERR_INVALID, "empty offsets");
   FV_HIP(hipStreamSynchronize(t->stream));
-  fv_trainer_free_corpus(t);
+  fv_trainer_forget_corpus(t);
   const uint64_t n_chunks = n_offsets - 1;
   uint64_t *off_dev = nullptr;
-  int rc = FV_OK;
-  hipError_t e = hipMalloc((void **)&t->corpus, n_tokens * sizeof(int32_t));
-  if (e == hipSuccess) e = hipMalloc((void **)&t->invf, t->V * sizeof(float));
-  if (e == hipSuccess) e = hipMalloc((void **)&off_dev, n_offsets * sizeof(uint64_t));
-  if (e == hipSuccess)
-    e = hipMemcpyAsync(t->corpus, tokens, n_tokens * sizeof(int32_t), hipMemcpyHostToDevice, t->stream);
-  if (e == hipSuccess)
-    e = hipMemcpyAsync(off_dev, offsets, n_offsets * sizeof(uint64_t), hipMemcpyHostToDevice, t->stream);
-  if (e != hipSuccess) rc = fv_fail(FV_ERR_HIP, "corpus upload failed: %s", hipGetErrorString(e));
+  int rc = fv_trainer_reserve_corpus(t, n_tokens);
+  hipError_t e = hipSuccess;
+  if (rc == FV_OK) {
+    e = hipMalloc((void **)&off_dev, n_offsets * sizeof(uint64_t));
+    if (e != hipSuccess) rc = fv_fail(FV_ERR_HIP, "corpus allocation failed: %s", hipGetErrorString(e));
+  }
+  if (rc == FV_OK) rc = fv_copy_up(t->corpus, tokens, n_tokens * sizeof(int32_t), t->stream);
+  if (rc == FV_OK) rc = fv_copy_up(off_dev, offsets, n_offsets * sizeof(uint64_t), t->stream);
 
   int32_t lo = 0, hi = 0;
   if (rc == FV_OK) rc = fv_dev_inverse_frequency(t->corpus, n_tokens, t->V, t->invf, &lo, &hi, t->stream);
@@ -466,10 +501,7 @@ extern "C" int fv_trainer_set_corpus(fv_trainer *t, const int32_t *tokens, uint6
   uint64_t nwin = 0;
   if (rc == FV_OK) rc = fv_dev_count_windows(off_dev, n_chunks, t->w, &nwin, t->stream);
   if (rc == FV_OK && nwin) {
-    e = hipMalloc((void **)&t->starts, nwin * sizeof(uint64_t));
-    if (e == hipSuccess) e = hipMalloc((void **)&t->perm, nwin * sizeof(uint64_t));
-    if (e == hipSuccess) e = hipMalloc((void **)&t->pstart, nwin * sizeof(uint64_t));
-    if (e != hipSuccess) rc = fv_fail(FV_ERR_HIP, "window table allocation failed: %s", hipGetErrorString(e));
+    rc = fv_trainer_reserve_windows(t, nwin);
     if (rc == FV_OK) {
       // Starts are sums of chunk lengths: with non-decreasing offsets that span no more than the
       // corpus, every window lies inside it (the kernels never read past n_tokens).
@@ -514,30 +546,22 @@ extern "C" int fv_trainer_set_corpus_starts(fv_trainer *t, const int32_t *tokens
                "window %llu starts at token %llu: it does not fit the corpus of %llu", (unsigned long long)i,
                (unsigned long long)starts[i], (unsigned long long)n_tokens);
   FV_HIP(hipStreamSynchronize(t->stream));
-  fv_trainer_free_corpus(t);
-  int rc = FV_OK;
-  hipError_t e = hipMalloc((void **)&t->corpus, n_tokens * sizeof(int32_t));
-  if (e == hipSuccess) e = hipMalloc((void **)&t->invf, t->V * sizeof(float));
-  if (e == hipSuccess)
-    e = hipMemcpyAsync(t->corpus, tokens, n_tokens * sizeof(int32_t), hipMemcpyHostToDevice, t->stream);
-  if (e != hipSuccess) rc = fv_fail(FV_ERR_HIP, "corpus upload failed: %s", hipGetErrorString(e));
+  fv_trainer_forget_corpus(t);
+  int rc = fv_trainer_reserve_corpus(t, n_tokens);
+  if (rc == FV_OK) rc = fv_copy_up(t->corpus, tokens, n_tokens * sizeof(int32_t), t->stream);
   int32_t lo = 0, hi = 0;
   if (rc == FV_OK) rc = fv_dev_inverse_frequency(t->corpus, n_tokens, t->V, t->invf, &lo, &hi, t->stream);
   if (rc == FV_OK && (lo < -1 || (hi >= 0 && (uint64_t)hi >= t->V)))
     rc = fv_fail(FV_ERR_DATA, "token ids span [%d, %d]; allowed are -1 (masked) and 0..%llu", lo, hi,
                  (unsigned long long)(t->V - 1));
   if (rc == FV_OK && n_windows) {
-    e = hipMalloc((void **)&t->starts, n_windows * sizeof(uint64_t));
-    if (e == hipSuccess) e = hipMalloc((void **)&t->perm, n_windows * sizeof(uint64_t));
-    if (e == hipSuccess) e = hipMalloc((void **)&t->pstart, n_windows * sizeof(uint64_t));
-    if (e == hipSuccess)
-      e = hipMemcpyAsync(t->starts, starts, n_windows * sizeof(uint64_t), hipMemcpyHostToDevice, t->stream);
-    if (e != hipSuccess) rc = fv_fail(FV_ERR_HIP, "window table upload failed: %s", hipGetErrorString(e));
+    rc = fv_trainer_reserve_windows(t, n_windows);
+    if (rc == FV_OK) rc = fv_copy_up(t->starts, starts, n_windows * sizeof(uint64_t), t->stream);
     if (rc == FV_OK) {
       hipLaunchKernelGGL(fv_identity_kernel, dim3(fv_perm_blocks(n_windows)), dim3(256), 0, t->stream, t->perm, n_windows);
       hipLaunchKernelGGL(fv_order_starts_kernel, dim3(fv_perm_blocks(n_windows)), dim3(256), 0, t->stream, t->perm,
                          t->starts, t->pstart, n_windows);
-      e = hipStreamSynchronize(t->stream);
+      const hipError_t e = hipStreamSynchronize(t->stream);
       if (e != hipSuccess) rc = fv_fail(FV_ERR_HIP, "permutation fill failed: %s", hipGetErrorString(e));
     }
   }
@@ -565,8 +589,7 @@ extern "C" int fv_trainer_get_window_starts(fv_trainer *t, uint64_t *out_starts,
              (unsigned long long)capacity, (unsigned long long)t->n_windows);
   if (t->n_windows) {
     FV_REQUIRE(out_starts, FV_ERR_INVALID, "null output");
-    FV_HIP(hipStreamSynchronize(t->stream));
-    FV_HIP(hipMemcpy(out_starts, t->starts, t->n_windows * sizeof(uint64_t), hipMemcpyDeviceToHost));
+    FV_TRY(fv_copy_down(out_starts, t->starts, t->n_windows * sizeof(uint64_t), t->stream));
   }
   return FV_OK;
 }
@@ -599,7 +622,7 @@ extern "C" int fv_trainer_shuffle(fv_trainer *t, uint64_t seed) {
   FV_REQUIRE(t->have_corpus, FV_ERR_STATE, "no corpus set");
   const uint64_t n = t->n_windows;
   if (n == 0) return FV_OK;
-  if (!t->perm_alt) FV_HIP(hipMalloc((void **)&t->perm_alt, n * sizeof(uint64_t)));
+  if (!t->perm_alt) FV_HIP(hipMalloc((void **)&t->perm_alt, t->windows_cap * sizeof(uint64_t)));
   // every call draws a different bijection, also under one seed
   const fv_feistel f = fv_feistel_make(n, seed ^ (0xD1B54A32D192ED03ull * (t->shuffle_calls + 1)));
   hipLaunchKernelGGL(fv_shuffle_kernel, dim3(fv_perm_blocks(n)), dim3(256), 0, t->stream, t->perm, t->perm_alt, n, f);
@@ -623,8 +646,7 @@ extern "C" int fv_trainer_set_permutation(fv_trainer *t, const uint64_t *perm, u
   for (uint64_t i = 0; i < n; ++i)
     FV_REQUIRE(perm[i] < n, FV_ERR_DATA, "permutation entry %llu = %llu is not a window index",
                (unsigned long long)i, (unsigned long long)perm[i]);
-  FV_HIP(hipStreamSynchronize(t->stream));
-  FV_HIP(hipMemcpy(t->perm, perm, n * sizeof(uint64_t), hipMemcpyHostToDevice));
+  FV_TRY(fv_copy_up(t->perm, perm, n * sizeof(uint64_t), t->stream));
   t->ahead_valid = false;  // sampled in the old order
   hipLaunchKernelGGL(fv_order_starts_kernel, dim3(fv_perm_blocks(n)), dim3(256), 0, t->stream, t->perm, t->starts,
                      t->pstart, n);
@@ -638,8 +660,7 @@ extern "C" int fv_trainer_get_permutation(fv_trainer *t, uint64_t *out_perm, uin
   FV_REQUIRE(capacity >= t->n_windows, FV_ERR_INVALID, "capacity too small");
   if (t->n_windows) {
     FV_REQUIRE(out_perm, FV_ERR_INVALID, "null output");
-    FV_HIP(hipStreamSynchronize(t->stream));
-    FV_HIP(hipMemcpy(out_perm, t->perm, t->n_windows * sizeof(uint64_t), hipMemcpyDeviceToHost));
+    FV_TRY(fv_copy_down(out_perm, t->perm, t->n_windows * sizeof(uint64_t), t->stream));
   }
   return FV_OK;
 }

@@ -45,6 +45,7 @@ struct fv_trainer {
   uint64_t *pstart;    // starts[perm[i]]: where the i-th window of the current order begins
   uint64_t *perm_alt;  // second permutation buffer, allocated by the first shuffle
   uint64_t n_windows;
+  uint64_t corpus_cap, windows_cap;  // tokens / windows the buffers above have room for
   float *invf;
   int32_t *idx;     // B rows of idx_stride column indices of the current minibatch (w used, the rest -1)
   uint32_t idx_stride;  // w rounded up to 4: rows are read 16 bytes at a time

@@ -49,6 +49,11 @@ int fv_device_memory(uint64_t *out_free_bytes, uint64_t *out_total_bytes);
 int fv_host_alloc_pinned(size_t bytes, void **out_ptr);
 int fv_host_free_pinned(void *ptr);
 
+/* Transfers to and from ordinary host memory go through up to 32 MB of page-locked memory that the library keeps for
+ * the transfers that follow. This returns what no transfer is using to the system (the next one takes it anew). No
+ * counterpart in the reference. */
+int fv_host_staging_release(void);
+
 /* flyvec/src/cuda_helpers.cu:8 do_gpu_cudaMallocManaged -- the reference keeps every
  * buffer in managed memory; here device buffers are explicit.  Used by callers that
  * keep hash inputs / outputs resident in HBM (the *_dev entry points). */

@@ -1,0 +1,144 @@
+"""Transfers between the device and host memory of either kind: large pageable ones go through page-locked slots in
+pieces, small hash batches through one page-locked buffer, batches of codes in chunks. Whatever the route, the bytes
+are the same."""
+import threading
+
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+SLOT_COLUMNS = 16384  # columns of a 64-row tile that fills a slot of 4 MB
+
+
+@pytest.mark.parametrize("K,N", [(1, 2), (64, 2 * SLOT_COLUMNS), (65, 2 * SLOT_COLUMNS + 2), (63, SLOT_COLUMNS - 2),
+                                 (130, 5 * SLOT_COLUMNS + 6), (400, 2)])
+def test_matrices_through_the_slots(gpu, K, N):
+    """Upload and download at tile edges (rows beside 64, columns beside a slot's), pageable and page-locked on either
+    side; the pad columns of the device's rows are zero again after a larger matrix's upload has been read."""
+    from flyvec_amd import Hasher, Trainer, _lib
+    W = np.random.default_rng(K).standard_normal((K, N), dtype=np.float32)
+    locked = _lib.pinned_empty(W.shape, np.float32)
+    locked[...] = W
+    for source in (W, locked):
+        t = Trainer(N // 2, K, 3, 16)
+        t.set_weights(source)
+        assert np.array_equal(t.get_weights().view(np.uint32), W.view(np.uint32))
+        out = _lib.pinned_empty(W.shape, np.float32)
+        assert np.array_equal(t.get_weights(out).view(np.uint32), W.view(np.uint32))
+        t.close()
+    if K > 1:
+        h = Hasher(W)
+        assert np.array_equal(h.weights(), W)
+        h.close()
+    assert _lib.load().fv_host_staging_release() == 0
+
+
+@pytest.mark.parametrize("n", [1, (1 << 18) - 1, 1 << 18, (1 << 19) + 5, (1 << 22) + 3])
+def test_orders_through_the_slots(gpu, n):
+    """Window tables and orders of n 64-bit entries: below and above the size from which pieces are taken, whole and
+    broken last pieces of either length."""
+    from flyvec_amd import Trainer
+    rng = np.random.default_rng(n)
+    tokens = rng.integers(0, 50, size=1000, dtype=np.int32)
+    starts = rng.integers(0, 990, size=n).astype(np.uint64)
+    perm = rng.permutation(n).astype(np.uint64)
+    t = Trainer(50, 8, 5, 16)
+    t.set_corpus_starts(tokens, starts)
+    assert np.array_equal(t.window_starts(), starts)
+    t.set_permutation(perm)
+    assert np.array_equal(t.get_permutation(), perm)
+    t.close()
+
+
+def test_more_transfers_at_once_than_there_are_slots(gpu):
+    """Six threads, each with a trainer of its own, hold up to four of eight slots each: they wait for each other's and
+    all finish with their own matrix."""
+    from flyvec_amd import Trainer
+    K, V = 130, 30000
+    bad = []
+
+    def work(seed):
+        W = np.random.default_rng(seed).standard_normal((K, 2 * V), dtype=np.float32)
+        t = Trainer(V, K, 3, 16)
+        for _ in range(3):
+            t.set_weights(W)
+            if not np.array_equal(t.get_weights(), W):
+                bad.append(seed)
+        t.close()
+
+    threads = [threading.Thread(target=work, args=(s,)) for s in range(6)]
+    for th in threads:
+        th.start()
+    for th in threads:
+        th.join()
+    assert not bad
+
+
+@pytest.mark.parametrize("K,w,n", [(400, 1, 1), (400, 1, 648), (400, 1, 649), (400, 1, 20000), (70, 11, 2300),
+                                   (70, 11, 2301), (70, 11, 100003), (400, 11, 40001)])
+@pytest.mark.parametrize("locked", [False, True])
+def test_hash_batches_of_every_route(gpu, K, w, n, locked):
+    """Codes and packed codes from host arrays, beside the largest batch that goes through the one buffer (2^18 bytes of
+    indices and codes: 648 targets of 400 neurons, 2299 windows of 11 with 70 neurons and two words), one chunk and
+    several, against the device-resident call on the same indices. An index out of range is reported by every route
+    and leaves the next call clean."""
+    from flyvec_amd import Hasher, _lib
+    V = 500
+    rng = np.random.default_rng(n)
+    h = Hasher(rng.standard_normal((K, 2 * V), dtype=np.float32))
+    idx = rng.integers(-1, 2 * V, size=(n, w)).astype(np.int32)
+    if w == 1:
+        idx[:] = rng.integers(0, V, size=(n, 1))
+    dev, bits_dev = _lib.DeviceBuffer.from_numpy(idx), _lib.DeviceBuffer(n * h.words * 8)
+    codes_dev = _lib.DeviceBuffer(n * K)
+    h.hash_windows_dev(dev, n, w, 9, bits_dev, codes_dev)
+    h.sync()
+    bits, codes = bits_dev.to_numpy(np.uint64, (n, h.words)), codes_dev.to_numpy(np.int8, (n, K))
+    src = idx
+    out = {}
+    if locked:
+        src = _lib.pinned_empty(idx.shape, np.int32)
+        src[...] = idx
+        out = dict(out_bits=_lib.pinned_empty(bits.shape, np.uint64), out_codes=_lib.pinned_empty(codes.shape, np.int8))
+    for bad in (False, True, False):
+        if bad:
+            kept = src[n // 2, 0]
+            src[n // 2, 0] = 2 * V
+            with pytest.raises(_lib.FlyvecError):
+                h.hash_windows(src, 9, packed=True, codes=True, **out)
+            src[n // 2, 0] = kept
+        else:
+            got_bits, got_codes = h.hash_windows(src, 9, packed=True, codes=True, **out)
+            assert np.array_equal(got_bits, bits) and np.array_equal(got_codes, codes)
+    assert np.array_equal(h.hash_windows(src, 9, packed=False, codes=True), codes)
+    if w == 1:
+        idx += V  # the target block's columns
+        dev2 = _lib.DeviceBuffer.from_numpy(idx)
+        h.hash_windows_dev(dev2, n, 1, 9, None, codes_dev)
+        h.sync()
+        assert np.array_equal(h.hash_targets(idx[:, 0] - V, 9), codes_dev.to_numpy(np.int8, (n, K)))
+    h.close()
+
+
+def test_one_corpus_after_another(gpu, oracle_lib):
+    """A trainer given corpora of other sizes in turn (a little smaller: the buffers are used again; much smaller, larger:
+    they are not), with reshuffles between, samples what a new trainer would."""
+    from flyvec_amd import Trainer
+    from conftest import small_corpus
+    V, w = 300, 7
+    t = Trainer(V, 16, w, 64)
+    for i, n in enumerate((20000, 19000, 4000, 4000, 60000, 55000)):
+        tokens, offsets = small_corpus(n, V, seed=i)
+        t.set_corpus(tokens, offsets)
+        starts = oracle_lib.window_starts(offsets, w)
+        assert t.num_windows == len(starts) and np.array_equal(t.window_starts(), starts)
+        assert np.array_equal(t.get_permutation(), np.arange(len(starts), dtype=np.uint64))
+        assert np.array_equal(t.inverse_frequency(), oracle_lib.inverse_frequency(tokens, V))
+        t.shuffle(i)
+        assert np.array_equal(np.sort(t.get_permutation()), np.arange(len(starts), dtype=np.uint64))
+    with pytest.raises(Exception):
+        t.set_corpus(np.full(100, V, dtype=np.int32), np.array([0, 50, 100], dtype=np.uint64))
+    with pytest.raises(Exception):
+        t.num_windows  # the corpus before the refused one is gone, as before
+    t.close()

@@ -125,6 +125,20 @@ def test_normalize_matches_numpy(gpu):
         h.close()
 
 
+@pytest.mark.parametrize("N", [1, 7, 8, 128, 129, 136, 263, 4103, 8190, 8191, 8192, 8193, 16384, 20487, 40001])
+def test_row_sums_of_every_tree_shape(gpu, N):
+    """The tree of a run of numpy's pairwise sum: one leaf, leaves that rounding pushed over 128 and split once more,
+    whole runs, a last run of one element; numbers of neurons around the sixteen of a block."""
+    from flyvec_amd import Hasher
+    from oracle import hash_oracle as ho
+    for K in (2, 15, 16, 17):
+        W = np.random.default_rng(N + K).standard_normal((K, N), dtype=np.float32)
+        h = Hasher(W)
+        h.normalize()
+        assert np.array_equal(h.weights(), ho.normalize_synapses(W)), K
+        h.close()
+
+
 @pytest.mark.parametrize("p", [1, 2, 3, 4, 7])
 def test_normalize_with_another_exponent(gpu, p):
     """flyvec/core.py:23 takes the exponent of the norm. p = 1 and p = 2 are numpy's fast paths (the value, the

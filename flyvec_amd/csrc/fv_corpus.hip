@@ -76,44 +76,62 @@ __global__ __launch_bounds__(FV_SCAN_THREADS) void fv_scan_totals_kernel(uint64_
   if (threadIdx.x == 0) totals[n_tiles] = carry;
 }
 
-// Pass 3: each thread rescans its FV_SCAN_ITEMS chunks and writes their window starts.
+// Pass 3: FV_SCAN_PARTS blocks per tile. Each scans the tile's chunks again and writes its part of the tile's window starts,
+// neighbouring threads neighbouring starts, each thread finding a start's chunk by a search in the scan. (A block per tile whose
+// threads wrote their own eight chunks' starts, one 8-byte store per chunk and turn, took 59 us for 2.6 M windows of
+// 160000 chunks: 78 blocks, every store a line of its own; so it takes 19.)
+#define FV_SCAN_PARTS 8u
 __global__ __launch_bounds__(FV_SCAN_THREADS) void fv_expand_starts_kernel(
     const uint64_t *__restrict__ off, uint64_t n_chunks, uint64_t w,
     const uint64_t *__restrict__ tile_base, uint64_t *__restrict__ starts, uint64_t n_windows) {
-  __shared__ uint64_t part[FV_SCAN_THREADS];
-  const uint64_t base = (uint64_t)blockIdx.x * FV_SCAN_TILE + (uint64_t)threadIdx.x * FV_SCAN_ITEMS;
-  uint64_t cnt[FV_SCAN_ITEMS];
-  uint64_t mine = 0;
+  __shared__ uint32_t part[FV_SCAN_THREADS];
+  __shared__ uint32_t before[FV_SCAN_TILE];  // windows of the tile in front of each chunk (a tile has fewer than 2^19)
+  __shared__ uint64_t first[FV_SCAN_TILE];   // corpus position of each chunk
+  const uint64_t tile = blockIdx.x / FV_SCAN_PARTS;
+  const uint32_t tid = threadIdx.x, own = tid * FV_SCAN_ITEMS;
+  const uint64_t base = tile * FV_SCAN_TILE + own;
+  const uint64_t off0 = off[0];
+  uint32_t cnt[FV_SCAN_ITEMS];
+  uint32_t mine = 0;
 #pragma unroll
   for (int j = 0; j < FV_SCAN_ITEMS; ++j) {
-    cnt[j] = fv_chunk_windows(off, base + j, n_chunks, w);
+    cnt[j] = (uint32_t)fv_chunk_windows(off, base + j, n_chunks, w);
+    first[own + j] = base + j < n_chunks ? off[base + j] - off0 : 0;
     mine += cnt[j];
   }
-  part[threadIdx.x] = mine;
+  part[tid] = mine;
   __syncthreads();
-  for (int d = 1; d < FV_SCAN_THREADS; d <<= 1) {
-    uint64_t add = threadIdx.x >= (unsigned)d ? part[threadIdx.x - d] : 0;
+  for (uint32_t d = 1; d < FV_SCAN_THREADS; d <<= 1) {
+    const uint32_t add = tid >= d ? part[tid - d] : 0;
     __syncthreads();
-    part[threadIdx.x] += add;
+    part[tid] += add;
     __syncthreads();
   }
-  uint64_t out = tile_base[blockIdx.x] + part[threadIdx.x] - mine;
-  const uint64_t off0 = off[0];
+  const uint32_t total = part[FV_SCAN_THREADS - 1];
+  uint32_t at = part[tid] - mine;
 #pragma unroll
   for (int j = 0; j < FV_SCAN_ITEMS; ++j) {
-    if (cnt[j]) {
-      uint64_t first = off[base + j] - off0;
-      for (uint64_t i = 0; i < cnt[j]; ++i)
-        if (out + i < n_windows) starts[out + i] = first + i;
-      out += cnt[j];
-    }
+    before[own + j] = at;
+    at += cnt[j];
+  }
+  __syncthreads();
+  const uint32_t p = blockIdx.x % FV_SCAN_PARTS;
+  const uint32_t lo = (uint32_t)((uint64_t)total * p / FV_SCAN_PARTS), hi = (uint32_t)((uint64_t)total * (p + 1) / FV_SCAN_PARTS);
+  const uint64_t out0 = tile_base[tile];
+  for (uint32_t i = lo + tid; i < hi; i += FV_SCAN_THREADS) {
+    // the last chunk with no more than i windows in front of it (of several, those before it have no windows)
+    uint32_t c = 0;
+#pragma unroll
+    for (uint32_t step = FV_SCAN_TILE / 2; step; step >>= 1)
+      if (before[c + step] <= i) c += step;
+    if (out0 + i < n_windows) starts[out0 + i] = first[c] + (i - before[c]);
   }
 }
 
 static int fv_scan_windows(const uint64_t *offsets_dev, uint64_t n_chunks, uint64_t w,
                            uint64_t **out_tile_base, uint64_t *out_total, hipStream_t stream) {
   const uint64_t n_tiles = (n_chunks + FV_SCAN_TILE - 1) / FV_SCAN_TILE;
-  FV_REQUIRE(n_tiles < (1ull << 31), FV_ERR_INVALID, "too many chunks (%llu)",
+  FV_REQUIRE(n_tiles < (1ull << 31) / FV_SCAN_PARTS, FV_ERR_INVALID, "too many chunks (%llu)",
              (unsigned long long)n_chunks);
   uint64_t *totals = nullptr;
   FV_HIP(hipMalloc((void **)&totals, (n_tiles + 1) * sizeof(uint64_t)));
@@ -153,7 +171,7 @@ int fv_dev_build_window_starts(const uint64_t *offsets_dev, uint64_t n_chunks, u
                  (unsigned long long)n_windows, (unsigned long long)total);
   } else if (n_chunks) {
     const uint64_t n_tiles = (n_chunks + FV_SCAN_TILE - 1) / FV_SCAN_TILE;
-    hipLaunchKernelGGL(fv_expand_starts_kernel, dim3((unsigned)n_tiles), dim3(FV_SCAN_THREADS), 0,
+    hipLaunchKernelGGL(fv_expand_starts_kernel, dim3((unsigned)n_tiles * FV_SCAN_PARTS), dim3(FV_SCAN_THREADS), 0,
                        stream, offsets_dev, n_chunks, w, tile_base, starts_dev, n_windows);
     hipError_t e = hipGetLastError();
     if (e == hipSuccess) e = hipStreamSynchronize(stream);
@@ -221,9 +239,22 @@ __global__ __launch_bounds__(256) void fv_histogram_kernel(const int32_t *__rest
     lo = ol < lo ? ol : lo;
     hi = oh > hi ? oh : hi;
   }
-  if ((threadIdx.x & 63) == 0 && lo <= hi) {
-    atomicMin(&minmax[0], lo);
-    atomicMax(&minmax[1], hi);
+  // one pair of atomics per block: they all meet at two addresses (a pair per wave: 112 us at 4 M tokens, so 52)
+  __shared__ int32_t block_lo[4], block_hi[4];
+  if ((threadIdx.x & 63) == 0) {
+    block_lo[threadIdx.x >> 6] = lo;
+    block_hi[threadIdx.x >> 6] = hi;
+  }
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    for (int i = 1; i < 4; ++i) {
+      lo = block_lo[i] < lo ? block_lo[i] : lo;
+      hi = block_hi[i] > hi ? block_hi[i] : hi;
+    }
+    if (lo <= hi) {
+      atomicMin(&minmax[0], lo);
+      atomicMax(&minmax[1], hi);
+    }
   }
 }
 

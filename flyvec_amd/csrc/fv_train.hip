@@ -91,19 +91,27 @@ __global__ __launch_bounds__(64) void fv_row_norm_kernel(const double *__restric
 
 // ---- window order ------------------------------------------------------------------------------
 
-__global__ __launch_bounds__(256) void fv_identity_kernel(uint64_t *__restrict__ perm, uint64_t n) {
-  for (uint64_t i = (uint64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (uint64_t)gridDim.x * 256) perm[i] = i;
+// The sampler's two look-ups (order -> window -> start) are folded into one table whenever the order changes.
+
+// The identity: the table is the starts themselves.
+__global__ __launch_bounds__(256) void fv_identity_kernel(const uint64_t *__restrict__ starts, uint64_t *__restrict__ perm,
+                                                          uint64_t *__restrict__ pstart, uint64_t n) {
+  for (uint64_t i = (uint64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (uint64_t)gridDim.x * 256) {
+    perm[i] = i;
+    pstart[i] = starts[i];
+  }
 }
 
 // The reshuffle of flyvec/src/model_arrays.cu:451-465 rearranges the current order, cumulatively
-// over the epochs; here out[i] = in[sigma(i)] with sigma a keyed bijection computed per index.
+// over the epochs; here out[i] = in[sigma(i)] with sigma a keyed bijection computed per index. (The table in a launch
+// of its own behind it: two random reads one behind the other in one launch took 97 us for 2.6 M windows, the two
+// launches 45 + 29.)
 __global__ __launch_bounds__(256) void fv_shuffle_kernel(const uint64_t *__restrict__ in, uint64_t *__restrict__ out,
                                                          uint64_t n, fv_feistel f) {
   for (uint64_t i = (uint64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (uint64_t)gridDim.x * 256)
     out[i] = in[fv_permute_index(&f, i, n)];
 }
 
-// The sampler's two look-ups (order -> window -> start) folded into one table whenever the order changes.
 __global__ __launch_bounds__(256) void fv_order_starts_kernel(const uint64_t *__restrict__ perm,
                                                               const uint64_t *__restrict__ starts,
                                                               uint64_t *__restrict__ pstart, uint64_t n) {
@@ -515,9 +523,8 @@ extern "C" int fv_trainer_set_corpus(fv_trainer *t, const int32_t *tokens, uint6
     }
     if (rc == FV_OK) rc = fv_dev_build_window_starts(off_dev, n_chunks, t->w, t->starts, nwin, t->stream);
     if (rc == FV_OK) {
-      hipLaunchKernelGGL(fv_identity_kernel, dim3(fv_perm_blocks(nwin)), dim3(256), 0, t->stream, t->perm, nwin);
-      hipLaunchKernelGGL(fv_order_starts_kernel, dim3(fv_perm_blocks(nwin)), dim3(256), 0, t->stream, t->perm,
-                         t->starts, t->pstart, nwin);
+      hipLaunchKernelGGL(fv_identity_kernel, dim3(fv_perm_blocks(nwin)), dim3(256), 0, t->stream, t->starts, t->perm,
+                         t->pstart, nwin);
       e = hipStreamSynchronize(t->stream);
       if (e != hipSuccess) rc = fv_fail(FV_ERR_HIP, "permutation fill failed: %s", hipGetErrorString(e));
     }
@@ -558,9 +565,8 @@ extern "C" int fv_trainer_set_corpus_starts(fv_trainer *t, const int32_t *tokens
     rc = fv_trainer_reserve_windows(t, n_windows);
     if (rc == FV_OK) rc = fv_copy_up(t->starts, starts, n_windows * sizeof(uint64_t), t->stream);
     if (rc == FV_OK) {
-      hipLaunchKernelGGL(fv_identity_kernel, dim3(fv_perm_blocks(n_windows)), dim3(256), 0, t->stream, t->perm, n_windows);
-      hipLaunchKernelGGL(fv_order_starts_kernel, dim3(fv_perm_blocks(n_windows)), dim3(256), 0, t->stream, t->perm,
-                         t->starts, t->pstart, n_windows);
+      hipLaunchKernelGGL(fv_identity_kernel, dim3(fv_perm_blocks(n_windows)), dim3(256), 0, t->stream, t->starts, t->perm,
+                         t->pstart, n_windows);
       const hipError_t e = hipStreamSynchronize(t->stream);
       if (e != hipSuccess) rc = fv_fail(FV_ERR_HIP, "permutation fill failed: %s", hipGetErrorString(e));
     }

@@ -34,6 +34,19 @@ def test_window_table_against_checker(gpu, oracle_lib, seed, w, n_chunks):
     assert np.array_equal(window_starts(off, w), oracle_lib.window_starts(off, w))
 
 
+@pytest.mark.parametrize("n_chunks", [1, 7, 2047, 2048, 2049, 4097])
+def test_window_table_at_tile_edges(gpu, oracle_lib, n_chunks):
+    """Chunks around the 2048 of a tile: many without windows (short, too long) in front, between and behind, fewer
+    windows than a tile has blocks, the most a tile can have."""
+    from flyvec_amd.engine import window_starts
+    w = 5
+    rng = np.random.default_rng(n_chunks)
+    for lengths in (rng.choice([0, 1, 4, 5, 6, 25, 213, 214, 300], size=n_chunks), np.full(n_chunks, 213),
+                    np.full(n_chunks, 4), np.r_[np.full(n_chunks - 1, 2), 7], np.r_[6, np.full(n_chunks - 1, 214)]):
+        offsets = np.r_[0, np.cumsum(lengths)].astype(np.uint64)
+        assert np.array_equal(window_starts(offsets, w), oracle_lib.window_starts(offsets, w))
+
+
 def test_empty_and_degenerate_offsets(gpu):
     from flyvec_amd import count_windows, window_starts
     assert count_windows(np.array([0], dtype=np.uint64), 11) == 0

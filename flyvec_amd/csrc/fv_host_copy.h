@@ -175,6 +175,7 @@ int fv_pipe_down(uint64_t n_pieces, hipStream_t stream, Produce produce, Piece p
   return rc;
 }
 
-// Plain copies; the stream has drained when they return. Page-locked memory and small sizes go through the runtime.
+// Plain copies. Page-locked memory and small sizes go through the runtime. Upwards the caller waits for the stream before
+// its own caller may change the source; downwards the host memory is filled on return.
 int fv_copy_up(void *dst_dev, const void *src_host, size_t bytes, hipStream_t stream);
 int fv_copy_down(void *dst_host, const void *src_dev, size_t bytes, hipStream_t stream);

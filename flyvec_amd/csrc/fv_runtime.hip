@@ -261,7 +261,6 @@ int fv_copy_up(void *dst_dev, const void *src_host, size_t bytes, hipStream_t st
   if (bytes == 0) return FV_OK;
   if (!fv_stages(src_host, bytes)) {
     FV_HIP(hipMemcpyAsync(dst_dev, src_host, bytes, hipMemcpyHostToDevice, stream));
-    FV_HIP(hipStreamSynchronize(stream));
     return FV_OK;
   }
   const size_t slot = bytes >= 4 * FV_STAGE_SLOT_BYTES ? FV_STAGE_SLOT_BYTES : FV_STAGE_SLOT_BYTES / 8;

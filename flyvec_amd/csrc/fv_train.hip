@@ -254,9 +254,7 @@ extern "C" int fv_trainer_destroy(fv_trainer *t) {
   (void)hipFree(t->top2_part);
   (void)hipFree(t->row_hits);
   (void)hipFree(t->path_count);
-  (void)hipFree(t->norm_part);
   if (t->norms) (void)hipHostFree(t->norms);
-  if (t->onepass_status) (void)hipHostFree(t->onepass_status);
   if (t->stream) (void)hipStreamDestroy(t->stream);
   fv_trainer_leaves_flight(t);
   delete t;
@@ -331,14 +329,18 @@ static int fv_trainer_alloc(fv_trainer *t) {
       FV_HIP(hipMalloc((void **)&t->slots_blocks, region * t->K * FV_NB_CLASSES * sizeof(fv_slot)));
     }
   }
-  FV_HIP(hipMalloc((void **)&t->scalars, 16 * sizeof(float)));
+  // behind the sixteen scalars the workspace of fv_trainer_row_norms, and its results in page-locked memory with the
+  // status word behind them
+  FV_HIP(hipMalloc((void **)&t->scalars, 16 * sizeof(float) + (size_t)t->K * FV_NORM_BLOCKS * sizeof(double)));
+  t->norm_part = (double *)(t->scalars + 16);
+  FV_HIP(hipHostMalloc((void **)&t->norms, t->K * sizeof(double) + sizeof(uint32_t), hipHostMallocDefault));
   FV_HIP(hipMemsetAsync(t->Wt, 0, elems * sizeof(float), t->stream));
   FV_HIP(hipMemsetAsync(t->xx, 0, (size_t)t->ldk * sizeof(float), t->stream));
   FV_HIP(hipMemsetAsync(t->scalars, 0, 16 * sizeof(float), t->stream));
   if (t->onepass_blocks) {
     FV_HIP(hipMalloc((void **)&t->arrive, ((size_t)t->onepass_blocks + 1) * sizeof(unsigned long long)));
     FV_HIP(hipMemsetAsync(t->arrive, 0, ((size_t)t->onepass_blocks + 1) * sizeof(unsigned long long), t->stream));
-    FV_HIP(hipHostMalloc((void **)&t->onepass_status, sizeof(uint32_t), hipHostMallocDefault));
+    t->onepass_status = (uint32_t *)(t->norms + t->K);
     *t->onepass_status = 0;
   }
   FV_HIP(hipStreamSynchronize(t->stream));
@@ -653,6 +655,7 @@ extern "C" int fv_trainer_set_permutation(fv_trainer *t, const uint64_t *perm, u
     FV_REQUIRE(perm[i] < n, FV_ERR_DATA, "permutation entry %llu = %llu is not a window index",
                (unsigned long long)i, (unsigned long long)perm[i]);
   FV_TRY(fv_copy_up(t->perm, perm, n * sizeof(uint64_t), t->stream));
+  FV_HIP(hipStreamSynchronize(t->stream));  // `perm` is the caller's again
   t->ahead_valid = false;  // sampled in the old order
   hipLaunchKernelGGL(fv_order_starts_kernel, dim3(fv_perm_blocks(n)), dim3(256), 0, t->stream, t->perm, t->starts,
                      t->pstart, n);
@@ -1290,17 +1293,6 @@ extern "C" int fv_trainer_row_norms(fv_trainer *t, uint32_t n_rows, double *out_
   FV_REQUIRE(t->have_weights, FV_ERR_STATE, "no weights set");
   if (n_rows > t->K) n_rows = t->K;
   if (n_rows == 0) return FV_OK;
-  // the blocks' sums, and the norms in page-locked memory: kept for as many rows as have been asked for
-  if (t->norm_rows < n_rows) {
-    FV_HIP(hipStreamSynchronize(t->stream));
-    (void)hipFree(t->norm_part);
-    if (t->norms) (void)hipHostFree(t->norms);
-    t->norm_part = t->norms = nullptr;
-    t->norm_rows = 0;
-    FV_HIP(hipMalloc((void **)&t->norm_part, (size_t)n_rows * FV_NORM_BLOCKS * sizeof(double)));
-    FV_HIP(hipHostMalloc((void **)&t->norms, n_rows * sizeof(double), hipHostMallocDefault));
-    t->norm_rows = n_rows;
-  }
   const uint64_t want = (t->N + 15) / 16;
   const uint32_t blocks = (uint32_t)(want < FV_NORM_BLOCKS ? want : FV_NORM_BLOCKS);
   hipLaunchKernelGGL(fv_row_squares_kernel, dim3(blocks, (n_rows + 15) / 16), dim3(256), 0, t->stream, t->Wt, t->N, t->ldk,

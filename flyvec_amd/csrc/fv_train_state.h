@@ -132,10 +132,9 @@ struct fv_trainer {
   unsigned long long *arrive;
   uint32_t onepass_epoch;
   uint32_t onepass_spin_limit;
-  uint32_t *onepass_status;  // pinned host word: 0, or the tag of the first launch that gave up
+  uint32_t *onepass_status;  // pinned host word (in the allocation of norms): 0, or the tag of the first launch that gave up
   uint32_t step_tag;         // tag of the step being enqueued: run_epoch numbers its steps from 1, else 0
   uint64_t giveups_recovered;  // epochs in which run_epoch took up again behind a launch that gave up
-  double *norm_part, *norms;   // workspace of fv_trainer_row_norms: FV_NORM_BLOCKS sums per row; page-locked results
-  uint32_t norm_rows;          // rows they hold
+  double *norm_part, *norms;  // workspace of fv_trainer_row_norms: FV_NORM_BLOCKS sums per row; page-locked results
   float update_cut;  // largest fp32 <= 1e-10
 };

@@ -51,7 +51,7 @@ struct fv_hasher {
   hipStream_t stream;
   float *Wt;
   uint32_t *err;  // flag in page-locked memory: a column index outside [-1, N) was met
-  char *direct;   // page-locked, FV_HASH_DIRECT_BYTES (null until the first small batch)
+  char *direct;   // behind it, FV_HASH_DIRECT_BYTES for small batches
   unsigned max_blocks;
   fv_hash_lane lane[FV_HASH_LANES];  // lane 0 runs on `stream`
 };
@@ -233,7 +233,6 @@ extern "C" int fv_hasher_destroy(fv_hasher *h) {
   }
   (void)hipFree(h->Wt);
   if (h->err) (void)hipHostFree(h->err);
-  if (h->direct) (void)hipHostFree(h->direct);
   if (h->stream) (void)hipStreamDestroy(h->stream);
   delete h;
   return FV_OK;
@@ -265,8 +264,11 @@ extern "C" int fv_hasher_create(const float *W, uint32_t hid, uint64_t n_columns
     if (e == hipSuccess) e = hipMalloc((void **)&h->Wt, (size_t)fv_matrix_alloc_elems(h->K, h->N) * sizeof(float));
     if (e == hipSuccess)
       e = hipMemsetAsync(h->Wt + (size_t)h->N * h->ldk, 0, (size_t)fv_matrix_pad_elems(h->K) * sizeof(float), h->stream);
-    if (e == hipSuccess) e = hipHostMalloc((void **)&h->err, sizeof(uint32_t), hipHostMallocCoherent);
-    if (e == hipSuccess) *h->err = 0;
+    if (e == hipSuccess) e = hipHostMalloc((void **)&h->err, 64 + FV_HASH_DIRECT_BYTES, hipHostMallocCoherent);
+    if (e == hipSuccess) {
+      *h->err = 0;
+      h->direct = (char *)h->err + 64;
+    }
     if (e != hipSuccess) rc = fv_fail(FV_ERR_HIP, "hasher allocation failed: %s", hipGetErrorString(e));
   }
   if (rc == FV_OK) rc = fv_upload_weights(W, h->Wt, h->K, h->N, h->ldk, h->stream);
@@ -326,7 +328,6 @@ static int fv_hash_reserve_pinned(char **buf, size_t *cap, size_t bytes) {
 // A small batch: the kernel reads the indices from, and writes its results to, one page-locked buffer.
 static int fv_hash_direct(fv_hasher *h, const int32_t *idx, uint64_t n, uint32_t w, uint32_t k, int32_t shift,
                           uint64_t *out_bits, int8_t *out_codes) {
-  if (!h->direct) FV_HIP(hipHostMalloc((void **)&h->direct, FV_HASH_DIRECT_BYTES, hipHostMallocCoherent));
   const size_t bits_bytes = out_bits ? n * ((h->K + 63) / 64) * sizeof(uint64_t) : 0;
   const size_t idx_bytes = n * w * sizeof(int32_t), codes_bytes = out_codes ? n * h->K : 0;
   uint64_t *bits = (uint64_t *)h->direct;
@@ -346,7 +347,7 @@ static int fv_hash_direct(fv_hasher *h, const int32_t *idx, uint64_t n, uint32_t
 // chunk is copied in, hashed and copied out in stream order, so the copies of one chunk overlap the kernel
 // of the other. Host buffers from fv_host_alloc_pinned are copied by DMA as they are. Outputs that go to
 // pageable memory are copied by DMA into the lane's page-locked staging and from there by host threads
-// (fv_copy_ring) while the device goes on; pageable inputs are copied into the lane's staging by the calling thread.
+// (fv_copy_ring) while the device goes on; pageable inputs are copied into the lane's staging by the same threads.
 // Nothing is allocated once the lanes' buffers have reached the chunk size. (100003 windows, K = 400, pageable: 4.0 ms
 // as one chunk through the runtime's copies.)
 static int fv_hash_host(fv_hasher *h, const int32_t *idx, uint64_t n, uint32_t w, uint32_t k, int32_t shift,
@@ -358,16 +359,21 @@ static int fv_hash_host(fv_hasher *h, const int32_t *idx, uint64_t n, uint32_t w
   const uint64_t out_row = (out_bits ? bits_row : 0) + (out_codes ? codes_row : 0);
   if (n <= FV_HASH_DIRECT_BYTES && n * (w * sizeof(int32_t) + out_row) <= FV_HASH_DIRECT_BYTES)
     return fv_hash_direct(h, idx, n, w, k, shift, out_bits, out_codes);
-  uint64_t chunk = (n + FV_HASH_CHUNKS - 1) / FV_HASH_CHUNKS;
-  const uint64_t least = FV_HASH_CHUNK_MIN_BYTES / (out_row ? out_row : 1) + 1;
-  chunk = chunk < least ? least : chunk;
-  chunk = chunk < FV_HASH_CHUNK ? chunk : FV_HASH_CHUNK;
+  // Small chunks and the host threads where results of some size go to memory that the device cannot reach by DMA; the
+  // indices then take the same way. Else the runtime's copies, in as few pieces as the lanes' buffers allow.
+  const bool crew = n * out_row >= FV_STAGE_MIN_BYTES && ((out_bits && fv_is_pageable(out_bits)) ||
+                                                          (out_codes && fv_is_pageable(out_codes)));
+  uint64_t chunk = FV_HASH_CHUNK;
+  if (crew) {
+    const uint64_t share = (n + FV_HASH_CHUNKS - 1) / FV_HASH_CHUNKS, least = FV_HASH_CHUNK_MIN_BYTES / out_row + 1;
+    chunk = share > least ? share : least;
+    chunk = chunk < FV_HASH_CHUNK ? chunk : FV_HASH_CHUNK;
+  }
   chunk = chunk < n ? chunk : n;
   const int lanes = n > chunk ? FV_HASH_LANES : 1;
-  const bool stage_idx = fv_is_pageable(idx);
-  // staging pays off for outputs of some size that the device cannot reach by DMA
-  const bool stage_bits = out_bits && lanes > 1 && fv_is_pageable(out_bits);
-  const bool stage_codes = out_codes && lanes > 1 && fv_is_pageable(out_codes);
+  const bool stage_bits = crew && out_bits && lanes > 1 && fv_is_pageable(out_bits);
+  const bool stage_codes = crew && out_codes && lanes > 1 && fv_is_pageable(out_codes);
+  const bool stage_idx = (stage_bits || stage_codes) && fv_is_pageable(idx);
   FV_HIP(hipStreamSynchronize(h->stream));  // what the caller enqueued on the hasher's stream comes first
   for (int l = 0; l < lanes; ++l) {
     fv_hash_lane &ln = h->lane[l];
@@ -387,7 +393,7 @@ static int fv_hash_host(fv_hasher *h, const int32_t *idx, uint64_t n, uint32_t w
   }
   const uint64_t n_chunks = (n + chunk - 1) / chunk;
   std::unique_ptr<fv_copy_ring> ring;
-  if (stage_bits || stage_codes) ring.reset(new fv_copy_ring(2 * n_chunks));
+  if (stage_bits || stage_codes) ring.reset(new fv_copy_ring(3 * n_chunks, crew));
   std::vector<uint32_t> last_item(n_chunks, 0xffffffffu);  // the last copy item of every chunk
   int rc = FV_OK;
   // chunk c's staged outputs are handed to the host threads once its copies have landed (one iteration later,
@@ -409,7 +415,10 @@ static int fv_hash_host(fv_hasher *h, const int32_t *idx, uint64_t n, uint32_t w
     if (stage_idx) {
       // the lane's chunk before this one has been copied in
       if (c >= (uint64_t)lanes) e = hipEventSynchronize(ln.done);
-      if (e == hipSuccess) from = (const int32_t *)memcpy(ln.stage_idx, from, m * w * sizeof(int32_t));
+      if (e == hipSuccess) {
+        ring->wait(ring->publish((const char *)from, ln.stage_idx, m * w * sizeof(int32_t)));
+        from = (const int32_t *)ln.stage_idx;
+      }
     }
     if (e == hipSuccess) e = hipMemcpyAsync(ln.idx, from, m * w * sizeof(int32_t), hipMemcpyHostToDevice, ln.stream);
     if (e != hipSuccess) {

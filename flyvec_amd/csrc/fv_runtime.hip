@@ -266,7 +266,7 @@ int fv_copy_up(void *dst_dev, const void *src_host, size_t bytes, hipStream_t st
   const size_t slot = bytes >= 4 * FV_STAGE_SLOT_BYTES ? FV_STAGE_SLOT_BYTES : FV_STAGE_SLOT_BYTES / 8;
   const auto length = [&](uint64_t t) { return bytes - t * slot < slot ? bytes - t * slot : slot; };
   return fv_pipe_up(
-      (bytes + slot - 1) / slot, stream,
+      (bytes + slot - 1) / slot, bytes, stream,
       [&](uint64_t t, char *p) {
         return fv_copy_ring::item{(const char *)src_host + t * slot, p, length(t), 0, 0, 1};
       },
@@ -286,7 +286,7 @@ int fv_copy_down(void *dst_host, const void *src_dev, size_t bytes, hipStream_t 
   const size_t slot = bytes >= 4 * FV_STAGE_SLOT_BYTES ? FV_STAGE_SLOT_BYTES : FV_STAGE_SLOT_BYTES / 8;
   const auto length = [&](uint64_t t) { return bytes - t * slot < slot ? bytes - t * slot : slot; };
   return fv_pipe_down(
-      (bytes + slot - 1) / slot, stream,
+      (bytes + slot - 1) / slot, bytes, stream,
       [&](uint64_t t, char *p) -> int {
         FV_HIP(hipMemcpyAsync(p, (const char *)src_dev + t * slot, length(t), hipMemcpyDeviceToHost, stream));
         return FV_OK;
@@ -323,7 +323,7 @@ int fv_upload_weights(const float *W_host, float *Wt_dev, uint32_t K, uint64_t N
   } else if (fv_is_pageable(W_host) && fv_is_pageable((const char *)W_host + bytes - 1)) {
     const fv_weight_tiles tiles(K, N);
     return fv_pipe_up(
-        tiles.n, stream,
+        tiles.n, bytes, stream,
         [&](uint64_t t, char *p) {
           return fv_copy_ring::item{(const char *)(W_host + tiles.h(t) * N + tiles.i(t)), p, tiles.cols(t) * sizeof(float),
                                     N * sizeof(float), tiles.pitch(t) * sizeof(float), tiles.rows(t)};
@@ -356,7 +356,7 @@ int fv_download_weights(const float *Wt_dev, float *W_host, uint32_t K, uint64_t
   } else if (fv_is_pageable(W_host) && fv_is_pageable((const char *)W_host + bytes - 1)) {
     const fv_weight_tiles tiles(K, N);
     return fv_pipe_down(
-        tiles.n, stream,
+        tiles.n, bytes, stream,
         [&](uint64_t t, char *p) {
           return fv_launch_to_row_major(Wt_dev + tiles.i(t) * ldk + tiles.h(t), (float *)p, tiles.pitch(t), tiles.rows(t),
                                         tiles.cols(t), ldk, stream);

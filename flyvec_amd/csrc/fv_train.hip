@@ -200,6 +200,14 @@ static void fv_trainer_leaves_flight(fv_trainer *t) {
   t->in_flight = false;
 }
 
+// Waits for the trainer's stream. Every wait of this file goes through here, so that a trainer whose steps have been
+// waited for by whatever call is out of the count.
+static hipError_t fv_trainer_drain(fv_trainer *t) {
+  const hipError_t e = hipStreamSynchronize(t->stream);
+  if (e == hipSuccess) fv_trainer_leaves_flight(t);
+  return e;
+}
+
 // After a single dense launch has given up: the trainer goes on with two launches per step, and the marks
 // the launch left (status word, "dead" flag for the launches behind it) are cleared. Returns the tag.
 static int fv_trainer_take_giveup(fv_trainer *t, uint32_t *out_tag) {
@@ -211,14 +219,13 @@ static int fv_trainer_take_giveup(fv_trainer *t, uint32_t *out_tag) {
   t->top2_valid = false;
   t->ahead_valid = false;
   FV_HIP(hipMemsetAsync(t->scalars + 1, 0, sizeof(float), t->stream));
-  FV_HIP(hipStreamSynchronize(t->stream));
+  FV_HIP(fv_trainer_drain(t));
   return FV_OK;
 }
 
 // Waits for the trainer's stream; reports a single dense launch that gave up waiting for its other blocks.
 static int fv_trainer_wait(fv_trainer *t) {
-  FV_HIP(hipStreamSynchronize(t->stream));
-  fv_trainer_leaves_flight(t);
+  FV_HIP(fv_trainer_drain(t));
   uint32_t tag = 0;
   FV_TRY(fv_trainer_take_giveup(t, &tag));
   if (tag)
@@ -343,7 +350,7 @@ static int fv_trainer_alloc(fv_trainer *t) {
     t->onepass_status = (uint32_t *)(t->norms + t->K);
     *t->onepass_status = 0;
   }
-  FV_HIP(hipStreamSynchronize(t->stream));
+  FV_HIP(fv_trainer_drain(t));
   return FV_OK;
 }
 
@@ -490,7 +497,7 @@ extern "C" int fv_trainer_set_corpus(fv_trainer *t, const int32_t *tokens, uint6
   FV_REQUIRE(t, FV_ERR_INVALID, "null trainer");
   FV_REQUIRE(tokens && n_tokens > 0, FV_ERR_INVALID, "empty corpus");
   FV_REQUIRE(offsets && n_offsets >= 1, FV_ERR_INVALID, "empty offsets");
-  FV_HIP(hipStreamSynchronize(t->stream));
+  FV_HIP(fv_trainer_drain(t));
   fv_trainer_forget_corpus(t);
   const uint64_t n_chunks = n_offsets - 1;
   uint64_t *off_dev = nullptr;
@@ -527,7 +534,7 @@ extern "C" int fv_trainer_set_corpus(fv_trainer *t, const int32_t *tokens, uint6
     if (rc == FV_OK) {
       hipLaunchKernelGGL(fv_identity_kernel, dim3(fv_perm_blocks(nwin)), dim3(256), 0, t->stream, t->starts, t->perm,
                          t->pstart, nwin);
-      e = hipStreamSynchronize(t->stream);
+      e = fv_trainer_drain(t);
       if (e != hipSuccess) rc = fv_fail(FV_ERR_HIP, "permutation fill failed: %s", hipGetErrorString(e));
     }
   }
@@ -554,7 +561,7 @@ extern "C" int fv_trainer_set_corpus_starts(fv_trainer *t, const int32_t *tokens
     FV_REQUIRE(starts[i] <= n_tokens && t->w <= n_tokens - starts[i], FV_ERR_DATA,
                "window %llu starts at token %llu: it does not fit the corpus of %llu", (unsigned long long)i,
                (unsigned long long)starts[i], (unsigned long long)n_tokens);
-  FV_HIP(hipStreamSynchronize(t->stream));
+  FV_HIP(fv_trainer_drain(t));
   fv_trainer_forget_corpus(t);
   int rc = fv_trainer_reserve_corpus(t, n_tokens);
   if (rc == FV_OK) rc = fv_copy_up(t->corpus, tokens, n_tokens * sizeof(int32_t), t->stream);
@@ -569,7 +576,7 @@ extern "C" int fv_trainer_set_corpus_starts(fv_trainer *t, const int32_t *tokens
     if (rc == FV_OK) {
       hipLaunchKernelGGL(fv_identity_kernel, dim3(fv_perm_blocks(n_windows)), dim3(256), 0, t->stream, t->starts, t->perm,
                          t->pstart, n_windows);
-      const hipError_t e = hipStreamSynchronize(t->stream);
+      const hipError_t e = fv_trainer_drain(t);
       if (e != hipSuccess) rc = fv_fail(FV_ERR_HIP, "permutation fill failed: %s", hipGetErrorString(e));
     }
   }
@@ -598,6 +605,7 @@ extern "C" int fv_trainer_get_window_starts(fv_trainer *t, uint64_t *out_starts,
   if (t->n_windows) {
     FV_REQUIRE(out_starts, FV_ERR_INVALID, "null output");
     FV_TRY(fv_copy_down(out_starts, t->starts, t->n_windows * sizeof(uint64_t), t->stream));
+    fv_trainer_leaves_flight(t);  // (the stream has drained)
   }
   return FV_OK;
 }
@@ -605,7 +613,7 @@ extern "C" int fv_trainer_get_window_starts(fv_trainer *t, uint64_t *out_starts,
 extern "C" int fv_trainer_get_inverse_frequency(fv_trainer *t, float *out_invf) {
   FV_REQUIRE(t && out_invf, FV_ERR_INVALID, "null argument");
   FV_REQUIRE(t->have_corpus, FV_ERR_STATE, "no corpus set");
-  FV_HIP(hipStreamSynchronize(t->stream));
+  FV_HIP(fv_trainer_drain(t));
   FV_HIP(hipMemcpy(out_invf, t->invf, t->V * sizeof(float), hipMemcpyDeviceToHost));
   return FV_OK;
 }
@@ -613,6 +621,7 @@ extern "C" int fv_trainer_get_inverse_frequency(fv_trainer *t, float *out_invf) 
 extern "C" int fv_trainer_set_weights(fv_trainer *t, const float *W) {
   FV_REQUIRE(t && W, FV_ERR_INVALID, "null argument");
   FV_TRY(fv_upload_weights(W, t->Wt, t->K, t->N, t->ldk, t->stream));
+  fv_trainer_leaves_flight(t);  // (the stream has drained)
   t->have_weights = true;
   t->top2_valid = false;  // the first single dense launch on the new matrix makes the pass for max|ds|
   return FV_OK;
@@ -655,7 +664,7 @@ extern "C" int fv_trainer_set_permutation(fv_trainer *t, const uint64_t *perm, u
     FV_REQUIRE(perm[i] < n, FV_ERR_DATA, "permutation entry %llu = %llu is not a window index",
                (unsigned long long)i, (unsigned long long)perm[i]);
   FV_TRY(fv_copy_up(t->perm, perm, n * sizeof(uint64_t), t->stream));
-  FV_HIP(hipStreamSynchronize(t->stream));  // `perm` is the caller's again
+  FV_HIP(fv_trainer_drain(t));  // `perm` is the caller's again
   t->ahead_valid = false;  // sampled in the old order
   hipLaunchKernelGGL(fv_order_starts_kernel, dim3(fv_perm_blocks(n)), dim3(256), 0, t->stream, t->perm, t->starts,
                      t->pstart, n);
@@ -670,6 +679,7 @@ extern "C" int fv_trainer_get_permutation(fv_trainer *t, uint64_t *out_perm, uin
   if (t->n_windows) {
     FV_REQUIRE(out_perm, FV_ERR_INVALID, "null output");
     FV_TRY(fv_copy_down(out_perm, t->perm, t->n_windows * sizeof(uint64_t), t->stream));
+    fv_trainer_leaves_flight(t);  // (the stream has drained)
   }
   return FV_OK;
 }
@@ -1031,6 +1041,7 @@ static int fv_enqueue_step(fv_trainer *t, uint64_t first, uint32_t n, float eps,
   else fv_launch_onepass<U, false>(d, t->onepass_blocks, smem1, t->stream);
       // no other trainer in flight: one launch that exchanges the blocks' maxima itself where it needs them; else the
       // launch twice, in the form that waits for nobody (both with this step's launch number)
+      t->dense_forms[alone ? 0 : 1]++;
       for (uint32_t phase = alone ? 0u : 1u; phase <= (alone ? 0u : 2u); ++phase) {
         d.phase = phase;
         if (t->onepass_stream) {
@@ -1126,7 +1137,7 @@ extern "C" int fv_trainer_get_second_winners(fv_trainer *t, int32_t *out_seconds
   FV_REQUIRE(t->win2 && t->last_delta != 0.0f, FV_ERR_STATE, "the last step had no anti-Hebbian term");
   FV_REQUIRE(capacity >= t->last_n, FV_ERR_INVALID, "capacity %u below the %u windows of the last step", capacity,
              t->last_n);
-  FV_HIP(hipStreamSynchronize(t->stream));
+  FV_HIP(fv_trainer_drain(t));
   FV_HIP(hipMemcpy(out_seconds, t->win2, (size_t)t->last_n * sizeof(int32_t), hipMemcpyDeviceToHost));
   return FV_OK;
 }
@@ -1164,8 +1175,7 @@ extern "C" int fv_trainer_run_epoch(fv_trainer *t, uint64_t epoch_id, uint64_t n
     }
     t->step_tag = 0;
     FV_TRY(rc);
-    FV_HIP(hipStreamSynchronize(t->stream));
-    fv_trainer_leaves_flight(t);
+    FV_HIP(fv_trainer_drain(t));
     uint32_t tag = 0;
     FV_TRY(fv_trainer_take_giveup(t, &tag));
     if (!tag) return FV_OK;
@@ -1250,10 +1260,17 @@ extern "C" int fv_trainer_get_dense_launches(fv_trainer *t, uint32_t *out_launch
 extern "C" int fv_trainer_get_dense_path_counts(fv_trainer *t, uint64_t *out_known, uint64_t *out_pass) {
   FV_REQUIRE(t && out_known && out_pass, FV_ERR_INVALID, "null argument");
   uint32_t c[2] = {0, 0};
-  FV_HIP(hipStreamSynchronize(t->stream));
+  FV_HIP(fv_trainer_drain(t));
   FV_HIP(hipMemcpy(c, t->path_count, sizeof c, hipMemcpyDeviceToHost));
   *out_known = c[0];
   *out_pass = c[1];
+  return FV_OK;
+}
+
+extern "C" int fv_trainer_get_dense_forms(fv_trainer *t, uint64_t *out_one, uint64_t *out_two) {
+  FV_REQUIRE(t && out_one && out_two, FV_ERR_INVALID, "null argument");
+  *out_one = t->dense_forms[0];
+  *out_two = t->dense_forms[1];
   return FV_OK;
 }
 
@@ -1272,7 +1289,7 @@ extern "C" int fv_trainer_get_winners(fv_trainer *t, int32_t *out_winners, uint3
   FV_REQUIRE(t && out_winners, FV_ERR_INVALID, "null argument");
   FV_REQUIRE(capacity >= t->last_n, FV_ERR_INVALID, "capacity %u < %u windows of the last step", capacity,
              t->last_n);
-  FV_HIP(hipStreamSynchronize(t->stream));
+  FV_HIP(fv_trainer_drain(t));
   if (t->last_n)
     FV_HIP(hipMemcpy(out_winners, t->win, (size_t)t->last_n * sizeof(int32_t), hipMemcpyDeviceToHost));
   return FV_OK;
@@ -1280,7 +1297,7 @@ extern "C" int fv_trainer_get_winners(fv_trainer *t, int32_t *out_winners, uint3
 
 extern "C" int fv_trainer_get_step_stats(fv_trainer *t, float *out_xx, float *out_max_abs_ds) {
   FV_REQUIRE(t, FV_ERR_INVALID, "null trainer");
-  FV_HIP(hipStreamSynchronize(t->stream));
+  FV_HIP(fv_trainer_drain(t));
   if (out_xx) FV_HIP(hipMemcpy(out_xx, t->xx, (size_t)t->K * sizeof(float), hipMemcpyDeviceToHost));
   if (out_max_abs_ds) {
     FV_HIP(hipMemcpy(out_max_abs_ds, t->scalars, sizeof(float), hipMemcpyDeviceToHost));
@@ -1299,7 +1316,7 @@ extern "C" int fv_trainer_row_norms(fv_trainer *t, uint32_t n_rows, double *out_
                      n_rows, t->norm_part);
   hipLaunchKernelGGL(fv_row_norm_kernel, dim3(n_rows), dim3(64), 0, t->stream, t->norm_part, blocks, t->norms);
   FV_HIP(hipGetLastError());
-  FV_HIP(hipStreamSynchronize(t->stream));
+  FV_HIP(fv_trainer_drain(t));
   memcpy(out_norms, t->norms, n_rows * sizeof(double));
   return FV_OK;
 }
@@ -1316,12 +1333,12 @@ extern "C" int fv_trainer_time_steps(fv_trainer *t, uint64_t first_window, uint3
   FV_HIP(hipEventCreate(&e0));
   FV_HIP(hipEventCreate(&e1));
   int rc = FV_OK;
-  FV_HIP(hipStreamSynchronize(t->stream));
+  FV_HIP(fv_trainer_drain(t));
   FV_HIP(hipEventRecord(e0, t->stream));
   for (uint32_t s = 0; s < n_steps && rc == FV_OK; ++s)
     rc = fv_enqueue_step(t, first_window + (uint64_t)s * t->B, t->B, eps, 0.0f, nullptr);
   FV_HIP(hipEventRecord(e1, t->stream));
-  FV_HIP(hipStreamSynchronize(t->stream));
+  FV_HIP(fv_trainer_drain(t));
   FV_HIP(hipEventElapsedTime(out_total_ms, e0, e1));
   (void)hipEventDestroy(e0);
   (void)hipEventDestroy(e1);
@@ -1334,7 +1351,7 @@ extern "C" int fv_trainer_time_steps(fv_trainer *t, uint64_t first_window, uint3
   for (auto &e : ev) FV_HIP(hipEventCreate(&e));
   for (uint32_t s = 0; s < n_steps && rc == FV_OK; ++s)
     rc = fv_enqueue_step(t, first_window + (uint64_t)s * t->B, t->B, eps, 0.0f, &ev[(size_t)s * per]);
-  FV_HIP(hipStreamSynchronize(t->stream));
+  FV_HIP(fv_trainer_drain(t));
   for (int k = 0; k < FV_TRAIN_KERNELS; ++k) out_kernel_ms[k] = 0.0f;
   if (rc == FV_OK) {
     for (uint32_t s = 0; s < n_steps; ++s)
@@ -1361,7 +1378,7 @@ extern "C" int fv_trainer_time_steps_graph(fv_trainer *t, uint64_t first_window,
   FV_REQUIRE(first_window + (uint64_t)n_steps * t->B <= t->n_windows, FV_ERR_INVALID,
              "%u steps of %u windows from %llu exceed the %llu available", n_steps, t->B,
              (unsigned long long)first_window, (unsigned long long)t->n_windows);
-  FV_HIP(hipStreamSynchronize(t->stream));
+  FV_HIP(fv_trainer_drain(t));
   std::vector<hipGraphExec_t> execs;
   int rc = FV_OK;
   hipError_t e = hipSuccess;
@@ -1387,7 +1404,7 @@ extern "C" int fv_trainer_time_steps_graph(fv_trainer *t, uint64_t first_window,
     e = hipEventRecord(e0, t->stream);
     for (size_t i = 0; i < execs.size() && e == hipSuccess; ++i) e = hipGraphLaunch(execs[i], t->stream);
     if (e == hipSuccess) e = hipEventRecord(e1, t->stream);
-    if (e == hipSuccess) e = hipStreamSynchronize(t->stream);
+    if (e == hipSuccess) e = fv_trainer_drain(t);
     if (e == hipSuccess) e = hipEventElapsedTime(out_total_ms, e0, e1);
   }
   for (hipGraphExec_t x : execs) (void)hipGraphExecDestroy(x);
@@ -1405,7 +1422,7 @@ extern "C" int fv_trainer_time_kernel(fv_trainer *t, uint32_t kernel_index, uint
   hipEvent_t e0, e1;
   FV_HIP(hipEventCreate(&e0));
   FV_HIP(hipEventCreate(&e1));
-  FV_HIP(hipStreamSynchronize(t->stream));
+  FV_HIP(fv_trainer_drain(t));
   int rc = fv_enqueue_step(t, t->last_first, t->last_n, t->last_eps, t->last_delta, nullptr, 1u << kernel_index);  // warm-up
   FV_HIP(hipEventRecord(e0, t->stream));
   for (uint32_t r = 0; r < reps && rc == FV_OK; ++r)
@@ -1414,8 +1431,7 @@ extern "C" int fv_trainer_time_kernel(fv_trainer *t, uint32_t kernel_index, uint
   // the repeated winner launches have counted every window many times: once more from cleared buffers
   if (kernel_index == 0 && rc == FV_OK)
     rc = fv_enqueue_step(t, t->last_first, t->last_n, t->last_eps, t->last_delta, nullptr, 1u);
-  FV_HIP(hipStreamSynchronize(t->stream));
-  fv_trainer_leaves_flight(t);
+  FV_HIP(fv_trainer_drain(t));
   float ms = 0.0f;
   FV_HIP(hipEventElapsedTime(&ms, e0, e1));
   *out_mean_ms = ms / (float)reps;

@@ -100,6 +100,7 @@ struct fv_trainer {
   float last_eps;
   uint64_t shuffle_calls;
   bool have_corpus, have_weights;
+  uint64_t dense_forms[2];  // single dense launches enqueued as one launch, as two that wait for nobody
   bool in_flight;  // steps have been enqueued since the stream was last known to have drained
   unsigned dense_blocks;   // blocks of the absmax launch
   unsigned update_blocks;  // blocks of the dense update launch

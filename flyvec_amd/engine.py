@@ -223,6 +223,13 @@ class Trainer:
         check(self.lib.fv_trainer_get_dense_path_counts(self.handle, C.byref(known), C.byref(made)))
         return known.value, made.value
 
+    @property
+    def dense_form_counts(self):
+        """(steps enqueued with one dense launch, steps enqueued with the two that wait for nobody)."""
+        one, two = C.c_uint64(0), C.c_uint64(0)
+        check(self.lib.fv_trainer_get_dense_forms(self.handle, C.byref(one), C.byref(two)))
+        return one.value, two.value
+
     def _set_wait_limit(self, rounds):
         check(self.lib.fv_trainer_set_wait_limit(self.handle, int(rounds)))
 

@@ -221,9 +221,11 @@ int fv_trainer_get_giveups_recovered(fv_trainer *t, uint64_t *out_count);
  * there is none), 3 for its streaming form whatever the matrix size, 2 for separate launches (maximum, update,
  * sparse elements), 0 returns to the choice made at creation. Results are bit-identical in all forms. Where the
  * single launch has to make the pass for max|ds| its blocks exchange their maxima inside the launch and need the
- * whole device for themselves; a step that finds steps of another trainer of the process in flight (enqueued and
- * not yet waited for) therefore enqueues the launch twice in a form that waits for nobody: the first does the whole step when max|ds| is known beforehand (the
- * usual case) and the second ends at once, else the first makes the pass and the second the update. */
+ * whole device for themselves; a step that finds steps of another trainer of the process in flight (enqueued, and
+ * no call on that trainer has waited for its stream since: sync, run_epoch and destroy do, and every call that
+ * returns something of the device's or sets weights, corpus or order) therefore enqueues the launch twice in a form
+ * that waits for nobody: the first does the whole step when max|ds| is known beforehand (the usual case) and the
+ * second ends at once, else the first makes the pass and the second the update. */
 int fv_trainer_set_dense_launches(fv_trainer *t, uint32_t launches);
 /* The single launch carries the two largest |W| of every row from step to step; from them and from what
  * the sparse-element launch reports it usually knows max|ds| (flyvec/src/cu_special_reduction.cu:241) before
@@ -231,6 +233,10 @@ int fv_trainer_set_dense_launches(fv_trainer *t, uint32_t launches);
  * maximum first, on registers. Counts of single launches so far that knew it / that made the pass (the
  * first step on a new matrix always makes it). Same results either way. No counterpart in the reference. */
 int fv_trainer_get_dense_path_counts(fv_trainer *t, uint64_t *out_known, uint64_t *out_pass);
+/* How many of the trainer's steps have been enqueued with the dense part as one launch, and as the two launches that
+ * wait for nobody (above; neither counts a step in separate launches). Reads host counters, waits for nothing. No
+ * counterpart in the reference. */
+int fv_trainer_get_dense_forms(fv_trainer *t, uint64_t *out_one, uint64_t *out_two);
 /* The form the next step takes: 1 = the single launch (after fv_trainer_set_dense_launches(1) or (3), its
  * register or its streaming form, as the matrix size and that call decide), 2 = separate launches. */
 int fv_trainer_get_dense_launches(fv_trainer *t, uint32_t *out_launches);

@@ -504,6 +504,45 @@ def test_steps_while_another_trainer_is_in_flight(gpu, oracle_lib, launches):
     other.close()
 
 
+WAITING_CALLS = {
+    "sync": lambda t, w, c: t.sync(), "winners": lambda t, w, c: t.winners(16), "step_stats": lambda t, w, c: t.step_stats(),
+    "second_winners": lambda t, w, c: t.second_winners(16), "row_norms": lambda t, w, c: t.row_norms(3),
+    "dense_path_counts": lambda t, w, c: t.dense_path_counts, "get_weights": lambda t, w, c: t.get_weights(),
+    "set_weights": lambda t, w, c: t.set_weights(w), "set_corpus": lambda t, w, c: t.set_corpus(*c),
+    "get_permutation": lambda t, w, c: t.get_permutation(), "window_starts": lambda t, w, c: t.window_starts(),
+    "set_permutation": lambda t, w, c: t.set_permutation(np.arange(t.num_windows, dtype=np.uint64)),
+    "inverse_frequency": lambda t, w, c: t.inverse_frequency(), "run_epoch": lambda t, w, c: t.run_epoch(0, 2),
+    "time_steps": lambda t, w, c: t.time_steps(0, 2, 1e-4), "close": lambda t, w, c: t.close()}
+
+
+@pytest.mark.parametrize("call", sorted(WAITING_CALLS))
+def test_whatever_waits_for_a_trainers_steps_takes_it_out_of_flight(gpu, call):
+    """A step beside another trainer's enqueued steps is enqueued as the two dense launches that wait for nobody, and
+    as one launch again once any call on that trainer has waited for its stream."""
+    from flyvec_amd import Trainer, synthetic
+    V, K, w, B = 300, 16, 7, 16
+    corpus = small_corpus(4000, V)
+    pair = []
+    for seed in (1, 2):
+        t = Trainer(V, K, w, B)
+        t.set_corpus(*corpus)
+        t.set_weights(synthetic.synapses(K, V, seed=seed))
+        pair.append(t)
+    t, other = pair
+    assert t.dense_launches == 1 and t.dense_form_counts == (0, 0)
+    other.step(0, B, 1e-4, 0.1)
+    t.step(0, B, 1e-4)
+    assert t.dense_form_counts == (0, 1)
+    other.shuffle(3)                                # waits for nothing
+    t.step(B, B, 1e-4)
+    assert t.dense_form_counts == (0, 2)
+    WAITING_CALLS[call](other, synthetic.synapses(K, V, seed=3), corpus)
+    t.step(2 * B, B, 1e-4)
+    assert t.dense_form_counts == (1, 2)
+    t.close()
+    other.close()
+
+
 @pytest.mark.parametrize("K,V", [(1, 1), (17, 3), (64, 505), (130, 2049), (400, 1)])
 def test_row_norms_and_page_locked_checkpoints(gpu, K, V):
     """Row norms over fewer and more columns than a turn of the launch's blocks takes, for numbers of rows around the

@@ -32,8 +32,9 @@ def gpu():
 
 @pytest.fixture(autouse=True)
 def _no_trainer_left_over():
-    """A trainer that an earlier test left to the garbage collector (inside an exception's traceback, say)
-    still counts as alive in the library, and a second live trainer switches the single dense launch off."""
+    """A trainer that an earlier test left to the garbage collector (inside an exception's traceback, say) with steps
+    that nobody has waited for still counts as in flight, and every other trainer's steps take the form of the dense
+    launch that waits for nobody."""
     import gc
     gc.collect()
     yield

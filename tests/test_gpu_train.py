@@ -388,10 +388,10 @@ def test_steps_in_any_order_and_across_order_changes(gpu, oracle_lib, launches):
 
 def test_two_trainers_side_by_side(gpu, oracle_lib):
     """Where the single dense launch has to make the pass for max|ds| its blocks exchange their maxima inside the
-    launch and want every compute unit, so while a process holds two trainers a step enqueues the launch twice in
-    the form that waits for nobody (steps of both are enqueued without a synchronisation in between here). Both
-    trainers, the first steps on a new matrix (the pass) and the later ones (max|ds| known) included, train to the
-    checker's bits; alone again, a trainer returns to the one launch."""
+    launch and want every compute unit, so a step that finds another trainer's steps in flight enqueues the launch
+    twice in the form that waits for nobody (steps of both are enqueued without a synchronisation in between here).
+    Both trainers, the first steps on a new matrix (the pass) and the later ones (max|ds| known) included, train to
+    the checker's bits; with the other one gone, a trainer returns to the one launch."""
     from flyvec_amd import synthetic
     to = oracle_lib
     V, K, w, B = 300, 64, 7, 128
@@ -405,6 +405,8 @@ def test_two_trainers_side_by_side(gpu, oracle_lib):
     for s in range(6):
         a.step(s * B, B, 1e-3)
         b.step(s * B, B, 1e-3)
+    # a's first step found nobody, all others the other trainer's steps
+    assert a.dense_form_counts == (1, 5) and b.dense_form_counts == (0, 6)
     b.sync()
     known, made = b.dense_path_counts
     assert known + made == 6 and made >= 1 and known >= 3
@@ -418,17 +420,18 @@ def test_two_trainers_side_by_side(gpu, oracle_lib):
     Wo = Wa.copy()
     to.train_steps(Wo, tokens, starts, perm_a, 0, B, 9, w, invf, 1e-3)
     assert np.array_equal(a.get_weights(), Wo)
-    assert sum(a.dense_path_counts) == 9
+    assert sum(a.dense_path_counts) == 9 and a.dense_form_counts == (4, 5)
     a.close()
 
 
+@pytest.mark.parametrize("delta", [0.0, 0.3])
 @pytest.mark.parametrize("launches", [1, 3])
-def test_second_trainer_alive_while_the_pass_for_the_maximum_is_needed(gpu, oracle_lib, launches):
-    """The form of the single dense launch that waits for nobody (a second trainer exists in the process), on
+def test_second_trainer_alive_while_the_pass_for_the_maximum_is_needed(gpu, oracle_lib, launches, delta):
+    """The form of the single dense launch that waits for nobody (another trainer's step is in flight all the time), on
     weights whose largest entries sit on the most frequent tokens: nearly every step has to make the pass for
     max|ds|, which the first of the two launches then makes and the second follows with the update. Step by
-    step against the checker, in the register and in the streaming form, run_epoch's partial last minibatch
-    included."""
+    step against the checker, in the register and in the streaming form, with and without the anti-Hebbian term,
+    run_epoch's partial last minibatch included."""
     from flyvec_amd import Trainer, synthetic
     to = oracle_lib
     V, K, w, B = 800, 96, 9, 2000
@@ -438,29 +441,35 @@ def test_second_trainer_alive_while_the_pass_for_the_maximum_is_needed(gpu, orac
     hot = np.argsort(-np.bincount(tokens[tokens >= 0], minlength=V))[:6]
     planted = synthetic.synapses(K, V, seed=9)
     planted[:, hot[:3]] = np.float32(7.0)
-    other = Trainer(50, 8, 3, 16)                    # idle, but alive
-    t = Trainer(V, K, w, B, initial_learning_rate=1e-3)
+    other = Trainer(V, 8, w, 16)
+    other.set_corpus(tokens, offsets)
+    other.set_weights(synthetic.synapses(8, V, seed=1))
+    t = Trainer(V, K, w, B, initial_learning_rate=1e-3, delta=delta)
     t.set_dense_launches(launches)
     t.set_corpus(tokens, offsets)
     t.set_permutation(perm)
     t.set_weights(planted)
     assert t.dense_launches == 1
+    other.step(0, 16, 1e-4)                          # in flight until somebody waits for it
     Wo = planted.copy()
     for s in range(8):
-        t.step(s * B, B, 1e-3)
-        ref = to.train_step(Wo, to.inflate(tokens, starts, perm, s * B, B, w, V), invf, 1e-3)
+        t.step(s * B, B, 1e-3, delta)
+        ref = to.train_step(Wo, to.inflate(tokens, starts, perm, s * B, B, w, V), invf, 1e-3, delta=delta)
         xx, nc = t.step_stats()
         assert np.array_equal(t.winners(B), ref["winners"]) and np.array_equal(xx, ref["xx"]), s
         assert nc == ref["nc"], s
     assert np.array_equal(t.get_weights().view(np.uint32), Wo.view(np.uint32))
     known, made = t.dense_path_counts
     assert known + made == 8 and made >= 4
+    assert t.dense_form_counts == (0, 8)
     t.set_weights(planted)
     t.run_epoch(3, 15)
     Wo = planted.copy()
-    to.train_steps(Wo, tokens, starts, perm, 0, B, len(starts) // B + 1, w, invf, to.epoch_eps(1e-3, 3, 15))
+    steps = len(starts) // B + 1
+    to.train_steps(Wo, tokens, starts, perm, 0, B, steps, w, invf, to.epoch_eps(1e-3, 3, 15),
+                   delta=t.epoch_delta(3, 15))
     assert len(starts) % B != 0 and np.array_equal(t.get_weights().view(np.uint32), Wo.view(np.uint32))
-    assert t.giveups_recovered == 0
+    assert t.dense_form_counts == (0, 8 + steps) and t.giveups_recovered == 0
     t.close()
     other.close()
 
@@ -500,6 +509,7 @@ def test_steps_while_another_trainer_is_in_flight(gpu, oracle_lib, launches):
         t.sync()                                     # out of flight: the next step of `other` may be the only one
     assert np.array_equal(t.get_weights().view(np.uint32), Wo.view(np.uint32))
     assert sum(t.dense_path_counts) == 9 and t.dense_path_counts[1] >= 4
+    assert t.dense_form_counts == (3, 6)             # two of every three steps beside the other's
     t.close()
     other.close()
 

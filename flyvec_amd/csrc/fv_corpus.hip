@@ -14,11 +14,9 @@
 
 #include "fv_internal.h"
 #include "fv_histogram.h"
+#include "fv_window_scan.h"
 
 #define FV_MAXLEN 214ull  // flyvec/src/prune_input.cpp:7
-#define FV_SCAN_THREADS 256
-#define FV_SCAN_ITEMS 8
-#define FV_SCAN_TILE (FV_SCAN_THREADS * FV_SCAN_ITEMS)
 
 __device__ __forceinline__ uint64_t fv_chunk_windows(const uint64_t *__restrict__ off, uint64_t s,
                                                      uint64_t n_chunks, uint64_t w) {
@@ -80,14 +78,13 @@ __global__ __launch_bounds__(FV_SCAN_THREADS) void fv_scan_totals_kernel(uint64_
 // neighbouring threads neighbouring starts, each thread finding a start's chunk by a search in the scan. (A block per tile whose
 // threads wrote their own eight chunks' starts, one 8-byte store per chunk and turn, took 59 us for 2.6 M windows of
 // 160000 chunks: 78 blocks, every store a line of its own; so it takes 19.)
-#define FV_SCAN_PARTS 8u
 __global__ __launch_bounds__(FV_SCAN_THREADS) void fv_expand_starts_kernel(
     const uint64_t *__restrict__ off, uint64_t n_chunks, uint64_t w,
     const uint64_t *__restrict__ tile_base, uint64_t *__restrict__ starts, uint64_t n_windows) {
   __shared__ uint32_t part[FV_SCAN_THREADS];
   __shared__ uint32_t before[FV_SCAN_TILE];  // windows of the tile in front of each chunk (a tile has fewer than 2^19)
   __shared__ uint64_t first[FV_SCAN_TILE];   // corpus position of each chunk
-  const uint64_t tile = blockIdx.x / FV_SCAN_PARTS;
+  const uint64_t tile = blockIdx.x;
   const uint32_t tid = threadIdx.x, own = tid * FV_SCAN_ITEMS;
   const uint64_t base = tile * FV_SCAN_TILE + own;
   const uint64_t off0 = off[0];
@@ -115,7 +112,7 @@ __global__ __launch_bounds__(FV_SCAN_THREADS) void fv_expand_starts_kernel(
     at += cnt[j];
   }
   __syncthreads();
-  const uint32_t p = blockIdx.x % FV_SCAN_PARTS;
+  const uint32_t p = blockIdx.y;
   const uint32_t lo = (uint32_t)((uint64_t)total * p / FV_SCAN_PARTS), hi = (uint32_t)((uint64_t)total * (p + 1) / FV_SCAN_PARTS);
   const uint64_t out0 = tile_base[tile];
   for (uint32_t i = lo + tid; i < hi; i += FV_SCAN_THREADS) {
@@ -130,14 +127,16 @@ __global__ __launch_bounds__(FV_SCAN_THREADS) void fv_expand_starts_kernel(
 
 static int fv_scan_windows(const uint64_t *offsets_dev, uint64_t n_chunks, uint64_t w,
                            uint64_t **out_tile_base, uint64_t *out_total, hipStream_t stream) {
-  const uint64_t n_tiles = (n_chunks + FV_SCAN_TILE - 1) / FV_SCAN_TILE;
-  FV_REQUIRE(n_tiles < (1ull << 31) / FV_SCAN_PARTS, FV_ERR_INVALID, "too many chunks (%llu)",
+  const uint64_t n_tiles = fv_scan_tiles(n_chunks);
+  FV_REQUIRE(n_tiles <= FV_SCAN_MAX_TILES, FV_ERR_INVALID, "too many chunks (%llu)",
              (unsigned long long)n_chunks);
   uint64_t *totals = nullptr;
   FV_HIP(hipMalloc((void **)&totals, (n_tiles + 1) * sizeof(uint64_t)));
-  if (n_tiles)
-    hipLaunchKernelGGL(fv_tile_totals_kernel, dim3((unsigned)n_tiles), dim3(FV_SCAN_THREADS), 0,
+  if (n_tiles) {
+    const fv_scan_grid grid = fv_scan_totals_grid(n_tiles);
+    hipLaunchKernelGGL(fv_tile_totals_kernel, dim3(grid.x, grid.y), dim3(FV_SCAN_THREADS), 0,
                        stream, offsets_dev, n_chunks, w, totals);
+  }
   hipLaunchKernelGGL(fv_scan_totals_kernel, dim3(1), dim3(FV_SCAN_THREADS), 0, stream, totals,
                      n_tiles);
   hipError_t e = hipGetLastError();
@@ -170,8 +169,8 @@ int fv_dev_build_window_starts(const uint64_t *offsets_dev, uint64_t n_chunks, u
     rc = fv_fail(FV_ERR_INVALID, "window table capacity %llu does not match the %llu windows found",
                  (unsigned long long)n_windows, (unsigned long long)total);
   } else if (n_chunks) {
-    const uint64_t n_tiles = (n_chunks + FV_SCAN_TILE - 1) / FV_SCAN_TILE;
-    hipLaunchKernelGGL(fv_expand_starts_kernel, dim3((unsigned)n_tiles * FV_SCAN_PARTS), dim3(FV_SCAN_THREADS), 0,
+    const fv_scan_grid grid = fv_scan_expand_grid(fv_scan_tiles(n_chunks));
+    hipLaunchKernelGGL(fv_expand_starts_kernel, dim3(grid.x, grid.y), dim3(FV_SCAN_THREADS), 0,
                        stream, offsets_dev, n_chunks, w, tile_base, starts_dev, n_windows);
     hipError_t e = hipGetLastError();
     if (e == hipSuccess) e = hipStreamSynchronize(stream);

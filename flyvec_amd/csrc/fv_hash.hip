@@ -29,6 +29,8 @@
 // kernel, copies out and host copies then overlap also for batches that fit one chunk.
 #define FV_HASH_CHUNKS 8
 #define FV_HASH_CHUNK_MIN_BYTES ((uint64_t)3 << 19)
+// Results of this size and more, for pageable memory, are worth the host threads.
+#define FV_HASH_CREW_BYTES ((uint64_t)4 << 20)
 // Batches whose indices and codes take no more than this go through one page-locked buffer that the kernel itself
 // reads and writes: a launch and a wait, where two copies and their waits took 30 us of 44.
 #define FV_HASH_DIRECT_BYTES ((uint64_t)1 << 18)
@@ -361,7 +363,7 @@ static int fv_hash_host(fv_hasher *h, const int32_t *idx, uint64_t n, uint32_t w
     return fv_hash_direct(h, idx, n, w, k, shift, out_bits, out_codes);
   // Small chunks and the host threads where results of some size go to memory that the device cannot reach by DMA; the
   // indices then take the same way. Else the runtime's copies, in as few pieces as the lanes' buffers allow.
-  const bool crew = n * out_row >= FV_STAGE_MIN_BYTES && ((out_bits && fv_is_pageable(out_bits)) ||
+  const bool crew = n * out_row >= FV_HASH_CREW_BYTES && ((out_bits && fv_is_pageable(out_bits)) ||
                                                           (out_codes && fv_is_pageable(out_codes)));
   uint64_t chunk = FV_HASH_CHUNK;
   if (crew) {
@@ -393,7 +395,7 @@ static int fv_hash_host(fv_hasher *h, const int32_t *idx, uint64_t n, uint32_t w
   }
   const uint64_t n_chunks = (n + chunk - 1) / chunk;
   std::unique_ptr<fv_copy_ring> ring;
-  if (stage_bits || stage_codes) ring.reset(new fv_copy_ring(3 * n_chunks, crew));
+  if (stage_bits || stage_codes) ring.reset(new fv_copy_ring(3 * n_chunks));
   std::vector<uint32_t> last_item(n_chunks, 0xffffffffu);  // the last copy item of every chunk
   int rc = FV_OK;
   // chunk c's staged outputs are handed to the host threads once its copies have landed (one iteration later,

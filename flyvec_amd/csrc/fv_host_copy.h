@@ -13,15 +13,10 @@
 #include <thread>
 #include <vector>
 
+#include "fv_host_plan.h"
 #include "fv_internal.h"
 
 #define FV_COPY_THREADS 4
-#define FV_STAGE_SLOT_BYTES ((size_t)4 << 20)
-#define FV_STAGE_SLOTS_MAX 8    // of the process: 32 MB
-#define FV_STAGE_SLOTS_LEASED 4 // by one transfer
-// From here on a transfer is worth the threads: four of them start and end in about 100 us, in which the runtime moves
-// more than 1 MB (a corpus of 1.2 MB set up on a new trainer: 810 us with them, 680 without).
-#define FV_STAGE_MIN_BYTES ((size_t)4 << 20)
 
 // Ordinary (pageable) host memory, which the device cannot reach by DMA? (fv_runtime.hip)
 bool fv_is_pageable(const void *p);
@@ -42,11 +37,11 @@ struct fv_copy_ring {
   std::vector<std::thread> workers;
   uint32_t crew = 0;  // threads that started (none: publish copies by itself)
 
-  fv_copy_ring(size_t max_items, bool threads) : items(max_items), finished(new std::atomic<uint32_t>[max_items]) {
+  explicit fv_copy_ring(size_t max_items) : items(max_items), finished(new std::atomic<uint32_t>[max_items]) {
     for (size_t i = 0; i < max_items; ++i) finished[i].store(0);
     std::atomic<uint32_t> *go = &started;
     try {
-      for (uint32_t p = 0; threads && p < FV_COPY_THREADS; ++p) {
+      for (uint32_t p = 0; p < FV_COPY_THREADS; ++p) {
         workers.emplace_back([this, p, go] {
           while (go->load(std::memory_order_acquire) == 0) std::this_thread::yield();
           run(p);
@@ -105,10 +100,10 @@ struct fv_stage_lease {
   fv_stage_lease &operator=(const fv_stage_lease &) = delete;
 };
 
-// Host memory -> device, `bytes` in n_pieces: piece(t, slot) says what to copy into the slot, consume(t, slot) enqueues the device's
+// Host memory -> device in n_pieces: piece(t, slot) says what to copy into the slot, consume(t, slot) enqueues the device's
 // reading of it on `stream`. Returns when everything has been enqueued and the slots have been read.
 template <typename Piece, typename Consume>
-int fv_pipe_up(uint64_t n_pieces, size_t bytes, hipStream_t stream, Piece piece, Consume consume) {
+int fv_pipe_up(uint64_t n_pieces, hipStream_t stream, Piece piece, Consume consume) {
   fv_stage_lease lease((unsigned)(n_pieces < FV_STAGE_SLOTS_LEASED ? n_pieces : FV_STAGE_SLOTS_LEASED));
   FV_TRY(lease.rc);
   const uint64_t S = lease.slots.size();
@@ -119,7 +114,7 @@ int fv_pipe_up(uint64_t n_pieces, size_t bytes, hipStream_t stream, Piece piece,
     FV_HIP(hipStreamSynchronize(stream));
     return FV_OK;
   }
-  fv_copy_ring ring(n_pieces, bytes >= FV_STAGE_MIN_BYTES);
+  fv_copy_ring ring(n_pieces);
   int rc = FV_OK;
   for (uint64_t t = 0; t < n_pieces + S - 1 && rc == FV_OK; ++t) {
     if (t < n_pieces) {
@@ -141,10 +136,10 @@ int fv_pipe_up(uint64_t n_pieces, size_t bytes, hipStream_t stream, Piece piece,
   return rc;
 }
 
-// Device -> host memory, `bytes` in n_pieces: produce(t, slot) enqueues the device's writing of the slot on `stream`, piece(t, slot)
+// Device -> host memory in n_pieces: produce(t, slot) enqueues the device's writing of the slot on `stream`, piece(t, slot)
 // says where its contents go. Returns when the host memory holds everything.
 template <typename Produce, typename Piece>
-int fv_pipe_down(uint64_t n_pieces, size_t bytes, hipStream_t stream, Produce produce, Piece piece) {
+int fv_pipe_down(uint64_t n_pieces, hipStream_t stream, Produce produce, Piece piece) {
   fv_stage_lease lease((unsigned)(n_pieces < FV_STAGE_SLOTS_LEASED ? n_pieces : FV_STAGE_SLOTS_LEASED));
   FV_TRY(lease.rc);
   const uint64_t S = lease.slots.size();
@@ -155,7 +150,7 @@ int fv_pipe_down(uint64_t n_pieces, size_t bytes, hipStream_t stream, Produce pr
     fv_copy_ring::copy_share(it, 0, 1);
     return FV_OK;
   }
-  fv_copy_ring ring(n_pieces, bytes >= FV_STAGE_MIN_BYTES);
+  fv_copy_ring ring(n_pieces);
   const uint64_t ahead = S > 1 ? S - 1 : 1;  // pieces the device may be ahead of the host threads by
   int rc = FV_OK;
   for (uint64_t t = 0; t < n_pieces + ahead && rc == FV_OK; ++t) {
@@ -176,7 +171,7 @@ int fv_pipe_down(uint64_t n_pieces, size_t bytes, hipStream_t stream, Produce pr
   return rc;
 }
 
-// Plain copies. Page-locked memory and small sizes go through the runtime. Upwards the caller waits for the stream before
+// Plain copies. Page-locked memory and sizes below fv_host_plan.h's go through the runtime. Upwards the caller waits for the stream before
 // its own caller may change the source; downwards the host memory is filled on return.
 int fv_copy_up(void *dst_dev, const void *src_host, size_t bytes, hipStream_t stream);
 int fv_copy_down(void *dst_host, const void *src_dev, size_t bytes, hipStream_t stream);

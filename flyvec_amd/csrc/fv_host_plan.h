@@ -1,0 +1,88 @@
+// Which way a transfer between the device and ordinary (pageable) host memory goes, and in which pieces: the rules and
+// the arithmetic of fv_host_copy.h, shared with the CPU test-suite. Plain C.
+//
+// The other way is the runtime's copy of such memory, for a matrix with a staging matrix on the device. Both sides
+// measured with pauses and new arrays between the calls, as set-up calls come (microseconds, runtime against slots; two
+// runs each; back to back the slots do a little better):
+//   upload    8 MB 486-490, 782-876;  16 MB 966-969, 1022-1197;  24 MB 1572-1587, 1515-1659;  32 MB 2053-2124,
+//             1863-1872;  64 MB 4120, 3680: the runtime reads the caller's pages at 17 GB/s, four threads at little more
+//   download  8 MB 478-492, 477-509;  12 MB 698-748, 702-718 (both in pieces of 512 KB);  16 MB 927-946, 497 (whole
+//             slots);  64 MB 6300, 1950 (the result's pages are touched for the first time, by four threads)
+//   matrix up, K = 400: 6 MB 314-337, 314-335, with the hasher around it 368-412, 415-496;  8 MB 376-411, 346-381 and
+//             426-471, 432-521;  12 MB 519-530, 442-456 and 558-611, 535-562;  64 MB 2430, 1680 and 2500, 1900.  In one
+//             piece: 0.25 MB 52, 50;  1 MB 70-81, 77;  4 MB 232-254, 228
+//   matrix down, K = 400: 8 MB 539-560, 320-347;  12 MB 800, 415;  64 MB 6550, 2700.  In one piece: 0.25 MB 56, 47;
+//             1 MB 82-87, 81;  4 MB 324-330, 210
+// A matrix that fits a slot goes as one piece, moved by the calling thread: cut into tiles of 64 rows, as the larger ones
+// are, 1 MB at K = 400 took 235 us, and page-locked four slots for it.
+#pragma once
+
+#include <stddef.h>
+#include <stdint.h>
+
+#define FV_STAGE_SLOT_BYTES ((size_t)4 << 20)
+#define FV_STAGE_SLOTS_MAX 8    /* of the process: 32 MB */
+#define FV_STAGE_SLOTS_LEASED 4 /* by one transfer */
+#define FV_STAGE_TILE_ROWS 64u  /* of a matrix that goes in several pieces */
+
+#define FV_STAGE_UP_BYTES ((size_t)32 << 20)        /* plain uploads through the slots from here on */
+#define FV_STAGE_DOWN_BYTES ((size_t)16 << 20)      /* plain downloads */
+#define FV_STAGE_MATRIX_UP_BYTES ((size_t)8 << 20)  /* matrices upwards, and those that fit one slot; downwards all */
+
+static inline int fv_upload_staged(size_t bytes) { return bytes >= FV_STAGE_UP_BYTES; }
+static inline int fv_download_staged(size_t bytes) { return bytes >= FV_STAGE_DOWN_BYTES; }
+static inline int fv_matrix_upload_staged(size_t bytes) {
+  return bytes <= FV_STAGE_SLOT_BYTES || bytes >= FV_STAGE_MATRIX_UP_BYTES;
+}
+
+/* Pieces of a plain copy: whole slots and a rest. */
+static inline uint64_t fv_copy_pieces(size_t bytes) { return (bytes + FV_STAGE_SLOT_BYTES - 1) / FV_STAGE_SLOT_BYTES; }
+static inline size_t fv_copy_piece_bytes(size_t bytes, uint64_t t) {
+  const size_t left = bytes - (size_t)t * FV_STAGE_SLOT_BYTES;
+  return left < FV_STAGE_SLOT_BYTES ? left : FV_STAGE_SLOT_BYTES;
+}
+
+/* Pieces of a K x N row-major matrix of floats: the whole of it as it lies in memory if it fits a slot, else tiles of
+ * FV_STAGE_TILE_ROWS rows by as many columns as a slot holds. Piece t: `rows` rows from row `h`, `cols` columns from
+ * column `i`, rows of `pitch` floats in the slot. */
+typedef struct fv_matrix_pieces {
+  uint32_t K;
+  uint64_t N, columns, across, n;
+} fv_matrix_pieces;
+
+typedef struct fv_matrix_piece {
+  uint32_t h, rows;
+  uint64_t i, cols, pitch;
+} fv_matrix_piece;
+
+static inline fv_matrix_pieces fv_cut_matrix(uint32_t K, uint64_t N) {
+  fv_matrix_pieces p;
+  p.K = K;
+  p.N = N;
+  if (N <= FV_STAGE_SLOT_BYTES / sizeof(float) / K) {
+    p.columns = N;
+    p.across = p.n = 1;
+  } else {
+    p.columns = FV_STAGE_SLOT_BYTES / (FV_STAGE_TILE_ROWS * sizeof(float));
+    p.across = (N + p.columns - 1) / p.columns;
+    p.n = p.across * ((K + FV_STAGE_TILE_ROWS - 1) / FV_STAGE_TILE_ROWS);
+  }
+  return p;
+}
+
+static inline fv_matrix_piece fv_matrix_piece_at(const fv_matrix_pieces *p, uint64_t t) {
+  fv_matrix_piece m;
+  if (p->n == 1) {
+    m.h = 0;
+    m.rows = p->K;
+    m.i = 0;
+    m.cols = m.pitch = p->N;
+    return m;
+  }
+  m.h = (uint32_t)(t / p->across) * FV_STAGE_TILE_ROWS;
+  m.rows = p->K - m.h < FV_STAGE_TILE_ROWS ? p->K - m.h : FV_STAGE_TILE_ROWS;
+  m.i = t % p->across * p->columns;
+  m.cols = p->N - m.i < p->columns ? p->N - m.i : p->columns;
+  m.pitch = (m.cols + FV_STAGE_TILE_ROWS - 1) / FV_STAGE_TILE_ROWS * FV_STAGE_TILE_ROWS;
+  return m;
+}

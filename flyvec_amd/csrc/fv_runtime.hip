@@ -195,7 +195,7 @@ bool fv_is_pageable(const void *p) {
 }
 
 // The process's page-locked slots: made when first needed, up to FV_STAGE_SLOTS_MAX, kept for the transfers that follow
-// (page-locking 4 MB takes as long as moving 20) until fv_host_staging_release.
+// (page-locking 4 MB takes 0.1 to 0.8 ms) until fv_host_staging_release.
 static std::mutex fv_stage_mutex;
 static std::condition_variable fv_stage_returned;
 static std::vector<char *> fv_stage_idle;
@@ -244,6 +244,13 @@ fv_stage_lease::~fv_stage_lease() {
   fv_stage_returned.notify_all();
 }
 
+extern "C" int fv_host_staging_held(size_t *out_bytes) {
+  FV_REQUIRE(out_bytes, FV_ERR_INVALID, "null argument");
+  std::lock_guard<std::mutex> lock(fv_stage_mutex);
+  *out_bytes = fv_stage_made * FV_STAGE_SLOT_BYTES;
+  return FV_OK;
+}
+
 extern "C" int fv_host_staging_release(void) {
   std::lock_guard<std::mutex> lock(fv_stage_mutex);
   for (char *p : fv_stage_idle) (void)hipHostFree(p);
@@ -252,86 +259,77 @@ extern "C" int fv_host_staging_release(void) {
   return FV_OK;
 }
 
-static bool fv_stages(const void *host, size_t bytes) {
-  // both ends: the range may begin or end inside page-locked memory of the caller's
-  return bytes >= FV_STAGE_MIN_BYTES && fv_is_pageable(host) && fv_is_pageable((const char *)host + bytes - 1);
+// Both ends: the range may begin or end inside page-locked memory of the caller's.
+static bool fv_pageable_range(const void *host, size_t bytes) {
+  return fv_is_pageable(host) && fv_is_pageable((const char *)host + bytes - 1);
 }
 
 int fv_copy_up(void *dst_dev, const void *src_host, size_t bytes, hipStream_t stream) {
   if (bytes == 0) return FV_OK;
-  if (!fv_stages(src_host, bytes)) {
+  if (!fv_upload_staged(bytes) || !fv_pageable_range(src_host, bytes)) {
     FV_HIP(hipMemcpyAsync(dst_dev, src_host, bytes, hipMemcpyHostToDevice, stream));
     return FV_OK;
   }
-  const size_t slot = bytes >= 4 * FV_STAGE_SLOT_BYTES ? FV_STAGE_SLOT_BYTES : FV_STAGE_SLOT_BYTES / 8;
-  const auto length = [&](uint64_t t) { return bytes - t * slot < slot ? bytes - t * slot : slot; };
   return fv_pipe_up(
-      (bytes + slot - 1) / slot, bytes, stream,
+      fv_copy_pieces(bytes), stream,
       [&](uint64_t t, char *p) {
-        return fv_copy_ring::item{(const char *)src_host + t * slot, p, length(t), 0, 0, 1};
+        return fv_copy_ring::item{(const char *)src_host + t * FV_STAGE_SLOT_BYTES, p, fv_copy_piece_bytes(bytes, t), 0, 0, 1};
       },
       [&](uint64_t t, char *p) -> int {
-        FV_HIP(hipMemcpyAsync((char *)dst_dev + t * slot, p, length(t), hipMemcpyHostToDevice, stream));
+        FV_HIP(hipMemcpyAsync((char *)dst_dev + t * FV_STAGE_SLOT_BYTES, p, fv_copy_piece_bytes(bytes, t),
+                              hipMemcpyHostToDevice, stream));
         return FV_OK;
       });
 }
 
 int fv_copy_down(void *dst_host, const void *src_dev, size_t bytes, hipStream_t stream) {
   if (bytes == 0) return FV_OK;
-  if (!fv_stages(dst_host, bytes)) {
+  if (!fv_download_staged(bytes) || !fv_pageable_range(dst_host, bytes)) {
     FV_HIP(hipMemcpyAsync(dst_host, src_dev, bytes, hipMemcpyDeviceToHost, stream));
     FV_HIP(hipStreamSynchronize(stream));
     return FV_OK;
   }
-  const size_t slot = bytes >= 4 * FV_STAGE_SLOT_BYTES ? FV_STAGE_SLOT_BYTES : FV_STAGE_SLOT_BYTES / 8;
-  const auto length = [&](uint64_t t) { return bytes - t * slot < slot ? bytes - t * slot : slot; };
   return fv_pipe_down(
-      (bytes + slot - 1) / slot, bytes, stream,
+      fv_copy_pieces(bytes), stream,
       [&](uint64_t t, char *p) -> int {
-        FV_HIP(hipMemcpyAsync(p, (const char *)src_dev + t * slot, length(t), hipMemcpyDeviceToHost, stream));
+        FV_HIP(hipMemcpyAsync(p, (const char *)src_dev + t * FV_STAGE_SLOT_BYTES, fv_copy_piece_bytes(bytes, t),
+                              hipMemcpyDeviceToHost, stream));
         return FV_OK;
       },
-      [&](uint64_t t, char *p) { return fv_copy_ring::item{p, (char *)dst_host + t * slot, length(t), 0, 0, 1}; });
+      [&](uint64_t t, char *p) {
+        return fv_copy_ring::item{p, (char *)dst_host + t * FV_STAGE_SLOT_BYTES, fv_copy_piece_bytes(bytes, t), 0, 0, 1};
+      });
 }
 
-// A K x N host matrix goes through the slots in tiles of FV_TT rows by as many columns as a slot holds; the layout
-// change reads and writes the slots over the link. Tile t: rows from h, columns from i.
-struct fv_weight_tiles {
-  uint32_t K;
-  uint64_t N, columns, across, n;
-  fv_weight_tiles(uint32_t K_, uint64_t N_) : K(K_), N(N_) {
-    columns = FV_STAGE_SLOT_BYTES / (FV_TT * sizeof(float));
-    across = (N + columns - 1) / columns;
-    n = across * ((K + FV_TT - 1) / FV_TT);
-  }
-  uint32_t h(uint64_t t) const { return (uint32_t)(t / across) * FV_TT; }
-  uint64_t i(uint64_t t) const { return t % across * columns; }
-  uint32_t rows(uint64_t t) const { return K - h(t) < FV_TT ? K - h(t) : FV_TT; }
-  uint64_t cols(uint64_t t) const { return N - i(t) < columns ? N - i(t) : columns; }
-  uint64_t pitch(uint64_t t) const { return (cols(t) + FV_TT - 1) / FV_TT * FV_TT; }  // of the slot's rows
-};
+// One piece of a matrix between the caller's memory (rows of N floats) and a slot (rows of m.pitch floats). Row by row
+// also where the rows touch: one memcpy of 4 MB goes past the caches (232 us for an upload, 195 by rows).
+static fv_copy_ring::item fv_matrix_item(const fv_matrix_piece &m, uint64_t N, const float *from, float *to, bool up) {
+  const size_t row = m.cols * sizeof(float), caller = N * sizeof(float), slot = m.pitch * sizeof(float);
+  return {(const char *)from, (char *)to, row, up ? caller : slot, up ? slot : caller, m.rows};
+}
 
-// Page-locked matrices are read and written in place by the layout change, and pageable ones through page-locked slots:
-// there is no staging matrix on the device, whose allocation and release (which waits for the device) cost more than
-// the copy of a small matrix, and no second pass over it. Memory of any other kind takes the runtime's copies.
+// Page-locked matrices are read and written in place by the layout change, and pageable ones of the sizes that
+// fv_host_plan.h names through page-locked slots: there is no staging matrix on the device, whose allocation and release
+// (which waits for the device) cost more than the copy of a small matrix, and no second pass over it. The others, and
+// memory of any other kind, take the runtime's copies.
 int fv_upload_weights(const float *W_host, float *Wt_dev, uint32_t K, uint64_t N, uint32_t ldk,
                       hipStream_t stream) {
   const size_t bytes = (size_t)K * N * sizeof(float);
   int rc = FV_OK;
   if (const float *view = (const float *)fv_device_view(W_host, bytes)) {
     rc = fv_launch_to_token_major(view, N, Wt_dev, K, N, ldk, ldk, stream);
-  } else if (fv_is_pageable(W_host) && fv_is_pageable((const char *)W_host + bytes - 1)) {
-    const fv_weight_tiles tiles(K, N);
+  } else if (fv_matrix_upload_staged(bytes) && fv_pageable_range(W_host, bytes)) {
+    const fv_matrix_pieces pieces = fv_cut_matrix(K, N);
     return fv_pipe_up(
-        tiles.n, bytes, stream,
+        pieces.n, stream,
         [&](uint64_t t, char *p) {
-          return fv_copy_ring::item{(const char *)(W_host + tiles.h(t) * N + tiles.i(t)), p, tiles.cols(t) * sizeof(float),
-                                    N * sizeof(float), tiles.pitch(t) * sizeof(float), tiles.rows(t)};
+          const fv_matrix_piece m = fv_matrix_piece_at(&pieces, t);
+          return fv_matrix_item(m, N, W_host + m.h * N + m.i, (float *)p, true);
         },
         [&](uint64_t t, char *p) {
-          const uint32_t h = tiles.h(t), rows = tiles.rows(t);
-          return fv_launch_to_token_major((const float *)p, tiles.pitch(t), Wt_dev + tiles.i(t) * ldk + h, rows,
-                                          tiles.cols(t), ldk, h + rows == K ? ldk - h : rows, stream);
+          const fv_matrix_piece m = fv_matrix_piece_at(&pieces, t);
+          return fv_launch_to_token_major((const float *)p, m.pitch, Wt_dev + m.i * ldk + m.h, m.rows, m.cols, ldk,
+                                          m.h + m.rows == K ? ldk - m.h : m.rows, stream);
         });
   } else {
     float *stage = nullptr;
@@ -353,17 +351,17 @@ int fv_download_weights(const float *Wt_dev, float *W_host, uint32_t K, uint64_t
   int rc = FV_OK;
   if (float *view = (float *)fv_device_view(W_host, bytes)) {
     rc = fv_launch_to_row_major(Wt_dev, view, N, K, N, ldk, stream);
-  } else if (fv_is_pageable(W_host) && fv_is_pageable((const char *)W_host + bytes - 1)) {
-    const fv_weight_tiles tiles(K, N);
+  } else if (fv_pageable_range(W_host, bytes)) {
+    const fv_matrix_pieces pieces = fv_cut_matrix(K, N);
     return fv_pipe_down(
-        tiles.n, bytes, stream,
+        pieces.n, stream,
         [&](uint64_t t, char *p) {
-          return fv_launch_to_row_major(Wt_dev + tiles.i(t) * ldk + tiles.h(t), (float *)p, tiles.pitch(t), tiles.rows(t),
-                                        tiles.cols(t), ldk, stream);
+          const fv_matrix_piece m = fv_matrix_piece_at(&pieces, t);
+          return fv_launch_to_row_major(Wt_dev + m.i * ldk + m.h, (float *)p, m.pitch, m.rows, m.cols, ldk, stream);
         },
         [&](uint64_t t, char *p) {
-          return fv_copy_ring::item{p, (char *)(W_host + tiles.h(t) * N + tiles.i(t)), tiles.cols(t) * sizeof(float),
-                                    tiles.pitch(t) * sizeof(float), N * sizeof(float), tiles.rows(t)};
+          const fv_matrix_piece m = fv_matrix_piece_at(&pieces, t);
+          return fv_matrix_item(m, N, (const float *)p, W_host + m.h * N + m.i, false);
         });
   } else {
     float *stage = nullptr;

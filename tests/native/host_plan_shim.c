@@ -1,0 +1,19 @@
+/* Host build of flyvec_amd/csrc/fv_host_plan.h for the CPU test-suite. */
+#include "fv_host_plan.h"
+
+uint64_t fvt_slot_bytes(void) { return FV_STAGE_SLOT_BYTES; }
+int fvt_upload_staged(uint64_t bytes) { return fv_upload_staged(bytes); }
+int fvt_download_staged(uint64_t bytes) { return fv_download_staged(bytes); }
+int fvt_matrix_upload_staged(uint64_t bytes) { return fv_matrix_upload_staged(bytes); }
+uint64_t fvt_copy_pieces(uint64_t bytes) { return fv_copy_pieces(bytes); }
+uint64_t fvt_copy_piece_bytes(uint64_t bytes, uint64_t t) { return fv_copy_piece_bytes(bytes, t); }
+uint64_t fvt_matrix_pieces(uint32_t K, uint64_t N) { return fv_cut_matrix(K, N).n; }
+void fvt_matrix_piece(uint32_t K, uint64_t N, uint64_t t, uint64_t *out) {
+  const fv_matrix_pieces p = fv_cut_matrix(K, N);
+  const fv_matrix_piece m = fv_matrix_piece_at(&p, t);
+  out[0] = m.h;
+  out[1] = m.rows;
+  out[2] = m.i;
+  out[3] = m.cols;
+  out[4] = m.pitch;
+}

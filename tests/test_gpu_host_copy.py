@@ -12,10 +12,11 @@ SLOT_COLUMNS = 16384  # columns of a 64-row tile that fills a slot of 4 MB
 
 
 @pytest.mark.parametrize("K,N", [(1, 2), (64, 2 * SLOT_COLUMNS), (65, 2 * SLOT_COLUMNS + 2), (63, SLOT_COLUMNS - 2),
-                                 (130, 5 * SLOT_COLUMNS + 6), (400, 2)])
+                                 (130, 5 * SLOT_COLUMNS + 6), (400, 2), (64, SLOT_COLUMNS), (64, SLOT_COLUMNS + 2),
+                                 (2048, 512), (2047, 514), (400, 5242), (400, 5244)])
 def test_matrices_through_the_slots(gpu, K, N):
-    """Upload and download at tile edges (rows beside 64, columns beside a slot's), pageable and page-locked on either
-    side; the pad columns of the device's rows are zero again after a larger matrix's upload has been read."""
+    """Upload and download at tile edges (rows beside 64, columns beside a slot's), beside the largest matrix that goes
+    in one piece (4 MB) and the smallest that goes up in tiles (8 MB), pageable and page-locked on either side; the pad columns of the device's rows are zero again after a larger matrix's upload has been read."""
     from flyvec_amd import Hasher, Trainer, _lib
     W = np.random.default_rng(K).standard_normal((K, N), dtype=np.float32)
     locked = _lib.pinned_empty(W.shape, np.float32)
@@ -34,10 +35,11 @@ def test_matrices_through_the_slots(gpu, K, N):
     assert _lib.load().fv_host_staging_release() == 0
 
 
-@pytest.mark.parametrize("n", [1, (1 << 18) - 1, 1 << 18, (1 << 19) + 5, (1 << 22) + 3])
+@pytest.mark.parametrize("n", [1, (1 << 18) - 1, 1 << 18, (1 << 19) + 5, (1 << 21) - 1, 1 << 21, (1 << 21) + 1,
+                               (1 << 22) - 1, 1 << 22, (1 << 22) + 3])
 def test_orders_through_the_slots(gpu, n):
-    """Window tables and orders of n 64-bit entries: below and above the size from which pieces are taken, whole and
-    broken last pieces of either length."""
+    """Window tables and orders of n 64-bit entries: beside the sizes from which pieces are taken (16 MB downwards, 32 MB
+    upwards), whole and broken last pieces."""
     from flyvec_amd import Trainer
     rng = np.random.default_rng(n)
     tokens = rng.integers(0, 50, size=1000, dtype=np.int32)
@@ -49,6 +51,40 @@ def test_orders_through_the_slots(gpu, n):
     t.set_permutation(perm)
     assert np.array_equal(t.get_permutation(), perm)
     t.close()
+
+
+def held():
+    import ctypes as C
+    from flyvec_amd import _lib
+    out = C.c_size_t(0)
+    _lib.check(_lib.load().fv_host_staging_held(C.byref(out)))
+    return out.value
+
+
+def test_what_transfers_page_lock(gpu):
+    """Small and middling transfers page-lock one slot at most (a matrix of 3 MB took four, so did a corpus of 8 MB);
+    large ones keep four for those that follow, until they are given back."""
+    from flyvec_amd import Trainer, _lib
+    slot = 4 << 20
+    assert _lib.load().fv_host_staging_release() == 0 and held() == 0
+    rng = np.random.default_rng(0)
+    t = Trainer(50, 8, 5, 16)
+    t.set_corpus(rng.integers(0, 50, 2 << 20).astype(np.int32), np.arange(0, (2 << 20) + 1, 64, dtype=np.uint64))
+    t.set_permutation(rng.permutation(t.num_windows).astype(np.uint64))
+    t.get_permutation()
+    t.close()
+    assert held() == 0
+    t = Trainer(937, 400, 5, 16)
+    W = rng.standard_normal((400, 2 * 937), dtype=np.float32)
+    t.set_weights(W)
+    assert held() == slot and np.array_equal(t.get_weights(), W) and held() == slot
+    t.close()
+    t = Trainer(4000, 400, 5, 16)
+    W = rng.standard_normal((400, 2 * 4000), dtype=np.float32)
+    t.set_weights(W)
+    assert held() == 4 * slot and np.array_equal(t.get_weights(), W) and held() == 4 * slot
+    t.close()
+    assert _lib.load().fv_host_staging_release() == 0 and held() == 0
 
 
 def test_more_transfers_at_once_than_there_are_slots(gpu):

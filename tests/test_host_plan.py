@@ -1,0 +1,63 @@
+"""flyvec_amd/csrc/fv_host_plan.h on the host: which transfers go through the page-locked slots, and that their pieces
+cover what they carry once, each inside a slot."""
+import ctypes as C
+import os
+import subprocess
+
+import numpy as np
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+MB = 1 << 20
+
+
+@pytest.fixture(scope="module")
+def shim(tmp_path_factory):
+    out = tmp_path_factory.mktemp("host_plan") / "libplan.so"
+    subprocess.run(["gcc", "-O2", "-shared", "-fPIC", "-I", os.path.join(ROOT, "flyvec_amd", "csrc"),
+                    os.path.join(ROOT, "tests", "native", "host_plan_shim.c"), "-o", str(out)], check=True)
+    lib = C.CDLL(str(out))
+    u64, u32 = C.c_uint64, C.c_uint32
+    for name, args in (("fvt_slot_bytes", []), ("fvt_copy_pieces", [u64]), ("fvt_copy_piece_bytes", [u64, u64]),
+                       ("fvt_matrix_pieces", [u32, u64])):
+        getattr(lib, name).restype = u64
+        getattr(lib, name).argtypes = args
+    for name in ("fvt_upload_staged", "fvt_download_staged", "fvt_matrix_upload_staged"):
+        getattr(lib, name).argtypes = [u64]
+    lib.fvt_matrix_piece.argtypes = [u32, u64, u64, C.POINTER(u64)]
+    return lib
+
+
+def test_small_and_middling_transfers_stay_with_the_runtime(shim):
+    """Where the slots were measured to be no faster: uploads below 32 MB, downloads below 16 MB, matrices between one
+    slot and 8 MB upwards."""
+    for up, down, matrix, size in ((0, 0, 1, 1), (0, 0, 1, 4 * MB), (0, 0, 0, 4 * MB + 4), (0, 0, 0, 8 * MB - 4),
+                                   (0, 0, 1, 8 * MB), (0, 0, 1, 16 * MB - 1), (0, 1, 1, 16 * MB), (0, 1, 1, 32 * MB - 1),
+                                   (1, 1, 1, 32 * MB), (1, 1, 1, 1 << 40)):
+        got = shim.fvt_upload_staged(size), shim.fvt_download_staged(size), shim.fvt_matrix_upload_staged(size)
+        assert tuple(map(bool, got)) == (bool(up), bool(down), bool(matrix)), size
+
+
+@pytest.mark.parametrize("size", [16 * MB, 16 * MB + 1, 20 * MB - 1, 33 * MB + 24])
+def test_pieces_of_a_plain_copy(shim, size):
+    n = shim.fvt_copy_pieces(size)
+    sizes = [shim.fvt_copy_piece_bytes(size, t) for t in range(n)]
+    assert sum(sizes) == size and min(sizes) > 0 and max(sizes) <= shim.fvt_slot_bytes()
+    assert all(s == shim.fvt_slot_bytes() for s in sizes[:-1])
+
+
+@pytest.mark.parametrize("K,N", [(1, 2), (2048, 2), (400, 1874), (400, 2620), (400, 2622), (64, 16384), (64, 16386),
+                                 (63, 16644), (63, 16646), (65, 16130), (65, 32770), (2048, 512), (2048, 514),
+                                 (130, 81926), (1, 1048576), (1, 1048578)])
+def test_pieces_of_a_matrix_cover_it_once(shim, K, N):
+    seen = np.zeros((K, N), np.uint8)
+    n = shim.fvt_matrix_pieces(K, N)
+    assert (n == 1) == (K * N * 4 <= shim.fvt_slot_bytes())  # what fits a slot goes in one piece
+    m = (C.c_uint64 * 5)()
+    for t in range(n):
+        shim.fvt_matrix_piece(K, N, t, m)
+        h, rows, i, cols, pitch = m
+        assert rows and cols and h + rows <= K and i + cols <= N and pitch >= cols
+        assert ((rows - 1) * pitch + cols) * 4 <= shim.fvt_slot_bytes()
+        seen[h:h + rows, i:i + cols] += 1
+    assert (seen == 1).all()

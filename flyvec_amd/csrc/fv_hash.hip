@@ -24,16 +24,6 @@
 // chunk's copies run while the other's kernel does: per stream a device buffer for the chunk's indices and
 // one for each kind of output, kept from call to call (grown when a call needs more).
 #define FV_HASH_LANES 2
-#define FV_HASH_CHUNK (1u << 17)  // most windows per chunk
-// A batch is cut into about this many chunks, of output that takes the link some 30 us or more: one call's copies in,
-// kernel, copies out and host copies then overlap also for batches that fit one chunk.
-#define FV_HASH_CHUNKS 8
-#define FV_HASH_CHUNK_MIN_BYTES ((uint64_t)3 << 19)
-// Results of this size and more, for pageable memory, are worth the host threads.
-#define FV_HASH_CREW_BYTES ((uint64_t)4 << 20)
-// Batches whose indices and codes take no more than this go through one page-locked buffer that the kernel itself
-// reads and writes: a launch and a wait, where two copies and their waits took 30 us of 44.
-#define FV_HASH_DIRECT_BYTES ((uint64_t)1 << 18)
 
 struct fv_hash_lane {
   hipStream_t stream;
@@ -358,23 +348,13 @@ static int fv_hash_host(fv_hasher *h, const int32_t *idx, uint64_t n, uint32_t w
   FV_REQUIRE(idx, FV_ERR_INVALID, "null index buffer");
   const uint32_t words = (h->K + 63) / 64;
   const size_t bits_row = words * sizeof(uint64_t), codes_row = h->K;
-  const uint64_t out_row = (out_bits ? bits_row : 0) + (out_codes ? codes_row : 0);
-  if (n <= FV_HASH_DIRECT_BYTES && n * (w * sizeof(int32_t) + out_row) <= FV_HASH_DIRECT_BYTES)
-    return fv_hash_direct(h, idx, n, w, k, shift, out_bits, out_codes);
-  // Small chunks and the host threads where results of some size go to memory that the device cannot reach by DMA; the
-  // indices then take the same way. Else the runtime's copies, in as few pieces as the lanes' buffers allow.
-  const bool crew = n * out_row >= FV_HASH_CREW_BYTES && ((out_bits && fv_is_pageable(out_bits)) ||
-                                                          (out_codes && fv_is_pageable(out_codes)));
-  uint64_t chunk = FV_HASH_CHUNK;
-  if (crew) {
-    const uint64_t share = (n + FV_HASH_CHUNKS - 1) / FV_HASH_CHUNKS, least = FV_HASH_CHUNK_MIN_BYTES / out_row + 1;
-    chunk = share > least ? share : least;
-    chunk = chunk < FV_HASH_CHUNK ? chunk : FV_HASH_CHUNK;
-  }
-  chunk = chunk < n ? chunk : n;
+  const uint64_t want_bits = out_bits ? bits_row : 0, want_codes = out_codes ? codes_row : 0;
+  if (fv_hash_is_direct(n, w, want_bits + want_codes)) return fv_hash_direct(h, idx, n, w, k, shift, out_bits, out_codes);
+  const bool bits_pageable = out_bits && fv_is_pageable(out_bits), codes_pageable = out_codes && fv_is_pageable(out_codes);
+  const fv_hash_plan plan = fv_plan_hash(n, want_bits, want_codes, bits_pageable, codes_pageable);
+  const uint64_t chunk = plan.chunk;
   const int lanes = n > chunk ? FV_HASH_LANES : 1;
-  const bool stage_bits = crew && out_bits && lanes > 1 && fv_is_pageable(out_bits);
-  const bool stage_codes = crew && out_codes && lanes > 1 && fv_is_pageable(out_codes);
+  const bool stage_bits = plan.crew && bits_pageable && lanes > 1, stage_codes = plan.crew && codes_pageable && lanes > 1;
   const bool stage_idx = (stage_bits || stage_codes) && fv_is_pageable(idx);
   FV_HIP(hipStreamSynchronize(h->stream));  // what the caller enqueued on the hasher's stream comes first
   for (int l = 0; l < lanes; ++l) {

@@ -86,3 +86,44 @@ static inline fv_matrix_piece fv_matrix_piece_at(const fv_matrix_pieces *p, uint
   m.pitch = (m.cols + FV_STAGE_TILE_ROWS - 1) / FV_STAGE_TILE_ROWS * FV_STAGE_TILE_ROWS;
   return m;
 }
+
+/* ---- batches of codes from host arrays ---- */
+
+#define FV_HASH_CHUNK (1u << 17) /* most windows per chunk */
+/* A batch is cut into about this many chunks, of output that takes the link some 30 us or more: one call's copies in,
+ * kernel, copies out and host copies then overlap also for batches that fit one chunk. */
+#define FV_HASH_CHUNKS 8
+#define FV_HASH_CHUNK_MIN_BYTES ((uint64_t)3 << 19)
+/* Results of this size and more, for pageable memory, are worth the host threads. */
+#define FV_HASH_CREW_BYTES ((uint64_t)4 << 20)
+/* Batches whose indices and codes take no more than this go through one page-locked buffer that the kernel itself
+ * reads and writes: a launch and a wait, where two copies and their waits took 30 us of 44. */
+#define FV_HASH_DIRECT_BYTES ((uint64_t)1 << 18)
+
+static inline int fv_hash_is_direct(uint64_t n, uint32_t w, uint64_t out_row) {
+  return n <= FV_HASH_DIRECT_BYTES && n * (w * sizeof(int32_t) + out_row) <= FV_HASH_DIRECT_BYTES;
+}
+
+typedef struct fv_hash_plan {
+  int crew;       /* host threads and page-locked staging */
+  uint64_t chunk; /* windows per chunk */
+} fv_hash_plan;
+
+/* The other batches. n windows; bits_row, codes_row: bytes of a window's packed and plain codes, 0 where not asked for.
+ * Host threads where results for pageable memory are large, or come in more than FV_HASH_CHUNK windows: there the
+ * chunks overlap on two streams, and the runtime's copies of pageable memory, which the host waits for, would take
+ * that away (500000 windows to 4 MB of packed codes: 835 us, 1230 with the runtime's copies; 200000 to 3 MB: 580, 640). */
+static inline fv_hash_plan fv_plan_hash(uint64_t n, uint64_t bits_row, uint64_t codes_row, int bits_pageable,
+                                        int codes_pageable) {
+  fv_hash_plan p = {0, FV_HASH_CHUNK};
+  const uint64_t out_row = bits_row + codes_row;
+  p.crew = ((bits_row && bits_pageable) || (codes_row && codes_pageable)) &&
+           (n > FV_HASH_CHUNK || n * out_row >= FV_HASH_CREW_BYTES);
+  if (p.crew) {
+    const uint64_t share = (n + FV_HASH_CHUNKS - 1) / FV_HASH_CHUNKS, least = FV_HASH_CHUNK_MIN_BYTES / out_row + 1;
+    const uint64_t want = share > least ? share : least;
+    p.chunk = want < FV_HASH_CHUNK ? want : FV_HASH_CHUNK;
+  }
+  if (p.chunk > n) p.chunk = n;
+  return p;
+}

@@ -17,3 +17,10 @@ void fvt_matrix_piece(uint32_t K, uint64_t N, uint64_t t, uint64_t *out) {
   out[3] = m.cols;
   out[4] = m.pitch;
 }
+void fvt_plan_hash(uint64_t n, uint32_t w, uint64_t bits_row, uint64_t codes_row, int bits_pageable, int codes_pageable,
+                   uint64_t *out) {
+  const fv_hash_plan p = fv_plan_hash(n, bits_row, codes_row, bits_pageable, codes_pageable);
+  out[0] = (uint64_t)fv_hash_is_direct(n, w, bits_row + codes_row);
+  out[1] = !out[0] && p.crew;
+  out[2] = p.chunk;
+}

@@ -24,6 +24,7 @@ def shim(tmp_path_factory):
         getattr(lib, name).argtypes = args
     for name in ("fvt_upload_staged", "fvt_download_staged", "fvt_matrix_upload_staged"):
         getattr(lib, name).argtypes = [u64]
+    lib.fvt_plan_hash.argtypes = [u64, u32, u64, u64, C.c_int, C.c_int, C.POINTER(u64)]
     lib.fvt_matrix_piece.argtypes = [u32, u64, u64, C.POINTER(u64)]
     return lib
 
@@ -61,3 +62,43 @@ def test_pieces_of_a_matrix_cover_it_once(shim, K, N):
         assert ((rows - 1) * pitch + cols) * 4 <= shim.fvt_slot_bytes()
         seen[h:h + rows, i:i + cols] += 1
     assert (seen == 1).all()
+
+
+def plan(shim, n, w, K, bits=False, codes=False, pageable=True):
+    out = (C.c_uint64 * 3)()
+    shim.fvt_plan_hash(n, w, -(-K // 64) * 8 if bits else 0, K if codes else 0, pageable, pageable, out)
+    return bool(out[0]), bool(out[1]), out[2]
+
+
+@pytest.mark.parametrize("K,w,bits,codes,largest", [(400, 1, False, True, 648), (400, 1, True, True, 569), (70, 11, False, True, 2299),
+                                                    (70, 11, True, True, 2016), (2, 1, True, False, 21845), (2048, 64, True, True, 102)])
+def test_largest_batch_of_the_one_buffer(shim, K, w, bits, codes, largest):
+    """2^18 bytes of indices and codes."""
+    for pageable in (True, False):
+        assert plan(shim, largest, w, K, bits, codes, pageable) == (True, False, largest)
+        assert plan(shim, largest + 1, w, K, bits, codes, pageable) == (False, False, largest + 1)
+
+
+def test_batches_that_get_host_threads(shim):
+    """Large results for ordinary memory, and any of more windows than a chunk: two streams' chunks overlap only if the
+    host does not wait for each copy. Page-locked arrays need neither."""
+    chunk = 1 << 17
+    for n, K, kw in ((200000, 64, dict(bits=True)), (500000, 64, dict(bits=True)), (chunk + 1, 2, dict(bits=True)),
+                     (200000, 20, dict(codes=True)), (10486, 400, dict(codes=True)), (1 << 20, 400, dict(bits=True, codes=True))):
+        direct, crew, size = plan(shim, n, 11, K, **kw)
+        assert not direct and crew and 0 < size <= chunk and size < n, (n, K)
+        assert plan(shim, n, 11, K, pageable=False, **kw) == (False, False, min(n, chunk))
+    for n, K, kw in ((chunk, 64, dict(bits=True)), (10485, 400, dict(codes=True)), (50000, 400, dict(bits=True)),
+                     (1 << 20, 400, {})):
+        assert plan(shim, n, 11, K, **kw) == (False, False, min(n, chunk)), (n, K)
+
+
+@pytest.mark.parametrize("K,w,bits,codes", [(400, 1, False, True), (400, 11, True, False), (1000, 15, True, True), (2, 1, True, False),
+                                            (2048, 64, False, True)])
+def test_chunks_of_a_batch(shim, K, w, bits, codes):
+    row = (-(-K // 64) * 8 if bits else 0) + (K if codes else 0)
+    for n in (1, 655, 10486, 20000, (1 << 17) - 1, 1 << 17, (1 << 17) + 1, 1 << 20, 10_000_019):
+        direct, crew, size = plan(shim, n, w, K, bits, codes)
+        assert 1 <= size <= min(n, 1 << 17)
+        if crew:
+            assert size * row >= 3 << 19 or size == 1 << 17  # a chunk is worth its launch and its copies

@@ -20,23 +20,6 @@
 
 #include "fv_host_copy.h"
 
-// Host-buffer batches go through the device in chunks on two streams of equal priority, so that one
-// chunk's copies run while the other's kernel does: per stream a device buffer for the chunk's indices and
-// one for each kind of output, kept from call to call (grown when a call needs more).
-#define FV_HASH_LANES 2
-
-struct fv_hash_lane {
-  hipStream_t stream;
-  int32_t *idx;
-  uint64_t *bits;
-  int8_t *codes;
-  size_t idx_cap, bits_cap, codes_cap;  // bytes
-  // page-locked staging for indices and outputs in pageable host memory, and the event behind a chunk's copies
-  char *stage_idx, *stage_bits, *stage_codes;
-  size_t stage_idx_cap, stage_bits_cap, stage_codes_cap;
-  hipEvent_t done;
-};
-
 struct fv_hasher {
   uint32_t K, ldk;
   uint64_t N;
@@ -45,7 +28,13 @@ struct fv_hasher {
   uint32_t *err;  // flag in page-locked memory: a column index outside [-1, N) was met
   char *direct;   // behind it, FV_HASH_DIRECT_BYTES for small batches
   unsigned max_blocks;
-  fv_hash_lane lane[FV_HASH_LANES];  // lane 0 runs on `stream`
+  // Host-buffer batches go through the device in chunks, FV_HASH_LANES of them in flight: device memory for the chunks'
+  // indices and codes, kept from call to call (made anew when a call needs more), and an event per lane behind its
+  // chunk's copies.
+  char *work;
+  size_t work_cap;
+  bool batches_in_chunks;  // there has been one
+  hipEvent_t done[FV_HASH_LANES];
 };
 
 struct fv_hash_args {
@@ -209,20 +198,9 @@ static int fv_check_hash_args(fv_hasher *h, uint32_t w, uint32_t k) {
 extern "C" int fv_hasher_destroy(fv_hasher *h) {
   if (!h) return FV_OK;
   if (h->stream) (void)hipStreamSynchronize(h->stream);
-  for (int l = 0; l < FV_HASH_LANES; ++l) {
-    fv_hash_lane &ln = h->lane[l];
-    if (ln.stream && ln.stream != h->stream) {
-      (void)hipStreamSynchronize(ln.stream);
-      (void)hipStreamDestroy(ln.stream);
-    }
-    (void)hipFree(ln.idx);
-    (void)hipFree(ln.bits);
-    (void)hipFree(ln.codes);
-    if (ln.stage_idx) (void)hipHostFree(ln.stage_idx);
-    if (ln.stage_bits) (void)hipHostFree(ln.stage_bits);
-    if (ln.stage_codes) (void)hipHostFree(ln.stage_codes);
-    if (ln.done) (void)hipEventDestroy(ln.done);
-  }
+  (void)hipFree(h->work);
+  for (hipEvent_t done : h->done)
+    if (done) (void)hipEventDestroy(done);
   (void)hipFree(h->Wt);
   if (h->err) (void)hipHostFree(h->err);
   if (h->stream) (void)hipStreamDestroy(h->stream);
@@ -295,28 +273,6 @@ extern "C" int fv_hash_windows_dev(fv_hasher *h, const int32_t *idx_dev, uint64_
   return fv_enqueue_hash(h, idx_dev, n, w, k, 0, out_bits_dev, out_codes_dev);
 }
 
-// Makes a lane's buffer hold at least `bytes` (freed and allocated anew when it does not).
-template <typename P>
-static int fv_hash_reserve(P **buf, size_t *cap, size_t bytes) {
-  if (*cap >= bytes) return FV_OK;
-  (void)hipFree(*buf);
-  *buf = nullptr;
-  *cap = 0;
-  FV_HIP(hipMalloc((void **)buf, bytes));
-  *cap = bytes;
-  return FV_OK;
-}
-
-static int fv_hash_reserve_pinned(char **buf, size_t *cap, size_t bytes) {
-  if (*cap >= bytes) return FV_OK;
-  if (*buf) (void)hipHostFree(*buf);
-  *buf = nullptr;
-  *cap = 0;
-  FV_HIP(hipHostMalloc((void **)buf, bytes, hipHostMallocDefault));
-  *cap = bytes;
-  return FV_OK;
-}
-
 // A small batch: the kernel reads the indices from, and writes its results to, one page-locked buffer.
 static int fv_hash_direct(fv_hasher *h, const int32_t *idx, uint64_t n, uint32_t w, uint32_t k, int32_t shift,
                           uint64_t *out_bits, int8_t *out_codes) {
@@ -335,13 +291,18 @@ static int fv_hash_direct(fv_hasher *h, const int32_t *idx, uint64_t n, uint32_t
   return rc;
 }
 
-// A batch in host memory: chunks of up to FV_HASH_CHUNK windows alternate between the lanes; on its lane a
-// chunk is copied in, hashed and copied out in stream order, so the copies of one chunk overlap the kernel
-// of the other. Host buffers from fv_host_alloc_pinned are copied by DMA as they are. Outputs that go to
-// pageable memory are copied by DMA into the lane's page-locked staging and from there by host threads
-// (fv_copy_ring) while the device goes on; pageable inputs are copied into the lane's staging by the same threads.
-// Nothing is allocated once the lanes' buffers have reached the chunk size. (100003 windows, K = 400, pageable: 4.0 ms
-// as one chunk through the runtime's copies.)
+// A batch in host memory: its chunks take turns on a few lanes and two streams of equal priority; on its lane a chunk is
+// copied in, hashed and copied out in stream order, so the copies of one chunk overlap the kernel of another. Host
+// buffers from fv_host_alloc_pinned are copied by DMA as they are. Outputs that go to pageable memory are copied by DMA
+// into page-locked staging and from there by host threads (fv_copy_ring) while the device goes on; pageable inputs take
+// the staging too. (100003 windows, K = 400, pageable: 4.1 ms as one chunk through the runtime's copies, 1.44 ms so;
+// 20000 targets 500 and 340 us.) Nothing is allocated once the hasher's device memory has reached the chunks' size.
+//
+// The staging and the second stream are the process's, borrowed for the call: of the hasher's own, the first batch on
+// every hasher made a stream and page-locked some megabytes, which took longer than the batch (20000 targets on a new
+// hasher: 0.6 to 2.8 ms, 13 ms on the process's first; a table of a whole vocabulary is such a batch and is made once).
+// For the same reason a hasher's first batch does with one stream if it has no more than FV_HASH_CHUNK windows and the
+// process has no idle one (a stream takes up to 4 ms to make, and saves such a batch some 10 %).
 static int fv_hash_host(fv_hasher *h, const int32_t *idx, uint64_t n, uint32_t w, uint32_t k, int32_t shift,
                         uint64_t *out_bits, int8_t *out_codes) {
   if (n == 0) return FV_OK;
@@ -351,87 +312,99 @@ static int fv_hash_host(fv_hasher *h, const int32_t *idx, uint64_t n, uint32_t w
   const uint64_t want_bits = out_bits ? bits_row : 0, want_codes = out_codes ? codes_row : 0;
   if (fv_hash_is_direct(n, w, want_bits + want_codes)) return fv_hash_direct(h, idx, n, w, k, shift, out_bits, out_codes);
   const bool bits_pageable = out_bits && fv_is_pageable(out_bits), codes_pageable = out_codes && fv_is_pageable(out_codes);
-  const fv_hash_plan plan = fv_plan_hash(n, want_bits, want_codes, bits_pageable, codes_pageable);
-  const uint64_t chunk = plan.chunk;
-  const int lanes = n > chunk ? FV_HASH_LANES : 1;
-  const bool stage_bits = plan.crew && bits_pageable && lanes > 1, stage_codes = plan.crew && codes_pageable && lanes > 1;
-  const bool stage_idx = (stage_bits || stage_codes) && fv_is_pageable(idx);
-  FV_HIP(hipStreamSynchronize(h->stream));  // what the caller enqueued on the hasher's stream comes first
-  for (int l = 0; l < lanes; ++l) {
-    fv_hash_lane &ln = h->lane[l];
-    if (!ln.stream) {
-      if (l == 0)
-        ln.stream = h->stream;
-      else
-        FV_HIP(hipStreamCreate(&ln.stream));
-    }
-    if (!ln.done) FV_HIP(hipEventCreateWithFlags(&ln.done, hipEventDisableTiming));
-    FV_TRY(fv_hash_reserve(&ln.idx, &ln.idx_cap, chunk * w * sizeof(int32_t)));
-    if (stage_idx) FV_TRY(fv_hash_reserve_pinned(&ln.stage_idx, &ln.stage_idx_cap, chunk * w * sizeof(int32_t)));
-    if (out_bits) FV_TRY(fv_hash_reserve(&ln.bits, &ln.bits_cap, chunk * bits_row));
-    if (out_codes) FV_TRY(fv_hash_reserve(&ln.codes, &ln.codes_cap, chunk * codes_row));
-    if (stage_bits) FV_TRY(fv_hash_reserve_pinned(&ln.stage_bits, &ln.stage_bits_cap, chunk * bits_row));
-    if (stage_codes) FV_TRY(fv_hash_reserve_pinned(&ln.stage_codes, &ln.stage_codes_cap, chunk * codes_row));
+  fv_hash_plan plan = fv_plan_hash(n, want_bits, want_codes, bits_pageable, codes_pageable);
+  const bool stage_bits = plan.crew && bits_pageable, stage_codes = plan.crew && codes_pageable;
+  const bool stage_idx = plan.crew && fv_is_pageable(idx);
+  const uint64_t in_row = stage_idx ? w * sizeof(int32_t) : 0, out_row = (stage_bits ? bits_row : 0) + (stage_codes ? codes_row : 0);
+  std::unique_ptr<fv_stage_lease> lease;
+  fv_hash_staging staging = {};
+  staging.lanes = 2;  // (not staged, a chunk may take hundreds of megabytes of the device)
+  if (plan.crew) {
+    lease.reset(new fv_stage_lease(fv_hash_stage_slots(&plan, in_row, out_row)));
+    FV_TRY(lease->rc);
+    staging = fv_hash_stage(&plan, in_row, out_row, (unsigned)lease->slots.size());
   }
-  const uint64_t n_chunks = (n + chunk - 1) / chunk;
+  const uint64_t chunk = plan.chunk, n_chunks = (n + chunk - 1) / chunk;
+  const uint64_t lanes = n_chunks < (uint64_t)staging.lanes ? n_chunks : (uint64_t)staging.lanes;
+  // a lane's device memory: packed codes, indices, plain codes
+  const auto up64 = [](size_t bytes) { return (bytes + 63) & ~(size_t)63; };
+  const size_t idx_at = up64(chunk * want_bits), codes_at = idx_at + up64(chunk * w * sizeof(int32_t));
+  const size_t lane_bytes = codes_at + up64(chunk * want_codes);
+  FV_HIP(hipStreamSynchronize(h->stream));  // what the caller enqueued on the hasher's stream comes first
+  fv_stream_lease second;
+  if (lanes > 1) {
+    FV_TRY(second.take(n > FV_HASH_CHUNK || h->batches_in_chunks));
+    h->batches_in_chunks = true;
+  }
+  for (uint64_t l = 0; l < lanes; ++l)
+    if (!h->done[l]) FV_HIP(hipEventCreateWithFlags(&h->done[l], hipEventDisableTiming));
+  if (h->work_cap < lanes * lane_bytes) {
+    (void)hipFree(h->work);
+    h->work = nullptr;
+    h->work_cap = 0;
+    FV_HIP(hipMalloc((void **)&h->work, lanes * lane_bytes));
+    h->work_cap = lanes * lane_bytes;
+  }
+  const auto stage = [&](uint64_t c) { return lease->slots[staging.slot[c % lanes]] + staging.at[c % lanes]; };
+  const auto stage_in = [&](uint64_t c) { return lease->slots[staging.in_slot[c % lanes]] + staging.in_at[c % lanes]; };
+  const size_t stage_codes_at = stage_bits ? chunk * bits_row : 0;  // (behind the packed codes)
   std::unique_ptr<fv_copy_ring> ring;
-  if (stage_bits || stage_codes) ring.reset(new fv_copy_ring(3 * n_chunks));
+  if (lease) ring.reset(new fv_copy_ring(3 * n_chunks));
   std::vector<uint32_t> last_item(n_chunks, 0xffffffffu);  // the last copy item of every chunk
   int rc = FV_OK;
-  // chunk c's staged outputs are handed to the host threads once its copies have landed (one iteration later,
-  // while the device works on chunk c + 1), and have left the staging before chunk c + 2 is copied into it
+  // chunk c's staged outputs are handed to the host threads once its copies have landed (one iteration later, while the
+  // device works on chunk c + 1), and have left the staging before the lane's next chunk is copied into it
   auto hand_over = [&](uint64_t c) -> int {
-    fv_hash_lane &ln = h->lane[c % lanes];
-    FV_HIP(hipEventSynchronize(ln.done));
+    FV_HIP(hipEventSynchronize(h->done[c % lanes]));
     const uint64_t first = c * chunk, m = n - first < chunk ? n - first : chunk;
-    if (stage_bits) last_item[c] = ring->publish(ln.stage_bits, (char *)out_bits + first * bits_row, m * bits_row);
-    if (stage_codes) last_item[c] = ring->publish(ln.stage_codes, (char *)out_codes + first * codes_row, m * codes_row);
+    if (stage_bits) last_item[c] = ring->publish(stage(c), (char *)out_bits + first * bits_row, m * bits_row);
+    if (stage_codes) last_item[c] = ring->publish(stage(c) + stage_codes_at, (char *)out_codes + first * codes_row, m * codes_row);
     return FV_OK;
   };
   for (uint64_t c = 0; c < n_chunks && rc == FV_OK; ++c) {
-    fv_hash_lane &ln = h->lane[c % lanes];
+    const hipStream_t s = second.stream && (c & 1) ? second.stream : h->stream;
+    char *dev = h->work + c % lanes * lane_bytes;
     const uint64_t first = c * chunk, m = n - first < chunk ? n - first : chunk;
-    if (ring && c >= (uint64_t)lanes && last_item[c - lanes] != 0xffffffffu) ring->wait(last_item[c - lanes]);
-    const int32_t *from = idx + first * w;
-    hipError_t e = hipSuccess;
-    if (stage_idx) {
-      // the lane's chunk before this one has been copied in
-      if (c >= (uint64_t)lanes) e = hipEventSynchronize(ln.done);
-      if (e == hipSuccess) {
-        ring->wait(ring->publish((const char *)from, ln.stage_idx, m * w * sizeof(int32_t)));
-        from = (const int32_t *)ln.stage_idx;
-      }
+    if (ring && c >= lanes && last_item[c - lanes] != 0xffffffffu) ring->wait(last_item[c - lanes]);
+    const char *from = (const char *)(idx + first * w);
+    if (stage_idx) {  // (the lane's chunk before this one has been copied in: its outputs have been handed over)
+      char *to = stage_in(c);
+      if (staging.light)
+        memcpy(to, from, m * w * sizeof(int32_t));
+      else
+        ring->wait(ring->publish(from, to, m * w * sizeof(int32_t)));
+      from = to;
     }
-    if (e == hipSuccess) e = hipMemcpyAsync(ln.idx, from, m * w * sizeof(int32_t), hipMemcpyHostToDevice, ln.stream);
+    hipError_t e = hipMemcpyAsync(dev + idx_at, from, m * w * sizeof(int32_t), hipMemcpyHostToDevice, s);
     if (e != hipSuccess) {
       rc = fv_fail(FV_ERR_HIP, "hash upload failed: %s", hipGetErrorString(e));
       break;
     }
-    rc = fv_enqueue_hash(h, ln.idx, m, w, k, shift, out_bits ? ln.bits : nullptr, out_codes ? ln.codes : nullptr,
-                         ln.stream);
+    rc = fv_enqueue_hash(h, (const int32_t *)(dev + idx_at), m, w, k, shift, out_bits ? (uint64_t *)dev : nullptr,
+                         out_codes ? (int8_t *)(dev + codes_at) : nullptr, s);
     if (rc == FV_OK && out_bits) {
-      void *dst = stage_bits ? (void *)ln.stage_bits : (void *)((char *)out_bits + first * bits_row);
-      e = hipMemcpyAsync(dst, ln.bits, m * bits_row, hipMemcpyDeviceToHost, ln.stream);
+      void *dst = stage_bits ? (void *)stage(c) : (void *)((char *)out_bits + first * bits_row);
+      e = hipMemcpyAsync(dst, dev, m * bits_row, hipMemcpyDeviceToHost, s);
       if (e != hipSuccess) rc = fv_fail(FV_ERR_HIP, "download failed: %s", hipGetErrorString(e));
     }
     if (rc == FV_OK && out_codes) {
-      void *dst = stage_codes ? (void *)ln.stage_codes : (void *)((char *)out_codes + first * codes_row);
-      e = hipMemcpyAsync(dst, ln.codes, m * codes_row, hipMemcpyDeviceToHost, ln.stream);
+      void *dst = stage_codes ? (void *)(stage(c) + stage_codes_at) : (void *)((char *)out_codes + first * codes_row);
+      e = hipMemcpyAsync(dst, dev + codes_at, m * codes_row, hipMemcpyDeviceToHost, s);
       if (e != hipSuccess) rc = fv_fail(FV_ERR_HIP, "download failed: %s", hipGetErrorString(e));
     }
-    if (rc == FV_OK) {
-      e = hipEventRecord(ln.done, ln.stream);
+    if (rc == FV_OK && ring) {
+      e = hipEventRecord(h->done[c % lanes], s);
       if (e != hipSuccess) rc = fv_fail(FV_ERR_HIP, "event record failed: %s", hipGetErrorString(e));
-      if (rc == FV_OK && ring && c >= 1) rc = hand_over(c - 1);
+      if (rc == FV_OK && c >= 1) rc = hand_over(c - 1);
     }
   }
   if (rc == FV_OK && ring) rc = hand_over(n_chunks - 1);
   ring.reset();  // waits for the host threads' copies
-  for (int l = 1; l < lanes; ++l) {
-    const hipError_t e = hipStreamSynchronize(h->lane[l].stream);
+  if (second.stream) {
+    const hipError_t e = hipStreamSynchronize(second.stream);
     if (e != hipSuccess && rc == FV_OK) rc = fv_fail(FV_ERR_HIP, "hash stream failed: %s", hipGetErrorString(e));
   }
-  const int rs = fv_hasher_sync(h);  // lane 0, and the flag for indices out of range
+  const int rs = fv_hasher_sync(h);  // the first stream, and the flag for indices out of range
   return rc == FV_OK ? rs : rc;
 }
 

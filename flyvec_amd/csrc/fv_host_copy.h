@@ -100,6 +100,18 @@ struct fv_stage_lease {
   fv_stage_lease &operator=(const fv_stage_lease &) = delete;
 };
 
+// A stream of the current device, borrowed from the process's pool for the length of one call, which leaves it idle.
+// (Making a stream takes up to 4 ms while the process has few.)
+struct fv_stream_lease {
+  hipStream_t stream = nullptr;
+  int device = 0;
+  int take(bool make);  // an idle one; if there is none and `make`, a new one, else none. Once per object.
+  fv_stream_lease() = default;
+  ~fv_stream_lease();
+  fv_stream_lease(const fv_stream_lease &) = delete;
+  fv_stream_lease &operator=(const fv_stream_lease &) = delete;
+};
+
 // Host memory -> device in n_pieces: piece(t, slot) says what to copy into the slot, consume(t, slot) enqueues the device's
 // reading of it on `stream`. Returns when everything has been enqueued and the slots have been read.
 template <typename Piece, typename Consume>

@@ -90,6 +90,7 @@ static inline fv_matrix_piece fv_matrix_piece_at(const fv_matrix_pieces *p, uint
 /* ---- batches of codes from host arrays ---- */
 
 #define FV_HASH_CHUNK (1u << 17) /* most windows per chunk */
+#define FV_HASH_LANES 4          /* most chunks in flight */
 /* A batch is cut into about this many chunks, of output that takes the link some 30 us or more: one call's copies in,
  * kernel, copies out and host copies then overlap also for batches that fit one chunk. */
 #define FV_HASH_CHUNKS 8
@@ -126,4 +127,51 @@ static inline fv_hash_plan fv_plan_hash(uint64_t n, uint64_t bits_row, uint64_t 
   }
   if (p.chunk > n) p.chunk = n;
   return p;
+}
+
+/* The staging of the chunks in flight, in_row bytes of indices and out_row of codes per window (0 where not staged).
+ * Light indices (a fourth of the codes and less): four chunks in flight, each in a region of its own for both, and the
+ * calling thread copies the indices itself, so that the host threads copy codes all the time (100003 windows of 444 bytes,
+ * 40 MB of codes: 1.44 ms, with two chunks and the threads copying both 1.75; 20000 targets 340 us and 376; three chunks in
+ * flight are in between). Heavy ones: two chunks in flight, the indices in slots of their own where the chunks are large,
+ * so that they may be nearly twice as large (1 M windows of 44 and 56 bytes: 3.46 ms; in the other layout 4.03). */
+typedef struct fv_hash_staging {
+  int lanes;                      /* chunks in flight */
+  int light;                      /* the calling thread copies the indices */
+  uint32_t slot[FV_HASH_LANES];   /* that holds the lane's codes */
+  size_t at[FV_HASH_LANES];       /* where in the slot they begin */
+  uint32_t in_slot[FV_HASH_LANES];/* the same of its indices */
+  size_t in_at[FV_HASH_LANES];
+} fv_hash_staging;
+
+static inline int fv_hash_indices_light(uint64_t in_row, uint64_t out_row) { return 4 * in_row <= out_row; }
+
+/* Slots that the staging asks the pool for. */
+static inline unsigned fv_hash_stage_slots(const fv_hash_plan *p, uint64_t in_row, uint64_t out_row) {
+  const uint64_t bytes = p->chunk * (in_row + out_row) + 128;
+  if (fv_hash_indices_light(in_row, out_row)) {
+    const uint64_t want = (FV_HASH_LANES * bytes + FV_STAGE_SLOT_BYTES - 1) / FV_STAGE_SLOT_BYTES;
+    return (unsigned)(want < FV_HASH_LANES ? want : FV_HASH_LANES);
+  }
+  if (2 * bytes <= FV_STAGE_SLOT_BYTES) return 1;
+  return bytes <= FV_STAGE_SLOT_BYTES ? 2 : 4;
+}
+
+/* Where the staging lies in the `slots` (1 .. that many) that the pool gave; the chunk shrinks to what they hold. */
+static inline fv_hash_staging fv_hash_stage(fv_hash_plan *p, uint64_t in_row, uint64_t out_row, unsigned slots) {
+  fv_hash_staging s;
+  s.light = fv_hash_indices_light(in_row, out_row);
+  s.lanes = s.light ? FV_HASH_LANES : 2;
+  const int apart = !s.light && slots >= 4;
+  const unsigned per_slot = apart ? 1 : ((unsigned)s.lanes + slots - 1) / slots;
+  const size_t region = FV_STAGE_SLOT_BYTES / per_slot & ~(size_t)63;
+  const uint64_t widest = !apart ? in_row + out_row : in_row > out_row ? in_row : out_row;
+  if (p->chunk > (region - 64) / widest) p->chunk = (region - 64) / widest;
+  for (uint32_t l = 0; l < (uint32_t)s.lanes; ++l) {
+    s.slot[l] = l / per_slot;
+    s.at[l] = l % per_slot * region;
+    s.in_slot[l] = apart ? l + 2 : s.slot[l];
+    s.in_at[l] = apart ? 0 : s.at[l] + ((p->chunk * out_row + 63) & ~(size_t)63);
+  }
+  return s;
 }

@@ -244,6 +244,38 @@ fv_stage_lease::~fv_stage_lease() {
   fv_stage_returned.notify_all();
 }
 
+// Idle streams, each with its device; as many are made as calls have held at once, and kept until
+// fv_host_staging_release.
+struct fv_idle_stream {
+  int device;
+  hipStream_t stream;
+};
+static std::vector<fv_idle_stream> fv_streams_idle;
+
+int fv_stream_lease::take(bool make) {
+  FV_HIP(hipGetDevice(&device));
+  {
+    std::lock_guard<std::mutex> lock(fv_stage_mutex);
+    for (size_t i = 0; i < fv_streams_idle.size(); ++i)
+      if (fv_streams_idle[i].device == device) {
+        stream = fv_streams_idle[i].stream;
+        fv_streams_idle.erase(fv_streams_idle.begin() + (ptrdiff_t)i);
+        return FV_OK;
+      }
+  }
+  if (make) FV_HIP(hipStreamCreate(&stream));
+  return FV_OK;
+}
+
+fv_stream_lease::~fv_stream_lease() {
+  if (!stream) return;
+  std::lock_guard<std::mutex> lock(fv_stage_mutex);
+  if (fv_streams_idle.size() < FV_STAGE_SLOTS_MAX)
+    fv_streams_idle.push_back({device, stream});
+  else
+    (void)hipStreamDestroy(stream);
+}
+
 extern "C" int fv_host_staging_held(size_t *out_bytes) {
   FV_REQUIRE(out_bytes, FV_ERR_INVALID, "null argument");
   std::lock_guard<std::mutex> lock(fv_stage_mutex);
@@ -256,6 +288,8 @@ extern "C" int fv_host_staging_release(void) {
   for (char *p : fv_stage_idle) (void)hipHostFree(p);
   fv_stage_made -= (unsigned)fv_stage_idle.size();
   fv_stage_idle.clear();
+  for (const fv_idle_stream &idle : fv_streams_idle) (void)hipStreamDestroy(idle.stream);
+  fv_streams_idle.clear();
   return FV_OK;
 }
 

@@ -24,3 +24,20 @@ void fvt_plan_hash(uint64_t n, uint32_t w, uint64_t bits_row, uint64_t codes_row
   out[1] = !out[0] && p.crew;
   out[2] = p.chunk;
 }
+/* the same with the staging: slots asked for, then places where the pool gives `got` (0: as many) */
+void fvt_hash_stage(uint64_t n, uint64_t bits_row, uint64_t codes_row, uint64_t in_row, uint64_t out_row, unsigned got,
+                    uint64_t *out) {
+  fv_hash_plan p = fv_plan_hash(n, bits_row, codes_row, 1, 1);
+  const unsigned want = fv_hash_stage_slots(&p, in_row, out_row), slots = got && got < want ? got : want;
+  const fv_hash_staging s = fv_hash_stage(&p, in_row, out_row, slots);
+  out[0] = want;
+  out[1] = slots;
+  out[2] = p.chunk;
+  out[3] = (uint64_t)s.lanes;
+  for (int l = 0; l < s.lanes; ++l) {
+    out[4 + 4 * l] = s.slot[l];
+    out[5 + 4 * l] = s.at[l];
+    out[6 + 4 * l] = s.in_slot[l];
+    out[7 + 4 * l] = s.in_at[l];
+  }
+}

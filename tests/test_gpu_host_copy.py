@@ -87,6 +87,57 @@ def test_what_transfers_page_lock(gpu):
     assert _lib.load().fv_host_staging_release() == 0 and held() == 0
 
 
+@pytest.mark.parametrize("n,slots", [(30000, 2), (60000, 4)])
+def test_hash_batches_borrow_their_staging(gpu, n, slots):
+    """Batches of codes for ordinary memory on one hasher after another page-lock two slots in all (four chunks of 1.7 MB) or
+    four (of 3.2 MB); the results are the device-resident call's, on a hasher's first batch (one stream) and on later ones
+    (two), and while other threads' transfers hold slots."""
+    from flyvec_amd import Hasher, Trainer, _lib
+    K = 400
+    assert _lib.load().fv_host_staging_release() == 0
+    rng = np.random.default_rng(5)
+    W = rng.standard_normal((K, 200), dtype=np.float32)
+    idx = rng.integers(0, 200, size=(n, 7)).astype(np.int32)
+    want = None
+    for i in range(3):
+        h = Hasher(W)
+        got = h.hash_windows(idx, 20, packed=False, codes=True)
+        if want is None:
+            dev, codes = _lib.DeviceBuffer.from_numpy(idx), _lib.DeviceBuffer(n * K)
+            h.hash_windows_dev(dev, n, 7, 20, None, codes)
+            h.sync()
+            want = codes.to_numpy(np.int8, (n, K))
+        assert np.array_equal(got, want) and held() == slots * (4 << 20)
+        if i:
+            assert np.array_equal(h.hash_windows(idx, 20, packed=False, codes=True), want) and held() == slots * (4 << 20)
+        h.close()
+    bad = []
+
+    def matrices(seed):
+        V = 40000
+        M = np.random.default_rng(seed).standard_normal((130, 2 * V), dtype=np.float32)
+        t = Trainer(V, 130, 3, 16)
+        for _ in range(3):
+            t.set_weights(M)
+            if not np.array_equal(t.get_weights(), M):
+                bad.append(seed)
+        t.close()
+
+    def hashes(seed):
+        h = Hasher(W)
+        for _ in range(6):
+            if not np.array_equal(h.hash_windows(idx, 20, packed=False, codes=True), want):
+                bad.append(seed)
+        h.close()
+
+    threads = [threading.Thread(target=matrices if s % 2 else hashes, args=(s,)) for s in range(6)]
+    for th in threads:
+        th.start()
+    for th in threads:
+        th.join()
+    assert not bad
+
+
 def test_more_transfers_at_once_than_there_are_slots(gpu):
     """Six threads, each with a trainer of its own, hold up to four of eight slots each: they wait for each other's and
     all finish with their own matrix."""

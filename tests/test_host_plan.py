@@ -25,6 +25,7 @@ def shim(tmp_path_factory):
     for name in ("fvt_upload_staged", "fvt_download_staged", "fvt_matrix_upload_staged"):
         getattr(lib, name).argtypes = [u64]
     lib.fvt_plan_hash.argtypes = [u64, u32, u64, u64, C.c_int, C.c_int, C.POINTER(u64)]
+    lib.fvt_hash_stage.argtypes = [u64, u64, u64, u64, u64, u32, C.POINTER(u64)]
     lib.fvt_matrix_piece.argtypes = [u32, u64, u64, C.POINTER(u64)]
     return lib
 
@@ -102,3 +103,29 @@ def test_chunks_of_a_batch(shim, K, w, bits, codes):
         assert 1 <= size <= min(n, 1 << 17)
         if crew:
             assert size * row >= 3 << 19 or size == 1 << 17  # a chunk is worth its launch and its copies
+
+
+@pytest.mark.parametrize("n,K,w,bits,codes", [(20000, 400, 1, False, True), (10486, 400, 11, False, True), (100003, 400, 11, True, False),
+                                              (100003, 400, 11, True, True), (1 << 20, 400, 11, True, False),
+                                              (5000, 2048, 64, True, True), (200000, 2, 64, True, False)])
+@pytest.mark.parametrize("got", [0, 1, 2, 3])
+@pytest.mark.parametrize("indices", [False, True])
+def test_staging_of_a_batch_fits_its_slots(shim, n, K, w, bits, codes, got, indices):
+    """The chunks in flight take up to four slots, whatever the pool gives; what they write lies inside the slots and
+    nowhere twice."""
+    bits_row, codes_row = -(-K // 64) * 8 if bits else 0, K if codes else 0
+    in_row, out_row = 4 * w if indices else 0, bits_row + codes_row
+    out = (C.c_uint64 * 20)()
+    shim.fvt_hash_stage(n, bits_row, codes_row, in_row, out_row, got, out)
+    want, slots, chunk, lanes = out[:4]
+    assert 1 <= want <= 4 and slots == (min(got, want) if got else want) and 1 <= chunk < n
+    assert lanes == (4 if 4 * in_row <= out_row else 2)
+    parts = []
+    for lane in range(lanes):
+        slot, at, in_slot, in_at = out[4 + 4 * lane:8 + 4 * lane]
+        parts += [(slot, at, chunk * out_row), (in_slot, in_at, chunk * in_row)]
+    for slot, at, size in parts:
+        assert slot < slots and at + size <= shim.fvt_slot_bytes()
+    for i, (slot, at, size) in enumerate(parts):
+        for other, o_at, o_size in parts[i + 1:]:
+            assert slot != other or at + size <= o_at or o_at + o_size <= at or not size or not o_size

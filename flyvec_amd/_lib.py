@@ -54,6 +54,7 @@ SIGNATURES = {
     "fv_host_free_pinned": [_vp],
     "fv_host_staging_release": [],
     "fv_host_staging_held": [C.POINTER(C.c_size_t)],
+    "fv_host_staging_limit": [C.c_size_t],
     "fv_dev_alloc": [C.c_size_t, _pp],
     "fv_dev_free": [_vp],
     "fv_dev_upload": [_vp, _vp, C.c_size_t],

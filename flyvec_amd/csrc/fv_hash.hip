@@ -313,16 +313,16 @@ static int fv_hash_host(fv_hasher *h, const int32_t *idx, uint64_t n, uint32_t w
   if (fv_hash_is_direct(n, w, want_bits + want_codes)) return fv_hash_direct(h, idx, n, w, k, shift, out_bits, out_codes);
   const bool bits_pageable = out_bits && fv_is_pageable(out_bits), codes_pageable = out_codes && fv_is_pageable(out_codes);
   fv_hash_plan plan = fv_plan_hash(n, want_bits, want_codes, bits_pageable, codes_pageable);
-  const bool stage_bits = plan.crew && bits_pageable, stage_codes = plan.crew && codes_pageable;
-  const bool stage_idx = plan.crew && fv_is_pageable(idx);
+  bool stage_bits = plan.crew && bits_pageable, stage_codes = plan.crew && codes_pageable, stage_idx = plan.crew && fv_is_pageable(idx);
   const uint64_t in_row = stage_idx ? w * sizeof(int32_t) : 0, out_row = (stage_bits ? bits_row : 0) + (stage_codes ? codes_row : 0);
-  std::unique_ptr<fv_stage_lease> lease;
+  fv_stage_lease lease(plan.crew ? fv_hash_stage_slots(&plan, in_row, out_row) : 0);
   fv_hash_staging staging = {};
   staging.lanes = 2;  // (not staged, a chunk may take hundreds of megabytes of the device)
-  if (plan.crew) {
-    lease.reset(new fv_stage_lease(fv_hash_stage_slots(&plan, in_row, out_row)));
-    FV_TRY(lease->rc);
-    staging = fv_hash_stage(&plan, in_row, out_row, (unsigned)lease->slots.size());
+  if (lease.n) {
+    staging = fv_hash_stage(&plan, in_row, out_row, lease.n);
+  } else {  // the runtime's copies, in as few pieces as may be
+    stage_bits = stage_codes = stage_idx = false;
+    plan.chunk = n < FV_HASH_CHUNK ? n : FV_HASH_CHUNK;
   }
   const uint64_t chunk = plan.chunk, n_chunks = (n + chunk - 1) / chunk;
   const uint64_t lanes = n_chunks < (uint64_t)staging.lanes ? n_chunks : (uint64_t)staging.lanes;
@@ -345,11 +345,11 @@ static int fv_hash_host(fv_hasher *h, const int32_t *idx, uint64_t n, uint32_t w
     FV_HIP(hipMalloc((void **)&h->work, lanes * lane_bytes));
     h->work_cap = lanes * lane_bytes;
   }
-  const auto stage = [&](uint64_t c) { return lease->slots[staging.slot[c % lanes]] + staging.at[c % lanes]; };
-  const auto stage_in = [&](uint64_t c) { return lease->slots[staging.in_slot[c % lanes]] + staging.in_at[c % lanes]; };
+  const auto stage = [&](uint64_t c) { return lease.slots[staging.slot[c % lanes]] + staging.at[c % lanes]; };
+  const auto stage_in = [&](uint64_t c) { return lease.slots[staging.in_slot[c % lanes]] + staging.in_at[c % lanes]; };
   const size_t stage_codes_at = stage_bits ? chunk * bits_row : 0;  // (behind the packed codes)
   std::unique_ptr<fv_copy_ring> ring;
-  if (lease) ring.reset(new fv_copy_ring(3 * n_chunks));
+  if (lease.n) ring.reset(new fv_copy_ring(3 * n_chunks));
   std::vector<uint32_t> last_item(n_chunks, 0xffffffffu);  // the last copy item of every chunk
   int rc = FV_OK;
   // chunk c's staged outputs are handed to the host threads once its copies have landed (one iteration later, while the

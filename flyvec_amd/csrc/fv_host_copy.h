@@ -88,12 +88,14 @@ struct fv_copy_ring {
   std::atomic<uint32_t> started{0};
 };
 
-// Page-locked slots of FV_STAGE_SLOT_BYTES, borrowed from the process's pool for the length of one transfer (at least
-// one; waits while other threads hold all of them) and returned by the destructor. `events`: one per slot.
+// Page-locked slots of FV_STAGE_SLOT_BYTES, borrowed from the process's pool for the length of one transfer and returned by
+// the destructor: n of up to FV_STAGE_SLOTS_LEASED wanted, at least one (waits while other threads hold all of them) unless the
+// system gives no page-locked memory or the pool may hold none; the transfer then goes the runtime's way. `events`:
+// one per slot.
 struct fv_stage_lease {
-  std::vector<char *> slots;
-  std::vector<hipEvent_t> events;
-  int rc;
+  char *slots[FV_STAGE_SLOTS_LEASED];
+  hipEvent_t events[FV_STAGE_SLOTS_LEASED];
+  unsigned n = 0;
   explicit fv_stage_lease(unsigned want);
   ~fv_stage_lease();
   fv_stage_lease(const fv_stage_lease &) = delete;
@@ -112,13 +114,11 @@ struct fv_stream_lease {
   fv_stream_lease &operator=(const fv_stream_lease &) = delete;
 };
 
-// Host memory -> device in n_pieces: piece(t, slot) says what to copy into the slot, consume(t, slot) enqueues the device's
+// Host memory -> device in n_pieces through the lease's slots: piece(t, slot) says what to copy into the slot, consume(t, slot) enqueues the device's
 // reading of it on `stream`. Returns when everything has been enqueued and the slots have been read.
 template <typename Piece, typename Consume>
-int fv_pipe_up(uint64_t n_pieces, hipStream_t stream, Piece piece, Consume consume) {
-  fv_stage_lease lease((unsigned)(n_pieces < FV_STAGE_SLOTS_LEASED ? n_pieces : FV_STAGE_SLOTS_LEASED));
-  FV_TRY(lease.rc);
-  const uint64_t S = lease.slots.size();
+int fv_pipe_up(fv_stage_lease &lease, uint64_t n_pieces, hipStream_t stream, Piece piece, Consume consume) {
+  const uint64_t S = lease.n;
   if (n_pieces == 1) {
     const fv_copy_ring::item it = piece(0, lease.slots[0]);
     fv_copy_ring::copy_share(it, 0, 1);
@@ -148,13 +148,11 @@ int fv_pipe_up(uint64_t n_pieces, hipStream_t stream, Piece piece, Consume consu
   return rc;
 }
 
-// Device -> host memory in n_pieces: produce(t, slot) enqueues the device's writing of the slot on `stream`, piece(t, slot)
+// Device -> host memory in n_pieces through the lease's slots: produce(t, slot) enqueues the device's writing of the slot on `stream`, piece(t, slot)
 // says where its contents go. Returns when the host memory holds everything.
 template <typename Produce, typename Piece>
-int fv_pipe_down(uint64_t n_pieces, hipStream_t stream, Produce produce, Piece piece) {
-  fv_stage_lease lease((unsigned)(n_pieces < FV_STAGE_SLOTS_LEASED ? n_pieces : FV_STAGE_SLOTS_LEASED));
-  FV_TRY(lease.rc);
-  const uint64_t S = lease.slots.size();
+int fv_pipe_down(fv_stage_lease &lease, uint64_t n_pieces, hipStream_t stream, Produce produce, Piece piece) {
+  const uint64_t S = lease.n;
   if (n_pieces == 1) {
     FV_TRY(produce(0, lease.slots[0]));
     FV_HIP(hipStreamSynchronize(stream));

@@ -70,6 +70,10 @@ static inline fv_matrix_pieces fv_cut_matrix(uint32_t K, uint64_t N) {
   return p;
 }
 
+static inline unsigned fv_matrix_slots(const fv_matrix_pieces *p) {
+  return p->n < FV_STAGE_SLOTS_LEASED ? (unsigned)p->n : FV_STAGE_SLOTS_LEASED;
+}
+
 static inline fv_matrix_piece fv_matrix_piece_at(const fv_matrix_pieces *p, uint64_t t) {
   fv_matrix_piece m;
   if (p->n == 1) {

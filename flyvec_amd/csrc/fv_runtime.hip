@@ -194,52 +194,55 @@ bool fv_is_pageable(const void *p) {
   return at.type == hipMemoryTypeUnregistered;
 }
 
-// The process's page-locked slots: made when first needed, up to FV_STAGE_SLOTS_MAX, kept for the transfers that follow
+// The process's page-locked slots: made when first needed, up to fv_stage_most, kept for the transfers that follow
 // (page-locking 4 MB takes 0.1 to 0.8 ms) until fv_host_staging_release.
 static std::mutex fv_stage_mutex;
 static std::condition_variable fv_stage_returned;
-static std::vector<char *> fv_stage_idle;
-static unsigned fv_stage_made = 0;
+static char *fv_stage_idle[FV_STAGE_SLOTS_MAX];
+static unsigned fv_stage_n_idle = 0, fv_stage_made = 0, fv_stage_most = FV_STAGE_SLOTS_MAX;
 
-fv_stage_lease::fv_stage_lease(unsigned want) : rc(FV_OK) {
-  {
-    std::unique_lock<std::mutex> lock(fv_stage_mutex);
-    while (slots.size() < want) {
-      if (!fv_stage_idle.empty()) {
-        slots.push_back(fv_stage_idle.back());
-        fv_stage_idle.pop_back();
-      } else if (fv_stage_made < FV_STAGE_SLOTS_MAX) {
-        char *p = nullptr;
-        const hipError_t e = hipHostMalloc((void **)&p, FV_STAGE_SLOT_BYTES, hipHostMallocPortable | hipHostMallocCoherent);
-        if (e != hipSuccess) {
-          (void)hipGetLastError();
-          if (slots.empty()) rc = fv_fail(FV_ERR_HIP, "page-locked staging memory: %s", hipGetErrorString(e));
-          break;  // with fewer than wanted
-        }
-        fv_stage_made++;
-        slots.push_back(p);
-      } else if (slots.empty()) {
-        fv_stage_returned.wait(lock);
-      } else {
-        break;
-      }
-    }
+// (with the lock held)
+static void fv_stage_trim(unsigned keep) {
+  while (fv_stage_n_idle && fv_stage_made > keep) {
+    (void)hipHostFree(fv_stage_idle[--fv_stage_n_idle]);
+    fv_stage_made--;
   }
-  for (size_t i = 0; i < slots.size() && rc == FV_OK; ++i) {
-    hipEvent_t ev = nullptr;
-    const hipError_t e = hipEventCreateWithFlags(&ev, hipEventDisableTiming);
-    if (e != hipSuccess)
-      rc = fv_fail(FV_ERR_HIP, "staging event: %s", hipGetErrorString(e));
-    else
-      events.push_back(ev);
+}
+
+fv_stage_lease::fv_stage_lease(unsigned want) {
+  std::unique_lock<std::mutex> lock(fv_stage_mutex);
+  while (n < want && n < FV_STAGE_SLOTS_LEASED) {
+    char *p = nullptr;
+    if (fv_stage_n_idle) {
+      p = fv_stage_idle[--fv_stage_n_idle];
+    } else if (fv_stage_made < fv_stage_most) {
+      if (hipHostMalloc((void **)&p, FV_STAGE_SLOT_BYTES, hipHostMallocPortable | hipHostMallocCoherent) != hipSuccess) {
+        (void)hipGetLastError();
+        break;  // with fewer than wanted, or none
+      }
+      fv_stage_made++;
+    } else if (n == 0 && fv_stage_made) {
+      fv_stage_returned.wait(lock);
+      continue;
+    } else {
+      break;
+    }
+    if (hipEventCreateWithFlags(&events[n], hipEventDisableTiming) != hipSuccess) {
+      (void)hipGetLastError();
+      fv_stage_idle[fv_stage_n_idle++] = p;
+      fv_stage_returned.notify_all();
+      break;
+    }
+    slots[n++] = p;
   }
 }
 
 fv_stage_lease::~fv_stage_lease() {
-  for (hipEvent_t ev : events) (void)hipEventDestroy(ev);
+  for (unsigned i = 0; i < n; ++i) (void)hipEventDestroy(events[i]);
   {
     std::lock_guard<std::mutex> lock(fv_stage_mutex);
-    for (char *p : slots) fv_stage_idle.push_back(p);
+    for (unsigned i = 0; i < n; ++i) fv_stage_idle[fv_stage_n_idle++] = slots[i];
+    fv_stage_trim(fv_stage_most);
   }
   fv_stage_returned.notify_all();
 }
@@ -283,11 +286,18 @@ extern "C" int fv_host_staging_held(size_t *out_bytes) {
   return FV_OK;
 }
 
+extern "C" int fv_host_staging_limit(size_t bytes) {
+  std::lock_guard<std::mutex> lock(fv_stage_mutex);
+  const size_t slots = bytes / FV_STAGE_SLOT_BYTES;
+  fv_stage_most = slots < FV_STAGE_SLOTS_MAX ? (unsigned)slots : FV_STAGE_SLOTS_MAX;
+  fv_stage_trim(fv_stage_most);
+  fv_stage_returned.notify_all();
+  return FV_OK;
+}
+
 extern "C" int fv_host_staging_release(void) {
   std::lock_guard<std::mutex> lock(fv_stage_mutex);
-  for (char *p : fv_stage_idle) (void)hipHostFree(p);
-  fv_stage_made -= (unsigned)fv_stage_idle.size();
-  fv_stage_idle.clear();
+  fv_stage_trim(0);
   for (const fv_idle_stream &idle : fv_streams_idle) (void)hipStreamDestroy(idle.stream);
   fv_streams_idle.clear();
   return FV_OK;
@@ -300,12 +310,13 @@ static bool fv_pageable_range(const void *host, size_t bytes) {
 
 int fv_copy_up(void *dst_dev, const void *src_host, size_t bytes, hipStream_t stream) {
   if (bytes == 0) return FV_OK;
-  if (!fv_upload_staged(bytes) || !fv_pageable_range(src_host, bytes)) {
+  fv_stage_lease lease(fv_upload_staged(bytes) && fv_pageable_range(src_host, bytes) ? FV_STAGE_SLOTS_LEASED : 0);
+  if (!lease.n) {
     FV_HIP(hipMemcpyAsync(dst_dev, src_host, bytes, hipMemcpyHostToDevice, stream));
     return FV_OK;
   }
   return fv_pipe_up(
-      fv_copy_pieces(bytes), stream,
+      lease, fv_copy_pieces(bytes), stream,
       [&](uint64_t t, char *p) {
         return fv_copy_ring::item{(const char *)src_host + t * FV_STAGE_SLOT_BYTES, p, fv_copy_piece_bytes(bytes, t), 0, 0, 1};
       },
@@ -318,13 +329,14 @@ int fv_copy_up(void *dst_dev, const void *src_host, size_t bytes, hipStream_t st
 
 int fv_copy_down(void *dst_host, const void *src_dev, size_t bytes, hipStream_t stream) {
   if (bytes == 0) return FV_OK;
-  if (!fv_download_staged(bytes) || !fv_pageable_range(dst_host, bytes)) {
+  fv_stage_lease lease(fv_download_staged(bytes) && fv_pageable_range(dst_host, bytes) ? FV_STAGE_SLOTS_LEASED : 0);
+  if (!lease.n) {
     FV_HIP(hipMemcpyAsync(dst_host, src_dev, bytes, hipMemcpyDeviceToHost, stream));
     FV_HIP(hipStreamSynchronize(stream));
     return FV_OK;
   }
   return fv_pipe_down(
-      fv_copy_pieces(bytes), stream,
+      lease, fv_copy_pieces(bytes), stream,
       [&](uint64_t t, char *p) -> int {
         FV_HIP(hipMemcpyAsync(p, (const char *)src_dev + t * FV_STAGE_SLOT_BYTES, fv_copy_piece_bytes(bytes, t),
                               hipMemcpyDeviceToHost, stream));
@@ -342,6 +354,12 @@ static fv_copy_ring::item fv_matrix_item(const fv_matrix_piece &m, uint64_t N, c
   return {(const char *)from, (char *)to, row, up ? caller : slot, up ? slot : caller, m.rows};
 }
 
+static int fv_finish_matrix(int rc, hipStream_t stream, const char *what) {
+  const hipError_t e = hipStreamSynchronize(stream);
+  if (rc == FV_OK && e != hipSuccess) rc = fv_fail(FV_ERR_HIP, "weight %s failed: %s", what, hipGetErrorString(e));
+  return rc;
+}
+
 // Page-locked matrices are read and written in place by the layout change, and pageable ones of the sizes that
 // fv_host_plan.h names through page-locked slots: there is no staging matrix on the device, whose allocation and release
 // (which waits for the device) cost more than the copy of a small matrix, and no second pass over it. The others, and
@@ -352,10 +370,13 @@ int fv_upload_weights(const float *W_host, float *Wt_dev, uint32_t K, uint64_t N
   int rc = FV_OK;
   if (const float *view = (const float *)fv_device_view(W_host, bytes)) {
     rc = fv_launch_to_token_major(view, N, Wt_dev, K, N, ldk, ldk, stream);
-  } else if (fv_matrix_upload_staged(bytes) && fv_pageable_range(W_host, bytes)) {
-    const fv_matrix_pieces pieces = fv_cut_matrix(K, N);
+    return fv_finish_matrix(rc, stream, "upload");
+  }
+  const fv_matrix_pieces pieces = fv_cut_matrix(K, N);
+  fv_stage_lease lease(fv_matrix_upload_staged(bytes) && fv_pageable_range(W_host, bytes) ? fv_matrix_slots(&pieces) : 0);
+  if (lease.n) {
     return fv_pipe_up(
-        pieces.n, stream,
+        lease, pieces.n, stream,
         [&](uint64_t t, char *p) {
           const fv_matrix_piece m = fv_matrix_piece_at(&pieces, t);
           return fv_matrix_item(m, N, W_host + m.h * N + m.i, (float *)p, true);
@@ -365,17 +386,14 @@ int fv_upload_weights(const float *W_host, float *Wt_dev, uint32_t K, uint64_t N
           return fv_launch_to_token_major((const float *)p, m.pitch, Wt_dev + m.i * ldk + m.h, m.rows, m.cols, ldk,
                                           m.h + m.rows == K ? ldk - m.h : m.rows, stream);
         });
-  } else {
-    float *stage = nullptr;
-    FV_HIP(hipMalloc((void **)&stage, bytes));
-    const hipError_t e = hipMemcpyAsync(stage, W_host, bytes, hipMemcpyHostToDevice, stream);
-    if (e != hipSuccess) rc = fv_fail(FV_ERR_HIP, "weight upload failed: %s", hipGetErrorString(e));
-    if (rc == FV_OK) rc = fv_launch_to_token_major(stage, N, Wt_dev, K, N, ldk, ldk, stream);
-    (void)hipStreamSynchronize(stream);
-    (void)hipFree(stage);
   }
-  const hipError_t e = hipStreamSynchronize(stream);
-  if (rc == FV_OK && e != hipSuccess) rc = fv_fail(FV_ERR_HIP, "weight upload failed: %s", hipGetErrorString(e));
+  float *on_device = nullptr;
+  FV_HIP(hipMalloc((void **)&on_device, bytes));
+  const hipError_t e = hipMemcpyAsync(on_device, W_host, bytes, hipMemcpyHostToDevice, stream);
+  if (e != hipSuccess) rc = fv_fail(FV_ERR_HIP, "weight upload failed: %s", hipGetErrorString(e));
+  if (rc == FV_OK) rc = fv_launch_to_token_major(on_device, N, Wt_dev, K, N, ldk, ldk, stream);
+  rc = fv_finish_matrix(rc, stream, "upload");
+  (void)hipFree(on_device);
   return rc;
 }
 
@@ -385,10 +403,13 @@ int fv_download_weights(const float *Wt_dev, float *W_host, uint32_t K, uint64_t
   int rc = FV_OK;
   if (float *view = (float *)fv_device_view(W_host, bytes)) {
     rc = fv_launch_to_row_major(Wt_dev, view, N, K, N, ldk, stream);
-  } else if (fv_pageable_range(W_host, bytes)) {
-    const fv_matrix_pieces pieces = fv_cut_matrix(K, N);
+    return fv_finish_matrix(rc, stream, "download");
+  }
+  const fv_matrix_pieces pieces = fv_cut_matrix(K, N);
+  fv_stage_lease lease(fv_pageable_range(W_host, bytes) ? fv_matrix_slots(&pieces) : 0);
+  if (lease.n) {
     return fv_pipe_down(
-        pieces.n, stream,
+        lease, pieces.n, stream,
         [&](uint64_t t, char *p) {
           const fv_matrix_piece m = fv_matrix_piece_at(&pieces, t);
           return fv_launch_to_row_major(Wt_dev + m.i * ldk + m.h, (float *)p, m.pitch, m.rows, m.cols, ldk, stream);
@@ -397,19 +418,16 @@ int fv_download_weights(const float *Wt_dev, float *W_host, uint32_t K, uint64_t
           const fv_matrix_piece m = fv_matrix_piece_at(&pieces, t);
           return fv_matrix_item(m, N, (const float *)p, W_host + m.h * N + m.i, false);
         });
-  } else {
-    float *stage = nullptr;
-    FV_HIP(hipMalloc((void **)&stage, bytes));
-    rc = fv_launch_to_row_major(Wt_dev, stage, N, K, N, ldk, stream);
-    if (rc == FV_OK) {
-      const hipError_t e = hipMemcpyAsync(W_host, stage, bytes, hipMemcpyDeviceToHost, stream);
-      if (e != hipSuccess) rc = fv_fail(FV_ERR_HIP, "weight download failed: %s", hipGetErrorString(e));
-    }
-    (void)hipStreamSynchronize(stream);
-    (void)hipFree(stage);
   }
-  const hipError_t e = hipStreamSynchronize(stream);
-  if (rc == FV_OK && e != hipSuccess) rc = fv_fail(FV_ERR_HIP, "weight download failed: %s", hipGetErrorString(e));
+  float *on_device = nullptr;
+  FV_HIP(hipMalloc((void **)&on_device, bytes));
+  rc = fv_launch_to_row_major(Wt_dev, on_device, N, K, N, ldk, stream);
+  if (rc == FV_OK) {
+    const hipError_t e = hipMemcpyAsync(W_host, on_device, bytes, hipMemcpyDeviceToHost, stream);
+    if (e != hipSuccess) rc = fv_fail(FV_ERR_HIP, "weight download failed: %s", hipGetErrorString(e));
+  }
+  rc = fv_finish_matrix(rc, stream, "download");
+  (void)hipFree(on_device);
   return rc;
 }
 

@@ -52,10 +52,12 @@ int fv_host_free_pinned(void *ptr);
 /* Matrices (upwards those of up to 4 MB and of 8 MB and more), other uploads of 32 MB, downloads of 16 MB and batches with
  * codes of 4 MB and more between the device and ordinary host memory go through page-locked memory, up to 32 MB of it,
  * that the library keeps for the transfers that follow, with a stream per batch in flight. release returns what no
- * transfer is using to the system (the next one takes it anew); held tells how much memory there is. No counterpart in
- * the reference. */
+ * transfer is using to the system (the next one takes it anew); held tells how much memory there is; limit sets the most
+ * there may be (in whole 4 MB, 32 MB by default), 0 for none: transfers then go through the runtime's copies, as they do
+ * where the system gives no page-locked memory. Process-wide; results are the same. No counterpart in the reference. */
 int fv_host_staging_release(void);
 int fv_host_staging_held(size_t *out_bytes);
+int fv_host_staging_limit(size_t bytes);
 
 /* flyvec/src/cuda_helpers.cu:8 do_gpu_cudaMallocManaged -- the reference keeps every
  * buffer in managed memory; here device buffers are explicit.  Used by callers that

@@ -138,6 +138,44 @@ def test_hash_batches_borrow_their_staging(gpu, n, slots):
     assert not bad
 
 
+@pytest.mark.parametrize("slots", [0, 1, 3])
+def test_every_route_with_fewer_slots_or_none(gpu, slots):
+    """Where the process may page-lock nothing (as where the system gives nothing) every transfer goes the runtime's way,
+    with one slot or three it waits for what there is: the same bytes. A limit below what is held gives back what is idle."""
+    from flyvec_amd import Hasher, Trainer, _lib
+    lib = _lib.load()
+    slot = 4 << 20
+    rng = np.random.default_rng(8)
+    try:
+        assert lib.fv_host_staging_limit(slots * slot + 5) == 0 and held() <= slots * slot
+        for K, V in ((64, 500), (400, 1500), (130, 20000)):     # one piece; between; tiles
+            W = rng.standard_normal((K, 2 * V), dtype=np.float32)
+            t = Trainer(V, K, 3, 16)
+            t.set_weights(W)
+            assert np.array_equal(t.get_weights(), W)
+            t.close()
+        t = Trainer(50, 8, 5, 16)
+        n = (1 << 22) + 3
+        starts, perm = rng.integers(0, 990, size=n).astype(np.uint64), rng.permutation(n).astype(np.uint64)
+        t.set_corpus_starts(rng.integers(0, 50, 1000).astype(np.int32), starts)
+        t.set_permutation(perm)
+        assert np.array_equal(t.window_starts(), starts) and np.array_equal(t.get_permutation(), perm)
+        t.close()
+        h = Hasher(rng.standard_normal((70, 400), dtype=np.float32))
+        for n, w in ((30000, 3), (100003, 3), (140001, 11)):    # light indices twice, heavy ones on two streams
+            idx = rng.integers(0, 400, size=(n, w)).astype(np.int32)
+            dev, bits, codes = _lib.DeviceBuffer.from_numpy(idx), _lib.DeviceBuffer(n * 16), _lib.DeviceBuffer(n * 70)
+            h.hash_windows_dev(dev, n, w, 9, bits, codes)
+            h.sync()
+            got = h.hash_windows(idx, 9, packed=True, codes=True)
+            assert np.array_equal(got[0], bits.to_numpy(np.uint64, (n, 2))) and np.array_equal(got[1], codes.to_numpy(np.int8, (n, 70)))
+            assert np.array_equal(h.hash_windows(idx, 9, packed=True), got[0])
+        h.close()
+        assert held() == slots * slot
+    finally:
+        assert lib.fv_host_staging_limit(1 << 40) == 0
+
+
 def test_more_transfers_at_once_than_there_are_slots(gpu):
     """Six threads, each with a trainer of its own, hold up to four of eight slots each: they wait for each other's and
     all finish with their own matrix."""

@@ -153,13 +153,23 @@ static void fv_trainer_forget_corpus(fv_trainer *t) {
 // larger than needed.
 static bool fv_fits_kept(uint64_t need, uint64_t cap) { return need <= cap && cap - need <= need / 4; }
 
+template <typename P>
+static int fv_corpus_alloc(fv_trainer *t, P **out, uint64_t n) {
+  const hipError_t e = t->fail_alloc && --t->fail_alloc == 0 ? hipErrorOutOfMemory : hipMalloc((void **)out, n * sizeof(P));
+  if (e != hipSuccess) {
+    (void)hipGetLastError();
+    return fv_fail(FV_ERR_HIP, "corpus allocation of %llu bytes failed: %s", (unsigned long long)(n * sizeof(P)), hipGetErrorString(e));
+  }
+  return FV_OK;
+}
+
 static int fv_trainer_reserve_corpus(fv_trainer *t, uint64_t n_tokens) {
   if (!fv_fits_kept(n_tokens, t->corpus_cap)) {
     fv_trainer_free_corpus(t);  // the window tables too: the new corpus finds the memory it would find in a new trainer
-    FV_HIP(hipMalloc((void **)&t->corpus, n_tokens * sizeof(int32_t)));
+    FV_TRY(fv_corpus_alloc(t, &t->corpus, n_tokens));
     t->corpus_cap = n_tokens;
   }
-  if (!t->invf) FV_HIP(hipMalloc((void **)&t->invf, t->V * sizeof(float)));
+  if (!t->invf) FV_TRY(fv_corpus_alloc(t, &t->invf, t->V));
   return FV_OK;
 }
 
@@ -171,11 +181,32 @@ static int fv_trainer_reserve_windows(fv_trainer *t, uint64_t n_windows) {
   (void)hipFree(t->pstart);
   t->starts = t->perm = t->perm_alt = t->pstart = nullptr;
   t->windows_cap = 0;
-  FV_HIP(hipMalloc((void **)&t->starts, n_windows * sizeof(uint64_t)));
-  FV_HIP(hipMalloc((void **)&t->perm, n_windows * sizeof(uint64_t)));
-  FV_HIP(hipMalloc((void **)&t->pstart, n_windows * sizeof(uint64_t)));
+  FV_TRY(fv_corpus_alloc(t, &t->starts, n_windows));
+  FV_TRY(fv_corpus_alloc(t, &t->perm, n_windows));
+  FV_TRY(fv_corpus_alloc(t, &t->pstart, n_windows));
   t->windows_cap = n_windows;
   return FV_OK;
+}
+
+// Sets a corpus with `load`. If that fails in the runtime while buffers of an earlier corpus are kept (the device's memory
+// may have been too little for both) they are given back and it is done once more as on a new trainer: what fits there
+// fits here. A corpus that is refused leaves the trainer without one, and without its buffers.
+template <typename Load>
+static int fv_trainer_load_corpus(fv_trainer *t, uint64_t n_tokens, Load load) {
+  fv_trainer_forget_corpus(t);
+  for (bool kept = t->corpus != nullptr;; kept = false) {
+    uint64_t n_windows = 0;
+    const int rc = load(&n_windows);
+    if (rc == FV_OK) {
+      t->n_tokens = n_tokens;
+      t->n_windows = n_windows;
+      t->have_corpus = true;
+      return FV_OK;
+    }
+    fv_trainer_free_corpus(t);
+    if (rc != FV_ERR_HIP || !kept) return rc;
+    (void)hipGetLastError();
+  }
 }
 
 // Trainers of this process with steps enqueued that nobody has waited for yet. The single dense launch, where it has
@@ -492,23 +523,21 @@ extern "C" int fv_trainer_create(const fv_train_config *cfg, fv_trainer **out_tr
   return FV_OK;
 }
 
-extern "C" int fv_trainer_set_corpus(fv_trainer *t, const int32_t *tokens, uint64_t n_tokens,
-                                     const uint64_t *offsets, uint64_t n_offsets) {
-  FV_REQUIRE(t, FV_ERR_INVALID, "null trainer");
-  FV_REQUIRE(tokens && n_tokens > 0, FV_ERR_INVALID, "empty corpus");
-  FV_REQUIRE(offsets && n_offsets >= 1, FV_ERR_INVALID, "empty offsets");
+// The identity order over the window starts, and its table; waits for the stream.
+static int fv_trainer_identity_order(fv_trainer *t, uint64_t n_windows) {
+  hipLaunchKernelGGL(fv_identity_kernel, dim3(fv_perm_blocks(n_windows)), dim3(256), 0, t->stream, t->starts, t->perm,
+                     t->pstart, n_windows);
   FV_HIP(fv_trainer_drain(t));
-  fv_trainer_forget_corpus(t);
-  const uint64_t n_chunks = n_offsets - 1;
+  return FV_OK;
+}
+
+static int fv_trainer_build_corpus(fv_trainer *t, const int32_t *tokens, uint64_t n_tokens, const uint64_t *offsets,
+                                   uint64_t n_chunks, uint64_t *out_windows) {
+  FV_TRY(fv_trainer_reserve_corpus(t, n_tokens));
   uint64_t *off_dev = nullptr;
-  int rc = fv_trainer_reserve_corpus(t, n_tokens);
-  hipError_t e = hipSuccess;
-  if (rc == FV_OK) {
-    e = hipMalloc((void **)&off_dev, n_offsets * sizeof(uint64_t));
-    if (e != hipSuccess) rc = fv_fail(FV_ERR_HIP, "corpus allocation failed: %s", hipGetErrorString(e));
-  }
-  if (rc == FV_OK) rc = fv_copy_up(t->corpus, tokens, n_tokens * sizeof(int32_t), t->stream);
-  if (rc == FV_OK) rc = fv_copy_up(off_dev, offsets, n_offsets * sizeof(uint64_t), t->stream);
+  FV_TRY(fv_corpus_alloc(t, &off_dev, n_chunks + 1));
+  int rc = fv_copy_up(t->corpus, tokens, n_tokens * sizeof(int32_t), t->stream);
+  if (rc == FV_OK) rc = fv_copy_up(off_dev, offsets, (n_chunks + 1) * sizeof(uint64_t), t->stream);
 
   int32_t lo = 0, hi = 0;
   if (rc == FV_OK) rc = fv_dev_inverse_frequency(t->corpus, n_tokens, t->V, t->invf, &lo, &hi, t->stream);
@@ -531,22 +560,23 @@ extern "C" int fv_trainer_set_corpus(fv_trainer *t, const int32_t *tokens, uint6
                      (unsigned long long)span, (unsigned long long)n_tokens);
     }
     if (rc == FV_OK) rc = fv_dev_build_window_starts(off_dev, n_chunks, t->w, t->starts, nwin, t->stream);
-    if (rc == FV_OK) {
-      hipLaunchKernelGGL(fv_identity_kernel, dim3(fv_perm_blocks(nwin)), dim3(256), 0, t->stream, t->starts, t->perm,
-                         t->pstart, nwin);
-      e = fv_trainer_drain(t);
-      if (e != hipSuccess) rc = fv_fail(FV_ERR_HIP, "permutation fill failed: %s", hipGetErrorString(e));
-    }
+    if (rc == FV_OK) rc = fv_trainer_identity_order(t, nwin);
   }
+  if (rc != FV_OK) (void)hipStreamSynchronize(t->stream);  // (before the offsets go)
   (void)hipFree(off_dev);
-  if (rc != FV_OK) {
-    fv_trainer_free_corpus(t);
-    return rc;
-  }
-  t->n_tokens = n_tokens;
-  t->n_windows = nwin;
-  t->have_corpus = true;
-  return FV_OK;
+  *out_windows = nwin;
+  return rc;
+}
+
+extern "C" int fv_trainer_set_corpus(fv_trainer *t, const int32_t *tokens, uint64_t n_tokens,
+                                     const uint64_t *offsets, uint64_t n_offsets) {
+  FV_REQUIRE(t, FV_ERR_INVALID, "null trainer");
+  FV_REQUIRE(tokens && n_tokens > 0, FV_ERR_INVALID, "empty corpus");
+  FV_REQUIRE(offsets && n_offsets >= 1, FV_ERR_INVALID, "empty offsets");
+  FV_HIP(fv_trainer_drain(t));
+  return fv_trainer_load_corpus(t, n_tokens, [&](uint64_t *out_windows) {
+    return fv_trainer_build_corpus(t, tokens, n_tokens, offsets, n_offsets - 1, out_windows);
+  });
 }
 
 // The same with the window table given instead of built: what the reference's driver hands over
@@ -562,32 +592,19 @@ extern "C" int fv_trainer_set_corpus_starts(fv_trainer *t, const int32_t *tokens
                "window %llu starts at token %llu: it does not fit the corpus of %llu", (unsigned long long)i,
                (unsigned long long)starts[i], (unsigned long long)n_tokens);
   FV_HIP(fv_trainer_drain(t));
-  fv_trainer_forget_corpus(t);
-  int rc = fv_trainer_reserve_corpus(t, n_tokens);
-  if (rc == FV_OK) rc = fv_copy_up(t->corpus, tokens, n_tokens * sizeof(int32_t), t->stream);
-  int32_t lo = 0, hi = 0;
-  if (rc == FV_OK) rc = fv_dev_inverse_frequency(t->corpus, n_tokens, t->V, t->invf, &lo, &hi, t->stream);
-  if (rc == FV_OK && (lo < -1 || (hi >= 0 && (uint64_t)hi >= t->V)))
-    rc = fv_fail(FV_ERR_DATA, "token ids span [%d, %d]; allowed are -1 (masked) and 0..%llu", lo, hi,
-                 (unsigned long long)(t->V - 1));
-  if (rc == FV_OK && n_windows) {
-    rc = fv_trainer_reserve_windows(t, n_windows);
-    if (rc == FV_OK) rc = fv_copy_up(t->starts, starts, n_windows * sizeof(uint64_t), t->stream);
-    if (rc == FV_OK) {
-      hipLaunchKernelGGL(fv_identity_kernel, dim3(fv_perm_blocks(n_windows)), dim3(256), 0, t->stream, t->starts, t->perm,
-                         t->pstart, n_windows);
-      const hipError_t e = fv_trainer_drain(t);
-      if (e != hipSuccess) rc = fv_fail(FV_ERR_HIP, "permutation fill failed: %s", hipGetErrorString(e));
-    }
-  }
-  if (rc != FV_OK) {
-    fv_trainer_free_corpus(t);
-    return rc;
-  }
-  t->n_tokens = n_tokens;
-  t->n_windows = n_windows;
-  t->have_corpus = true;
-  return FV_OK;
+  return fv_trainer_load_corpus(t, n_tokens, [&](uint64_t *out_windows) -> int {
+    FV_TRY(fv_trainer_reserve_corpus(t, n_tokens));
+    FV_TRY(fv_copy_up(t->corpus, tokens, n_tokens * sizeof(int32_t), t->stream));
+    int32_t lo = 0, hi = 0;
+    FV_TRY(fv_dev_inverse_frequency(t->corpus, n_tokens, t->V, t->invf, &lo, &hi, t->stream));
+    FV_REQUIRE(lo >= -1 && (hi < 0 || (uint64_t)hi < t->V), FV_ERR_DATA,
+               "token ids span [%d, %d]; allowed are -1 (masked) and 0..%llu", lo, hi, (unsigned long long)(t->V - 1));
+    *out_windows = n_windows;
+    if (!n_windows) return FV_OK;
+    FV_TRY(fv_trainer_reserve_windows(t, n_windows));
+    FV_TRY(fv_copy_up(t->starts, starts, n_windows * sizeof(uint64_t), t->stream));
+    return fv_trainer_identity_order(t, n_windows);
+  });
 }
 
 extern "C" int fv_trainer_num_windows(fv_trainer *t, uint64_t *out_count) {
@@ -1271,6 +1288,12 @@ extern "C" int fv_trainer_get_dense_forms(fv_trainer *t, uint64_t *out_one, uint
   FV_REQUIRE(t && out_one && out_two, FV_ERR_INVALID, "null argument");
   *out_one = t->dense_forms[0];
   *out_two = t->dense_forms[1];
+  return FV_OK;
+}
+
+extern "C" int fv_trainer_fail_allocation(fv_trainer *t, uint32_t nth) {
+  FV_REQUIRE(t, FV_ERR_INVALID, "null trainer");
+  t->fail_alloc = nth;
   return FV_OK;
 }
 

@@ -45,6 +45,7 @@ struct fv_trainer {
   uint64_t *pstart;    // starts[perm[i]]: where the i-th window of the current order begins
   uint64_t *perm_alt;  // second permutation buffer, allocated by the first shuffle
   uint64_t n_windows;
+  uint32_t fail_alloc;  // fv_trainer_fail_allocation: allocations of a corpus until one is refused, 0 for none
   uint64_t corpus_cap, windows_cap;  // tokens / windows the buffers above have room for
   float *invf;
   int32_t *idx;     // B rows of idx_stride column indices of the current minibatch (w used, the rest -1)

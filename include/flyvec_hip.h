@@ -163,6 +163,10 @@ int fv_trainer_set_corpus(fv_trainer *t, const int32_t *tokens, uint64_t n_token
  * FV_ERR_DATA); builds 1/frequency and the identity permutation like fv_trainer_set_corpus. */
 int fv_trainer_set_corpus_starts(fv_trainer *t, const int32_t *tokens, uint64_t n_tokens,
                                  const uint64_t *starts, uint64_t n_windows);
+/* A trainer given another corpus keeps its buffers where they are at most a quarter larger than needed; where the device's
+ * memory does not allow that they are given back first. Test hook: the nth allocation from here on of set_corpus /
+ * set_corpus_starts on this trainer is refused as if the memory were full (0: none). No counterpart in the reference. */
+int fv_trainer_fail_allocation(fv_trainer *t, uint32_t nth);
 int fv_trainer_num_windows(fv_trainer *t, uint64_t *out_count);
 /* Read-back of what set_corpus built (parity hooks). */
 int fv_trainer_get_window_starts(fv_trainer *t, uint64_t *out_starts, uint64_t capacity);

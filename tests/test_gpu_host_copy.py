@@ -267,3 +267,50 @@ def test_one_corpus_after_another(gpu, oracle_lib):
     with pytest.raises(Exception):
         t.num_windows  # the corpus before the refused one is gone, as before
     t.close()
+
+
+@pytest.mark.parametrize("n,nth", [(20000, 1), (20000, 2), (20000, 3), (20000, 4), (55000, 1)])
+def test_a_corpus_that_fits_a_new_trainer_fits_one_that_has_a_corpus(gpu, oracle_lib, n, nth):
+    """Where the device's memory does not hold what the call needs beside the buffers kept from the corpus before, they are
+    given back and the corpus is set as on a new trainer: whichever allocation is refused (the second corpus much smaller, so
+    that nothing is kept but while it fails, or a little, so that only the offsets' memory is new). On a new trainer the refusal
+    stands, and the next corpus is set as ever."""
+    from flyvec_amd import Trainer, _lib
+    from conftest import small_corpus
+    V, w = 300, 7
+    big, tokens_offsets = small_corpus(60000, V, seed=1), small_corpus(n, V, seed=2)
+    starts = oracle_lib.window_starts(tokens_offsets[1], w)
+
+    def refuse(t):
+        _lib.check(_lib.load().fv_trainer_fail_allocation(t.handle, nth))
+
+    def check(t):
+        assert np.array_equal(t.window_starts(), starts)
+        assert np.array_equal(t.get_permutation(), np.arange(len(starts), dtype=np.uint64))
+        assert np.array_equal(t.inverse_frequency(), oracle_lib.inverse_frequency(tokens_offsets[0], V))
+
+    for given in (False, True):
+        def set_corpus(t):
+            if given:
+                t.set_corpus_starts(tokens_offsets[0], starts)
+            else:
+                t.set_corpus(*tokens_offsets)
+        t = Trainer(V, 16, w, 64)
+        t.set_corpus(*big)
+        t.shuffle(1)
+        refuse(t)
+        set_corpus(t)
+        check(t)
+        t.shuffle(2)
+        assert np.array_equal(np.sort(t.get_permutation()), np.arange(len(starts), dtype=np.uint64))
+        t.close()
+        t = Trainer(V, 16, w, 64)
+        refuse(t)
+        with pytest.raises(_lib.FlyvecError) as e:
+            set_corpus(t)
+        assert e.value.code == _lib.FV_ERR_HIP and "allocation" in str(e.value)
+        with pytest.raises(_lib.FlyvecError):
+            t.num_windows
+        set_corpus(t)
+        check(t)
+        t.close()

@@ -1,9 +1,9 @@
 // Large transfers between the device and ordinary (pageable) host memory.
 //
-// The runtime copies such memory through a staging buffer of its own with one thread: 10 to 16 GB/s, and the caller's
+// The runtime copies such memory through a staging buffer of its own with one thread: 10 to 17 GB/s, and the caller's
 // fresh pages are touched for the first time by that thread, against some 55 GB/s of the link. Here a few host
 // threads move pieces between the caller's memory and page-locked slots while the device fills or empties the other
-// slots.
+// slots. fv_host_plan.h says from which sizes on that is the faster way.
 #pragma once
 
 #include <string.h>
@@ -16,6 +16,8 @@
 #include "fv_host_plan.h"
 #include "fv_internal.h"
 
+// Four: with two, 100003 windows to 40 MB of int8 codes take 2.0 ms instead of 1.45 and a matrix of 64 MB down 3.9 instead of
+// 2.7; with six 1.3 and 2.55, but 20000 targets (8 MB) 380 us instead of 340, with eight 435: starting them costs that.
 #define FV_COPY_THREADS 4
 
 // Ordinary (pageable) host memory, which the device cannot reach by DMA? (fv_runtime.hip)

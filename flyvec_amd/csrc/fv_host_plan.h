@@ -96,13 +96,17 @@ static inline fv_matrix_piece fv_matrix_piece_at(const fv_matrix_pieces *p, uint
 #define FV_HASH_CHUNK (1u << 17) /* most windows per chunk */
 #define FV_HASH_LANES 4          /* most chunks in flight */
 /* A batch is cut into about this many chunks, of output that takes the link some 30 us or more: one call's copies in,
- * kernel, copies out and host copies then overlap also for batches that fit one chunk. */
+ * kernel, copies out and host copies then overlap also for batches that fit one chunk. (4 or 16 chunks: the same within
+ * the runs' differences, 20000 targets 365 and 339 us, 340 with 8; chunks of 0.75 MB 394, of 3 MB 333, for twice the
+ * page-locked memory.) */
 #define FV_HASH_CHUNKS 8
 #define FV_HASH_CHUNK_MIN_BYTES ((uint64_t)3 << 19)
 /* Results of this size and more, for pageable memory, are worth the host threads. */
 #define FV_HASH_CREW_BYTES ((uint64_t)4 << 20)
 /* Batches whose indices and codes take no more than this go through one page-locked buffer that the kernel itself
- * reads and writes: a launch and a wait, where two copies and their waits took 30 us of 44. */
+ * reads and writes: a launch and a wait, where two copies and their waits took 30 us of 44 (126 KB: 24 us against 82, 252
+ * KB: 29 against 49). It is still faster beyond (513 KB: 41 against 54, 1 MB: 66 against 80, 2 MB: 125 against 145);
+ * the line lies where it does because every hasher page-locks that much when it is made. */
 #define FV_HASH_DIRECT_BYTES ((uint64_t)1 << 18)
 
 static inline int fv_hash_is_direct(uint64_t n, uint32_t w, uint64_t out_row) {

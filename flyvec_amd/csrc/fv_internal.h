@@ -47,9 +47,6 @@ int fv_upload_weights(const float *W_host, float *Wt_dev, uint32_t K, uint64_t N
 int fv_download_weights(const float *Wt_dev, float *W_host, uint32_t K, uint64_t N, uint32_t ldk,
                         hipStream_t stream);
 
-// The device's address of page-locked host memory, null for any other kind (fv_runtime.hip).
-void *fv_device_view(const void *p, size_t bytes);
-
 // ---- corpus kernels (fv_corpus.hip) ----------------------------------------------
 // All pointers are device memory.
 int fv_dev_count_windows(const uint64_t *offsets_dev, uint64_t n_chunks, uint64_t w,

@@ -172,7 +172,7 @@ static int fv_launch_to_row_major(const float *Wt, float *W, uint64_t pitch, uin
 
 // The device's address of `bytes` of page-locked host memory at p (hipHostMalloc), or null where the range is anything
 // else: pageable, or not inside one allocation.
-void *fv_device_view(const void *p, size_t bytes) {
+static void *fv_device_view(const void *p, size_t bytes) {
   hipPointerAttribute_t at;
   void *base = nullptr;
   size_t size = 0;

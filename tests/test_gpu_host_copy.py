@@ -16,7 +16,7 @@ SLOT_COLUMNS = 16384  # columns of a 64-row tile that fills a slot of 4 MB
                                  (2048, 512), (2047, 514), (400, 5242), (400, 5244)])
 def test_matrices_through_the_slots(gpu, K, N):
     """Upload and download at tile edges (rows beside 64, columns beside a slot's), beside the largest matrix that goes
-    in one piece (4 MB) and the smallest that goes up in tiles (8 MB), pageable and page-locked on either side; the pad columns of the device's rows are zero again after a larger matrix's upload has been read."""
+    in one piece (4 MB) and the smallest that goes up in tiles (8 MB), pageable and page-locked on either side."""
     from flyvec_amd import Hasher, Trainer, _lib
     W = np.random.default_rng(K).standard_normal((K, N), dtype=np.float32)
     locked = _lib.pinned_empty(W.shape, np.float32)
@@ -200,14 +200,15 @@ def test_more_transfers_at_once_than_there_are_slots(gpu):
     assert not bad
 
 
-@pytest.mark.parametrize("K,w,n", [(400, 1, 1), (400, 1, 648), (400, 1, 649), (400, 1, 20000), (70, 11, 2300),
-                                   (70, 11, 2301), (70, 11, 100003), (400, 11, 40001)])
+@pytest.mark.parametrize("K,w,n", [(400, 1, 1), (400, 1, 569), (400, 1, 570), (400, 1, 648), (400, 1, 649), (400, 1, 20000),
+                                   (70, 11, 2016), (70, 11, 2017), (70, 11, 2299), (70, 11, 2300), (70, 11, 2301),
+                                   (70, 11, 100003), (400, 11, 40001)])
 @pytest.mark.parametrize("locked", [False, True])
 def test_hash_batches_of_every_route(gpu, K, w, n, locked):
-    """Codes and packed codes from host arrays, beside the largest batch that goes through the one buffer (2^18 bytes of
-    indices and codes: 648 targets of 400 neurons, 2299 windows of 11 with 70 neurons and two words), one chunk and
-    several, against the device-resident call on the same indices. An index out of range is reported by every route
-    and leaves the next call clean."""
+    """Codes and packed codes from host arrays, beside the largest batches that go through the one buffer (2^18 bytes of
+    indices and codes: of one target with 400 neurons 569 with both kinds of code and 648 with plain codes only, of
+    windows of 11 with 70 neurons 2016 and 2299), one chunk and several, against the device-resident call on the same
+    indices. An index out of range is reported by every route and leaves the next call clean."""
     from flyvec_amd import Hasher, _lib
     V = 500
     rng = np.random.default_rng(n)

@@ -4,10 +4,12 @@
 // The other way is the runtime's copy of such memory, for a matrix with a staging matrix on the device. Both sides
 // measured with pauses and new arrays between the calls, as set-up calls come (microseconds, runtime against slots; two
 // runs each; back to back the slots do a little better):
-//   upload    8 MB 486-490, 782-876;  16 MB 966-969, 1022-1197;  24 MB 1572-1587, 1515-1659;  32 MB 2053-2124,
-//             1863-1872;  64 MB 4120, 3680: the runtime reads the caller's pages at 17 GB/s, four threads at little more
-//   download  8 MB 478-492, 477-509;  12 MB 698-748, 702-718 (both in pieces of 512 KB);  16 MB 927-946, 497 (whole
-//             slots);  64 MB 6300, 1950 (the result's pages are touched for the first time, by four threads)
+//   upload    8 MB 480-560, 590-650;  12 MB 700-850, 810-920;  16 MB on one machine 920-970, 1020-1045, on another 1120-1190,
+//             1040-1170;  24 MB 1570-1590, 1515-1660 and 1710-1800, 1490-1530;  32 MB 2030-2120, 1840-1990;  64 MB 4120,
+//             3680: the runtime reads the caller's pages at 17 GB/s, four threads at little more
+//   download  4 MB 250, 280 (in eight pieces);  5 MB 316-390, 213-242;  8 MB 480-610, 284-316;  16 MB 930-960, 470-505;
+//             64 MB 6300, 1950 (the result's pages are touched for the first time, by four threads). In pieces of 512 KB
+//             instead of whole slots 8 MB took 480-560 and 14 MB 775-800.
 //   matrix up, K = 400: 6 MB 314-337, 314-335, with the hasher around it 368-412, 415-496;  8 MB 376-411, 346-381 and
 //             426-471, 432-521;  12 MB 519-530, 442-456 and 558-611, 535-562;  64 MB 2430, 1680 and 2500, 1900.  In one
 //             piece: 0.25 MB 52, 50;  1 MB 70-81, 77;  4 MB 232-254, 228
@@ -25,8 +27,8 @@
 #define FV_STAGE_SLOTS_LEASED 4 /* by one transfer */
 #define FV_STAGE_TILE_ROWS 64u  /* of a matrix that goes in several pieces */
 
-#define FV_STAGE_UP_BYTES ((size_t)32 << 20)        /* plain uploads through the slots from here on */
-#define FV_STAGE_DOWN_BYTES ((size_t)16 << 20)      /* plain downloads */
+#define FV_STAGE_UP_BYTES ((size_t)24 << 20)        /* plain uploads through the slots from here on */
+#define FV_STAGE_DOWN_BYTES ((size_t)5 << 20)       /* plain downloads */
 #define FV_STAGE_MATRIX_UP_BYTES ((size_t)8 << 20)  /* matrices upwards, and those that fit one slot; downwards all */
 
 static inline int fv_upload_staged(size_t bytes) { return bytes >= FV_STAGE_UP_BYTES; }
@@ -37,6 +39,9 @@ static inline int fv_matrix_upload_staged(size_t bytes) {
 
 /* Pieces of a plain copy: whole slots and a rest. */
 static inline uint64_t fv_copy_pieces(size_t bytes) { return (bytes + FV_STAGE_SLOT_BYTES - 1) / FV_STAGE_SLOT_BYTES; }
+static inline unsigned fv_copy_slots(size_t bytes) {
+  return bytes < FV_STAGE_SLOTS_LEASED * FV_STAGE_SLOT_BYTES ? (unsigned)fv_copy_pieces(bytes) : FV_STAGE_SLOTS_LEASED;
+}
 static inline size_t fv_copy_piece_bytes(size_t bytes, uint64_t t) {
   const size_t left = bytes - (size_t)t * FV_STAGE_SLOT_BYTES;
   return left < FV_STAGE_SLOT_BYTES ? left : FV_STAGE_SLOT_BYTES;

@@ -310,7 +310,7 @@ static bool fv_pageable_range(const void *host, size_t bytes) {
 
 int fv_copy_up(void *dst_dev, const void *src_host, size_t bytes, hipStream_t stream) {
   if (bytes == 0) return FV_OK;
-  fv_stage_lease lease(fv_upload_staged(bytes) && fv_pageable_range(src_host, bytes) ? FV_STAGE_SLOTS_LEASED : 0);
+  fv_stage_lease lease(fv_upload_staged(bytes) && fv_pageable_range(src_host, bytes) ? fv_copy_slots(bytes) : 0);
   if (!lease.n) {
     FV_HIP(hipMemcpyAsync(dst_dev, src_host, bytes, hipMemcpyHostToDevice, stream));
     return FV_OK;
@@ -329,7 +329,7 @@ int fv_copy_up(void *dst_dev, const void *src_host, size_t bytes, hipStream_t st
 
 int fv_copy_down(void *dst_host, const void *src_dev, size_t bytes, hipStream_t stream) {
   if (bytes == 0) return FV_OK;
-  fv_stage_lease lease(fv_download_staged(bytes) && fv_pageable_range(dst_host, bytes) ? FV_STAGE_SLOTS_LEASED : 0);
+  fv_stage_lease lease(fv_download_staged(bytes) && fv_pageable_range(dst_host, bytes) ? fv_copy_slots(bytes) : 0);
   if (!lease.n) {
     FV_HIP(hipMemcpyAsync(dst_host, src_dev, bytes, hipMemcpyDeviceToHost, stream));
     FV_HIP(hipStreamSynchronize(stream));

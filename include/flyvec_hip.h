@@ -49,7 +49,7 @@ int fv_device_memory(uint64_t *out_free_bytes, uint64_t *out_total_bytes);
 int fv_host_alloc_pinned(size_t bytes, void **out_ptr);
 int fv_host_free_pinned(void *ptr);
 
-/* Matrices (upwards those of up to 4 MB and of 8 MB and more), other uploads of 32 MB, downloads of 16 MB and batches with
+/* Matrices (upwards those of up to 4 MB and of 8 MB and more), other uploads of 24 MB, downloads of 5 MB and batches with
  * codes of 4 MB and more between the device and ordinary host memory go through page-locked memory, up to 32 MB of it,
  * that the library keeps for the transfers that follow, with a stream per batch in flight. release returns what no
  * transfer is using to the system (the next one takes it anew); held tells how much memory there is; limit sets the most

@@ -6,6 +6,7 @@ int fvt_upload_staged(uint64_t bytes) { return fv_upload_staged(bytes); }
 int fvt_download_staged(uint64_t bytes) { return fv_download_staged(bytes); }
 int fvt_matrix_upload_staged(uint64_t bytes) { return fv_matrix_upload_staged(bytes); }
 uint64_t fvt_copy_pieces(uint64_t bytes) { return fv_copy_pieces(bytes); }
+uint64_t fvt_copy_slots(uint64_t bytes) { return fv_copy_slots(bytes); }
 uint64_t fvt_copy_piece_bytes(uint64_t bytes, uint64_t t) { return fv_copy_piece_bytes(bytes, t); }
 uint64_t fvt_matrix_pieces(uint32_t K, uint64_t N) { return fv_cut_matrix(K, N).n; }
 void fvt_matrix_piece(uint32_t K, uint64_t N, uint64_t t, uint64_t *out) {

@@ -35,10 +35,10 @@ def test_matrices_through_the_slots(gpu, K, N):
     assert _lib.load().fv_host_staging_release() == 0
 
 
-@pytest.mark.parametrize("n", [1, (1 << 18) - 1, 1 << 18, (1 << 19) + 5, (1 << 21) - 1, 1 << 21, (1 << 21) + 1,
-                               (1 << 22) - 1, 1 << 22, (1 << 22) + 3])
+@pytest.mark.parametrize("n", [1, (1 << 18) - 1, 1 << 18, (1 << 19) + 5, 5 * (1 << 17) - 1, 5 * (1 << 17),
+                               (1 << 20) + 1, 3 * (1 << 20) - 1, 3 * (1 << 20), (1 << 22) + 3])
 def test_orders_through_the_slots(gpu, n):
-    """Window tables and orders of n 64-bit entries: beside the sizes from which pieces are taken (16 MB downwards, 32 MB
+    """Window tables and orders of n 64-bit entries: beside the sizes from which pieces are taken (5 MB downwards, 24 MB
     upwards), whole and broken last pieces."""
     from flyvec_amd import Trainer
     rng = np.random.default_rng(n)
@@ -69,11 +69,11 @@ def test_what_transfers_page_lock(gpu):
     assert _lib.load().fv_host_staging_release() == 0 and held() == 0
     rng = np.random.default_rng(0)
     t = Trainer(50, 8, 5, 16)
-    t.set_corpus(rng.integers(0, 50, 2 << 20).astype(np.int32), np.arange(0, (2 << 20) + 1, 64, dtype=np.uint64))
-    t.set_permutation(rng.permutation(t.num_windows).astype(np.uint64))
+    t.set_corpus_starts(rng.integers(0, 50, 2 << 20).astype(np.int32), rng.integers(0, 2 << 20, 600000).astype(np.uint64) // 2)
+    t.set_permutation(rng.permutation(600000).astype(np.uint64))
     t.get_permutation()
-    t.close()
     assert held() == 0
+    t.close()
     t = Trainer(937, 400, 5, 16)
     W = rng.standard_normal((400, 2 * 937), dtype=np.float32)
     t.set_weights(W)

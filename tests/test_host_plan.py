@@ -18,7 +18,7 @@ def shim(tmp_path_factory):
                     os.path.join(ROOT, "tests", "native", "host_plan_shim.c"), "-o", str(out)], check=True)
     lib = C.CDLL(str(out))
     u64, u32 = C.c_uint64, C.c_uint32
-    for name, args in (("fvt_slot_bytes", []), ("fvt_copy_pieces", [u64]), ("fvt_copy_piece_bytes", [u64, u64]),
+    for name, args in (("fvt_slot_bytes", []), ("fvt_copy_pieces", [u64]), ("fvt_copy_slots", [u64]), ("fvt_copy_piece_bytes", [u64, u64]),
                        ("fvt_matrix_pieces", [u32, u64])):
         getattr(lib, name).restype = u64
         getattr(lib, name).argtypes = args
@@ -31,21 +31,22 @@ def shim(tmp_path_factory):
 
 
 def test_small_and_middling_transfers_stay_with_the_runtime(shim):
-    """Where the slots were measured to be no faster: uploads below 32 MB, downloads below 16 MB, matrices between one
+    """Where the slots were measured to be no faster: uploads below 24 MB, downloads below 5 MB, matrices between one
     slot and 8 MB upwards."""
-    for up, down, matrix, size in ((0, 0, 1, 1), (0, 0, 1, 4 * MB), (0, 0, 0, 4 * MB + 4), (0, 0, 0, 8 * MB - 4),
-                                   (0, 0, 1, 8 * MB), (0, 0, 1, 16 * MB - 1), (0, 1, 1, 16 * MB), (0, 1, 1, 32 * MB - 1),
-                                   (1, 1, 1, 32 * MB), (1, 1, 1, 1 << 40)):
+    for up, down, matrix, size in ((0, 0, 1, 1), (0, 0, 1, 4 * MB), (0, 0, 0, 4 * MB + 4), (0, 0, 0, 5 * MB - 1), (0, 1, 0, 5 * MB),
+                                   (0, 1, 0, 8 * MB - 4), (0, 1, 1, 8 * MB), (0, 1, 1, 24 * MB - 1), (1, 1, 1, 24 * MB),
+                                   (1, 1, 1, 1 << 40)):
         got = shim.fvt_upload_staged(size), shim.fvt_download_staged(size), shim.fvt_matrix_upload_staged(size)
         assert tuple(map(bool, got)) == (bool(up), bool(down), bool(matrix)), size
 
 
-@pytest.mark.parametrize("size", [16 * MB, 16 * MB + 1, 20 * MB - 1, 33 * MB + 24])
+@pytest.mark.parametrize("size", [5 * MB, 8 * MB, 8 * MB + 1, 16 * MB, 16 * MB + 1, 20 * MB - 1, 33 * MB + 24])
 def test_pieces_of_a_plain_copy(shim, size):
     n = shim.fvt_copy_pieces(size)
     sizes = [shim.fvt_copy_piece_bytes(size, t) for t in range(n)]
     assert sum(sizes) == size and min(sizes) > 0 and max(sizes) <= shim.fvt_slot_bytes()
     assert all(s == shim.fvt_slot_bytes() for s in sizes[:-1])
+    assert shim.fvt_copy_slots(size) == min(n, 4)
 
 
 @pytest.mark.parametrize("K,N", [(1, 2), (2048, 2), (400, 1874), (400, 2620), (400, 2622), (64, 16384), (64, 16386),

@@ -105,7 +105,7 @@ __global__ __launch_bounds__(256) void fv_identity_kernel(const uint64_t *__rest
 // The reshuffle of flyvec/src/model_arrays.cu:451-465 rearranges the current order, cumulatively
 // over the epochs; here out[i] = in[sigma(i)] with sigma a keyed bijection computed per index. (The table in a launch
 // of its own behind it: two random reads one behind the other in one launch took 97 us for 2.6 M windows, the two
-// launches 45 + 29.)
+// launches 46 + 45.)
 __global__ __launch_bounds__(256) void fv_shuffle_kernel(const uint64_t *__restrict__ in, uint64_t *__restrict__ out,
                                                          uint64_t n, fv_feistel f) {
   for (uint64_t i = (uint64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (uint64_t)gridDim.x * 256)

@@ -417,9 +417,7 @@ static void fv_choose_onepass(fv_trainer *t, uint64_t cu) {
     bool set = true;
 #define FV_SET(KERNEL)                                                                                              \
   set = set && hipFuncSetAttribute((const void *)KERNEL, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem) == hipSuccess;
-    FV_SET((fv_dense_stream_kernel<false, 0>)) FV_SET((fv_dense_stream_kernel<true, 0>))
-    FV_SET((fv_dense_stream_kernel<false, 1>)) FV_SET((fv_dense_stream_kernel<true, 1>))
-    FV_SET((fv_dense_stream_kernel<false, 2>)) FV_SET((fv_dense_stream_kernel<true, 2>))
+    FV_SET(fv_dense_stream_kernel<0>) FV_SET(fv_dense_stream_kernel<1>) FV_SET(fv_dense_stream_kernel<2>)
 #undef FV_SET
     if (set)
       t->stream_ok = fv_stream_fits(smem) != 0;
@@ -435,9 +433,9 @@ static void fv_choose_onepass(fv_trainer *t, uint64_t cu) {
       bool set = true;
 #define FV_SET(KERNEL)                                                                                              \
   set = set && hipFuncSetAttribute((const void *)KERNEL, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem) == hipSuccess;
-#define FV_SET_PHASES(U, DELTA) \
-  FV_SET((fv_dense_onepass_kernel<U, DELTA, 0>)) FV_SET((fv_dense_onepass_kernel<U, DELTA, 1>)) FV_SET((fv_dense_onepass_kernel<U, DELTA, 2>))
-      if (unroll == 8) { FV_SET_PHASES(8, false) FV_SET_PHASES(8, true) } else { FV_SET_PHASES(16, false) FV_SET_PHASES(16, true) }
+#define FV_SET_PHASES(U) \
+  FV_SET((fv_dense_onepass_kernel<U, 0>)) FV_SET((fv_dense_onepass_kernel<U, 1>)) FV_SET((fv_dense_onepass_kernel<U, 2>))
+      if (unroll == 8) { FV_SET_PHASES(8) } else { FV_SET_PHASES(16) }
 #undef FV_SET_PHASES
 #undef FV_SET
       if (!set) {
@@ -730,22 +728,19 @@ static void fv_trainer_free_delta(fv_trainer *t) {
   (void)hipFree(t->group_base2);
   (void)hipFree(t->group_count2);
   (void)hipFree(t->slots2);
-  (void)hipFree(t->slot_n2);
   (void)hipFree(t->won2[0]);
   (void)hipFree(t->slots2_blocks);
-  (void)hipFree(t->slot_n2_blocks);
   t->won2[0] = t->won2[1] = nullptr;
   t->slots2_blocks = nullptr;
-  t->slot_n2_blocks = nullptr;
   t->win2 = nullptr;
   t->win2_16 = nullptr;
   t->sc2 = nullptr;
-  t->order2 = t->group_base2 = t->group_count2 = t->slot_n2 = nullptr;
+  t->order2 = t->group_base2 = t->group_count2 = nullptr;
   t->slots2 = nullptr;
 }
 
 static int fv_trainer_alloc_delta(fv_trainer *t) {
-  if (t->slot_n2) return FV_OK;  // the last one allocated: all are there
+  if (t->slots2) return FV_OK;  // the last one allocated: all are there
   fv_trainer_free_delta(t);      // what an earlier, failed attempt left
   const size_t B = t->B, bw = (size_t)t->B * t->w;
   FV_HIP(hipMalloc((void **)&t->win2, B * sizeof(int32_t)));
@@ -755,7 +750,6 @@ static int fv_trainer_alloc_delta(fv_trainer *t) {
   FV_HIP(hipMalloc((void **)&t->order2, B * sizeof(uint32_t)));
   FV_HIP(hipMalloc((void **)&t->group_base2, (size_t)t->K * sizeof(uint32_t)));
   FV_HIP(hipMalloc((void **)&t->group_count2, (size_t)t->K * sizeof(uint32_t)));
-  FV_HIP(hipMalloc((void **)&t->slots2, 2 * FV_NB_CLASSES * bw * sizeof(fv_slot)));
   // The form that groups inside the sparse launch: bit rows for the second neurons, and a slot region per block. A
   // block writes at most one record per column of its class; the regions are that long only where a class has no
   // more columns than the minibatch has window positions (fv_trainer_alloc), else this form is not taken.
@@ -767,9 +761,8 @@ static int fv_trainer_alloc_delta(fv_trainer *t) {
     t->won2[1] = t->won2[0] + row_words;
     FV_HIP(hipMemsetAsync(t->won2[0], 0, 2 * row_words * sizeof(uint32_t), t->stream));
     FV_HIP(hipMalloc((void **)&t->slots2_blocks, records * sizeof(fv_slot)));
-    FV_HIP(hipMalloc((void **)&t->slot_n2_blocks, records * sizeof(uint32_t)));
   }
-  FV_HIP(hipMalloc((void **)&t->slot_n2, 2 * FV_NB_CLASSES * bw * sizeof(uint32_t)));
+  FV_HIP(hipMalloc((void **)&t->slots2, 2 * FV_NB_CLASSES * bw * sizeof(fv_slot)));
   return FV_OK;
 }
 
@@ -830,7 +823,7 @@ static int fv_enqueue_step(fv_trainer *t, uint64_t first, uint32_t n, float eps,
   // on the last step's pair, cleared here first unless it repeats the launch before it.
   // (beyond 64 windows per thread of a class block only with a slot region per block: without one every block
   // would count the lower neurons' windows in the whole winner array)
-  const bool can_group = fv_groups_in_sparse(t) && (!anti || (t->slot_n2_blocks && !t->no_block_regions));
+  const bool can_group = fv_groups_in_sparse(t) && (!anti || (t->slots2_blocks && !t->no_block_regions));
   const bool grouping_in_sparse = which == 0x3f ? can_group : (anti ? t->last_delta_grouped : t->last_grouped_in_sparse);
   if (which == 0x3f) (anti ? t->last_delta_grouped : t->last_grouped_in_sparse) = grouping_in_sparse;
   // the blocks of a sparse launch that groups for itself write their records to regions of their own, where
@@ -922,7 +915,6 @@ static int fv_enqueue_step(fv_trainer *t, uint64_t first, uint32_t n, float eps,
   sp.order2 = t->order2;
   sp.group_base2 = t->group_base2;
   sp.group_count2 = t->group_count2;
-  sp.slot_n2 = anti && slot_region ? t->slot_n2_blocks : t->slot_n2;
   sp.delta = delta;
   sp.lmid = t->cfg.lmid;
   sp.lbase = t->cfg.lbase;
@@ -983,7 +975,6 @@ static int fv_enqueue_step(fv_trainer *t, uint64_t first, uint32_t n, float eps,
   fv_dense_args d;
   d.Wt4 = (float4 *)t->Wt;
   d.xx = t->xx;
-  d.invf = t->invf;
   d.slots = anti ? (slot_region ? t->slots2_blocks : t->slots2) : slot_region ? t->slots_blocks : t->slots;
   d.slot_region = slot_region;
   {
@@ -994,15 +985,11 @@ static int fv_enqueue_step(fv_trainer *t, uint64_t first, uint32_t n, float eps,
   d.slot_count = t->slot_count;
   d.group_base = t->group_base;
   d.group_base2 = t->group_base2;
-  d.slot_n2 = anti && slot_region ? t->slot_n2_blocks : t->slot_n2;
-  d.delta = delta;
   d.w = t->w;
   d.arrive = nullptr;
   d.status = nullptr;
   d.phase = 0;
   d.epoch = d.spin_limit = d.step_tag = 0;
-  d.lmid = t->cfg.lmid;
-  d.lbase = t->cfg.lbase;
   d.corpus = t->corpus;
   d.pstart = t->pstart;
   d.idx_ahead = nullptr;
@@ -1053,20 +1040,15 @@ static int fv_enqueue_step(fv_trainer *t, uint64_t first, uint32_t n, float eps,
         t->ahead_n = d.ahead_n;
       }
       const size_t smem1 = fv_onepass_smem(t);
-#define FV_CASE(U)                                                                     \
-  if (anti) fv_launch_onepass<U, true>(d, t->onepass_blocks, smem1, t->stream);        \
-  else fv_launch_onepass<U, false>(d, t->onepass_blocks, smem1, t->stream);
       // no other trainer in flight: one launch that exchanges the blocks' maxima itself where it needs them; else the
       // launch twice, in the form that waits for nobody (both with this step's launch number)
       t->dense_forms[alone ? 0 : 1]++;
       for (uint32_t phase = alone ? 0u : 1u; phase <= (alone ? 0u : 2u); ++phase) {
         d.phase = phase;
-        if (t->onepass_stream) {
-          if (anti) fv_launch_stream<true>(d, t->onepass_blocks, fv_stream_smem(t), t->stream);
-          else fv_launch_stream<false>(d, t->onepass_blocks, fv_stream_smem(t), t->stream);
-        } else if (t->onepass_unroll == 8) { FV_CASE(8) } else { FV_CASE(16) }
+        if (t->onepass_stream) fv_launch_stream(d, t->onepass_blocks, fv_stream_smem(t), t->stream);
+        else if (t->onepass_unroll == 8) fv_launch_onepass<8>(d, t->onepass_blocks, smem1, t->stream);
+        else fv_launch_onepass<16>(d, t->onepass_blocks, smem1, t->stream);
       }
-#undef FV_CASE
       t->top2_valid = true;  // this launch leaves the shares of the matrix it writes
       t->top2_n_part = t->onepass_blocks;
       t->top2_merged = false;  // the next winner kernel's first blocks merge them

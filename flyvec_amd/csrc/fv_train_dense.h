@@ -9,14 +9,11 @@
 struct fv_dense_args {
   float4 *Wt4;
   const float *xx;
-  const float *invf;
   const fv_slot *slots;  // FV_NB_CLASSES regions of slot_stride records
   uint64_t slot_stride;
   const uint32_t *slot_count;  // records of each block of the sparse launch
   const uint32_t *group_base;
-  const uint32_t *group_base2;  // anti-Hebbian form only, like slot_n2 and delta
-  const uint32_t *slot_n2;
-  float delta;
+  const uint32_t *group_base2;  // anti-Hebbian form only
   float *bmax;           // n_bmax block maxima of |ds|: dense blocks, then the sparse kernel's blocks
   float *scalars;
   uint32_t total4, ldk4, ldk, V, K, w, n_bmax, dense_blocks;
@@ -26,7 +23,6 @@ struct fv_dense_args {
   uint32_t *status;
   uint32_t epoch, spin_limit;
   uint32_t step_tag;  // what a launch that gives up leaves in *status (not 0)
-  float lmid, lbase;  // weight of a window's centre position (elements p >= V * ldk) and of the others
   // the minibatch sampled ahead (ahead_n = 0: none)
   const int32_t *corpus;
   const uint64_t *pstart;
@@ -331,7 +327,7 @@ __global__ __launch_bounds__(TB) void fv_update_kernel(fv_dense_args a) {
 // The sparse elements are finished here as well, by the block that owns them: a thread that meets a
 // sentinel leaves it alone and notes (sentinel, element) in its wave's LDS list; when the wave has updated its
 // dense elements it deals its list over its lanes, each of which finds the record through the sentinel's
-// number, forms ds and writes the element. No other block ever reads or writes that element in this launch.
+// number and writes the element from its weight and ds. No other block ever reads or writes that element in this launch.
 // (A list per wave, not per block: the wave asks for its records as soon as its own last store is issued,
 // without a barrier, so the records travel while the stores drain -- a wave's loads and stores share one
 // counter, and a load asked for behind the block's barrier would begin its trip only when the drain is over.)
@@ -360,11 +356,17 @@ __device__ __forceinline__ void fv_top2_insert_lds(uint32_t *s1, uint32_t *s2, u
   atomicMax(&s2[h], min(old, b));
 }
 
+// The final value of a sparse element: its saved weight, updated where the update is not below the cut (ds is 0 in a row
+// with xx = 0, which is not updated) and the launch has not given up.
+__device__ __forceinline__ float fv_slot_final(const fv_slot &sl, float s, bool ok, float cut) {
+  const float d = __fmul_rn(s, sl.ds);
+  return ok && fabsf(d) > cut ? __fadd_rn(sl.wv, d) : sl.wv;
+}
+
 // The element p holds the sentinel `bits`: its final value from the record the sentinel names. The saved
 // weight goes back where the row is not updated (xx == 0) or the launch gave up, else the updated one.
-template <bool DELTA>
 __device__ __forceinline__ void fv_finish_sparse_element(const fv_dense_args &a, uint32_t bits, uint32_t p, float s,
-                                                         bool ok, const float *xs, uint32_t *sp1, uint32_t *sp2) {
+                                                         bool ok, uint32_t *sp1, uint32_t *sp2) {
   const uint32_t number = (bits & FV_SENTINEL_MAX) - 1u;
   if (number >= a.n_slots) return;  // a NaN of another origin stays what it is
   const uint32_t col = p / a.ldk, h = p - col * a.ldk;
@@ -375,15 +377,7 @@ __device__ __forceinline__ void fv_finish_sparse_element(const fv_dense_args &a,
                                     : number;
   const fv_slot sl = a.slots[at];
   if (sl.p != p) return;
-  const float x = xs[h];
-  float out = sl.wv;
-  if (ok && x != 0.0f) {
-    const float l = p >= a.V * a.ldk ? a.lmid : a.lbase;
-    const float ds = DELTA ? fv_sparse_ds2(x, sl.wv, sl.f, sl.n, a.delta, a.slot_n2[at], l)
-                           : fv_sparse_ds(x, sl.wv, sl.f, sl.n, l);
-    const float d = __fmul_rn(s, ds);
-    if (fabsf(d) > a.update_cut) out = __fadd_rn(sl.wv, d);
-  }
+  const float out = fv_slot_final(sl, s, ok, a.update_cut);
   ((float *)a.Wt4)[p] = out;
   fv_top2_insert_lds(sp1, sp2, h, fv_abs_or_zero(out));
 }
@@ -391,14 +385,11 @@ __device__ __forceinline__ void fv_finish_sparse_element(const fv_dense_args &a,
 // The sentinels of a list, dealt over `width` threads (this one is number `me` of them), four records in flight per
 // thread: a wave that has met a row of a frequent token holds a few hundred of them, and one after the other each
 // would be a trip to memory of its own.
-template <bool DELTA>
 __device__ __forceinline__ void fv_finish_sparse_elements(const fv_dense_args &a, const uint2 *list, uint32_t n, uint32_t me,
-                                                          uint32_t width, float s, bool ok, const float *xs, uint32_t *sp1,
-                                                          uint32_t *sp2) {
+                                                          uint32_t width, float s, bool ok, uint32_t *sp1, uint32_t *sp2) {
   for (uint32_t i0 = me; i0 < n; i0 += 4 * width) {
     uint2 hit[4];
     fv_slot sl[4];
-    uint32_t n2[4];
     bool mine[4];
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
@@ -410,22 +401,13 @@ __device__ __forceinline__ void fv_finish_sparse_elements(const fv_dense_args &a
                                                         a.slot_region, a.K * FV_NB_CLASSES)
                                         : number;
       sl[u] = a.slots[mine[u] ? at : 0];
-      n2[u] = DELTA ? a.slot_n2[mine[u] ? at : 0] : 0u;
     }
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
       const uint32_t p = hit[u].y;
       if (!mine[u] || sl[u].p != p) continue;
       const uint32_t h = p % a.ldk;
-      const float x = xs[h];
-      float out = sl[u].wv;
-      if (ok && x != 0.0f) {
-        const float l = p >= a.V * a.ldk ? a.lmid : a.lbase;
-        const float ds = DELTA ? fv_sparse_ds2(x, sl[u].wv, sl[u].f, sl[u].n, a.delta, n2[u], l)
-                               : fv_sparse_ds(x, sl[u].wv, sl[u].f, sl[u].n, l);
-        const float d = __fmul_rn(s, ds);
-        if (fabsf(d) > a.update_cut) out = __fadd_rn(sl[u].wv, d);
-      }
+      const float out = fv_slot_final(sl[u], s, ok, a.update_cut);
       ((float *)a.Wt4)[p] = out;
       fv_top2_insert_lds(sp1, sp2, h, fv_abs_or_zero(out));
     }
@@ -603,7 +585,7 @@ static_assert(FV_NB_CLASSES == 4, "a neuron's block maxima and hit counts are re
 
 // PHASE: fv_dense_args.phase, fixed at compile time (the branches of the other phases cost the register form
 // its last registers).
-template <int U, bool DELTA, int PHASE = 0>
+template <int U, int PHASE = 0>
 __global__ __launch_bounds__(FV_ONEPASS_THREADS) void fv_dense_onepass_kernel(fv_dense_args a) {
   constexpr uint32_t T = FV_ONEPASS_THREADS;
   constexpr int DEPTH = FV_ONEPASS_DEPTH < U ? FV_ONEPASS_DEPTH : U;
@@ -800,13 +782,13 @@ __global__ __launch_bounds__(FV_ONEPASS_THREADS) void fv_dense_onepass_kernel(fv
   __builtin_amdgcn_s_setprio(0);
   {
     const uint32_t n_hits = min(*wave_hits, a.hit_cap);
-    fv_finish_sparse_elements<DELTA>(a, wave_list, n_hits, tid & 63u, 64u, s, ok, xs, sp1, sp2);
+    fv_finish_sparse_elements(a, wave_list, n_hits, tid & 63u, 64u, s, ok, sp1, sp2);
   }
   while (beyond_list) {
     const uint32_t b = (uint32_t)__ffsll((long long)beyond_list) - 1u;
     beyond_list &= beyond_list - 1;
     const uint32_t at = 4u * ((row0 + (b >> 2) * row_step) * a.ldk4 + q) + (b & 3u);
-    fv_finish_sparse_element<DELTA>(a, __float_as_uint(((const float *)a.Wt4)[at]), at, s, ok, xs, sp1, sp2);
+    fv_finish_sparse_element(a, __float_as_uint(((const float *)a.Wt4)[at]), at, s, ok, sp1, sp2);
   }
   if (active) {
 #pragma unroll
@@ -836,7 +818,7 @@ __global__ __launch_bounds__(FV_ONEPASS_THREADS) void fv_dense_onepass_kernel(fv
 #endif
 #define FV_STREAM_HIT_CAP 8192  // sentinels a block notes in LDS (64 KB)
 
-template <bool DELTA, int PHASE = 0>
+template <int PHASE = 0>
 __global__ __launch_bounds__(FV_ONEPASS_THREADS) void fv_dense_stream_kernel(fv_dense_args a) {
   constexpr uint32_t T = FV_ONEPASS_THREADS;
   constexpr int D = FV_STREAM_DEPTH;
@@ -973,7 +955,7 @@ __global__ __launch_bounds__(FV_ONEPASS_THREADS) void fv_dense_stream_kernel(fv_
     if (k < a.hit_cap)                                                                         \
       hit_list[k] = make_uint2(__float_as_uint(v.member), 4u * p4 + lane4);                    \
     else                                                                                       \
-      fv_finish_sparse_element<DELTA>(a, __float_as_uint(v.member), 4u * p4 + lane4, s, ok, xs, sp1, sp2); \
+      fv_finish_sparse_element(a, __float_as_uint(v.member), 4u * p4 + lane4, s, ok, sp1, sp2); \
   }
   for (uint32_t c = 0; c < rounds; c += D) {
 #pragma unroll
@@ -1011,7 +993,7 @@ __global__ __launch_bounds__(FV_ONEPASS_THREADS) void fv_dense_stream_kernel(fv_
   const uint32_t n_hits = min(sh_hits, a.hit_cap);
   for (uint32_t i = tid; i < n_hits; i += T) {
     const uint2 hit = hit_list[i];
-    fv_finish_sparse_element<DELTA>(a, hit.x, hit.y, s, ok, xs, sp1, sp2);
+    fv_finish_sparse_element(a, hit.x, hit.y, s, ok, sp1, sp2);
   }
   __syncthreads();
   for (uint32_t h = tid; h < a.K; h += T) {
@@ -1026,50 +1008,44 @@ __global__ __launch_bounds__(FV_ONEPASS_THREADS) void fv_dense_stream_kernel(fv_
 }
 
 static int fv_stream_fits(size_t smem) {
-  int nb = 0, nb2 = 0;
-  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, (fv_dense_stream_kernel<false, 0>), FV_ONEPASS_THREADS, smem) !=
-          hipSuccess ||
-      hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb2, (fv_dense_stream_kernel<true, 0>), FV_ONEPASS_THREADS, smem) !=
-          hipSuccess) {
+  int nb = 0;
+  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, fv_dense_stream_kernel<0>, FV_ONEPASS_THREADS, smem) != hipSuccess) {
     (void)hipGetLastError();
     return 0;
   }
-  return nb >= 1 && nb2 >= 1;
+  return nb >= 1;
 }
 
-template <int U, bool DELTA>
+template <int U>
 static void fv_launch_onepass(const fv_dense_args &d, unsigned blocks, size_t smem, hipStream_t stream) {
   const dim3 grid(blocks), block(FV_ONEPASS_THREADS);
   if (d.phase == 0)
-    hipLaunchKernelGGL((fv_dense_onepass_kernel<U, DELTA, 0>), grid, block, smem, stream, d);
+    hipLaunchKernelGGL((fv_dense_onepass_kernel<U, 0>), grid, block, smem, stream, d);
   else if (d.phase == 1)
-    hipLaunchKernelGGL((fv_dense_onepass_kernel<U, DELTA, 1>), grid, block, smem, stream, d);
+    hipLaunchKernelGGL((fv_dense_onepass_kernel<U, 1>), grid, block, smem, stream, d);
   else
-    hipLaunchKernelGGL((fv_dense_onepass_kernel<U, DELTA, 2>), grid, block, smem, stream, d);
+    hipLaunchKernelGGL((fv_dense_onepass_kernel<U, 2>), grid, block, smem, stream, d);
 }
 
-template <bool DELTA>
 static void fv_launch_stream(const fv_dense_args &d, unsigned blocks, size_t smem, hipStream_t stream) {
   const dim3 grid(blocks), block(FV_ONEPASS_THREADS);
   if (d.phase == 0)
-    hipLaunchKernelGGL((fv_dense_stream_kernel<DELTA, 0>), grid, block, smem, stream, d);
+    hipLaunchKernelGGL(fv_dense_stream_kernel<0>, grid, block, smem, stream, d);
   else if (d.phase == 1)
-    hipLaunchKernelGGL((fv_dense_stream_kernel<DELTA, 1>), grid, block, smem, stream, d);
+    hipLaunchKernelGGL(fv_dense_stream_kernel<1>, grid, block, smem, stream, d);
   else
-    hipLaunchKernelGGL((fv_dense_stream_kernel<DELTA, 2>), grid, block, smem, stream, d);
+    hipLaunchKernelGGL(fv_dense_stream_kernel<2>, grid, block, smem, stream, d);
 }
 
 template <int U>
 static int fv_onepass_fits(size_t smem) {
-  int nb = 0, nb2 = 0;
-  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, (fv_dense_onepass_kernel<U, false, 0>), FV_ONEPASS_THREADS,
-                                                   smem) != hipSuccess ||
-      hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb2, (fv_dense_onepass_kernel<U, true, 0>), FV_ONEPASS_THREADS,
-                                                   smem) != hipSuccess) {
+  int nb = 0;
+  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, (fv_dense_onepass_kernel<U, 0>), FV_ONEPASS_THREADS, smem) !=
+      hipSuccess) {
     (void)hipGetLastError();
     return 0;
   }
-  return nb >= FV_ONEPASS_BLOCKS_PER_CU && nb2 >= FV_ONEPASS_BLOCKS_PER_CU;
+  return nb >= FV_ONEPASS_BLOCKS_PER_CU;
 }
 
 // Kernel 6: the final value of every sparse element goes over its sentinel. Runs after the dense
@@ -1095,29 +1071,16 @@ __global__ __launch_bounds__(256) void fv_slot_update_kernel(fv_dense_args a) {
   auto place_of = [&](uint32_t number) {
     return a.slot_region ? fv_slot_place(blockIdx.x, number, a.slot_region, gridDim.x) : slot_first + number;
   };
-  const float x = a.xx[h];
   const float nc = a.scalars[0];
   const float s = a.prec > nc ? a.eps / a.prec : a.eps / nc;
   for (uint32_t eb = threadIdx.x; eb < count; eb += 4 * 256) {  // four records in flight per thread
     fv_slot sl[4];
-    uint32_t n2[4];
 #pragma unroll
-    for (int u = 0; u < 4; ++u) {
-      const uint64_t place = place_of(min(eb + u * 256, count - 1));
-      sl[u] = a.slots[place];
-      n2[u] = DELTA ? a.slot_n2[place] : 0u;
-    }
+    for (int u = 0; u < 4; ++u) sl[u] = a.slots[place_of(min(eb + u * 256, count - 1))];
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
       if (eb + u * 256 >= count) break;
-      float out = sl[u].wv;  // a row with xx == 0 is not updated: the saved weight goes back
-      if (x != 0.0f) {
-        const float l = sl[u].p >= a.V * a.ldk ? a.lmid : a.lbase;
-        const float ds = DELTA ? fv_sparse_ds2(x, sl[u].wv, sl[u].f, sl[u].n, a.delta, n2[u], l)
-                               : fv_sparse_ds(x, sl[u].wv, sl[u].f, sl[u].n, l);
-        const float d = __fmul_rn(s, ds);
-        if (fabsf(d) > a.update_cut) out = __fadd_rn(sl[u].wv, d);
-      }
+      const float out = fv_slot_final(sl[u], s, true, a.update_cut);
       ((float *)a.Wt4)[sl[u].p] = out;
       fv_top2_insert(m1, m2, fv_abs_or_zero(out));
     }

@@ -8,8 +8,11 @@
 // FV_NB_CLASSES blocks per neuron h; block q owns the elements (h, column i) with
 // i mod FV_NB_CLASSES == q, so a neuron that won a large share of the minibatch is spread over
 // several blocks and no two blocks share an element.  A block counts the occurrences of each of
-// its columns over the neuron's windows in LDS, and for every distinct one saves
-// (element, count, weight) in a slot record and plants the sentinel in W.
+// its columns over the neuron's windows in LDS, and for every distinct one saves (element, weight, ds) in a slot
+// record and plants the sentinel in W. (ds with the record: the dense launch, which used to form it again from the
+// count, spent up to 7 us on that behind its stream, in the waves that held a frequent token's row. An epoch of 101
+// steps at K = 400, V = 20000, w = 11, B = 10000 took 6770 us and takes 6490, 41 steps with the anti-Hebbian term 4430
+// and 4100, 101 steps at K = 209, V = 7919, w = 7, B = 3001 3170 and 3030.)
 
 struct fv_sparse_args {
   const uint32_t *order;
@@ -30,12 +33,10 @@ struct fv_sparse_args {
   uint32_t *slot_count;  // records written per block
   uint32_t ldk, w, V, pad_row;  // pad_row: the row index just behind the index matrix
   uint32_t stride;              // entries per row of idx (a multiple of 4)
-  // anti-Hebbian form only: the windows in which the neuron came second, grouped like the others;
-  // the count of those occurrences of an element goes to slot_n2 beside its record
+  // anti-Hebbian form only: the windows in which the neuron came second, grouped like the others
   const uint32_t *order2;
   const uint32_t *group_base2;
   const uint32_t *group_count2;
-  uint32_t *slot_n2;
   float delta;
   float lmid, lbase;  // weight of a window's centre position (columns >= V) and of the others
   // grouping form only: the block finds the neuron's windows in the winner array itself
@@ -213,18 +214,19 @@ __device__ __forceinline__ void fv_sparse_light(const fv_sparse_args &a, uint32_
         cnt[at] = 0;  // zero again for the next class
       else
         atomicAnd(&cnt[at], 0xffff0000u >> shift);
+      a.Wt[p] = fv_sentinel(number);
       fv_slot rec;
       rec.p = p;
       rec.n = n;
       rec.wv = wv;
-      rec.f = f;
+      rec.ds = 0.0f;
+      if (x_h != 0.0f) {
+        rec.ds = DELTA ? fv_sparse_ds2(x_h, wv, f, n, a.delta, n2, l) : fv_sparse_ds(x_h, wv, f, n, l);
+        ds_max = fv_absmax_keep(ds_max, rec.ds);
+      }
       // (fv_slot_place for a number below the block's threads, which is below FV_SLOT_PRIMARY or below the region)
       const uint64_t place = ((h << FV_NB_CLASS_SHIFT) | q) * min(a.slot_region, FV_SLOT_PRIMARY) + number;
       a.slots[place] = rec;
-      if (DELTA) a.slot_n2[place] = n2;
-      a.Wt[p] = fv_sentinel(number);
-      if (x_h != 0.0f)
-        ds_max = fv_absmax_keep(ds_max, DELTA ? fv_sparse_ds2(x_h, wv, f, n, a.delta, n2, l) : fv_sparse_ds(x_h, wv, f, n, l));
     }
     const float aw = fabsf(wv);
     hits1 += (uint32_t)__popcll(__ballot(owner && aw == top2.x));
@@ -703,19 +705,20 @@ __device__ __forceinline__ void fv_sparse_block(const fv_sparse_args &a) {
             rec.p = pe[u];
             rec.n = ne[u];
             rec.wv = wv[u];
-            rec.f = fe[u];
+            rec.ds = 0.0f;
             const uint32_t number = emitted + eb + u * T;
             const uint64_t place = round_place + number;
-            a.slots[place] = rec;
-            if (DELTA) a.slot_n2[place] = n2e[u];
             a.Wt[pe[u]] = fv_sentinel(record0 + eb + u * T);
             // counted per wave from lane masks: the counts stay in scalar registers
             const float aw = fabsf(wv[u]);
             hits1 += (uint32_t)__popcll(__ballot(aw == top2.x));
             hits2 += (uint32_t)__popcll(__ballot(aw == top2.y && top2.y < top2.x));
-            if (x_h != 0.0f)
-              ds_max = fv_absmax_keep(ds_max, DELTA ? fv_sparse_ds2(x_h, wv[u], fe[u], ne[u], a.delta, n2e[u], le[u])
-                                                    : fv_sparse_ds(x_h, wv[u], fe[u], ne[u], le[u]));
+            if (x_h != 0.0f) {
+              rec.ds = DELTA ? fv_sparse_ds2(x_h, wv[u], fe[u], ne[u], a.delta, n2e[u], le[u])
+                             : fv_sparse_ds(x_h, wv[u], fe[u], ne[u], le[u]);
+              ds_max = fv_absmax_keep(ds_max, rec.ds);
+            }
+            a.slots[place] = rec;
           }
       }
       emitted += take;

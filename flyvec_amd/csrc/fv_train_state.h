@@ -27,9 +27,9 @@ __device__ __forceinline__ float fv_sentinel(uint32_t record) {
 
 struct __attribute__((aligned(16))) fv_slot {
   uint32_t p;  // element index i * ldk + h
-  uint32_t n;  // pending additions of 1/f
+  float ds;    // ds of the element: the dense term and its additions of 1/f (0 in a row with xx = 0)
   float wv;    // the weight the sentinel replaced
-  float f;     // 1/f of the element's token
+  uint32_t n;  // the additions of 1/f (with the anti-Hebbian term those of the first list); fills the 16 bytes
 };
 
 struct fv_trainer {
@@ -69,17 +69,14 @@ struct fv_trainer {
   // changes only with the steps that use the rows)
   uint32_t *won2[2];
   uint32_t won2_parity;
-  // records per block of the sparse launch when that form groups for itself (like slots_blocks) and their second counts
-  fv_slot *slots2_blocks;
-  uint32_t *slot_n2_blocks;
+  fv_slot *slots2_blocks;  // records per block of the sparse launch when that form groups for itself (like slots_blocks)
   bool last_delta_grouped;  // the form the last whole anti-Hebbian step took
   // anti-Hebbian form (delta != 0), allocated with the first such step: the second neuron of every
-  // window, its scaled activation, the windows grouped by it, the second count of every slot record
+  // window, its scaled activation, the windows grouped by it
   int32_t *win2;
   uint16_t *win2_16;
   float *sc2;
   uint32_t *order2, *group_base2, *group_count2;
-  uint32_t *slot_n2;
   fv_slot *slots2;  // records of a step with delta != 0: twice the room
   float last_delta;
   float *sc;        // B scaled activations at the winner

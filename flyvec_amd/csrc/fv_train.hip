@@ -28,10 +28,13 @@
 //                      step, and the launch is a single read-modify-write of the matrix; otherwise it
 //                      makes the pass for the maximum first (on registers where the matrix fits the
 //                      register file of the machine, by streaming the rows twice where it does not).
-//                      As separate launches (4a max, 5 update, 6 slot update) on request.
+//                      As separate launches (4a max, 5 update, 6 slot update) on request. Where steps follow
+//                      each other the single launch visits only the rows this step has touched and the next one
+//                      reads; the other rows get their updates, in order, when they are needed.
 //
 // The device code is in fv_train_gather.h (1), fv_train_group.h (2), fv_train_sparse.h (3),
-// fv_train_dense.h (4 to 6) and fv_train_top2.h (the carried largest weights); fv_train_state.h holds
+// fv_train_dense.h (4 to 6), fv_train_rows.h and fv_train_row_list.h (the rows of launch 4 as they are needed)
+// and fv_train_top2.h (the carried largest weights); fv_train_state.h holds
 // the trainer's state. This file has the small kernels of the window order and the host side.
 //
 // Every one of the n additions of 1/f onto ds[h][i] adds the same value, so the reference's
@@ -44,6 +47,7 @@
 #include "fv_train_group.h"
 #include "fv_train_sparse.h"
 #include "fv_train_dense.h"
+#include "fv_train_rows.h"
 
 // ---- row norms (log line of flyvec/src/cuda_funcs.cu:1234-1242) -------------------------------
 
@@ -127,6 +131,14 @@ static unsigned fv_perm_blocks(uint64_t n) {
 // ---- host side ------------------------------------------------------------------------------
 
 static void fv_trainer_free_delta(fv_trainer *t);
+
+// Dynamic LDS of the launches of fv_train_rows.h: the kept xx, and the sentinel lists or the threads' pairs.
+static size_t fv_rows_smem(const fv_trainer *t) {
+  return (size_t)t->rows_age * t->ldk * sizeof(float) + (size_t)(FV_ONEPASS_THREADS / 64) * t->rows_wave_hits * sizeof(uint2);
+}
+static size_t fv_rows_settle_smem(const fv_trainer *t) {
+  return (size_t)t->rows_age * t->ldk * sizeof(float) + (size_t)FV_ONEPASS_THREADS * 4 * sizeof(float2);
+}
 
 static void fv_trainer_free_corpus(fv_trainer *t) {
   (void)hipFree(t->corpus);
@@ -231,11 +243,66 @@ static void fv_trainer_leaves_flight(fv_trainer *t) {
   t->in_flight = false;
 }
 
-// Waits for the trainer's stream. Every wait of this file goes through here, so that a trainer whose steps have been
+// What the launches that visit rows (fv_train_rows.h) are told about them; `step` is the step the launch belongs to.
+static fv_rows_args fv_rows_describe(const fv_trainer *t, uint32_t step) {
+  fv_rows_args b = {};
+  b.list.need = t->row_need;
+  b.list.last = t->row_last;
+  b.list.list = t->row_list;
+  b.list.count = t->row_count;
+  b.list.cap = t->rows_cap;
+  b.list.n_dense = t->onepass_blocks;
+  b.list.step = step;
+  b.list.first = t->rows_first;
+  b.list.age = t->rows_age;
+  b.list.n_rows = (uint32_t)t->N;
+  b.list.dead = t->scalars + 1;
+  b.hist_xx = t->hist_xx;
+  b.hist_s = t->hist_s;
+  b.pieces = (t->ldk / 4 + 63) / 64;
+  b.piece_magic = (uint32_t)((1ull << 32) / b.pieces + 1);
+  b.rows_per_round = t->onepass_active / (t->ldk / 4);
+  // rounded upwards
+  b.drift = (float)(t->rows_drift * 1.0001 + 1e-30);
+  b.wave_hits = t->rows_wave_hits;
+  b.fallbacks = t->rows_fallback;
+  return b;
+}
+
+// Enqueues the launch that brings every row of the matrix up to date, if rows may lack updates.
+static hipError_t fv_trainer_settle(fv_trainer *t) {
+  if (!t->rows_behind) return hipSuccess;
+  const fv_rows_args b = fv_rows_describe(t, t->rows_step + 1);
+  fv_dense_args d;
+  memset(&d, 0, sizeof d);
+  d.Wt4 = (float4 *)t->Wt;
+  d.scalars = t->scalars;
+  d.K = t->K;
+  d.ldk = t->ldk;
+  d.ldk4 = t->ldk / 4;
+  d.n_rows = (uint32_t)t->N;
+  d.active = t->onepass_active;
+  d.update_cut = t->update_cut;
+  d.top2_part = t->top2_part;
+  hipLaunchKernelGGL(fv_rows_settle_kernel, dim3(t->onepass_blocks), dim3(FV_ONEPASS_THREADS), fv_rows_settle_smem(t),
+                     t->stream, d, b);
+  t->rows_behind = false;
+  t->rows_since = 0;
+  t->rows_drift = 0.0;
+  t->top2_valid = true;  // this launch leaves the shares of the matrix as it is
+  t->top2_n_part = t->onepass_blocks;
+  t->top2_merged = false;
+  t->last_top2_known = true;  // (what a launch of the last step on its own goes by)
+  return hipGetLastError();
+}
+
+// Waits for the trainer's stream, every row of the matrix up to date. Every wait of this file goes through here, so that a trainer whose steps have been
 // waited for by whatever call is out of the count.
 static hipError_t fv_trainer_drain(fv_trainer *t) {
-  const hipError_t e = hipStreamSynchronize(t->stream);
+  hipError_t e = fv_trainer_settle(t);
+  if (e == hipSuccess) e = hipStreamSynchronize(t->stream);
   if (e == hipSuccess) fv_trainer_leaves_flight(t);
+  t->in_a_row = 0;
   return e;
 }
 
@@ -248,6 +315,7 @@ static int fv_trainer_take_giveup(fv_trainer *t, uint32_t *out_tag) {
   *t->onepass_status = 0;
   t->onepass = false;
   t->top2_valid = false;
+  t->rows_behind = false;  // that launch has left every row as the step before it did
   t->ahead_valid = false;
   FV_HIP(hipMemsetAsync(t->scalars + 1, 0, sizeof(float), t->stream));
   FV_HIP(fv_trainer_drain(t));
@@ -271,8 +339,8 @@ extern "C" int fv_trainer_destroy(fv_trainer *t) {
   if (t->stream) (void)hipStreamSynchronize(t->stream);
   fv_trainer_free_corpus(t);
   (void)hipFree(t->Wt);
-  (void)hipFree(t->idx);
-  (void)hipFree(t->idx_ahead);
+  (void)hipFree(t->idx_all);
+  (void)hipFree(t->hist_xx);
   (void)hipFree(t->slots);
   (void)hipFree(t->slots_blocks);
   (void)hipFree(t->slot_count);
@@ -299,21 +367,47 @@ extern "C" int fv_trainer_destroy(fv_trainer *t) {
   return FV_OK;
 }
 
+// Whether the dense launch of a step should visit only the rows somebody needs, going by the sizes.
+static bool fv_rows_worth_it(const fv_trainer *t) {
+  return t->rows_ok && (uint64_t)t->B * t->w <= FV_ROWS_MOST_POSITIONS * t->N && (uint64_t)t->total4 * 16 >= FV_ROWS_LEAST_BYTES;
+}
+
+// Entries of an index matrix: a row per window of a minibatch, and the padding behind them.
+static size_t fv_idx_entries(const fv_trainer *t) { return (size_t)t->B * t->idx_stride + FV_IDX_PAD; }
+
+// What such steps take: with the trainer where the sizes call for them, else when they are asked for.
+static int fv_trainer_alloc_rows(fv_trainer *t) {
+  if (t->hist_xx || !t->rows_ok) return FV_OK;
+  const size_t padded = (t->N + FV_SP_THREADS - 1) / FV_SP_THREADS * FV_SP_THREADS;
+  const size_t kept = (size_t)t->rows_age * (t->ldk + 1), lists = 2 * (size_t)t->onepass_blocks * t->rows_cap;
+  // every part a multiple of 16 bytes; the third index matrix last
+  const size_t words = (kept + 2 * padded + 4 + lists + 3) & ~(size_t)3, idx_bytes = fv_idx_entries(t) * sizeof(int32_t);
+  FV_HIP(hipMalloc((void **)&t->hist_xx, words * sizeof(uint32_t) + idx_bytes));
+  FV_HIP(hipMemsetAsync(t->hist_xx, 0, words * sizeof(uint32_t), t->stream));
+  t->idx_ahead2 = (int32_t *)(t->hist_xx + words);
+  FV_HIP(hipMemsetAsync(t->idx_ahead2, 0xff, idx_bytes, t->stream));
+  t->hist_s = t->hist_xx + (size_t)t->rows_age * t->ldk;
+  t->row_need = (uint32_t *)(t->hist_xx + kept);
+  t->row_last = t->row_need + padded;
+  t->row_count = (unsigned long long *)(t->row_last + padded);
+  t->row_list = (uint32_t *)(t->row_count + 2);
+  return FV_OK;
+}
+
 static int fv_trainer_alloc(fv_trainer *t) {
   // zeros behind the matrix: what the gather reads for masked positions and in its lanes past K
   const size_t elems = (size_t)fv_matrix_alloc_elems(t->K, t->N);
   FV_REQUIRE(fv_matrix_gather_reach(t->K, t->N) <= elems, FV_ERR_INVALID,
              "a gather of a %u x %llu matrix would read past its allocation", t->K, (unsigned long long)t->N);
   FV_HIP(hipStreamCreate(&t->stream));
-  FV_HIP(hipMalloc((void **)&t->Wt, elems * sizeof(float)));
   t->idx_stride = (t->w + 3u) & ~3u;
-  const size_t idx_entries = (size_t)t->B * t->idx_stride + FV_IDX_PAD;
-  FV_HIP(hipMalloc((void **)&t->idx, idx_entries * sizeof(int32_t)));
-  FV_HIP(hipMemsetAsync(t->idx, 0xff, idx_entries * sizeof(int32_t), t->stream));
-  if (t->onepass_blocks) {
-    FV_HIP(hipMalloc((void **)&t->idx_ahead, idx_entries * sizeof(int32_t)));
-    FV_HIP(hipMemsetAsync(t->idx_ahead, 0xff, idx_entries * sizeof(int32_t), t->stream));
-  }
+  FV_HIP(hipMalloc((void **)&t->Wt, elems * sizeof(float)));
+  const size_t idx_entries = fv_idx_entries(t);
+  const size_t idx_matrices = t->onepass_blocks ? 2 : 1;  // the minibatch at hand and the next one change places
+  FV_HIP(hipMalloc((void **)&t->idx_all, idx_matrices * idx_entries * sizeof(int32_t)));
+  FV_HIP(hipMemsetAsync(t->idx_all, 0xff, idx_matrices * idx_entries * sizeof(int32_t), t->stream));
+  t->idx = t->idx_all;
+  if (t->onepass_blocks) t->idx_ahead = t->idx + idx_entries;
   FV_HIP(hipMalloc((void **)&t->win, ((size_t)t->B + 16) * sizeof(int32_t)));  // read in 16-byte pieces
   FV_HIP(hipMalloc((void **)&t->sc, (size_t)t->B * sizeof(float)));
   FV_HIP(hipMalloc((void **)&t->order, (size_t)t->B * sizeof(uint32_t)));
@@ -371,7 +465,15 @@ static int fv_trainer_alloc(fv_trainer *t) {
   // status word behind them
   FV_HIP(hipMalloc((void **)&t->scalars, 16 * sizeof(float) + (size_t)t->K * FV_NORM_BLOCKS * sizeof(double)));
   t->norm_part = (double *)(t->scalars + 16);
-  FV_HIP(hipHostMalloc((void **)&t->norms, t->K * sizeof(double) + sizeof(uint32_t), hipHostMallocDefault));
+  FV_HIP(hipHostMalloc((void **)&t->norms, t->K * sizeof(double) + 2 * sizeof(uint32_t), hipHostMallocDefault));
+  t->rows_fallback = (uint32_t *)(t->norms + t->K) + 1;
+  *t->rows_fallback = 0;
+  t->xx_last = t->xx;
+  if (fv_rows_worth_it(t) && fv_trainer_alloc_rows(t) != FV_OK) {  // (the trainer does without)
+    (void)hipGetLastError();
+    fv_clear_error();
+    t->rows_ok = false;
+  }
   FV_HIP(hipMemsetAsync(t->Wt, 0, elems * sizeof(float), t->stream));
   FV_HIP(hipMemsetAsync(t->xx, 0, (size_t)t->ldk * sizeof(float), t->stream));
   FV_HIP(hipMemsetAsync(t->scalars, 0, 16 * sizeof(float), t->stream));
@@ -452,6 +554,20 @@ static void fv_choose_onepass(fv_trainer *t, uint64_t cu) {
   t->onepass_active = rows_per_round * ldk4;
   t->onepass = true;
   t->onepass_stream = unroll == 0;
+  if (t->N > FV_ROWS_MASK) return;
+  t->rows_age = fv_rows_age(t->ldk);
+  t->rows_cap = (uint32_t)((t->N + blocks - 1) / blocks);
+  t->rows_wave_hits = 512u;
+  bool set = true;
+#define FV_SET(KERNEL, BYTES)                                                                                       \
+  set = set && hipFuncSetAttribute((const void *)KERNEL, hipFuncAttributeMaxDynamicSharedMemorySize, (int)(BYTES)) == hipSuccess;
+  FV_SET((fv_dense_rows_kernel<FV_ROWS_DEPTH, FV_ROWS_LATE>), fv_rows_smem(t))
+  FV_SET(fv_rows_settle_kernel, fv_rows_settle_smem(t))
+#undef FV_SET
+  if (set)
+    t->rows_ok = fv_rows_fit(fv_rows_smem(t), fv_rows_settle_smem(t)) != 0;
+  else
+    (void)hipGetLastError();
 }
 
 extern "C" int fv_trainer_create(const fv_train_config *cfg, fv_trainer **out_trainer) {
@@ -491,6 +607,7 @@ extern "C" int fv_trainer_create(const fv_train_config *cfg, fv_trainer **out_tr
   t->V = cfg->vocab;
   t->N = N;
   t->total4 = (uint32_t)(N * ldk / 4);
+  t->rows_hold_next = 16;
   float cut = (float)1.e-10;  // the reference compares fabs(fp32) > 1.e-10 in double
   if ((double)cut > 1.e-10) cut = nextafterf(cut, 0.0f);
   t->update_cut = cut;
@@ -635,6 +752,7 @@ extern "C" int fv_trainer_get_inverse_frequency(fv_trainer *t, float *out_invf) 
 
 extern "C" int fv_trainer_set_weights(fv_trainer *t, const float *W) {
   FV_REQUIRE(t && W, FV_ERR_INVALID, "null argument");
+  FV_HIP(fv_trainer_settle(t));
   FV_TRY(fv_upload_weights(W, t->Wt, t->K, t->N, t->ldk, t->stream));
   fv_trainer_leaves_flight(t);  // (the stream has drained)
   t->have_weights = true;
@@ -770,6 +888,29 @@ static int fv_trainer_alloc_delta(fv_trainer *t) {
 // (a minibatch of up to 64 windows per thread of a class block).
 static bool fv_groups_in_sparse(const fv_trainer *t) { return t->won[0] && !t->separate_grouping; }
 
+// Whether this step (a whole one, its dense passes in one launch) takes the form that visits the rows somebody needs.
+// A sequence of such steps begins where at least FV_ROWS_SEQUENCE steps follow each other without anybody looking
+// at the matrix in between (those enqueued and those the caller has announced): it costs a launch at its start and one at its end.
+static bool fv_rows_take(fv_trainer *t, float eps, bool alone) {
+  if (!t->hist_xx || t->rows_mode == 1 || t->cfg.prune_duplicates || t->capturing || !alone) return false;
+  if (t->rows_mode == 0 && !fv_rows_worth_it(t)) return false;
+  if (!(fabsf(eps) <= 1.0f)) return false;
+  const uint32_t fell_back = *(volatile uint32_t *)t->rows_fallback;
+  if (fell_back != t->rows_fallback_seen) {
+    // max|ds| was not the sparse elements' and the launch went over the matrix twice: every row in every step for a while,
+    // longer each time this happens again
+    t->rows_fallback_seen = fell_back;
+    t->rows_hold = t->rows_hold_next;
+    if (t->rows_hold_next < 4096) t->rows_hold_next *= 2;
+  }
+  if (t->rows_mode == 0 && t->rows_hold) {
+    t->rows_hold--;
+    return false;
+  }
+  if (t->rows_behind) return true;
+  return t->top2_valid && (t->rows_mode == 2 || t->to_come + t->in_a_row >= FV_ROWS_SEQUENCE);
+}
+
 // n_fresh < n: only the first n_fresh windows are sampled (from `first` on), the rows behind them are what
 // the index buffer of the previous step holds.
 static int fv_enqueue_step(fv_trainer *t, uint64_t first, uint32_t n, float eps, float delta, hipEvent_t *ev,
@@ -780,9 +921,62 @@ static int fv_enqueue_step(fv_trainer *t, uint64_t first, uint32_t n, float eps,
   // records the slot regions of this step hold; the single dense launch finds a record through the number in
   // its sentinel, so it is only taken when every record number fits one
   uint64_t n_slots = (uint64_t)FV_NB_CLASSES * t->B * t->w * (anti ? 2 : 1);
+  const bool can_group = fv_groups_in_sparse(t) && (!anti || (t->slots2_blocks && !t->no_block_regions));
+  const bool grouping_in_sparse = which == 0x3f ? can_group : (anti ? t->last_delta_grouped : t->last_grouped_in_sparse);
+  if (which == 0x3f) (anti ? t->last_delta_grouped : t->last_grouped_in_sparse) = grouping_in_sparse;
+  // the blocks of a sparse launch that groups for itself write their records to regions of their own, where
+  // the trainer has them, and a sentinel names a record inside its block's region
+  const uint32_t slot_region = grouping_in_sparse && !t->no_block_regions ? t->slot_region : 0u;
+  if (slot_region) n_slots = slot_region;
+  const bool onepass = t->onepass && n_slots + 1 < FV_SENTINEL_MAX;
+  fv_trainer_enters_flight(t);
+  const bool alone = fv_trainers_in_flight.load() == 1;
+  const bool rows = whole && onepass && n_fresh >= n && fv_rows_take(t, eps, alone);
+  const bool sampled_ahead = whole && t->ahead_valid && t->ahead_first == first && t->ahead_n == n && n_fresh >= n;
+  const bool rows_go_on = rows && sampled_ahead && t->ahead_marked;
+  if (whole && t->rows_behind && (!rows || !rows_go_on || t->rows_since >= FV_ROWS_REFRESH)) FV_HIP(fv_trainer_settle(t));
   // the rows' two largest weights are in hand if the last write of the matrix was a single dense launch
   const bool top2_known = whole ? t->top2_valid : t->last_top2_known;
   if (whole) t->last_top2_known = top2_known;
+  if (whole) t->in_a_row++;
+  // the windows that follow this step's, a full batch or what is left of the order, and the ones behind those
+  auto batch_at = [&](uint64_t at) {
+    return at >= t->n_windows ? 0u : (uint32_t)(t->n_windows - at < t->B ? t->n_windows - at : t->B);
+  };
+  const uint64_t next_first = first + n;
+  const uint32_t next_n = batch_at(next_first), next2_n = batch_at(next_first + next_n);
+  float *xx = t->xx_last;
+  if (whole) xx = t->xx_last = t->xx;
+  if (rows) {
+    t->rows_step += rows_go_on ? 1 : 3;  // (a sequence that ended has marked rows for two steps more)
+    if (!t->rows_behind) t->rows_first = t->rows_step;
+    if (rows_go_on) {
+      int32_t *const free_one = t->idx;
+      t->idx = t->idx_ahead;
+      t->idx_ahead = t->idx_ahead2;
+      t->idx_ahead2 = free_one;
+    } else {
+      fv_rows_start_args st;
+      st.corpus = t->corpus;
+      st.pstart = t->pstart;
+      st.stride = t->idx_stride;
+      st.w = t->w;
+      st.V = (uint32_t)t->V;
+      st.need = t->row_need;
+      st.count = t->row_count;
+      for (uint32_t k = 0; k < 2; ++k) {
+        st.idx = k ? t->idx_ahead : t->idx;
+        st.first = k ? next_first : first;
+        st.n = k ? next_n : n;
+        st.step = t->rows_step + k;
+        if (!st.n) break;
+        const uint64_t want = ((uint64_t)st.n * t->idx_stride + 255) / 256;
+        hipLaunchKernelGGL(fv_rows_start_kernel, dim3((unsigned)(want < 4096 ? want : 4096)), dim3(256), 0, t->stream, st);
+      }
+    }
+    xx = t->xx_last = t->hist_xx + (size_t)(t->rows_step & (t->rows_age - 1)) * t->ldk;
+  }
+  const fv_rows_args ra = fv_rows_describe(t, t->rows_step);
   fv_gather_args g;
   const uint32_t merge_groups = (t->K + FV_MERGE_NEURONS - 1) / FV_MERGE_NEURONS;
   g.merge_rows = (top2_known && !t->top2_merged && (whole || (which & 1u))) ? merge_groups : 0u;  // one chunk
@@ -823,16 +1017,6 @@ static int fv_enqueue_step(fv_trainer *t, uint64_t first, uint32_t n, float eps,
   // on the last step's pair, cleared here first unless it repeats the launch before it.
   // (beyond 64 windows per thread of a class block only with a slot region per block: without one every block
   // would count the lower neurons' windows in the whole winner array)
-  const bool can_group = fv_groups_in_sparse(t) && (!anti || (t->slots2_blocks && !t->no_block_regions));
-  const bool grouping_in_sparse = which == 0x3f ? can_group : (anti ? t->last_delta_grouped : t->last_grouped_in_sparse);
-  if (which == 0x3f) (anti ? t->last_delta_grouped : t->last_grouped_in_sparse) = grouping_in_sparse;
-  // the blocks of a sparse launch that groups for itself write their records to regions of their own, where
-  // the trainer has them, and a sentinel names a record inside its block's region
-  const uint32_t slot_region = grouping_in_sparse && !t->no_block_regions ? t->slot_region : 0u;
-  if (slot_region) n_slots = slot_region;
-  const bool onepass = t->onepass && n_slots + 1 < FV_SENTINEL_MAX;
-  fv_trainer_enters_flight(t);
-  const bool alone = fv_trainers_in_flight.load() == 1;
   g.won = nullptr;
   g.won2 = nullptr;
   g.won_words = t->won_words;
@@ -849,14 +1033,15 @@ static int fv_enqueue_step(fv_trainer *t, uint64_t first, uint32_t n, float eps,
     if (anti) g.won2 = t->won2[t->won2_parity];
   }
   // a whole step whose windows the previous one has sampled ahead takes that buffer
-  g.sampled = 0;
+  g.sampled = rows ? 1u : 0u;
+  g.idx = t->idx;
   if (whole) {
-    if (t->ahead_valid && t->ahead_first == first && t->ahead_n == n && n_fresh >= n) {
+    if (!rows && sampled_ahead) {
       std::swap(t->idx, t->idx_ahead);
       g.idx = t->idx;
       g.sampled = 1;
     }
-    t->ahead_valid = false;
+    t->ahead_valid = t->ahead_marked = false;
   }
   if (ev) FV_HIP(hipEventRecord(ev[0], t->stream));
   if (which & 1u) switch ((t->K + 63) / 64) {
@@ -876,7 +1061,7 @@ static int fv_enqueue_step(fv_trainer *t, uint64_t first, uint32_t n, float eps,
   gr.order = t->order;
   gr.group_base = t->group_base;
   gr.group_count = t->group_count;
-  gr.xx = t->xx;
+  gr.xx = xx;
   gr.n = n;
   gr.scale = 1.0f;
   gr.accumulate = 0;
@@ -918,12 +1103,12 @@ static int fv_enqueue_step(fv_trainer *t, uint64_t first, uint32_t n, float eps,
   sp.delta = delta;
   sp.lmid = t->cfg.lmid;
   sp.lbase = t->cfg.lbase;
-  sp.xx = t->xx;
+  sp.xx = xx;
   sp.invf = t->invf;
   sp.bmax_sparse = t->bmax + t->sparse_base;
   sp.row_top2 = t->row_top2;
   sp.row_hits = t->row_hits;
-  sp.top2_known = top2_known ? 1u : 0u;
+  sp.top2_known = top2_known && !rows ? 1u : 0u;
   sp.light = t->no_light_blocks ? 0u : 1u;
   sp.slot_count = t->slot_count;
   sp.pad_row = t->B;
@@ -945,9 +1130,10 @@ static int fv_enqueue_step(fv_trainer *t, uint64_t first, uint32_t n, float eps,
   sp.order_out = t->order;
   sp.group_base_out = t->group_base;
   sp.group_count_out = t->group_count;
-  sp.xx_out = t->xx;
+  sp.xx_out = xx;
+  sp.rows = ra.list;
   if (which & 4u) {
-    const dim3 sp_grid(t->K * FV_NB_CLASSES), sp_block(FV_SP_THREADS);
+    const dim3 sp_grid(t->K * FV_NB_CLASSES + (rows ? fv_rows_list_blocks(t->N) : 0u)), sp_block(FV_SP_THREADS);
     // the wider counter array where it saves a pass over the neuron's windows
     const uint32_t class_cols = (uint32_t)((t->N + FV_NB_CLASSES - 1) / FV_NB_CLASSES);
     // (counted for 16-bit counters, two to a word: what all but the heaviest neurons of a large minibatch use)
@@ -974,7 +1160,7 @@ static int fv_enqueue_step(fv_trainer *t, uint64_t first, uint32_t n, float eps,
   if (ev) FV_HIP(hipEventRecord(ev[3], t->stream));
   fv_dense_args d;
   d.Wt4 = (float4 *)t->Wt;
-  d.xx = t->xx;
+  d.xx = xx;
   d.slots = anti ? (slot_region ? t->slots2_blocks : t->slots2) : slot_region ? t->slots_blocks : t->slots;
   d.slot_region = slot_region;
   {
@@ -1020,7 +1206,31 @@ static int fv_enqueue_step(fv_trainer *t, uint64_t first, uint32_t n, float eps,
   d.prec = t->cfg.prec;
   d.update_cut = t->update_cut;
   const size_t smem = (size_t)t->ldk * sizeof(float);
-  if (onepass) {
+  if (rows) {
+    if (++t->onepass_epoch == 0) t->onepass_epoch = 1;
+    d.arrive = t->arrive;
+    d.status = t->onepass_status;
+    d.epoch = t->onepass_epoch;
+    d.spin_limit = t->onepass_spin_limit;
+    d.step_tag = t->step_tag ? t->step_tag : 0xffffffffu;
+    d.hit_cap = t->hit_cap_limit && t->hit_cap_limit < t->rows_wave_hits ? t->hit_cap_limit : t->rows_wave_hits;
+    d.ahead_first = next_first + next_n;
+    d.ahead_n = next2_n;
+    d.idx_ahead = t->idx_ahead2;
+    t->dense_forms[0]++;
+    hipLaunchKernelGGL((fv_dense_rows_kernel<FV_ROWS_DEPTH, FV_ROWS_LATE>), dim3(t->onepass_blocks), dim3(FV_ONEPASS_THREADS), fv_rows_smem(t),
+                       t->stream, d, ra);
+    t->ahead_valid = t->ahead_marked = next_n != 0;
+    t->ahead_first = next_first;
+    t->ahead_n = next_n;
+    t->rows_behind = true;
+    t->rows_since++;
+    t->rows_steps++;
+    t->rows_drift += fabs((double)eps);
+    t->top2_valid = false;    // row_top2 is that of the matrix rows_since steps ago,
+    t->top2_merged = true;    // and the winner kernel has merged it
+    if (ev) FV_HIP(hipEventRecord(ev[4], t->stream));
+  } else if (onepass) {
     // both dense passes in the launch that takes the place of the first one
     if (which & 8u) {
       if (++t->onepass_epoch == 0) t->onepass_epoch = 1;
@@ -1030,10 +1240,9 @@ static int fv_enqueue_step(fv_trainer *t, uint64_t first, uint32_t n, float eps,
       d.spin_limit = t->onepass_spin_limit;
       d.step_tag = t->step_tag ? t->step_tag : 0xffffffffu;
       // the windows that follow this step's, a full batch or what is left of the order
-      const uint64_t next_first = first + n;
-      if (whole && next_first < t->n_windows && !t->cfg.prune_duplicates) {  // the ahead sampler does not prune
+      if (whole && next_n && !t->cfg.prune_duplicates) {  // the ahead sampler does not prune
         d.ahead_first = next_first;
-        d.ahead_n = (uint32_t)(t->n_windows - next_first < t->B ? t->n_windows - next_first : t->B);
+        d.ahead_n = next_n;
         d.idx_ahead = t->idx_ahead;
         t->ahead_valid = true;
         t->ahead_first = next_first;
@@ -1165,6 +1374,8 @@ extern "C" int fv_trainer_run_epoch(fv_trainer *t, uint64_t epoch_id, uint64_t n
     for (uint64_t k = k_first; k < t->n_windows && rc == FV_OK; k += t->B) {
       const uint64_t n = t->n_windows - k < t->B ? t->n_windows - k : t->B;
       t->step_tag = (uint32_t)(k / t->B) + 1u;
+      const uint64_t behind = (t->n_windows - k - n + t->B - 1) / t->B;
+      t->to_come = behind < FV_ROWS_SEQUENCE ? (uint32_t)behind : FV_ROWS_SEQUENCE;
       if (n < t->B && k > 0 && t->stale_tail)
         // flyvec/src/cuda_funcs.cu:1679 against :1700-1732: only the sampler sees the remainder, the other
         // kernels run on all Num rows, those behind the remainder being the previous minibatch's
@@ -1173,6 +1384,7 @@ extern "C" int fv_trainer_run_epoch(fv_trainer *t, uint64_t epoch_id, uint64_t n
         rc = fv_enqueue_step(t, k, (uint32_t)n, eps, delta, nullptr);
     }
     t->step_tag = 0;
+    t->to_come = 0;
     FV_TRY(rc);
     FV_HIP(fv_trainer_drain(t));
     uint32_t tag = 0;
@@ -1241,6 +1453,21 @@ extern "C" int fv_trainer_set_light_blocks(fv_trainer *t, uint32_t on) {
   return FV_OK;
 }
 
+extern "C" int fv_trainer_set_row_updates(fv_trainer *t, uint32_t mode) {
+  FV_REQUIRE(t, FV_ERR_INVALID, "null trainer");
+  FV_REQUIRE(mode <= 2, FV_ERR_INVALID, "mode must be 0 (choose), 1 (every row in every step) or 2 (rows as they are needed)");
+  FV_HIP(fv_trainer_settle(t));
+  if (mode == 2) FV_TRY(fv_trainer_alloc_rows(t));
+  t->rows_mode = mode;
+  return FV_OK;
+}
+
+extern "C" int fv_trainer_get_row_updates(fv_trainer *t, uint64_t *out_steps) {
+  FV_REQUIRE(t && out_steps, FV_ERR_INVALID, "null argument");
+  *out_steps = t->rows_steps;
+  return FV_OK;
+}
+
 extern "C" int fv_trainer_get_grouping_launch(fv_trainer *t, uint32_t *out_separate) {
   FV_REQUIRE(t && out_separate, FV_ERR_INVALID, "null argument");
   *out_separate = fv_groups_in_sparse(t) ? 0u : 1u;
@@ -1303,7 +1530,7 @@ extern "C" int fv_trainer_get_winners(fv_trainer *t, int32_t *out_winners, uint3
 extern "C" int fv_trainer_get_step_stats(fv_trainer *t, float *out_xx, float *out_max_abs_ds) {
   FV_REQUIRE(t, FV_ERR_INVALID, "null trainer");
   FV_HIP(fv_trainer_drain(t));
-  if (out_xx) FV_HIP(hipMemcpy(out_xx, t->xx, (size_t)t->K * sizeof(float), hipMemcpyDeviceToHost));
+  if (out_xx) FV_HIP(hipMemcpy(out_xx, t->xx_last, (size_t)t->K * sizeof(float), hipMemcpyDeviceToHost));
   if (out_max_abs_ds) {
     FV_HIP(hipMemcpy(out_max_abs_ds, t->scalars, sizeof(float), hipMemcpyDeviceToHost));
   }
@@ -1315,6 +1542,7 @@ extern "C" int fv_trainer_row_norms(fv_trainer *t, uint32_t n_rows, double *out_
   FV_REQUIRE(t->have_weights, FV_ERR_STATE, "no weights set");
   if (n_rows > t->K) n_rows = t->K;
   if (n_rows == 0) return FV_OK;
+  FV_HIP(fv_trainer_settle(t));
   const uint64_t want = (t->N + 15) / 16;
   const uint32_t blocks = (uint32_t)(want < FV_NORM_BLOCKS ? want : FV_NORM_BLOCKS);
   hipLaunchKernelGGL(fv_row_squares_kernel, dim3(blocks, (n_rows + 15) / 16), dim3(256), 0, t->stream, t->Wt, t->N, t->ldk,
@@ -1340,8 +1568,12 @@ extern "C" int fv_trainer_time_steps(fv_trainer *t, uint64_t first_window, uint3
   int rc = FV_OK;
   FV_HIP(fv_trainer_drain(t));
   FV_HIP(hipEventRecord(e0, t->stream));
-  for (uint32_t s = 0; s < n_steps && rc == FV_OK; ++s)
+  for (uint32_t s = 0; s < n_steps && rc == FV_OK; ++s) {
+    t->to_come = n_steps - 1 - s;
     rc = fv_enqueue_step(t, first_window + (uint64_t)s * t->B, t->B, eps, 0.0f, nullptr);
+  }
+  t->to_come = 0;
+  FV_HIP(fv_trainer_settle(t));  // (part of what the steps take)
   FV_HIP(hipEventRecord(e1, t->stream));
   FV_HIP(fv_trainer_drain(t));
   FV_HIP(hipEventElapsedTime(out_total_ms, e0, e1));
@@ -1392,8 +1624,10 @@ extern "C" int fv_trainer_time_steps_graph(fv_trainer *t, uint64_t first_window,
     hipGraph_t graph = nullptr;
     e = hipStreamBeginCapture(t->stream, hipStreamCaptureModeRelaxed);
     if (e != hipSuccess) break;
+    t->capturing = true;
     for (uint32_t i = s; i < last && rc == FV_OK; ++i)
       rc = fv_enqueue_step(t, first_window + (uint64_t)i * t->B, t->B, eps, 0.0f, nullptr);
+    t->capturing = false;
     e = hipStreamEndCapture(t->stream, &graph);
     if (e == hipSuccess && rc == FV_OK) {
       hipGraphExec_t exec = nullptr;

@@ -364,7 +364,9 @@ __device__ __forceinline__ float fv_slot_final(const fv_slot &sl, float s, bool 
 }
 
 // The element p holds the sentinel `bits`: its final value from the record the sentinel names. The saved
-// weight goes back where the row is not updated (xx == 0) or the launch gave up, else the updated one.
+// weight goes back where the row is not updated (xx == 0) or the launch gave up, else the updated one. SHARES: the
+// launch keeps the two largest finished sparse elements of every neuron.
+template <bool SHARES = true>
 __device__ __forceinline__ void fv_finish_sparse_element(const fv_dense_args &a, uint32_t bits, uint32_t p, float s,
                                                          bool ok, uint32_t *sp1, uint32_t *sp2) {
   const uint32_t number = (bits & FV_SENTINEL_MAX) - 1u;
@@ -379,7 +381,7 @@ __device__ __forceinline__ void fv_finish_sparse_element(const fv_dense_args &a,
   if (sl.p != p) return;
   const float out = fv_slot_final(sl, s, ok, a.update_cut);
   ((float *)a.Wt4)[p] = out;
-  fv_top2_insert_lds(sp1, sp2, h, fv_abs_or_zero(out));
+  if (SHARES) fv_top2_insert_lds(sp1, sp2, h, fv_abs_or_zero(out));
 }
 
 // The sentinels of a list, dealt over `width` threads (this one is number `me` of them), four records in flight per

@@ -2,6 +2,7 @@
 #pragma once
 
 #include "fv_train_group.h"
+#include "fv_train_row_list.h"
 
 // ---- kernel 3: sparse elements -----------------------------------------------------------------------
 //
@@ -65,6 +66,8 @@ struct fv_sparse_args {
   // grouping form with a slot region per block: a neuron whose window positions are no more than the block has
   // threads is finished by its class-0 block alone, an entry per thread (fv_sparse_light); 0 switches that off
   uint32_t light;
+  // the blocks behind the first n_blocks list the rows that the dense launch visits (none: it visits all of them)
+  fv_rows_list_args rows;
 };
 
 // Counting pass of one class block over the windows whose ids are staged in LDS: ord[0 .. n_staged),
@@ -278,6 +281,10 @@ __device__ __forceinline__ void fv_sparse_block(const fv_sparse_args &a) {
   __shared__ float wave_max[16];
   __shared__ uint32_t red[17];
   constexpr uint32_t T = FV_SP_THREADS;
+  if (blockIdx.x >= a.n_blocks) {
+    fv_rows_list_block(a.rows, blockIdx.x - a.n_blocks, red);
+    return;
+  }
   const uint32_t h = blockIdx.x >> FV_NB_CLASS_SHIFT;
   const uint32_t q = GROUPING ? ((blockIdx.x & (FV_NB_CLASSES - 1)) + (blockIdx.x >> (FV_NB_CLASS_SHIFT + 1))) & (FV_NB_CLASSES - 1)
                               : blockIdx.x & (FV_NB_CLASSES - 1);

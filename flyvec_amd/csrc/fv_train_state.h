@@ -48,6 +48,7 @@ struct fv_trainer {
   uint32_t fail_alloc;  // fv_trainer_fail_allocation: allocations of a corpus until one is refused, 0 for none
   uint64_t corpus_cap, windows_cap;  // tokens / windows the buffers above have room for
   float *invf;
+  int32_t *idx_all; // the allocation of idx and idx_ahead, which change places with each other and with idx_ahead2
   int32_t *idx;     // B rows of idx_stride column indices of the current minibatch (w used, the rest -1)
   uint32_t idx_stride;  // w rounded up to 4: rows are read 16 bytes at a time
   // the single dense launch samples the column indices of the minibatch expected next (the windows
@@ -136,4 +137,26 @@ struct fv_trainer {
   uint64_t giveups_recovered;  // epochs in which run_epoch took up again behind a launch that gave up
   double *norm_part, *norms;  // workspace of fv_trainer_row_norms: FV_NORM_BLOCKS sums per row; page-locked results
   float update_cut;  // largest fp32 <= 1e-10
+  // Steps whose dense launch visits the rows somebody needs (fv_train_rows.h). They are numbered; such a step's xx and s
+  // are kept for rows_age steps.
+  bool rows_ok;             // this trainer has what they take
+  uint32_t rows_mode;       // fv_trainer_set_row_updates: 0 as the sizes say, 1 never, 2 wherever it can be
+  uint32_t rows_age, rows_cap, rows_wave_hits;
+  float *hist_xx, *hist_s;  // what fv_rows_list_args and fv_rows_args say of them; one allocation, null until it is needed
+  uint32_t *row_need, *row_last, *row_list;
+  unsigned long long *row_count;
+  uint32_t *rows_fallback;  // page-locked (in the allocation of norms): the last such launch that had to make the pass for max|ds|
+  uint32_t rows_fallback_seen, rows_hold, rows_hold_next;  // steps the trainer stays with visiting every row behind one
+  uint32_t rows_step;       // number of the newest such step
+  uint32_t rows_first;      // no row lacks the update of a step before this one
+  bool rows_behind;         // rows may lack updates: fv_trainer_settle before anybody else looks at the matrix
+  uint64_t rows_steps;      // such steps so far
+  uint32_t rows_since;      // such steps since row_top2 was exact, and the sum of their |eps|
+  double rows_drift;
+  int32_t *idx_ahead2;      // the minibatch after the next, sampled by such a step (room for it in the same allocation)
+  bool ahead_marked;        // idx_ahead and idx_ahead2 hold the next two minibatches, and row_need knows them
+  uint32_t to_come;         // steps the caller is going to enqueue behind the present one without looking at the matrix
+  bool capturing;           // steps are being captured into a graph
+  uint32_t in_a_row;        // steps enqueued since somebody waited for the stream
+  float *xx_last;           // xx of the last step
 };

@@ -198,6 +198,19 @@ class Trainer:
         Same results either way."""
         check(self.lib.fv_trainer_set_light_blocks(self.handle, 1 if on else 0))
 
+    def set_row_updates(self, mode):
+        """1: the single dense launch updates every row of the matrix in every step; 2: the rows the step has touched
+        or the next one reads, each with all the steps it lacks, where it can; 0 (the default): by the sizes.
+        Same results."""
+        check(self.lib.fv_trainer_set_row_updates(self.handle, int(mode)))
+
+    @property
+    def row_update_steps(self):
+        """Steps so far whose dense launch visited the rows somebody needed."""
+        out = C.c_uint64(0)
+        check(self.lib.fv_trainer_get_row_updates(self.handle, C.byref(out)))
+        return out.value
+
     def set_sentinel_list(self, entries):
         """Test hook: the single dense launch's LDS list of sparse elements counts as full after `entries`
         (0: its real size); the elements beyond are finished where they are met.  Same results."""

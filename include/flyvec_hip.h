@@ -269,6 +269,14 @@ int fv_trainer_set_slot_regions(fv_trainer *t, uint32_t per_block);
  * default; 0 keeps the four class blocks for every neuron. Results are bit-identical either way. No counterpart
  * in the reference. */
 int fv_trainer_set_light_blocks(fv_trainer *t, uint32_t on);
+/* How the single dense launch takes the rows of W (a row holds the weights of one token). mode 1: it updates every row
+ * in every step. mode 2: where it can (no other trainer in flight, no duplicate pruning) it visits the rows that this
+ * step has touched or the next one reads, and brings each up to date with all the steps it lacks; nothing is
+ * left undone when a call that waits for the trainer returns. mode 0, the default: by the sizes, where at least eight
+ * steps follow each other without such a call in between. Results are bit-identical. get: steps so far whose dense
+ * launch visited rows. No counterpart in the reference. */
+int fv_trainer_set_row_updates(fv_trainer *t, uint32_t mode);
+int fv_trainer_get_row_updates(fv_trainer *t, uint64_t *out_steps);
 /* Test hook. The single dense launch notes the sparse elements it meets (their sentinels) in LDS lists, one of
  * 256 entries per wave in the register form, one of 8192 per block in the streaming form, and finishes them when
  * its dense elements are done; an element that finds its list full is finished by its own thread. entries > 0

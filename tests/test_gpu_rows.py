@@ -1,0 +1,200 @@
+"""The dense launch that visits only the rows of the matrix somebody needs (fv_train_rows.h), against the checker."""
+import numpy as np
+import pytest
+
+from conftest import small_corpus
+
+pytestmark = pytest.mark.gpu
+
+
+def _trainer(tokens, offsets, V, K, w, B, W0, delta=0.0, lr0=1e-3, mode=2, **kw):
+    from flyvec_amd import Trainer
+    t = Trainer(V, K, w, B, initial_learning_rate=lr0, delta=delta, **kw)
+    t.set_row_updates(mode)
+    t.set_corpus(tokens, offsets)
+    perm = np.random.default_rng(6).permutation(t.num_windows).astype(np.uint64)
+    t.set_permutation(perm)
+    t.set_weights(W0)
+    return t, perm
+
+
+@pytest.mark.parametrize("V,K,w,B,n_tokens,delta", [
+    (3000, 100, 7, 40, 12000, 0.0),      # few rows touched: most lag until they are 16 steps behind
+    (3000, 100, 7, 40, 12000, 0.4),
+    (500, 400, 11, 512, 60000, 0.0),     # nearly every row touched in every step
+    (700, 209, 5, 333, 40000, 0.3),
+    (300, 1, 3, 7, 2000, 0.0),           # one neuron, one group of which three parts are padding
+    (200, 5, 1, 3, 900, 0.0),            # window of one position
+    (90, 2048, 7, 64, 6000, 0.0),        # the widest rows: xx kept for 8 steps, two threads per group of a round
+    (2000, 1025, 4, 100, 20000, 0.0),
+    (40000, 64, 5, 500, 60000, 0.0),     # more rounds of rows than a thread has groups in flight in the launch over all rows
+    (1500, 8, 6, 20000, 90000, 0.0),     # grouped by a launch of its own
+    (4100, 513, 6, 2000, 60000, 0.0),
+])
+def test_epochs_with_rows_updated_as_they_are_needed(gpu, oracle_lib, V, K, w, B, n_tokens, delta):
+    """Two epochs (partial last minibatch included) against the checker's, the log line's norms in between."""
+    from flyvec_amd import synthetic
+    to = oracle_lib
+    tokens, offsets = small_corpus(n_tokens, V, seed=K)
+    starts, invf = to.window_starts(offsets, w), to.inverse_frequency(tokens, V)
+    W0 = synthetic.synapses(K, V, seed=3, sigma=0.02)
+    t, perm = _trainer(tokens, offsets, V, K, w, B, W0, delta=delta)
+    Wo = W0.copy()
+    n_steps = (len(starts) + B - 1) // B
+    for ep in (3, 4):
+        norms = t.row_norms(K)
+        assert np.allclose(norms, np.sqrt((Wo.astype(np.float64) ** 2).sum(1)), rtol=1e-12)
+        t.run_epoch(ep, 15)
+        wo = to.train_steps(Wo, tokens, starts, perm, 0, B, n_steps, w, invf, to.epoch_eps(1e-3, ep, 15),
+                            delta=t.epoch_delta(ep, 15))
+        last = len(starts) - (n_steps - 1) * B
+        assert np.array_equal(t.winners(last), wo[-last:])
+        assert np.array_equal(t.get_weights().view(np.uint32), Wo.view(np.uint32)), ep
+    assert t.row_update_steps >= 2 * n_steps - 1      # the first step on a new matrix visits every row
+    assert sum(t.dense_path_counts) == 2 * n_steps and t.giveups_recovered == 0
+    t.close()
+
+
+def _planted(tokens, V, K):
+    """Weights whose largest entries sit on the most frequent tokens: the dense term decides max|ds|."""
+    from flyvec_amd import synthetic
+    W = synthetic.synapses(K, V, seed=9)
+    W[:, np.argsort(-np.bincount(tokens[tokens >= 0], minlength=V))[:3]] = np.float32(7.0)
+    return W
+
+
+@pytest.mark.parametrize("delta", [0.0, 0.3])
+@pytest.mark.parametrize("wait", [None, 0])
+def test_the_maximum_is_not_the_sparse_elements(gpu, oracle_lib, wait, delta):
+    """The launch then goes over every row twice, with an exchange between its blocks; where that gives up (a limit of zero
+    rounds: every block decides at once) run_epoch takes up again with the separate launches, and rows that lacked
+    updates have them."""
+    to = oracle_lib
+    V, K, w, B = 3000, 96, 9, 200
+    tokens, offsets = small_corpus(40000, V, seed=2)
+    starts, invf = to.window_starts(offsets, w), to.inverse_frequency(tokens, V)
+    W0 = _planted(tokens, V, K)
+    t, perm = _trainer(tokens, offsets, V, K, w, B, W0, delta=delta)
+    Wo = W0.copy()
+    steps = 25
+    eps = 1e-3
+    for s in range(steps):
+        if s == 10 and wait is not None:
+            break
+        t.step(s * B, B, eps, delta)
+    done = s if wait is not None and s == 10 else steps
+    to.train_steps(Wo, tokens, starts, perm, 0, B, done, w, invf, eps, delta=delta)
+    assert np.array_equal(t.get_weights().view(np.uint32), Wo.view(np.uint32))
+    known, made = t.dense_path_counts
+    assert t.row_update_steps >= done - 1 and made >= 3
+    if wait is not None:
+        t._set_wait_limit(wait)
+        t.run_epoch(3, 15)
+        n_steps = (len(starts) + B - 1) // B
+        to.train_steps(Wo, tokens, starts, perm, 0, B, n_steps, w, invf, to.epoch_eps(1e-3, 3, 15), delta=t.epoch_delta(3, 15))
+        assert np.array_equal(t.get_weights().view(np.uint32), Wo.view(np.uint32))
+        assert t.giveups_recovered == 1 and t.dense_launches == 2
+    t.close()
+
+
+def test_left_alone_where_the_maximum_keeps_failing(gpu, oracle_lib):
+    """Chosen by the sizes, the form is left for a while once its launches have had to make the pass for max|ds|."""
+    to = oracle_lib
+    V, K, w, B = 12000, 100, 5, 200
+    tokens, offsets = small_corpus(60000, V, seed=2)
+    starts, invf = to.window_starts(offsets, w), to.inverse_frequency(tokens, V)
+    W0 = _planted(tokens, V, K)
+    t, perm = _trainer(tokens, offsets, V, K, w, B, W0, mode=0)
+    Wo = W0.copy()
+    n_steps = (len(starts) + B - 1) // B
+    for ep in (3, 4, 5):
+        t.run_epoch(ep, 15)
+        to.train_steps(Wo, tokens, starts, perm, 0, B, n_steps, w, invf, to.epoch_eps(1e-3, ep, 15))
+        assert np.array_equal(t.get_weights().view(np.uint32), Wo.view(np.uint32)), ep
+    assert n_steps > 100 and 0 < t.row_update_steps < 3 * n_steps - 30
+    t.close()
+
+
+@pytest.mark.parametrize("entries", [1, 3])
+def test_more_sentinels_than_a_wave_notes(gpu, oracle_lib, entries):
+    from flyvec_amd import synthetic
+    to = oracle_lib
+    V, K, w, B = 700, 130, 9, 900
+    tokens, offsets = small_corpus(40000, V, seed=8)
+    starts, invf = to.window_starts(offsets, w), to.inverse_frequency(tokens, V)
+    W0 = synthetic.synapses(K, V, seed=2, sigma=0.02)
+    t, perm = _trainer(tokens, offsets, V, K, w, B, W0)
+    t.set_sentinel_list(entries)
+    Wo = W0.copy()
+    n_steps = (len(starts) + B - 1) // B
+    t.run_epoch(3, 15)
+    to.train_steps(Wo, tokens, starts, perm, 0, B, n_steps, w, invf, to.epoch_eps(1e-3, 3, 15))
+    assert np.array_equal(t.get_weights().view(np.uint32), Wo.view(np.uint32)) and t.row_update_steps >= n_steps - 1
+    t.close()
+
+
+def test_calls_between_steps_see_every_update(gpu, oracle_lib):
+    """Steps that visit rows, broken off in every way a caller can: look at the matrix, replace it, another order, another
+    place in it, another size of minibatch, another trainer's steps beside them, the separate launches."""
+    from flyvec_amd import Trainer, synthetic
+    to = oracle_lib
+    V, K, w, B = 2500, 61, 6, 150
+    tokens, offsets = small_corpus(30000, V, seed=5)
+    starts, invf = to.window_starts(offsets, w), to.inverse_frequency(tokens, V)
+    W0 = synthetic.synapses(K, V, seed=3, sigma=0.02)
+    t, perm = _trainer(tokens, offsets, V, K, w, B, W0)
+    other = Trainer(V, 8, w, 16)
+    other.set_corpus(tokens, offsets)
+    other.set_weights(synthetic.synapses(8, V, seed=1))
+    Wo = W0.copy()
+
+    def steps(first, n, count):
+        for s in range(count):
+            t.step(first + s * n, n, 1e-3)
+            to.train_step(Wo, to.inflate(tokens, starts, perm, first + s * n, n, w, V), invf, 1e-3)
+
+    def same(what):
+        assert np.array_equal(t.get_weights().view(np.uint32), Wo.view(np.uint32)), what
+
+    steps(0, B, 20)
+    assert np.allclose(t.row_norms(K), np.sqrt((Wo.astype(np.float64) ** 2).sum(1)), rtol=1e-12)
+    steps(20 * B, B, 7)
+    same("steps behind the norms")
+    steps(27 * B, B, 5)
+    Wo = synthetic.synapses(K, V, seed=4, sigma=0.02)
+    t.set_weights(Wo)
+    steps(32 * B, B, 9)
+    perm = np.random.default_rng(7).permutation(len(starts)).astype(np.uint64)
+    t.set_permutation(perm)
+    steps(0, B, 6)
+    t.shuffle(3)
+    perm = t.get_permutation()
+    steps(0, B, 6)
+    steps(50 * B + 3, B, 6)
+    steps(10 * B + 1, B - 7, 6)
+    same("another order, place and size")
+    steps(0, B, 6)
+    other.step(0, 16, 1e-4)
+    steps(6 * B, B, 4)
+    other.sync()
+    steps(10 * B, B, 4)
+    same("another trainer in flight")
+    steps(0, B, 6)
+    before = t.row_update_steps
+    t.set_dense_launches(2)
+    steps(6 * B, B, 3)
+    t.set_dense_launches(0)
+    steps(9 * B, B, 5)
+    xx, nc = t.step_stats()
+    ref = to.train_step(Wo.copy(), to.inflate(tokens, starts, perm, 0, B, w, V), invf, 1e-3)
+    steps(0, B, 1)
+    xx, nc = t.step_stats()
+    assert np.array_equal(xx, ref["xx"]) and nc == ref["nc"]
+    same("separate launches")
+    assert t.row_update_steps > before > 30
+    t.set_row_updates(1)
+    steps(0, B, 3)
+    same("every row")
+    assert t.time_steps(0, 20, 1e-3, per_kernel=False)[0] > 0 and t.time_steps_graph(0, 4, 1e-3, 2) > 0
+    t.close()
+    other.close()

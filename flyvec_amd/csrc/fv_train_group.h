@@ -38,6 +38,14 @@ struct fv_group_args {
   uint32_t *group_count;
   float *xx;
   uint32_t n;
+  // fv_group_bits_kernel: the rows of the winners' bits that the winner kernel has filled, the pair of the step before last (cleared here),
+  // how many windows the blocks of
+  // this launch have placed in order[] so far, and the neurons
+  const uint32_t *won;
+  uint32_t *won_clear;
+  uint32_t won_words;
+  uint32_t *placed;
+  uint32_t K;
   float scale;          // every scaled activation is multiplied by this first (1, or -delta for the second neurons)
   uint32_t accumulate;  // add the total to xx[h] instead of storing it
 };
@@ -350,3 +358,94 @@ __global__ __launch_bounds__(FV_NB_MAX_THREADS) void fv_group_kernel(fv_group_ar
   const float xx = fv_block_tree_sum(part, tree);
   if (tid == 0) a.xx[h] = a.accumulate ? __fadd_rn(a.xx[h], xx) : xx;
 }
+
+// The same from the neurons' rows of winner bits: 6 KB a neuron at 50000 windows, where every one of the K blocks above
+// reads the 100 KB of the winner array. 256 threads per neuron, four neurons per block. A thread takes FV_GROUP_RUN groups
+// of 64 windows, its subtree of the order of the totals xx. The windows' ids meet in LDS by rank, and from there the
+// activations are fetched (and order[] written) by all of the neuron's threads alike: a thread that fetched its
+// own matches' was one of the heaviest neuron's, batch behind batch. The number of windows that lower neurons won does not
+// come with the row: the block takes the next free place in order[] for its neurons. That changes where window ids and
+// slot records lie and no result. (One atomic per neuron on the one counter was most of the launch.)
+// K = 1000, V = 50000, B = 50000: 29.3 us from the winner array; a thread with its own matches 19.2, by rank 17.3, and
+// four neurons a block 10.8 (and the winner kernel, which marks the bits, 204.0 instead of 202.4).
+#define FV_GROUP_RUN 4
+#define FV_GROUP_NEURONS 4
+#define FV_GROUP_BITS_WINDOWS (64u * FV_GROUP_RUN * 256u)  // most windows of a step
+#define FV_GROUP_STAGE 3072  // windows of a neuron in LDS at a time
+__global__ __launch_bounds__(256 * FV_GROUP_NEURONS) void fv_group_bits_kernel(fv_group_args a) {
+  constexpr int R = FV_GROUP_RUN, M = FV_GROUP_NEURONS;
+  extern __shared__ uint32_t dyn[];  // ids and values of every neuron
+  __shared__ uint32_t wave_count[4 * M], sh_base;
+  __shared__ float wave_sum[4 * M];
+  const uint32_t tid = threadIdx.x & 255u, sub = __builtin_amdgcn_readfirstlane(threadIdx.x >> 8), wave = threadIdx.x >> 6;
+  const uint32_t h = blockIdx.x * M + sub;
+  const bool real = h < a.K;
+  uint32_t *ids = dyn + sub * 2 * FV_GROUP_STAGE;
+  float *val = (float *)(ids + FV_GROUP_STAGE);
+  uint64_t mask[R], left[R];
+  uint32_t eq = 0;
+#pragma unroll
+  for (int g = 0; g < R; ++g) {
+    const uint32_t word = 2 * (R * tid + g);
+    uint2 mw = make_uint2(0u, 0u);
+    if (real && word < a.won_words) {
+      mw = *(const uint2 *)(a.won + (uint64_t)h * a.won_words + word);
+      *(uint2 *)(a.won_clear + (uint64_t)h * a.won_words + word) = make_uint2(0u, 0u);
+    }
+    left[g] = mask[g] = (uint64_t)mw.x | ((uint64_t)mw.y << 32);
+    eq += (uint32_t)__popcll(mask[g]);
+  }
+  const uint32_t incl = fv_wave_inclusive_scan_u32(eq);
+  if ((threadIdx.x & 63u) == 63u) wave_count[wave] = incl;
+  fv_lds_barrier();
+  uint32_t my_off = incl - eq, c_h = 0, before = 0, all = 0, most = 0;
+#pragma unroll
+  for (uint32_t m = 0; m < M; ++m) {
+    uint32_t c = 0;
+#pragma unroll
+    for (uint32_t i = 0; i < 4; ++i) {
+      if (m == sub && m * 4 + i < wave) my_off += wave_count[m * 4 + i];
+      c += wave_count[m * 4 + i];
+    }
+    if (m < sub) before += c;
+    if (m == sub) c_h = c;
+    all += c;
+    most = max(most, c);
+  }
+  // (no more than n windows in all: the bound is for a launch repeated by itself)
+  if (threadIdx.x == 0) sh_base = all ? min(atomicAdd(a.placed, all), a.n - all) : 0u;
+  float part[R];
+#pragma unroll
+  for (int g = 0; g < R; ++g) part[g] = 0.0f;
+  uint32_t put = my_off, add = my_off;  // rank of the thread's next match to be staged, to be added
+  for (uint32_t j0 = 0; j0 < most; j0 += FV_GROUP_STAGE) {
+    const uint32_t j1 = min(c_h, j0 + FV_GROUP_STAGE);
+#pragma unroll
+    for (int g = 0; g < R; ++g)
+      for (; mask[g] && put < j1; mask[g] &= mask[g] - 1)
+        ids[put++ - j0] = 64 * (R * tid + g) + (uint32_t)__ffsll((long long)mask[g]) - 1;
+    __syncthreads();
+    uint32_t *order = a.order + sh_base + before;
+    for (uint32_t j = j0 + tid; j < j1; j += 256) {
+      const uint32_t r = ids[j - j0];
+      order[j] = r;
+      val[j - j0] = a.sc[r];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int g = 0; g < R; ++g)
+      for (; left[g] && add < j1; left[g] &= left[g] - 1) part[g] = __fadd_rn(part[g], val[add++ - j0]);
+    fv_lds_barrier();
+  }
+  static_assert(R == 4, "a thread's subtree");
+  const float ws = fv_wave_tree_sum(__fadd_rn(__fadd_rn(part[0], part[1]), __fadd_rn(part[2], part[3])));
+  if ((threadIdx.x & 63u) == 0) wave_sum[wave] = ws;
+  __syncthreads();
+  if (tid == 0 && real) {
+    const float *t = wave_sum + sub * 4;
+    a.group_base[h] = sh_base + before;
+    a.group_count[h] = c_h;
+    a.xx[h] = __fadd_rn(__fadd_rn(t[0], t[1]), __fadd_rn(t[2], t[3]));
+  }
+}
+#define FV_GROUP_BITS_LDS (2 * FV_GROUP_STAGE * FV_GROUP_NEURONS * sizeof(uint32_t))

@@ -11,8 +11,9 @@
 // additions; if all three results share a binade and the two differences are equal, the state
 // is steady and the remaining additions inside the binade are one integer multiply-add on the
 // bit pattern (stopping short of the binade's ends); binade crossings, including the passage
-// through zero, are taken with real additions.  Compiles for the host too, where the tests
-// check it against the plain loop.
+// through zero, are taken with real additions.  Fewer than FV_REPEAT_JUMP additions are simply made, eight to a turn:
+// a turn that looks for the steady state costs as much as sixty additions (the division), and the sums of an ordinary
+// minibatch have a few dozen.  Compiles for the host too, where the tests check it against the plain loop.
 #pragma once
 
 #include <stdint.h>
@@ -46,8 +47,12 @@ FV_HD float fv_add1(float a, float b) {
 #endif
 }
 
+#ifndef FV_REPEAT_JUMP
+#define FV_REPEAT_JUMP 96u
+#endif
+
 FV_HD float fv_add_repeat(float v, float f, uint32_t n) {
-  while (n >= 4) {
+  while (n >= FV_REPEAT_JUMP) {
     const float v1 = fv_add1(v, f), v2 = fv_add1(v1, f), v3 = fv_add1(v2, f);
     n -= 3;
     v = v3;
@@ -72,9 +77,12 @@ FV_HD float fv_add_repeat(float v, float f, uint32_t n) {
       }
     }
   }
-  while (n > 0) {
-    v = fv_add1(v, f);
-    --n;
+  for (; n >= 8; n -= 8) {
+    v = fv_add1(fv_add1(fv_add1(fv_add1(v, f), f), f), f);
+    v = fv_add1(fv_add1(fv_add1(fv_add1(v, f), f), f), f);
   }
+  if (n & 4u) v = fv_add1(fv_add1(fv_add1(fv_add1(v, f), f), f), f);
+  if (n & 2u) v = fv_add1(fv_add1(v, f), f);
+  if (n & 1u) v = fv_add1(v, f);
   return v;
 }

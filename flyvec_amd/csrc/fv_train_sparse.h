@@ -248,6 +248,14 @@ __device__ __forceinline__ void fv_sparse_light(const fv_sparse_args &a, uint32_
   if (tid < FV_NB_CLASSES) a.slot_count[(h << FV_NB_CLASS_SHIFT) | tid] = cls_n[tid];
 }
 
+// Bit 0: the low half of the word is not zero; bit 16: the high half. (Written as the instruction: the compiler makes two
+// comparisons, two selections and their joining of it.)
+__device__ __forceinline__ uint32_t fv_nonzero_halves(uint32_t word) {
+  uint32_t r;
+  asm("v_pk_min_u16 %0, %1, %2" : "=v"(r) : "v"(word), "s"(0x00010001u));
+  return r;
+}
+
 // DELTA: the neuron's elements are counted over two lists of windows, those it won and those in
 // which it came second, into two counter arrays; a record carries both counts.
 // GROUPING: no grouping launch has run. Every class block takes its neuron's windows from the bit row
@@ -302,8 +310,33 @@ __device__ __forceinline__ void fv_sparse_block(const fv_sparse_args &a) {
   // scaled activations a thread fetches before it knows how many it needs: four, or sixteen in a wave with a
   // thread that has more than four matches (a neuron that won a tenth of the minibatch has seven per thread)
   constexpr int PF = 4, PF_BIG = 16;
+  const uint32_t stage_cap = fv_sparse_stage_cap(a.stride);  // window ids staged in LDS at a time
   float pf[PF_BIG];
   float x_h = 0.0f;
+  // GROUPING: the window ids of ranks [j0, j0 + FV_SP_STAGE) into LDS, every thread those of its own matches (its
+  // ranks start at my_off; a neuron with more windows than LDS stages is staged part by part, each time
+  // from the bit row's words in registers)
+  auto stage_ids = [&](uint32_t j0, int second = 0) {
+    uint32_t at = (second ? my_off2 : my_off) - j0;  // wraps below 0 for the ranks in front of the part
+    // the two halves of a word one after the other, four matches between two branches, as many rounds as the
+    // wave's busiest thread needs (a taken branch costs a lone wave as much as four or five instructions)
+#pragma unroll
+    for (int half = 0; half < 2 * NW; ++half) {
+      uint32_t mm = (uint32_t)((second ? mask2 : mask[half >> 1]) >> (32 * (half & 1)));
+      const uint32_t first = r0 + 32u * half;
+      const uint32_t rounds = (fv_wave_max_u32((uint32_t)__popc(mm)) + 3u) >> 2;
+      for (uint32_t it = 0; it < rounds; ++it) {
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+          // (no branch around a match: one masked store, the rest by selects; a thread out of matches adds nothing)
+          const bool more = mm != 0;
+          if (more && at < stage_cap) ord[at] = (ord_t)(first + (uint32_t)__ffs((int)mm) - 1u);
+          at += more ? 1u : 0u;
+          mm &= mm - 1;
+        }
+      }
+    }
+  };
   if (GROUPING) {
     static_assert(NW == 1, "a thread's words are one group of 64 windows of the order of the totals xx");
     const uint32_t n = a.n;
@@ -405,6 +438,8 @@ __device__ __forceinline__ void fv_sparse_block(const fv_sparse_args &a) {
     // The launch lasts as long as its few heaviest blocks: their waves go first wherever they share a
     // SIMD with the waves of light blocks.
     if (c_h > FV_SP_HEAVY) __builtin_amdgcn_s_setprio(3);
+    // the window ids of the usual neuron go to LDS while the activations travel (the counting pass starts behind a barrier)
+    if (!DELTA && c_h <= stage_cap) stage_ids(0);
     // xx[h]: the thread's group first, in row order onto +0 (what was fetched, then, for a thread with more matches
     // than that, the rest one by one), then the tree over the threads
     {
@@ -501,15 +536,13 @@ __device__ __forceinline__ void fv_sparse_block(const fv_sparse_args &a) {
         }
         return;
       }
-      {
+      if (DELTA) {
         uint32_t at = my_off;  // the window ids by rank
 #pragma unroll
         for (int i = 0; i < NW; ++i)
           for (uint64_t mm = mask[i]; mm; mm &= mm - 1) ord[at++] = (ord_t)(r0 + 64 * i + (uint32_t)__ffsll((long long)mm) - 1);
-        if (DELTA) {
-          at = c_h + my_off2;  // behind them those in which the neuron came second
-          for (uint64_t mm = mask2; mm; mm &= mm - 1) ord[at++] = (ord_t)(r0 + (uint32_t)__ffsll((long long)mm) - 1);
-        }
+        at = c_h + my_off2;  // behind them those in which the neuron came second
+        for (uint64_t mm = mask2; mm; mm &= mm - 1) ord[at++] = (ord_t)(r0 + (uint32_t)__ffsll((long long)mm) - 1);
       }
       fv_sparse_light<DELTA, ord_t>(a, h, blk, c_h, c2_h, x_h, cnt, ord, red2, sh_hits, wave_max);
       return;
@@ -537,41 +570,11 @@ __device__ __forceinline__ void fv_sparse_block(const fv_sparse_args &a) {
   const uint64_t place_low = regions ? (uint64_t)blk * slot_primary : slot_first;
   const uint64_t place_high = regions ? fv_slot_place(blk, slot_primary, a.slot_region, a.n_blocks) - slot_primary : slot_first;
 
-  const uint32_t stage_cap = fv_sparse_stage_cap(a.stride);  // window ids staged in LDS at a time
   const bool staged_once = !DELTA && c_h <= stage_cap;  // the usual case: the neuron's window ids are staged here
   if (!GROUPING) {
     for (uint32_t i = tid; i < CW / 4; i += T) ((uint4 *)cnt)[i] = make_uint4(0, 0, 0, 0);
     if (DELTA)
       for (uint32_t i = tid; i < CW / 4; i += T) ((uint4 *)cnt2)[i] = make_uint4(0, 0, 0, 0);
-  }
-  // GROUPING: the window ids of ranks [j0, j0 + FV_SP_STAGE) into LDS, every thread those of its own matches (its
-  // ranks start at my_off; a neuron with more windows than LDS stages is staged part by part, each time
-  // from the bit row's words in registers)
-  auto stage_ids = [&](uint32_t j0, int second = 0) {
-    uint32_t at = (second ? my_off2 : my_off) - j0;  // wraps below 0 for the ranks in front of the part
-    // the two halves of a word one after the other, four matches between two branches, as many rounds as the
-    // wave's busiest thread needs (a taken branch costs a lone wave as much as four or five instructions)
-#pragma unroll
-    for (int half = 0; half < 2 * NW; ++half) {
-      uint32_t mm = (uint32_t)((second ? mask2 : mask[half >> 1]) >> (32 * (half & 1)));
-      const uint32_t first = r0 + 32u * half;
-      const uint32_t rounds = (fv_wave_max_u32((uint32_t)__popc(mm)) + 3u) >> 2;
-      for (uint32_t it = 0; it < rounds; ++it) {
-#pragma unroll
-        for (int u = 0; u < 4; ++u) {
-          // (no branch around a match: one masked store, the rest by selects; a thread out of matches adds nothing)
-          const bool more = mm != 0;
-          if (more && at < stage_cap) ord[at] = (ord_t)(first + (uint32_t)__ffs((int)mm) - 1u);
-          at += more ? 1u : 0u;
-          mm &= mm - 1;
-        }
-      }
-    }
-  };
-  if (GROUPING) {
-    if (staged_once) stage_ids(0);
-    // the counting pass starts behind a barrier
-  } else {
     if (staged_once)
       for (uint32_t i = tid; i < c_h; i += T) ord[i] = (ord_t)order[i];
     fv_lds_barrier();
@@ -616,7 +619,12 @@ __device__ __forceinline__ void fv_sparse_block(const fv_sparse_args &a) {
       if (tid == 0) sh_pos = 0;
       fv_lds_barrier();
       {
-        // bit 8 * i + u of `mine`: counter u of the thread's i-th group of four words is non-zero
+        // Bits 8 i .. 8 i + 7 of `mine`: the non-zero counters of the thread's i-th group of four words. narrow: the low
+        // halves of the words, then the high ones (a packed minimum with 1 leaves a word's two answers 16 bits apart: three
+        // instructions a word where there were eight). All blocks of a compute unit come through here at about the same
+        // time and the vector units are what they wait for: 1.6 to 1.9 us of every block's 7 to 12. With the plain
+        // additions of fv_add_repeat and the window ids staged while the activations travel, K = 400, V = 20000,
+        // B = 10000: 15.1 -> 14.2 us, with the anti-Hebbian term 31.0 -> 28.9, K = 209, V = 7919, B = 3001 11.2 -> 10.1.
         constexpr int n_groups = (CW / 4 + T - 1) / T;
         static_assert(n_groups <= 8, "a 64-bit mask holds eight groups");
         uint64_t mine = 0;
@@ -624,27 +632,19 @@ __device__ __forceinline__ void fv_sparse_block(const fv_sparse_args &a) {
         for (int i = 0; i < n_groups; ++i) {
           const uint32_t g4 = min(tid + i * T, (uint32_t)CW / 4 - 1);
           uint4 c4 = ((const uint4 *)cnt)[g4];
-          if (DELTA) {
+          if (DELTA) {  // a half or a word is non-zero in the union if it is in either array
             const uint4 d4 = ((const uint4 *)cnt2)[g4];
-            if (narrow) {
-              // a 16-bit half is non-zero in the union if it is in either word: OR keeps that
-              c4.x |= d4.x; c4.y |= d4.y; c4.z |= d4.z; c4.w |= d4.w;
-            } else {
-              c4.x |= d4.x; c4.y |= d4.y; c4.z |= d4.z; c4.w |= d4.w;
-            }
+            c4.x |= d4.x; c4.y |= d4.y; c4.z |= d4.z; c4.w |= d4.w;
           }
-          if (tid + i * T >= CW / 4) c4 = make_uint4(0, 0, 0, 0);
-          const uint32_t cw[4] = {c4.x, c4.y, c4.z, c4.w};
           uint32_t bits = 0;
-#pragma unroll
-          for (int u = 0; u < 4; ++u) {
-            if (narrow) {
-              bits |= ((cw[u] & 0xffffu) ? 1u : 0u) << (2 * u);
-              bits |= ((cw[u] >> 16) ? 1u : 0u) << (2 * u + 1);
-            } else {
-              bits |= (cw[u] ? 1u : 0u) << u;
-            }
+          if (narrow) {
+            const uint32_t both = fv_nonzero_halves(c4.x) | (fv_nonzero_halves(c4.y) << 1) | (fv_nonzero_halves(c4.z) << 2) |
+                                  (fv_nonzero_halves(c4.w) << 3);
+            bits = (both | (both >> 12)) & 0xffu;
+          } else {
+            bits = (c4.x ? 1u : 0u) | (c4.y ? 2u : 0u) | (c4.z ? 4u : 0u) | (c4.w ? 8u : 0u);
           }
+          if (i == n_groups - 1 && tid + i * T >= CW / 4) bits = 0;
           mine |= (uint64_t)bits << (8 * i);
         }
         // list positions: prefix sum inside the wave, one LDS atomic per wave
@@ -658,7 +658,9 @@ __device__ __forceinline__ void fv_sparse_block(const fv_sparse_args &a) {
         while (mine) {
           const uint32_t b = (uint32_t)__ffsll((long long)mine) - 1;
           mine &= mine - 1;
-          if (e < FV_SP_LIST_CAP) list[e] = (uint16_t)((tid + (b >> 3) * T) * (narrow ? 8u : 4u) + (b & 7u));
+          // (narrow: bits 0 to 3 are the counters 0, 2, 4, 6 of the group, bits 4 to 7 the counters 1, 3, 5, 7)
+          const uint32_t in_group = narrow ? 2u * (b & 3u) + ((b >> 2) & 1u) : b & 7u;
+          if (e < FV_SP_LIST_CAP) list[e] = (uint16_t)((tid + (b >> 3) * T) * (narrow ? 8u : 4u) + in_group);
           ++e;
         }
       }

@@ -16,15 +16,13 @@
 #include "fv_host_plan.h"
 #include "fv_internal.h"
 
-// Four: with two, 100003 windows to 40 MB of int8 codes take 2.0 ms instead of 1.45 and a matrix of 64 MB down 3.9 instead of
-// 2.7; with six 1.3 and 2.55, but 20000 targets (8 MB) 380 us instead of 340, with eight 435: starting them costs that.
-#define FV_COPY_THREADS 4
-
 // Ordinary (pageable) host memory, which the device cannot reach by DMA? (fv_runtime.hip)
 bool fv_is_pageable(const void *p);
 
 // Host threads that copy pieces for the length of one call. Pieces are published in order; every thread copies its
-// share of every piece.
+// share of every piece. The threads begin with start(), or with the first piece: starting them takes 70 to 100 us, which
+// a caller whose pieces come from the device spends while the first one is on its way (20000 targets 402 -> 349 us, 100003
+// windows 1615 -> 1533 with four threads).
 struct fv_copy_ring {
   struct item {  // `rows` rows of `bytes` bytes
     const char *src;
@@ -37,13 +35,20 @@ struct fv_copy_ring {
   std::atomic<uint32_t> published{0};
   std::atomic<bool> quit{false};
   std::vector<std::thread> workers;
+  uint32_t wanted;
+  bool begun = false;
   uint32_t crew = 0;  // threads that started (none: publish copies by itself)
 
-  explicit fv_copy_ring(size_t max_items) : items(max_items), finished(new std::atomic<uint32_t>[max_items]) {
+  fv_copy_ring(size_t max_items, uint32_t threads)
+      : items(max_items), finished(new std::atomic<uint32_t>[max_items]), wanted(threads) {
     for (size_t i = 0; i < max_items; ++i) finished[i].store(0);
+  }
+  void start() {
+    if (begun) return;
+    begun = true;
     std::atomic<uint32_t> *go = &started;
     try {
-      for (uint32_t p = 0; p < FV_COPY_THREADS; ++p) {
+      for (uint32_t p = 0; p < wanted; ++p) {
         workers.emplace_back([this, p, go] {
           while (go->load(std::memory_order_acquire) == 0) std::this_thread::yield();
           run(p);
@@ -70,6 +75,7 @@ struct fv_copy_ring {
     }
   }
   uint32_t publish(const item &it) {
+    start();
     const uint32_t i = published.load(std::memory_order_relaxed);
     items[i] = it;
     if (crew == 0) copy_share(it, 0, 1);
@@ -128,7 +134,7 @@ int fv_pipe_up(fv_stage_lease &lease, uint64_t n_pieces, hipStream_t stream, Pie
     FV_HIP(hipStreamSynchronize(stream));
     return FV_OK;
   }
-  fv_copy_ring ring(n_pieces);
+  fv_copy_ring ring(n_pieces, fv_copy_threads(n_pieces * FV_STAGE_SLOT_BYTES));
   int rc = FV_OK;
   for (uint64_t t = 0; t < n_pieces + S - 1 && rc == FV_OK; ++t) {
     if (t < n_pieces) {
@@ -162,7 +168,7 @@ int fv_pipe_down(fv_stage_lease &lease, uint64_t n_pieces, hipStream_t stream, P
     fv_copy_ring::copy_share(it, 0, 1);
     return FV_OK;
   }
-  fv_copy_ring ring(n_pieces);
+  fv_copy_ring ring(n_pieces, fv_copy_threads(n_pieces * FV_STAGE_SLOT_BYTES));
   const uint64_t ahead = S > 1 ? S - 1 : 1;  // pieces the device may be ahead of the host threads by
   int rc = FV_OK;
   for (uint64_t t = 0; t < n_pieces + ahead && rc == FV_OK; ++t) {
@@ -177,6 +183,7 @@ int fv_pipe_down(fv_stage_lease &lease, uint64_t n_pieces, hipStream_t stream, P
       rc = produce(t, lease.slots[t % S]);
       if (rc == FV_OK && hipEventRecord(lease.events[t % S], stream) != hipSuccess)
         rc = fv_fail(FV_ERR_HIP, "staged download: event record failed");
+      ring.start();
     }
   }
   (void)hipStreamSynchronize(stream);  // before the slots go back (an error is in rc already)

@@ -40,6 +40,8 @@
 // Every one of the n additions of 1/f onto ds[h][i] adds the same value, so the reference's
 // result for that element depends only on n; replaying n sequential fp32 adds reproduces it
 // exactly whatever order its atomics ran in.
+#include <thread>
+
 #include "fv_host_copy.h"
 #include "fv_train_state.h"
 #include "fv_train_top2.h"
@@ -200,6 +202,13 @@ static int fv_trainer_reserve_windows(fv_trainer *t, uint64_t n_windows) {
   return FV_OK;
 }
 
+// The matrix or the corpus is another: what the launches have said so far says nothing of it.
+static void fv_rows_forget_verdicts(fv_trainer *t) {
+  t->verdicts = t->verdicts_base = (uint32_t)(*(volatile unsigned long long *)t->rows_verdict >> 32);
+  t->verdicts_asked = false;
+  t->rows_clear = FV_ROWS_CLEAR;
+}
+
 // Sets a corpus with `load`. If that fails in the runtime while buffers of an earlier corpus are kept (the device's memory
 // may have been too little for both) they are given back and it is done once more as on a new trainer: what fits there
 // fits here. A corpus that is refused leaves the trainer without one, and without its buffers.
@@ -213,6 +222,7 @@ static int fv_trainer_load_corpus(fv_trainer *t, uint64_t n_tokens, Load load) {
       t->n_tokens = n_tokens;
       t->n_windows = n_windows;
       t->have_corpus = true;
+      fv_rows_forget_verdicts(t);
       return FV_OK;
     }
     fv_trainer_free_corpus(t);
@@ -265,7 +275,6 @@ static fv_rows_args fv_rows_describe(const fv_trainer *t, uint32_t step) {
   // rounded upwards
   b.drift = (float)(t->rows_drift * 1.0001 + 1e-30);
   b.wave_hits = t->rows_wave_hits;
-  b.fallbacks = t->rows_fallback;
   return b;
 }
 
@@ -369,7 +378,7 @@ extern "C" int fv_trainer_destroy(fv_trainer *t) {
 
 // Whether the dense launch of a step should visit only the rows somebody needs, going by the sizes.
 static bool fv_rows_worth_it(const fv_trainer *t) {
-  return t->rows_ok && (uint64_t)t->B * t->w <= FV_ROWS_MOST_POSITIONS * t->N && (uint64_t)t->total4 * 16 >= FV_ROWS_LEAST_BYTES;
+  return t->rows_ok && t->ldk >= FV_ROWS_LEAST_LDK && (uint64_t)t->B * t->w <= FV_ROWS_MOST_POSITIONS * t->N && (uint64_t)t->total4 * 16 >= FV_ROWS_LEAST_BYTES;
 }
 
 // Entries of an index matrix: a row per window of a minibatch, and the padding behind them.
@@ -467,9 +476,9 @@ static int fv_trainer_alloc(fv_trainer *t) {
   // status word behind them
   FV_HIP(hipMalloc((void **)&t->scalars, 16 * sizeof(float) + (size_t)t->K * FV_NORM_BLOCKS * sizeof(double)));
   t->norm_part = (double *)(t->scalars + 16);
-  FV_HIP(hipHostMalloc((void **)&t->norms, t->K * sizeof(double) + 2 * sizeof(uint32_t), hipHostMallocDefault));
-  t->rows_fallback = (uint32_t *)(t->norms + t->K) + 1;
-  *t->rows_fallback = 0;
+  FV_HIP(hipHostMalloc((void **)&t->norms, t->K * sizeof(double) + 2 * sizeof(unsigned long long), hipHostMallocDefault));
+  t->rows_verdict = (unsigned long long *)(t->norms + t->K) + 1;
+  *t->rows_verdict = 0;
   t->xx_last = t->xx;
   if (fv_rows_worth_it(t) && fv_trainer_alloc_rows(t) != FV_OK) {  // (the trainer does without)
     (void)hipGetLastError();
@@ -609,7 +618,7 @@ extern "C" int fv_trainer_create(const fv_train_config *cfg, fv_trainer **out_tr
   t->V = cfg->vocab;
   t->N = N;
   t->total4 = (uint32_t)(N * ldk / 4);
-  t->rows_hold_next = 16;
+  t->rows_clear = FV_ROWS_CLEAR;
   float cut = (float)1.e-10;  // the reference compares fabs(fp32) > 1.e-10 in double
   if ((double)cut > 1.e-10) cut = nextafterf(cut, 0.0f);
   t->update_cut = cut;
@@ -759,6 +768,7 @@ extern "C" int fv_trainer_set_weights(fv_trainer *t, const float *W) {
   fv_trainer_leaves_flight(t);  // (the stream has drained)
   t->have_weights = true;
   t->top2_valid = false;  // the first single dense launch on the new matrix makes the pass for max|ds|
+  fv_rows_forget_verdicts(t);
   return FV_OK;
 }
 
@@ -892,6 +902,15 @@ static bool fv_groups_in_sparse(const fv_trainer *t) {
   return t->won[0] && t->B <= 64 * FV_SP_THREADS && !t->separate_grouping;
 }
 
+// Waits until the device has done `launches` of the trainer's single dense launches, or everything it was given.
+static void fv_rows_wait_for(fv_trainer *t, uint32_t launches) {
+  while ((int32_t)((uint32_t)(*(volatile unsigned long long *)t->rows_verdict >> 32) - launches) < 0) {
+    if (hipStreamQuery(t->stream) != hipErrorNotReady) break;
+    std::this_thread::yield();
+  }
+  (void)hipGetLastError();  // ("not ready")
+}
+
 // Whether this step (a whole one, its dense passes in one launch) takes the form that visits the rows somebody needs.
 // A sequence of such steps begins where at least FV_ROWS_SEQUENCE steps follow each other without anybody looking
 // at the matrix in between (those enqueued and those the caller has announced): it costs a launch at its start and one at its end.
@@ -899,20 +918,24 @@ static bool fv_rows_take(fv_trainer *t, float eps, bool alone) {
   if (!t->hist_xx || t->rows_mode == 1 || t->cfg.prune_duplicates || t->capturing || !alone) return false;
   if (t->rows_mode == 0 && !fv_rows_worth_it(t)) return false;
   if (!(fabsf(eps) <= 1.0f)) return false;
-  const uint32_t fell_back = *(volatile uint32_t *)t->rows_fallback;
-  if (fell_back != t->rows_fallback_seen) {
-    // max|ds| was not the sparse elements' and the launch went over the matrix twice: every row in every step for a while,
-    // longer each time this happens again
-    t->rows_fallback_seen = fell_back;
-    t->rows_hold = t->rows_hold_next;
-    if (t->rows_hold_next < 4096) t->rows_hold_next *= 2;
-  }
-  if (t->rows_mode == 0 && t->rows_hold) {
-    t->rows_hold--;
+  if (t->rows_mode == 2) return t->rows_behind || t->top2_valid;
+  if (fabsf(eps) * FV_ROWS_DRIFT_STEPS > FV_ROWS_DRIFT) return false;
+  // As the sizes say, and only where the launches so far have found the maximum of |ds| to be the sparse elements' by far
+  // (a corpus of a few million tokens; on larger ones 1/f is small and the dense elements decide).
+  const uint32_t in_a_row = (uint32_t)*(volatile unsigned long long *)t->rows_verdict;
+  if (t->rows_behind) {
+    if (in_a_row != 0) return true;
+    if (t->rows_clear < FV_ROWS_CLEAR_MOST) t->rows_clear *= 2;
     return false;
   }
-  if (t->rows_behind) return true;
-  return t->top2_valid && (t->rows_mode == 2 || t->to_come + t->in_a_row >= FV_ROWS_SEQUENCE);
+  if (!t->top2_valid || t->to_come + t->in_a_row < FV_ROWS_SEQUENCE) return false;
+  if (!t->verdicts_asked && t->to_come >= FV_ROWS_SEQUENCE && t->verdicts - t->verdicts_base >= FV_ROWS_CLEAR + 2) {
+    // the first steps of an epoch on a new matrix: their answers are worth a short wait, the device has a step left to do
+    fv_rows_wait_for(t, t->verdicts - 1);
+    t->verdicts_asked = true;
+  }
+  const unsigned long long said = *(volatile unsigned long long *)t->rows_verdict;
+  return (int32_t)((uint32_t)(said >> 32) - t->verdicts_base) >= (int32_t)t->rows_clear && (uint32_t)said >= t->rows_clear;
 }
 
 // n_fresh < n: only the first n_fresh windows are sampled (from `first` on), the rows behind them are what
@@ -938,7 +961,16 @@ static int fv_enqueue_step(fv_trainer *t, uint64_t first, uint32_t n, float eps,
   const bool rows = whole && onepass && n_fresh >= n && fv_rows_take(t, eps, alone);
   const bool sampled_ahead = whole && t->ahead_valid && t->ahead_first == first && t->ahead_n == n && n_fresh >= n;
   const bool rows_go_on = rows && sampled_ahead && t->ahead_marked;
-  if (whole && t->rows_behind && (!rows || !rows_go_on || t->rows_since >= FV_ROWS_REFRESH)) FV_HIP(fv_trainer_settle(t));
+  const bool refresh = t->rows_since >= FV_ROWS_REFRESH || (t->rows_mode == 0 && t->rows_drift >= FV_ROWS_DRIFT);
+  if (whole && t->rows_behind && (!rows || !rows_go_on || refresh)) FV_HIP(fv_trainer_settle(t));
+  if (rows && refresh) {
+    // no further ahead of the device than to the refresh before the last: what its launches find has to be heard of
+    fv_rows_wait_for(t, t->rows_mark_before);
+    t->rows_mark_before = t->rows_mark;
+    t->rows_mark = t->verdicts;
+  } else if (rows && !t->rows_behind) {
+    t->rows_mark_before = t->rows_mark = t->verdicts;
+  }
   // the rows' two largest weights are in hand if the last write of the matrix was a single dense launch
   const bool top2_known = whole ? t->top2_valid : t->last_top2_known;
   if (whole) t->last_top2_known = top2_known;
@@ -1218,6 +1250,7 @@ static int fv_enqueue_step(fv_trainer *t, uint64_t first, uint32_t n, float eps,
   d.top2_part = t->top2_part;
   d.part_base = onepass ? 0u : t->update_blocks;
   d.path_count = t->path_count;
+  d.verdict = t->rows_verdict;
   d.eps = eps;
   d.prec = t->cfg.prec;
   d.update_cut = t->update_cut;
@@ -1234,6 +1267,7 @@ static int fv_enqueue_step(fv_trainer *t, uint64_t first, uint32_t n, float eps,
     d.ahead_n = next2_n;
     d.idx_ahead = t->idx_ahead2;
     t->dense_forms[0]++;
+    t->verdicts++;
     hipLaunchKernelGGL((fv_dense_rows_kernel<FV_ROWS_DEPTH, FV_ROWS_LATE>), dim3(t->onepass_blocks), dim3(FV_ONEPASS_THREADS), fv_rows_smem(t),
                        t->stream, d, ra);
     t->ahead_valid = t->ahead_marked = next_n != 0;
@@ -1268,6 +1302,7 @@ static int fv_enqueue_step(fv_trainer *t, uint64_t first, uint32_t n, float eps,
       // no other trainer in flight: one launch that exchanges the blocks' maxima itself where it needs them; else the
       // launch twice, in the form that waits for nobody (both with this step's launch number)
       t->dense_forms[alone ? 0 : 1]++;
+      t->verdicts++;
       for (uint32_t phase = alone ? 0u : 1u; phase <= (alone ? 0u : 2u); ++phase) {
         d.phase = phase;
         if (t->onepass_stream) fv_launch_stream(d, t->onepass_blocks, fv_stream_smem(t), t->stream);

@@ -53,7 +53,22 @@ struct fv_dense_args {
   // same rule on the same inputs) and in the second reads the words, all written when it starts, and makes the
   // update. phase 0: one launch, the blocks exchange their maxima inside it (they must be resident together).
   uint32_t phase;
+  // What a single dense launch leaves for the host to choose the form of later steps by (fv_rows_take): launches so far << 32
+  // | launches in a row whose sparse elements' maximum was at least twice every dense element's bound. Page-locked; the
+  // two counts themselves are at scalars[10].
+  unsigned long long *verdict;
 };
+
+// By one thread of the launch; `before`: the two counts it has found.
+__device__ __forceinline__ void fv_leave_verdict(const fv_dense_args &a, uint2 before, bool known, bool clear) {
+  const uint32_t launches = before.x + 1u, in_a_row = !known ? before.y : clear ? min(before.y + 1u, 0xffffu) : 0u;
+  *(uint2 *)(a.scalars + 10) = make_uint2(launches, in_a_row);
+  *a.verdict = ((unsigned long long)launches << 32) | in_a_row;
+}
+// Twice the bound, both as bit patterns of non-negative floats (a NaN is larger than any).
+__device__ __forceinline__ bool fv_clearly_sparse(uint32_t sparse, uint32_t dense) {
+  return dense < 0x7f000000u && dense + 0x00800000u <= sparse;
+}
 
 // ds of a dense element is -xx[h] * W (flyvec/src/cuda_funcs.cu:657-672 without the sparse term). No
 // test for a sentinel or for xx == 0 is needed in the two passes: a sentinel is a NaN and so are
@@ -628,6 +643,7 @@ __global__ __launch_bounds__(FV_ONEPASS_THREADS) void fv_dense_onepass_kernel(fv
   }
   // after one launch has given up, the launches already enqueued behind it neither wait nor update
   const bool dead = a.scalars[1] != 0.0f;
+  const uint2 verdict_before = *(const uint2 *)(a.scalars + 10);
   const uint32_t limit = dead ? 0u : a.spin_limit;
   float4 w[U];
   __builtin_amdgcn_sched_barrier(0);  // nothing that uses a small load moves up between the loads of W
@@ -681,6 +697,8 @@ __global__ __launch_bounds__(FV_ONEPASS_THREADS) void fv_dense_onepass_kernel(fv
   const bool fast = a.top2_known && F <= max(S, E);  // the same answer in every thread of every block
   const float4 xq = ((const float4 *)xs)[q];
   if (PHASE == 2 && fast) return;  // phase 1 has made the whole step
+  if (PHASE != 2 && blockIdx.x == 0 && tid == 0)
+    fv_leave_verdict(a, verdict_before, a.top2_known != 0, fv_clearly_sparse(S, max(E, F)));
   // the rows are streamed (loaded as their turn comes, updated, stored) rather than held from a pass for the maximum
   const bool streams = fast || PHASE == 2;
 
@@ -855,6 +873,7 @@ __global__ __launch_bounds__(FV_ONEPASS_THREADS) void fv_dense_stream_kernel(fv_
     smx[j] = ((const float4 *)(a.bmax + a.sparse_base))[h];
   }
   const bool dead = a.scalars[1] != 0.0f;
+  const uint2 verdict_before = *(const uint2 *)(a.scalars + 10);
   const uint32_t limit = dead ? 0u : a.spin_limit;
   float4 w[D];
   auto group_of = [&](uint32_t row) { return (row < a.n_rows ? row : row_inside) * a.ldk4 + q; };
@@ -901,6 +920,8 @@ __global__ __launch_bounds__(FV_ONEPASS_THREADS) void fv_dense_stream_kernel(fv_
   const bool fast = a.top2_known && F <= max(S, E);
   const float4 xq = ((const float4 *)xs)[q];
   if (PHASE == 2 && fast) return;  // phase 1 has made the whole step
+  if (PHASE != 2 && blockIdx.x == 0 && tid == 0)
+    fv_leave_verdict(a, verdict_before, a.top2_known != 0, fv_clearly_sparse(S, max(E, F)));
   // the next minibatch is sampled beside the update's stream rather than during a wait
   const bool streams = fast || PHASE == 2;
 

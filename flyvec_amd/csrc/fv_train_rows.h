@@ -43,6 +43,14 @@
 // Steps that must follow each other for a sequence to begin, and after how many the bound of |W| starts afresh.
 #define FV_ROWS_SEQUENCE 8u
 #define FV_ROWS_REFRESH 128u
+#define FV_ROWS_DRIFT 0.02  // or when |W| may have grown by this much, which takes at least FV_ROWS_DRIFT_STEPS steps
+#define FV_ROWS_DRIFT_STEPS 32
+// Launches in a row that have to find the sparse elements' maximum twice the dense bound before a sequence begins: at
+// first, and at most (twice as many each time a sequence ended because one of its launches did not). A launch that cannot
+// tell max|ds| goes over the matrix twice (at K = 400 on a corpus of 10 M tokens, where the dense elements decide in
+// half of the steps, a step took 61 us so and 54 with every row updated).
+#define FV_ROWS_CLEAR 3u
+#define FV_ROWS_CLEAR_MOST 1024u
 // Where visiting rows pays: at most so many window positions per row of the matrix, at least so many bytes of matrix.
 // Measured per step, every row / rows as needed (us; Zipf tokens unless "uniform"): 0.4 MB 24.3 / 23.0, 0.5 MB 22.0 / 22.4,
 // 4 MB 24.6 / 22.1, 8 MB and 0.1 positions a row 26.1 / 22.2, 9.6 MB and 7.5 positions 36.2 / 36.3, 30 positions 67.3 / 68.1,
@@ -50,6 +58,7 @@
 // 22 positions 183.3 / 178.2, 400 MB and 7.5 positions 441 / 400 (uniform 690 / 677).
 #define FV_ROWS_MOST_POSITIONS 24ull
 #define FV_ROWS_LEAST_BYTES (4ull << 20)
+#define FV_ROWS_LEAST_LDK 32u  // (the lists take 16 bytes per row: an eighth of a matrix this narrow)
 // Steps whose xx is kept (a power of two): what fits the dense launch's LDS beside its lists.
 static inline uint32_t fv_rows_age(uint32_t ldk) { return ldk <= 1024 ? 16u : 8u; }
 
@@ -61,7 +70,6 @@ struct fv_rows_args {
   uint32_t rows_per_round;  // rows a block takes at a time (active / ldk4)
   float drift;           // what |W| may have grown by since row_top2 was taken
   uint32_t wave_hits;    // sentinels a wave notes in LDS
-  uint32_t *fallbacks;   // page-locked: launches that had to make the pass for max|ds|
 };
 
 // The samplers of minibatches to come also say which rows they will read.
@@ -224,6 +232,7 @@ __global__ __launch_bounds__(FV_ONEPASS_THREADS) void fv_dense_rows_kernel(fv_de
   }
   const float s_kept = b.hist_s[tid & (b.list.age - 1u)];
   const bool dead = a.scalars[1] != 0.0f;
+  const uint2 verdict_before = *(const uint2 *)(a.scalars + 10);
   const uint32_t n_hist = b.list.age * a.ldk4;  // at most 4 T
   const float4 *hist = (const float4 *)b.hist_xx;
   const float4 hist0 = hist[min(tid, n_hist - 1)], hist1 = hist[min(tid + T, n_hist - 1)];
@@ -276,6 +285,7 @@ __global__ __launch_bounds__(FV_ONEPASS_THREADS) void fv_dense_rows_kernel(fv_de
     F = max(F, red2[i][1]);
   }
   const float4 xq = x4[here * a.ldk4 + q];
+  if (blockIdx.x == 0 && tid == 0) fv_leave_verdict(a, verdict_before, true, !dead && fv_clearly_sparse(S, F));
 
   float s;
   bool ok = true;
@@ -410,7 +420,6 @@ __global__ __launch_bounds__(FV_ONEPASS_THREADS) void fv_dense_rows_kernel(fv_de
     if (blockIdx.x == 0 && tid == 0) {
       b.hist_s[here] = s;
       b.list.count[(step + 1u) & 1u] = 0;
-      *b.fallbacks = step;
     }
     for (uint32_t c = 0; c < all_rounds; ++c) {
       const uint32_t row = row0 + c * row_step;

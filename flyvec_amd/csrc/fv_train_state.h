@@ -145,12 +145,17 @@ struct fv_trainer {
   float *hist_xx, *hist_s;  // what fv_rows_list_args and fv_rows_args say of them; one allocation, null until it is needed
   uint32_t *row_need, *row_last, *row_list;
   unsigned long long *row_count;
-  uint32_t *rows_fallback;  // page-locked (in the allocation of norms): the last such launch that had to make the pass for max|ds|
-  uint32_t rows_fallback_seen, rows_hold, rows_hold_next;  // steps the trainer stays with visiting every row behind one
+  // what the single dense launches say of themselves (fv_dense_args.verdict; in the allocation of norms), how many such
+  // launches were enqueued, at the last change of the matrix or the corpus from outside, and whether run_epoch has waited for the first answers since
+  unsigned long long *rows_verdict;
+  uint32_t verdicts, verdicts_base;
+  bool verdicts_asked;
+  uint32_t rows_clear;      // launches in a row that must have been clear for a sequence to begin
   uint32_t rows_step;       // number of the newest such step
   uint32_t rows_first;      // no row lacks the update of a step before this one
   bool rows_behind;         // rows may lack updates: fv_trainer_settle before anybody else looks at the matrix
   uint64_t rows_steps;      // such steps so far
+  uint32_t rows_mark, rows_mark_before;  // `verdicts` at the last two refreshes
   uint32_t rows_since;      // such steps since row_top2 was exact, and the sum of their |eps|
   double rows_drift;
   int32_t *idx_ahead2;      // the minibatch after the next, sampled by such a step (room for it in the same allocation)

@@ -98,7 +98,7 @@ def test_the_maximum_is_not_the_sparse_elements(gpu, oracle_lib, wait, delta):
 
 
 def test_left_alone_where_the_maximum_keeps_failing(gpu, oracle_lib):
-    """Chosen by the sizes, the form is left for a while once its launches have had to make the pass for max|ds|."""
+    """Chosen by the sizes, the form is not taken, or left again, where the launches have to make the pass for max|ds|."""
     to = oracle_lib
     V, K, w, B = 12000, 100, 5, 200
     tokens, offsets = small_corpus(60000, V, seed=2)
@@ -111,7 +111,7 @@ def test_left_alone_where_the_maximum_keeps_failing(gpu, oracle_lib):
         t.run_epoch(ep, 15)
         to.train_steps(Wo, tokens, starts, perm, 0, B, n_steps, w, invf, to.epoch_eps(1e-3, ep, 15))
         assert np.array_equal(t.get_weights().view(np.uint32), Wo.view(np.uint32)), ep
-    assert n_steps > 100 and 0 < t.row_update_steps < 3 * n_steps - 30
+    assert n_steps > 100 and t.row_update_steps < 3 * n_steps - 30
     t.close()
 
 

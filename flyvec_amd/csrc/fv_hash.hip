@@ -349,7 +349,7 @@ static int fv_hash_host(fv_hasher *h, const int32_t *idx, uint64_t n, uint32_t w
   const auto stage_in = [&](uint64_t c) { return lease.slots[staging.in_slot[c % lanes]] + staging.in_at[c % lanes]; };
   const size_t stage_codes_at = stage_bits ? chunk * bits_row : 0;  // (behind the packed codes)
   std::unique_ptr<fv_copy_ring> ring;
-  if (lease.n) ring.reset(new fv_copy_ring(3 * n_chunks, fv_copy_threads(n * out_row)));
+  if (lease.n) ring.reset(new fv_copy_ring(3 * n_chunks));
   std::vector<uint32_t> last_item(n_chunks, 0xffffffffu);  // the last copy item of every chunk
   int rc = FV_OK;
   // chunk c's staged outputs are handed to the host threads once its copies have landed (one iteration later, while the

@@ -35,12 +35,10 @@ struct fv_copy_ring {
   std::atomic<uint32_t> published{0};
   std::atomic<bool> quit{false};
   std::vector<std::thread> workers;
-  uint32_t wanted;
   bool begun = false;
   uint32_t crew = 0;  // threads that started (none: publish copies by itself)
 
-  fv_copy_ring(size_t max_items, uint32_t threads)
-      : items(max_items), finished(new std::atomic<uint32_t>[max_items]), wanted(threads) {
+  explicit fv_copy_ring(size_t max_items) : items(max_items), finished(new std::atomic<uint32_t>[max_items]) {
     for (size_t i = 0; i < max_items; ++i) finished[i].store(0);
   }
   void start() {
@@ -48,7 +46,7 @@ struct fv_copy_ring {
     begun = true;
     std::atomic<uint32_t> *go = &started;
     try {
-      for (uint32_t p = 0; p < wanted; ++p) {
+      for (uint32_t p = 0; p < FV_COPY_THREADS; ++p) {
         workers.emplace_back([this, p, go] {
           while (go->load(std::memory_order_acquire) == 0) std::this_thread::yield();
           run(p);
@@ -134,7 +132,7 @@ int fv_pipe_up(fv_stage_lease &lease, uint64_t n_pieces, hipStream_t stream, Pie
     FV_HIP(hipStreamSynchronize(stream));
     return FV_OK;
   }
-  fv_copy_ring ring(n_pieces, fv_copy_threads(n_pieces * FV_STAGE_SLOT_BYTES));
+  fv_copy_ring ring(n_pieces);
   int rc = FV_OK;
   for (uint64_t t = 0; t < n_pieces + S - 1 && rc == FV_OK; ++t) {
     if (t < n_pieces) {
@@ -168,7 +166,7 @@ int fv_pipe_down(fv_stage_lease &lease, uint64_t n_pieces, hipStream_t stream, P
     fv_copy_ring::copy_share(it, 0, 1);
     return FV_OK;
   }
-  fv_copy_ring ring(n_pieces, fv_copy_threads(n_pieces * FV_STAGE_SLOT_BYTES));
+  fv_copy_ring ring(n_pieces);
   const uint64_t ahead = S > 1 ? S - 1 : 1;  // pieces the device may be ahead of the host threads by
   int rc = FV_OK;
   for (uint64_t t = 0; t < n_pieces + ahead && rc == FV_OK; ++t) {

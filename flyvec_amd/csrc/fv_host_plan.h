@@ -39,13 +39,10 @@ static inline int fv_matrix_upload_staged(size_t bytes) {
 
 /* Host threads of a transfer, started while its first piece is on its way (fv_copy_ring). Four against six against eight
  * (microseconds): 20000 targets (8 MB) 349, 395, 443;  a corpus with its order and table read back (21 MB) 1531, 1609,
- * 1640;  100003 windows to 40 MB of codes 1533, 1435, 1485;  a matrix of 64 MB up and down 4790, 4590, 4540. */
+ * 1640;  100003 windows to 40 MB of codes 1533, 1435, 1485;  a matrix of 64 MB up and down 4790, 4590, 4540. Six for the large
+ * transfers alone made the first batch of four behind one slower (20000 targets on a new hasher 590 to 730 instead of
+ * 490 to 620). */
 #define FV_COPY_THREADS 4
-#define FV_COPY_THREADS_MAX 6
-#define FV_COPY_MORE_BYTES ((size_t)32 << 20)
-static inline uint32_t fv_copy_threads(uint64_t bytes) {
-  return bytes >= FV_COPY_MORE_BYTES ? FV_COPY_THREADS_MAX : FV_COPY_THREADS;
-}
 
 /* Pieces of a plain copy: whole slots and a rest. */
 static inline uint64_t fv_copy_pieces(size_t bytes) { return (bytes + FV_STAGE_SLOT_BYTES - 1) / FV_STAGE_SLOT_BYTES; }

@@ -182,6 +182,7 @@ def bench_train(steps, warmup, cpu_seconds, c=TRAIN, which="step", dense_launche
         t.step(s * c["B"], c["B"], eps)
     t.sync()
     known0, made0 = t.dense_path_counts
+    rows0 = t.row_update_steps
     # timed region: exactly `steps` steps, device idle before and after
     t0 = time.perf_counter()
     for s in range(steps):
@@ -189,6 +190,7 @@ def bench_train(steps, warmup, cpu_seconds, c=TRAIN, which="step", dense_launche
     t.sync()
     wall = time.perf_counter() - t0
     known1, made1 = t.dense_path_counts
+    rows1 = t.row_update_steps
     # the same number of steps again, timed by two HIP events on the trainer's stream
     total_ms, _ = t.time_steps((warmup + steps) * c["B"], steps, eps, per_kernel=False)
     ev_ms_per_step = total_ms / steps
@@ -273,8 +275,10 @@ def bench_train(steps, warmup, cpu_seconds, c=TRAIN, which="step", dense_launche
         out["hip_graph"] = graph
     if launches == 1:
         out["dense_launch_paths"] = {"knew_max_ds": known1 - known0, "made_the_pass": made1 - made0,
+                                     "visited_rows_as_needed": rows1 - rows0,
                                      "note": "timed steps whose single dense launch took max|ds| from the carried "
-                                             "row maxima / read the matrix for it first"}
+                                             "row maxima / read the matrix for it first; kernels.dense_update is the launch "
+                                             "over every row"}
     if cpu_seconds > 0:
         from oracle import train_oracle as to
         starts = to.window_starts(offsets, c["w"])
@@ -342,6 +346,7 @@ def bench_epoch(c=EPOCH):
     with tempfile.TemporaryDirectory() as d:
         t.save_weights(os.path.join(d, "flyvec_model_0.npy"))  # and of the checkpoint's page-locked buffer
     known0, made0 = t.dense_path_counts
+    rows0 = t.row_update_steps
     t0 = time.perf_counter()
     t.shuffle(2)
     t.sync()
@@ -355,6 +360,7 @@ def bench_epoch(c=EPOCH):
     t_ckpt = time.perf_counter() - t2
     total = time.perf_counter() - t0
     known1, made1 = t.dense_path_counts
+    rows1 = t.row_update_steps
     t.close()
     n_steps = (nwin + c["B"] - 1) // c["B"]
     model = step_byte_model(c["K"], 2 * c["V"], c["w"], c["B"])
@@ -368,7 +374,8 @@ def bench_epoch(c=EPOCH):
             "breakdown_s": {"shuffle": t_shuffle, "minibatch_loop": t_steps, "checkpoint": t_ckpt,
                             "setup_once": t_setup, "synthetic_corpus_generation": t_gen},
             "step_roofline_frac": (model * (nwin / c["B"]) / HBM_PEAK) / t_steps,
-            "dense_launch_paths": {"knew_max_ds": known1 - known0, "made_the_pass": made1 - made0}}
+            "dense_launch_paths": {"knew_max_ds": known1 - known0, "made_the_pass": made1 - made0,
+                                 "visited_rows_as_needed": rows1 - rows0}}
 
 
 def bench_reference_shaped_calls(h, W, c):

@@ -25,8 +25,8 @@
 //
 // max|ds|: no dense |ds| of neuron h exceeds |xx[h]| * (the largest |W[h][i]| when that was last known + the steps
 // since then x |eps|, what a step changes an element by at most). Where the largest |ds| of the sparse elements
-// is no less than that bound for every neuron, it is max|ds|. (The ratio of the two was measured at 0.02 to 0.29 on
-// the configurations named above.) Otherwise the launch brings every row up to date, takes the maximum over the matrix
+// is no less than that bound for every neuron, it is max|ds|. (The ratio of bound and maximum was measured at 0.02 to
+// 0.29 at the sizes named above on corpora of some millions of tokens; it grows with the corpus, as 1/f shrinks.) Otherwise the launch brings every row up to date, takes the maximum over the matrix
 // with an exchange between its blocks, and updates every row.
 #pragma once
 

@@ -48,12 +48,14 @@
 // Launches in a row that have to find the sparse elements' maximum twice the dense bound before a sequence begins: at
 // first, and at most (twice as many each time a sequence ended because one of its launches did not). A launch that cannot
 // tell max|ds| goes over the matrix twice (at K = 400 on a corpus of 10 M tokens, where the dense elements decide in
-// half of the steps, a step took 61 us so and 54 with every row updated).
+// half of the steps, a step took 61 us so and 54 with every row updated). With the rule, synapses of 1 to 40 times the usual
+// size (the bound grows with their square) at K = 400: 44.5 us up to 2.7 times, 49.6 at 2.9, 50.9 to 51.8 from 3.1 on, every row 51.9.
 #define FV_ROWS_CLEAR 3u
 #define FV_ROWS_CLEAR_MOST 1024u
 // Where visiting rows pays: at most so many window positions per row of the matrix, at least so many bytes of matrix.
 // Measured per step, every row / rows as needed (us; Zipf tokens unless "uniform"): 0.4 MB 24.3 / 23.0, 0.5 MB 22.0 / 22.4,
-// 4 MB 24.6 / 22.1, 8 MB and 0.1 positions a row 26.1 / 22.2, 9.6 MB and 7.5 positions 36.2 / 36.3, 30 positions 67.3 / 68.1,
+// 4 MB 24.6 / 22.1, 8 MB and 0.1 positions a row 26.1 / 22.2, 9.6 MB and 7.5 positions 36.2 / 36.3,
+// 16 MB and 2.75 positions 28.7 / 29.1, 30 positions 67.3 / 68.1,
 // 64 MB and 2.75 positions 52.7 / 45.0 (uniform 69.7 / 67.1), 11 positions 97.1 / 94.1, 80 MB and 0.2 positions 50.6 / 34.3,
 // 22 positions 183.3 / 178.2, 400 MB and 7.5 positions 441 / 400 (uniform 690 / 677).
 #define FV_ROWS_MOST_POSITIONS 24ull

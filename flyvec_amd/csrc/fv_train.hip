@@ -921,7 +921,7 @@ static bool fv_rows_take(fv_trainer *t, float eps, bool alone) {
   if (t->rows_mode == 2) return t->rows_behind || t->top2_valid;
   if (fabsf(eps) * FV_ROWS_DRIFT_STEPS > FV_ROWS_DRIFT) return false;
   // As the sizes say, and only where the launches so far have found the maximum of |ds| to be the sparse elements' by far
-  // (a corpus of a few million tokens; on larger ones 1/f is small and the dense elements decide).
+  // (the larger the synapses, the more often the dense elements decide).
   const uint32_t in_a_row = (uint32_t)*(volatile unsigned long long *)t->rows_verdict;
   if (t->rows_behind) {
     if (in_a_row != 0) return true;

@@ -26,7 +26,8 @@
 // max|ds|: no dense |ds| of neuron h exceeds |xx[h]| * (the largest |W[h][i]| when that was last known + the steps
 // since then x |eps|, what a step changes an element by at most). Where the largest |ds| of the sparse elements
 // is no less than that bound for every neuron, it is max|ds|. (The ratio of bound and maximum was measured at 0.02 to
-// 0.29 at the sizes named above on corpora of some millions of tokens; it grows with the corpus, as 1/f shrinks.) Otherwise the launch brings every row up to date, takes the maximum over the matrix
+// 0.29 at the sizes named above with normal synapses of the size the tests use; it grows with the square of theirs.)
+// Otherwise the launch brings every row up to date, takes the maximum over the matrix
 // with an exchange between its blocks, and updates every row.
 #pragma once
 
@@ -47,8 +48,8 @@
 #define FV_ROWS_DRIFT_STEPS 32
 // Launches in a row that have to find the sparse elements' maximum twice the dense bound before a sequence begins: at
 // first, and at most (twice as many each time a sequence ended because one of its launches did not). A launch that cannot
-// tell max|ds| goes over the matrix twice (at K = 400 on a corpus of 10 M tokens, where the dense elements decide in
-// half of the steps, a step took 61 us so and 54 with every row updated). With the rule, synapses of 1 to 40 times the usual
+// tell max|ds| goes over the matrix twice (at K = 400 on a corpus of 10 M tokens with larger synapses, where the dense elements
+// decide in half of the steps, a step took 61 us so and 54 with every row updated). With the rule, synapses of 1 to 40 times the usual
 // size (the bound grows with their square) at K = 400: 44.5 us up to 2.7 times, 49.6 at 2.9, 50.9 to 51.8 from 3.1 on, every row 51.9.
 #define FV_ROWS_CLEAR 3u
 #define FV_ROWS_CLEAR_MOST 1024u

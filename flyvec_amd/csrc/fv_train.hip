@@ -324,7 +324,6 @@ static int fv_trainer_take_giveup(fv_trainer *t, uint32_t *out_tag) {
   *t->onepass_status = 0;
   t->onepass = false;
   t->top2_valid = false;
-  t->rows_behind = false;  // that launch has left every row as the step before it did
   t->ahead_valid = false;
   FV_HIP(hipMemsetAsync(t->scalars + 1, 0, sizeof(float), t->stream));
   FV_HIP(fv_trainer_drain(t));
@@ -1474,6 +1473,7 @@ extern "C" int fv_trainer_set_dense_launches(fv_trainer *t, uint32_t launches) {
              "the streaming dense launch does not fit this device: the dense passes need separate launches");
   t->onepass = launches == 2 ? false : t->onepass_blocks != 0;
   t->onepass_stream = launches == 3 || t->onepass_unroll == 0;
+  FV_HIP(fv_trainer_settle(t));  // in front of the clearing: behind a launch that gave up no row lacks an update
   FV_HIP(hipMemsetAsync(t->scalars + 1, 0, sizeof(float), t->stream));  // "a launch has given up"
   return FV_OK;
 }

@@ -469,7 +469,8 @@ __global__ __launch_bounds__(FV_ONEPASS_THREADS) void fv_dense_rows_kernel(fv_de
 
 // Every row brought up to date to the steps before `step`, and every block's share of the rows' two largest weights
 // left as a dense launch leaves them: behind the last step of a sequence, and now and then inside one, so that the
-// bound of |W| starts afresh.
+// bound of |W| starts afresh. Behind a launch that gave up no row lacks an update (that launch has left every row as
+// the step before it did, and the steps enqueued behind it change nothing): the shares only.
 #ifndef FV_ROWS_SETTLE_DEPTH
 #define FV_ROWS_SETTLE_DEPTH 4
 #endif
@@ -480,7 +481,7 @@ __global__ __launch_bounds__(FV_ONEPASS_THREADS) void fv_rows_settle_kernel(fv_d
   float4 *x4 = dyn4;
   float2 *pairs = (float2 *)(x4 + b.list.age * a.ldk4);
   const uint32_t tid = threadIdx.x;
-  if (a.scalars[1] != 0.0f) return;  // behind a launch that gave up, which left every row as the step before it did
+  const bool dead = a.scalars[1] != 0.0f;
   const bool active = tid < a.active;
   const uint32_t q = tid % a.ldk4, r = tid / a.ldk4;
   const uint32_t rows_per_round = a.active / a.ldk4;
@@ -504,7 +505,7 @@ __global__ __launch_bounds__(FV_ONEPASS_THREADS) void fv_rows_settle_kernel(fv_d
     for (int u = 0; u < D; ++u) {
       const uint32_t row = row0 + (c + u) * row_step;
       const bool real = active && row < a.n_rows;
-      const uint32_t lacks = real ? b.list.step - max(last[u], b.list.first) : 0u;
+      const uint32_t lacks = real && !dead ? b.list.step - max(last[u], b.list.first) : 0u;
       const float4 v = fv_rows_catch_up(w[u], lacks, b.list.step, b.list.age, x4, s_kept, a.ldk4, q, a.update_cut);
       if (real) {
         if (lacks) a.Wt4[row * a.ldk4 + q] = v;

@@ -97,6 +97,57 @@ def test_the_maximum_is_not_the_sparse_elements(gpu, oracle_lib, wait, delta):
     t.close()
 
 
+@pytest.mark.parametrize("launches", [0, 1, 2])
+@pytest.mark.parametrize("drained", [False, True])
+def test_dense_launches_chosen_behind_a_launch_that_gave_up(gpu, oracle_lib, launches, drained):
+    """A launch that visits rows gives up (a limit of zero rounds), steps are enqueued behind it, more of them than steps
+    whose xx is kept, and the form of the dense launches is chosen anew before anybody has heard of it (drained: behind a
+    call that waits and does not report it, and more steps in front of the report). The matrix stays as the last step in
+    front of that launch left it, the report says so, and steps go on from there."""
+    from flyvec_amd._lib import FlyvecError
+    to = oracle_lib
+    V, K, w, B = 3000, 96, 9, 200
+    tokens, offsets = small_corpus(40000, V, seed=2)
+    starts, invf = to.window_starts(offsets, w), to.inverse_frequency(tokens, V)
+    W0 = _planted(tokens, V, K)
+    t, perm = _trainer(tokens, offsets, V, K, w, B, W0)
+    eps, live, behind = 1e-3, 10, 25
+    for s in range(live):
+        t.step(s * B, B, eps)
+    t.sync()
+    t._set_wait_limit(0)
+    for s in range(live, live + behind):
+        t.step(s * B, B, eps)
+    assert t.row_update_steps >= live + behind - 2
+    if drained:
+        t.winners(B)
+    t.set_dense_launches(launches)
+    t._set_wait_limit(1 << 14)
+
+    def six_steps(W):
+        to.train_steps(W, tokens, starts, perm, 40 * B, B, 6, w, invf, eps)
+        return W
+
+    if drained:
+        for s in range(40, 46):
+            t.step(s * B, B, eps)
+    with pytest.raises(FlyvecError, match="gave up"):
+        t.sync()
+    W = t.get_weights()
+    Wo, at = W0.copy(), None
+    for s in range(live + behind):
+        if s >= live and np.array_equal(W.view(np.uint32), (six_steps(Wo.copy()) if drained else Wo).view(np.uint32)):
+            at = s
+            break
+        to.train_steps(Wo, tokens, starts, perm, s * B, B, 1, w, invf, eps)
+    assert at is not None and at < live + behind - 17
+    if not drained:
+        for s in range(40, 46):
+            t.step(s * B, B, eps)
+        assert np.array_equal(t.get_weights().view(np.uint32), six_steps(Wo).view(np.uint32))
+    t.close()
+
+
 def test_left_alone_where_the_maximum_keeps_failing(gpu, oracle_lib):
     """Chosen by the sizes, the form is not taken, or left again, where the launches have to make the pass for max|ds|."""
     to = oracle_lib

@@ -453,20 +453,18 @@ static int fv_trainer_alloc(fv_trainer *t) {
   FV_HIP(hipMemsetAsync(t->win, 0, ((size_t)t->B + 16) * sizeof(int32_t), t->stream));
   FV_HIP(hipMalloc((void **)&t->win16, ((size_t)t->B + 64) * sizeof(uint16_t)));  // read in 16-byte pieces
   FV_HIP(hipMemsetAsync(t->win16, 0, ((size_t)t->B + 64) * sizeof(uint16_t), t->stream));
-  if (t->B > 64 * FV_SP_THREADS && t->B <= FV_GROUP_BITS_WINDOWS)
-    FV_HIP(hipFuncSetAttribute((const void *)fv_group_bits_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)FV_GROUP_BITS_LDS));
-  if (t->B <= FV_GROUP_BITS_WINDOWS) {  // steps of such a trainer are grouped from the winners' bits
+  if (t->B <= 64 * FV_SP_THREADS) {  // steps of such a trainer can be grouped inside the sparse launch
     t->won_words = 2 * ((t->B + 63) / 64);
     const size_t row_words = (size_t)t->K * t->won_words;
     FV_HIP(hipMalloc((void **)&t->won[0], 2 * row_words * sizeof(uint32_t)));
     t->won[1] = t->won[0] + row_words;
     FV_HIP(hipMemsetAsync(t->won[0], 0, 2 * row_words * sizeof(uint32_t), t->stream));
-    // A block of the sparse launch that groups for itself writes no more records than its class has columns, nor more than the step has
+    // A block of that launch writes no more records than its class has columns, nor more than the step has
     // window positions: with that much room of its own per block, no block has to count the windows of the
     // neurons before it to find its place. Left out where the regions would take more than a gigabyte.
     const uint64_t class_cols = (t->N + FV_NB_CLASSES - 1) / FV_NB_CLASSES, positions = (uint64_t)t->B * t->w;
     const uint64_t region = class_cols < positions ? class_cols : positions;
-    if (t->B <= 64 * FV_SP_THREADS && region * t->K * FV_NB_CLASSES * sizeof(fv_slot) <= FV_SLOT_REGIONS_MAX_BYTES && region + 1 < FV_SENTINEL_MAX) {
+    if (region * t->K * FV_NB_CLASSES * sizeof(fv_slot) <= FV_SLOT_REGIONS_MAX_BYTES && region + 1 < FV_SENTINEL_MAX) {
       t->slot_region = (uint32_t)region;
       FV_HIP(hipMalloc((void **)&t->slots_blocks, region * t->K * FV_NB_CLASSES * sizeof(fv_slot)));
     }
@@ -898,7 +896,7 @@ static int fv_trainer_alloc_delta(fv_trainer *t) {
 // Whether the sparse launch of a step without the anti-Hebbian term groups for itself: the trainer has the bit rows
 // (a minibatch of up to 64 windows per thread of a class block).
 static bool fv_groups_in_sparse(const fv_trainer *t) {
-  return t->won[0] && t->B <= 64 * FV_SP_THREADS && !t->separate_grouping;
+  return t->won[0] && !t->separate_grouping;
 }
 
 // Waits until the device has done `launches` of the trainer's single dense launches, or everything it was given.
@@ -1055,11 +1053,7 @@ static int fv_enqueue_step(fv_trainer *t, uint64_t first, uint32_t n, float eps,
   g.won = nullptr;
   g.won2 = nullptr;
   g.won_words = t->won_words;
-  // beyond that, up to 64 windows per thread of the grouping kernel, that one takes the bits (with the anti-Hebbian term it
-  // takes the winner arrays: the places of a neuron's two lists have to follow the neurons' order)
-  const bool bits_grouping = !grouping_in_sparse && !anti && t->won[0] && t->B > 64 * FV_SP_THREADS;
-  g.placed = bits_grouping ? (uint32_t *)(t->scalars + 8) : nullptr;
-  if (grouping_in_sparse || bits_grouping) {
+  if (grouping_in_sparse) {
     if (which == 0x3f) {
       t->won_parity ^= 1u;
       if (anti) t->won2_parity ^= 1u;
@@ -1104,13 +1098,10 @@ static int fv_enqueue_step(fv_trainer *t, uint64_t first, uint32_t n, float eps,
   gr.n = n;
   gr.scale = 1.0f;
   gr.accumulate = 0;
-  gr.won = t->won[t->won_parity];
-  gr.won_clear = t->won[t->won_parity ^ 1u];
-  gr.won_words = t->won_words;
-  gr.placed = (uint32_t *)(t->scalars + 8);
   gr.K = t->K;
   // a thread's run of the winner array should fit its 64-bit match mask
   const unsigned gr_threads = n <= 16384 ? 256 : FV_NB_MAX_THREADS;
+  const bool gr_small = n <= 64 * gr_threads && n < 65536;
   // with delta != 0 a second launch groups the windows by their second neuron and adds
   // -delta * (their scaled activations) to xx
   for (int l = 0; l < (anti ? 2 : 1); ++l) {
@@ -1124,13 +1115,14 @@ static int fv_enqueue_step(fv_trainer *t, uint64_t first, uint32_t n, float eps,
       gr.accumulate = 1;
     }
     if ((which & 2u) && !grouping_in_sparse) {
-      if (bits_grouping)
-        hipLaunchKernelGGL(fv_group_bits_kernel, dim3((t->K + FV_GROUP_NEURONS - 1) / FV_GROUP_NEURONS), dim3(256 * FV_GROUP_NEURONS),
-                           FV_GROUP_BITS_LDS, t->stream, gr);
-      else if (n <= 64 * gr_threads && n < 65536)
-        hipLaunchKernelGGL(fv_group_kernel<true>, dim3(t->K), dim3(gr_threads), 0, t->stream, gr);
+      if (gr_small && (n <= 16384 || t->K <= FV_GROUP_ONE_TO))
+        hipLaunchKernelGGL(fv_group_small_kernel<1>, dim3(t->K), dim3(gr_threads), 0, t->stream, gr);
+      else if (gr_small && t->K <= FV_GROUP_TWO_TO)
+        hipLaunchKernelGGL(fv_group_small_kernel<2>, dim3((t->K + 1) / 2), dim3(gr_threads), 0, t->stream, gr);
+      else if (gr_small)
+        hipLaunchKernelGGL(fv_group_small_kernel<4>, dim3((t->K + 3) / 4), dim3(gr_threads), 0, t->stream, gr);
       else
-        hipLaunchKernelGGL(fv_group_kernel<false>, dim3(t->K), dim3(gr_threads), 0, t->stream, gr);
+        hipLaunchKernelGGL(fv_group_kernel, dim3(t->K), dim3(gr_threads), 0, t->stream, gr);
     }
   }
   if (ev) FV_HIP(hipEventRecord(ev[2], t->stream));

@@ -16,7 +16,6 @@ struct fv_gather_args {
   uint32_t *won;        // not null: bit r of row hstar is set (atomic OR; the rows are zero before)
   uint32_t *won2;       // not null (anti-Hebbian form): the same for the window's second neuron
   uint32_t won_words;
-  uint32_t *placed;     // not null: the grouping kernel's counter, to be cleared (fv_group_args)
   float *sc;
   // anti-Hebbian form only: the second neuron of every window and its scaled activation
   int32_t *win2;
@@ -74,7 +73,7 @@ __global__ __launch_bounds__(256) void fv_gather_winner_kernel(fv_gather_args a)
   // first load of a window's ids.
   asm volatile("" ::"s"(a.Wt), "s"(a.idx), "s"(a.invf), "s"(a.win), "s"(a.win16), "s"(a.won), "s"(a.sc), "s"(a.n),
                "s"(a.K), "s"(a.ldk), "s"(a.w), "s"(a.V), "s"(a.tie_rule), "s"(a.stride), "s"(a.sampled),
-               "s"(a.n_fresh), "s"(a.won_words), "s"(a.merge_rows), "s"(a.placed));
+               "s"(a.n_fresh), "s"(a.won_words), "s"(a.merge_rows));
   if (blockIdx.x < a.merge_rows) {
     fv_merge_row_top2(a.merge, blockIdx.x);
     return;
@@ -190,7 +189,6 @@ __device__ __forceinline__ void fv_gather_one_window(const fv_gather_args &a, ui
   // the wave of the step's last window fills the 16-bit winners up to the next multiple of 64 with a
   // value no neuron has
   if (r == a.n - 1 && r + 1 + lane < ((a.n + 63) & ~63u)) a.win16[r + 1 + lane] = 0x7fffu;
-  if (r == a.n - 1 && lane == 0 && a.placed) *a.placed = 0;
   if (DELTA) {
     // flyvec/src/cuda_funcs.cu:495-548: the winner's activation becomes -9999.9999, the search repeats
     const uint32_t lost = fv_ord_key((float)-9999.9999);
@@ -205,5 +203,6 @@ __device__ __forceinline__ void fv_gather_one_window(const fv_gather_args &a, ui
       a.sc2[r] = s2;
       if (a.won2 && second < a.K) atomicOr(&a.won2[(uint64_t)second * a.won_words + (r >> 5)], 1u << (r & 31u));
     }
+    if (r == a.n - 1 && r + 1 + lane < ((a.n + 63) & ~63u)) a.win2_16[r + 1 + lane] = 0x7fffu;
   }
 }

@@ -1,6 +1,8 @@
 // Kernel 2 of the training step and the block-level helpers kernel 3 shares with it (device code of fv_train.hip).
 #pragma once
 
+#include <type_traits>
+
 #include "fv_train_state.h"
 
 // ---- kernel 2: group the windows by winner, xx ----------------------------------------------------
@@ -38,13 +40,6 @@ struct fv_group_args {
   uint32_t *group_count;
   float *xx;
   uint32_t n;
-  // fv_group_bits_kernel: the rows of the winners' bits that the winner kernel has filled, the pair of the step before last (cleared here),
-  // how many windows the blocks of
-  // this launch have placed in order[] so far, and the neurons
-  const uint32_t *won;
-  uint32_t *won_clear;
-  uint32_t won_words;
-  uint32_t *placed;
   uint32_t K;
   float scale;          // every scaled activation is multiplied by this first (1, or -delta for the second neurons)
   uint32_t accumulate;  // add the total to xx[h] instead of storing it
@@ -177,11 +172,7 @@ __device__ __forceinline__ uint32_t fv_block_scan_total(uint32_t v, uint32_t *sm
 // over the balanced binary tree on the group number (fv_wave_tree_sum, fv_block_tree_sum). A thread's run is one
 // group, or a power of two of them (its own subtree, which it adds up itself), so the thread number continues the
 // tree. The CPU checker states the same order.
-//
-// SMALL: a thread's run is one group and the minibatch has fewer than 2^16 windows. The run is then
-// fetched in one trip to memory (8 loads of 16 bytes in flight), the two counts travel through
-// one block scan as the halves of a word, and the scaled activations of a thread's first matches
-// are fetched while that scan runs.
+
 // Winner number q (0 .. 7) of a 16-byte load of 16-bit winners.
 __device__ __forceinline__ uint32_t fv_winner_of(const int4 &v, int q) {
   const uint32_t word = (uint32_t)((q >> 1) == 0 ? v.x : (q >> 1) == 1 ? v.y : (q >> 1) == 2 ? v.z : v.w);
@@ -197,87 +188,127 @@ __host__ __device__ __forceinline__ uint32_t fv_group_run_groups(uint32_t n, uin
   return m;
 }
 
-template <bool SMALL>
-__global__ __launch_bounds__(FV_NB_MAX_THREADS) void fv_group_kernel(fv_group_args a) {
-  __shared__ uint32_t red[17];
-  __shared__ float tree[16];
-
-  const uint32_t h = blockIdx.x;
-  const uint32_t tid = threadIdx.x, T = blockDim.x;
-  const uint32_t n = a.n;
-  const uint16_t *__restrict__ win = a.win;
-
-  // A thread's run is m groups of 64 windows (SMALL: one), read as 16-byte loads of 8 winners; matches among
-  // its first 64 windows are kept as a bit mask.
-  const uint32_t m_groups = SMALL ? 1u : fv_group_run_groups(n, T);
-  const uint32_t seg = 64u * m_groups;
-  const uint32_t r0 = (uint32_t)min((uint64_t)tid * seg, (uint64_t)n), r1 = (uint32_t)min((uint64_t)r0 + seg, (uint64_t)n);
-  const uint32_t n_pad = (n + 63) & ~63u;
-  uint32_t lt = 0, eq = 0;
-  uint64_t mask = 0;
-  uint32_t base, my_off, c_h;
-  constexpr int PF = 8;
-  float pf[PF];
-  if (SMALL) {
-    int4 wv4[8];
+// A run of one group per thread (up to 64 windows per thread and fewer than 2^16 in all), M neurons per block: the
+// winners are fetched in one trip to memory (8 loads of 16 bytes in flight), the counts travel through one block scan as
+// halves of words, and the scaled activations of a thread's first matches are fetched while that scan runs.
+//
+// What bounds it: every block reads the whole winner array (100 KB at 50000 windows) and looks at every winner; a thread
+// then fetches its matches eight at a time, so a neuron that wins everything takes eight such trips. Several neurons a
+// block read and look once for all of them, and cost a block the neurons' chains one behind the other. M is the least
+// with which the blocks are no more than a device's 256 compute units, as far as four. Grouping launch in us at 50000
+// windows, M = 1, 2, 4, light and with one neuron at 0.3 to 0.7 of the windows: K = 200 8.4 10.2 11.8 and 34.2 37.0 38.5;
+// K = 400 12.2 10.4 12.1 and 27.6 27.8 29.5; K = 1000 (V = 20000) 27.6 21.2 14.2 and 31.3 29.3 30.1. With runs read
+// straight by their threads (128 bytes a lane, every line asked for by eight loads) and M = 1 for all of them this launch
+// took 12.3, 18.7, 36.7 and 38.7, 34.2, 44.3. From rows of winner bits, which the winner kernel marks with an atomic a
+// window, it took 12.3 at K = 1000 but 288, 142 and 119 with the heavy neuron, and the winner kernel 1 to 5 us more (9 to
+// 20 with a heavy neuron, whose windows all mark the same words).
+#define FV_GROUP_ONE_TO 256u   // most neurons with one a block,
+#define FV_GROUP_TWO_TO 512u   // and with two
+template <int M>
+__global__ __launch_bounds__(FV_NB_MAX_THREADS) void fv_group_small_kernel(fv_group_args a) {
+  constexpr int NW = (M + 2) / 2;          // words of counts: windows of lower neurons, then of each of the M
+  constexpr int PF = M == 1 ? 8 : 4;
+  __shared__ uint32_t red[NW][16];
+  __shared__ float tree[M][16];
+  using piece_t = typename std::conditional<M == 1, uint8_t, uint32_t>::type;
+  __shared__ __attribute__((aligned(16))) piece_t bits[FV_NB_MAX_THREADS * 8];
+  const uint32_t h0 = blockIdx.x * M;
+  const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6, n_waves = blockDim.x >> 6;
+  const uint32_t n = a.n, n_pad = (n + 63) & ~63u, r0 = tid * 64;
+  // The wave's 4096 winners in eight loads of 1 KB side by side: lane l's piece of load j is the piece l mod 8 of the
+  // run of lane 8 j + l / 8, so the pieces' answers, eight windows to a byte, stand in LDS in the order of the runs.
+  uint32_t lt = 0;
+  int4 wv4[8];
 #pragma unroll
-    for (int q = 0; q < 8; ++q) wv4[q] = *(const int4 *)(win + min(r0 + 8 * q, n_pad - 8));
+  for (int j = 0; j < 8; ++j) wv4[j] = *(const int4 *)(a.win + min(wave * 4096 + 512 * j + 8 * lane, n_pad - 8));
 #pragma unroll
-    for (int q = 0; q < 64; ++q) {
-      const uint32_t wv = fv_winner_of(wv4[q >> 3], q & 7);
-      const bool in = r0 + q < r1;
-      lt += in && wv < h;
-      const bool hit = in && wv == h;
-      eq += hit;
-      mask |= (uint64_t)hit << q;
+  for (int j = 0; j < 8; ++j) {
+    // (the winners behind the last window, up to a whole group, are a value no neuron has)
+    const bool in = wave * 4096 + 512 * j + 8 * lane < n;
+    uint32_t bytes = 0;  // byte m: neuron m's windows of the piece
+#pragma unroll
+    for (int q = 0; q < 8; ++q) {
+      const uint32_t d = (in ? fv_winner_of(wv4[j], q) : 0xffffu) - h0;
+      lt += d >> 31;
+      bytes |= d < (uint32_t)M ? (1u << q) << (8 * d) : 0u;
     }
-    uint64_t mm = mask;
+    bits[wave * 512 + 64 * j + lane] = (piece_t)bytes;
+  }
+  fv_lds_barrier();
+  uint64_t mask[M];
+  if (M == 1) {
+    mask[0] = *(const uint64_t *)&bits[tid * 8];
+  } else {
+    uint32_t piece[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) piece[i] = bits[tid * 8 + i];
+#pragma unroll
+    for (int m = 0; m < M; ++m) {
+      uint32_t word2[2];
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        // byte m of four pieces, side by side
+        const uint32_t a01 = __builtin_amdgcn_perm(piece[4 * i + 1], piece[4 * i], 0x0c0c0400u + 0x0101u * m);
+        const uint32_t a23 = __builtin_amdgcn_perm(piece[4 * i + 3], piece[4 * i + 2], 0x0c0c0400u + 0x0101u * m);
+        word2[i] = a01 | (a23 << 16);
+      }
+      mask[m] = (uint64_t)word2[0] | ((uint64_t)word2[1] << 32);
+    }
+  }
+  uint32_t word[NW], half[2 * NW];
+  float pf[M][PF];
+#pragma unroll
+  for (int i = 0; i < 2 * NW; ++i) half[i] = 0;
+  half[0] = lt;
+#pragma unroll
+  for (int m = 0; m < M; ++m) {
+    half[1 + m] = (uint32_t)__popcll(mask[m]);
+    uint64_t mm = mask[m];
 #pragma unroll
     for (int q = 0; q < PF; ++q) {
-      const uint32_t r = mm ? r0 + (uint32_t)__ffsll((long long)mm) - 1 : r0;
-      pf[q] = __fmul_rn(a.scale, a.sc[min(r, n - 1)]);
+      const uint32_t r = mm ? r0 + (uint32_t)__ffsll((long long)mm) - 1 : 0u;  // (one address for all that have none)
+      pf[m][q] = __fmul_rn(a.scale, a.sc[r]);
       mm &= mm - 1;
     }
-    uint32_t total;
-    const uint32_t before = fv_block_scan_total(lt | (eq << 16), red, &total);
-    base = total & 0xffffu;
-    c_h = total >> 16;
-    my_off = before >> 16;
-  } else {
-    for (uint32_t rb = r0; rb < r1; rb += FV_NB_LOADS) {
-      int4 wv4[FV_NB_LOADS / 8];
+  }
 #pragma unroll
-      for (int q = 0; q < FV_NB_LOADS / 8; ++q) wv4[q] = *(const int4 *)(win + min(rb + 8 * q, n_pad - 8));
+  for (int i = 0; i < NW; ++i) {
+    word[i] = half[2 * i] | (half[2 * i + 1] << 16);
+    const uint32_t incl = fv_wave_inclusive_scan_u32(word[i]);
+    if (lane == 63u) red[i][wave] = incl;
+    word[i] = incl - word[i];
+  }
+  __syncthreads();
+  uint32_t all[NW];
 #pragma unroll
-      for (int q = 0; q < FV_NB_LOADS; ++q) {
-        const uint32_t wv = fv_winner_of(wv4[q >> 3], q & 7);
-        const bool in = rb + q < r1;
-        lt += in && wv < h;
-        const bool hit = in && wv == h;
-        eq += hit;
-        const uint32_t o = rb + q - r0;
-        mask |= o < 64 ? (uint64_t)hit << o : 0ull;
-      }
+  for (int i = 0; i < NW; ++i) {
+    all[i] = 0;
+    for (uint32_t v = 0; v < n_waves; ++v) {
+      const uint32_t t = red[i][v];
+      word[i] += v < wave ? t : 0u;
+      all[i] += t;
     }
-    base = fv_block_sum_u32(lt, red);  // windows won by lower neurons
-    my_off = fv_block_exclusive_scan(eq, red);
-    c_h = fv_block_sum_u32(eq, red);
   }
-  if (tid == 0) {
-    a.group_base[h] = base;
-    a.group_count[h] = c_h;
-  }
-  // the neuron's windows, ascending, into order[]; the thread's own part of xx beside it
-  uint32_t *order = a.order + base;
-  float part = 0.0f;
-  if (SMALL) {
-    uint32_t rank = my_off;
-    uint64_t mm = mask;
+  const auto of = [](const uint32_t *w, int i) { return (i & 1) ? w[i >> 1] >> 16 : w[i >> 1] & 0xffffu; };
+  uint32_t base = of(all, 0);
+#pragma unroll
+  for (int m = 0; m < M; ++m) {
+    const uint32_t c_h = of(all, 1 + m);
+    if (tid == 0 && h0 + m < a.K) {
+      a.group_base[h0 + m] = base;
+      a.group_count[h0 + m] = c_h;
+    }
+    // the neuron's windows, ascending, into order[]; the thread's own part of xx beside it
+    uint32_t *order = a.order + base;
+    base += c_h;
+    float part = 0.0f;
+    uint32_t rank = of(word, 1 + m);
+    uint64_t mm = mask[m];
 #pragma unroll
     for (int q = 0; q < PF; ++q) {
       if (mm) {
         order[rank++] = r0 + (uint32_t)__ffsll((long long)mm) - 1;
-        part = __fadd_rn(part, pf[q]);
+        part = __fadd_rn(part, pf[m][q]);
         mm &= mm - 1;
       }
     }
@@ -288,9 +319,9 @@ __global__ __launch_bounds__(FV_NB_MAX_THREADS) void fv_group_kernel(fv_group_ar
       uint64_t m2 = mm;
 #pragma unroll
       for (int q = 0; q < 8; ++q) {
-        r[q] = m2 ? r0 + (uint32_t)__ffsll((long long)m2) - 1 : r0;
+        r[q] = m2 ? r0 + (uint32_t)__ffsll((long long)m2) - 1 : 0u;
         m2 &= m2 - 1;
-        v[q] = __fmul_rn(a.scale, a.sc[min(r[q], n - 1)]);
+        v[q] = __fmul_rn(a.scale, a.sc[r[q]]);
       }
 #pragma unroll
       for (int q = 0; q < 8; ++q) {
@@ -301,151 +332,118 @@ __global__ __launch_bounds__(FV_NB_MAX_THREADS) void fv_group_kernel(fv_group_ar
         }
       }
     }
-  } else {
-    // the matches of the thread's first 64 windows are in the mask, the others are found again in the winner array
-    uint32_t rank = my_off;
-    for (uint64_t mm = mask; mm; mm &= mm - 1) order[rank++] = r0 + (uint32_t)__ffsll((long long)mm) - 1;
-    for (uint32_t r = r0 + 64; r < r1; ++r)
-      if ((uint32_t)win[r] == h) order[rank++] = r;
-    // the thread's groups one after the other; their sums meet on a stack that is the thread's subtree: a finished
-    // node of level k waits in stack[k] for its right sibling (static indices: the stack stays in registers)
-    float stack[16];  // n < 2^30 windows and 1024 threads: at most 2^14 groups per thread
-#pragma unroll
-    for (int k = 0; k < 16; ++k) stack[k] = 0.0f;
-    uint32_t j = my_off;  // next match of the thread, by rank (its own writes to order[] above)
-    const uint32_t j_end = my_off + eq;
-    for (uint32_t g = 0; g < m_groups; ++g) {
-      const uint32_t g_end = r0 + 64u * (g + 1);
-      float p_g = 0.0f;
-      while (j < j_end) {  // up to four values of the group fetched together
-        uint32_t r[4];
-        float v[4];
-#pragma unroll
-        for (int q = 0; q < 4; ++q) r[q] = order[min(j + q, j_end - 1)];
-#pragma unroll
-        for (int q = 0; q < 4; ++q) v[q] = __fmul_rn(a.scale, a.sc[r[q]]);
-        uint32_t took = 0;
-#pragma unroll
-        for (int q = 0; q < 4; ++q)
-          if (took == (uint32_t)q && j + q < j_end && r[q] < g_end) {
-            p_g = __fadd_rn(p_g, v[q]);
-            ++took;
-          }
-        j += took;
-        if (took < 4) break;
-      }
-      float carry = p_g;
-      bool placed = false;
-      uint32_t i = g;
-#pragma unroll
-      for (int k = 0; k < 16; ++k) {
-        if (!placed) {
-          if (i & 1u) {
-            carry = __fadd_rn(stack[k], carry);
-          } else {
-            stack[k] = carry;
-            placed = true;
-          }
-        }
-        i >>= 1;
-      }
-    }
-    // m_groups = 2^k: the last group's carry ended in stack[k], the root of the thread's subtree
-#pragma unroll
-    for (int k = 0; k < 16; ++k)
-      if (m_groups == (1u << k)) part = stack[k];
+    const float ws = fv_wave_tree_sum(part);
+    if (lane == 0) tree[m][wave] = ws;
   }
+  fv_lds_barrier();
+  if (tid < M && h0 + tid < a.K) {
+    float t[16];
+#pragma unroll
+    for (uint32_t i = 0; i < 16; ++i) t[i] = i < n_waves ? tree[tid][i] : 0.0f;
+#pragma unroll
+    for (uint32_t stride = 1; stride < 16; stride <<= 1)
+#pragma unroll
+      for (uint32_t i = 0; i < 16; i += 2 * stride) t[i] = __fadd_rn(t[i], t[i + stride]);
+    a.xx[h0 + tid] = a.accumulate ? __fadd_rn(a.xx[h0 + tid], t[0]) : t[0];
+  }
+}
+
+// The same for any number of windows, a neuron per block.
+__global__ __launch_bounds__(FV_NB_MAX_THREADS) void fv_group_kernel(fv_group_args a) {
+  __shared__ uint32_t red[17];
+  __shared__ float tree[16];
+
+  const uint32_t h = blockIdx.x;
+  const uint32_t tid = threadIdx.x, T = blockDim.x;
+  const uint32_t n = a.n;
+  const uint16_t *__restrict__ win = a.win;
+
+  // A thread's run is m groups of 64 windows, read as 16-byte loads of 8 winners; matches among
+  // its first 64 windows are kept as a bit mask.
+  const uint32_t m_groups = fv_group_run_groups(n, T);
+  const uint32_t seg = 64u * m_groups;
+  const uint32_t r0 = (uint32_t)min((uint64_t)tid * seg, (uint64_t)n), r1 = (uint32_t)min((uint64_t)r0 + seg, (uint64_t)n);
+  const uint32_t n_pad = (n + 63) & ~63u;
+  uint32_t lt = 0, eq = 0;
+  uint64_t mask = 0;
+  uint32_t base, my_off, c_h;
+  for (uint32_t rb = r0; rb < r1; rb += FV_NB_LOADS) {
+    int4 wv4[FV_NB_LOADS / 8];
+#pragma unroll
+    for (int q = 0; q < FV_NB_LOADS / 8; ++q) wv4[q] = *(const int4 *)(win + min(rb + 8 * q, n_pad - 8));
+#pragma unroll
+    for (int q = 0; q < FV_NB_LOADS; ++q) {
+      const uint32_t wv = fv_winner_of(wv4[q >> 3], q & 7);
+      const bool in = rb + q < r1;
+      lt += in && wv < h;
+      const bool hit = in && wv == h;
+      eq += hit;
+      const uint32_t o = rb + q - r0;
+      mask |= o < 64 ? (uint64_t)hit << o : 0ull;
+    }
+  }
+  base = fv_block_sum_u32(lt, red);  // windows won by lower neurons
+  my_off = fv_block_exclusive_scan(eq, red);
+  c_h = fv_block_sum_u32(eq, red);
+  if (tid == 0) {
+    a.group_base[h] = base;
+    a.group_count[h] = c_h;
+  }
+  // the neuron's windows, ascending, into order[]; the thread's own part of xx beside it
+  uint32_t *order = a.order + base;
+  float part = 0.0f;
+  // the matches of the thread's first 64 windows are in the mask, the others are found again in the winner array
+  uint32_t rank = my_off;
+  for (uint64_t mm = mask; mm; mm &= mm - 1) order[rank++] = r0 + (uint32_t)__ffsll((long long)mm) - 1;
+  for (uint32_t r = r0 + 64; r < r1; ++r)
+    if ((uint32_t)win[r] == h) order[rank++] = r;
+  // the thread's groups one after the other; their sums meet on a stack that is the thread's subtree: a finished
+  // node of level k waits in stack[k] for its right sibling (static indices: the stack stays in registers)
+  float stack[16];  // n < 2^30 windows and 1024 threads: at most 2^14 groups per thread
+#pragma unroll
+  for (int k = 0; k < 16; ++k) stack[k] = 0.0f;
+  uint32_t j = my_off;  // next match of the thread, by rank (its own writes to order[] above)
+  const uint32_t j_end = my_off + eq;
+  for (uint32_t g = 0; g < m_groups; ++g) {
+    const uint32_t g_end = r0 + 64u * (g + 1);
+    float p_g = 0.0f;
+    while (j < j_end) {  // up to four values of the group fetched together
+      uint32_t r[4];
+      float v[4];
+#pragma unroll
+      for (int q = 0; q < 4; ++q) r[q] = order[min(j + q, j_end - 1)];
+#pragma unroll
+      for (int q = 0; q < 4; ++q) v[q] = __fmul_rn(a.scale, a.sc[r[q]]);
+      uint32_t took = 0;
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+        if (took == (uint32_t)q && j + q < j_end && r[q] < g_end) {
+          p_g = __fadd_rn(p_g, v[q]);
+          ++took;
+        }
+      j += took;
+      if (took < 4) break;
+    }
+    float carry = p_g;
+    bool placed = false;
+    uint32_t i = g;
+#pragma unroll
+    for (int k = 0; k < 16; ++k) {
+      if (!placed) {
+        if (i & 1u) {
+          carry = __fadd_rn(stack[k], carry);
+        } else {
+          stack[k] = carry;
+          placed = true;
+        }
+      }
+      i >>= 1;
+    }
+  }
+  // m_groups = 2^k: the last group's carry ended in stack[k], the root of the thread's subtree
+#pragma unroll
+  for (int k = 0; k < 16; ++k)
+    if (m_groups == (1u << k)) part = stack[k];
   const float xx = fv_block_tree_sum(part, tree);
   if (tid == 0) a.xx[h] = a.accumulate ? __fadd_rn(a.xx[h], xx) : xx;
 }
-
-// The same from the neurons' rows of winner bits: 6 KB a neuron at 50000 windows, where every one of the K blocks above
-// reads the 100 KB of the winner array. 256 threads per neuron, four neurons per block. A thread takes FV_GROUP_RUN groups
-// of 64 windows, its subtree of the order of the totals xx. The windows' ids meet in LDS by rank, and from there the
-// activations are fetched (and order[] written) by all of the neuron's threads alike: a thread that fetched its
-// own matches' was one of the heaviest neuron's, batch behind batch. The number of windows that lower neurons won does not
-// come with the row: the block takes the next free place in order[] for its neurons. That changes where window ids and
-// slot records lie and no result. (One atomic per neuron on the one counter was most of the launch.)
-// K = 1000, V = 50000, B = 50000: 29.3 us from the winner array; a thread with its own matches 19.2, by rank 17.3, and
-// four neurons a block 10.8 (and the winner kernel, which marks the bits, 204.0 instead of 202.4).
-#define FV_GROUP_RUN 4
-#define FV_GROUP_NEURONS 4
-#define FV_GROUP_BITS_WINDOWS (64u * FV_GROUP_RUN * 256u)  // most windows of a step
-#define FV_GROUP_STAGE 3072  // windows of a neuron in LDS at a time
-__global__ __launch_bounds__(256 * FV_GROUP_NEURONS) void fv_group_bits_kernel(fv_group_args a) {
-  constexpr int R = FV_GROUP_RUN, M = FV_GROUP_NEURONS;
-  extern __shared__ uint32_t dyn[];  // ids and values of every neuron
-  __shared__ uint32_t wave_count[4 * M], sh_base;
-  __shared__ float wave_sum[4 * M];
-  const uint32_t tid = threadIdx.x & 255u, sub = __builtin_amdgcn_readfirstlane(threadIdx.x >> 8), wave = threadIdx.x >> 6;
-  const uint32_t h = blockIdx.x * M + sub;
-  const bool real = h < a.K;
-  uint32_t *ids = dyn + sub * 2 * FV_GROUP_STAGE;
-  float *val = (float *)(ids + FV_GROUP_STAGE);
-  uint64_t mask[R], left[R];
-  uint32_t eq = 0;
-#pragma unroll
-  for (int g = 0; g < R; ++g) {
-    const uint32_t word = 2 * (R * tid + g);
-    uint2 mw = make_uint2(0u, 0u);
-    if (real && word < a.won_words) {
-      mw = *(const uint2 *)(a.won + (uint64_t)h * a.won_words + word);
-      *(uint2 *)(a.won_clear + (uint64_t)h * a.won_words + word) = make_uint2(0u, 0u);
-    }
-    left[g] = mask[g] = (uint64_t)mw.x | ((uint64_t)mw.y << 32);
-    eq += (uint32_t)__popcll(mask[g]);
-  }
-  const uint32_t incl = fv_wave_inclusive_scan_u32(eq);
-  if ((threadIdx.x & 63u) == 63u) wave_count[wave] = incl;
-  fv_lds_barrier();
-  uint32_t my_off = incl - eq, c_h = 0, before = 0, all = 0, most = 0;
-#pragma unroll
-  for (uint32_t m = 0; m < M; ++m) {
-    uint32_t c = 0;
-#pragma unroll
-    for (uint32_t i = 0; i < 4; ++i) {
-      if (m == sub && m * 4 + i < wave) my_off += wave_count[m * 4 + i];
-      c += wave_count[m * 4 + i];
-    }
-    if (m < sub) before += c;
-    if (m == sub) c_h = c;
-    all += c;
-    most = max(most, c);
-  }
-  // (no more than n windows in all: the bound is for a launch repeated by itself)
-  if (threadIdx.x == 0) sh_base = all ? min(atomicAdd(a.placed, all), a.n - all) : 0u;
-  float part[R];
-#pragma unroll
-  for (int g = 0; g < R; ++g) part[g] = 0.0f;
-  uint32_t put = my_off, add = my_off;  // rank of the thread's next match to be staged, to be added
-  for (uint32_t j0 = 0; j0 < most; j0 += FV_GROUP_STAGE) {
-    const uint32_t j1 = min(c_h, j0 + FV_GROUP_STAGE);
-#pragma unroll
-    for (int g = 0; g < R; ++g)
-      for (; mask[g] && put < j1; mask[g] &= mask[g] - 1)
-        ids[put++ - j0] = 64 * (R * tid + g) + (uint32_t)__ffsll((long long)mask[g]) - 1;
-    __syncthreads();
-    uint32_t *order = a.order + sh_base + before;
-    for (uint32_t j = j0 + tid; j < j1; j += 256) {
-      const uint32_t r = ids[j - j0];
-      order[j] = r;
-      val[j - j0] = a.sc[r];
-    }
-    __syncthreads();
-#pragma unroll
-    for (int g = 0; g < R; ++g)
-      for (; left[g] && add < j1; left[g] &= left[g] - 1) part[g] = __fadd_rn(part[g], val[add++ - j0]);
-    fv_lds_barrier();
-  }
-  static_assert(R == 4, "a thread's subtree");
-  const float ws = fv_wave_tree_sum(__fadd_rn(__fadd_rn(part[0], part[1]), __fadd_rn(part[2], part[3])));
-  if ((threadIdx.x & 63u) == 0) wave_sum[wave] = ws;
-  __syncthreads();
-  if (tid == 0 && real) {
-    const float *t = wave_sum + sub * 4;
-    a.group_base[h] = sh_base + before;
-    a.group_count[h] = c_h;
-    a.xx[h] = __fadd_rn(__fadd_rn(t[0], t[1]), __fadd_rn(t[2], t[3]));
-  }
-}
-#define FV_GROUP_BITS_LDS (2 * FV_GROUP_STAGE * FV_GROUP_NEURONS * sizeof(uint32_t))

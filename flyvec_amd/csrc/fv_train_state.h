@@ -162,6 +162,6 @@ struct fv_trainer {
   bool ahead_marked;        // idx_ahead and idx_ahead2 hold the next two minibatches, and row_need knows them
   uint32_t to_come;         // steps the caller is going to enqueue behind the present one without looking at the matrix
   bool capturing;           // steps are being captured into a graph
-  uint32_t in_a_row;        // steps enqueued since somebody waited for the stream
+  uint32_t in_a_row;        // steps enqueued since somebody waited for the stream, each on the windows behind the last one's
   float *xx_last;           // xx of the last step
 };

@@ -166,6 +166,37 @@ def test_left_alone_where_the_maximum_keeps_failing(gpu, oracle_lib):
     t.close()
 
 
+@pytest.mark.parametrize("order", ["short", "strided", "again", "six and a jump", "twelve and a jump"])
+def test_steps_that_do_not_follow_each_other(gpu, oracle_lib, order):
+    """Steps on windows that are not the ones behind the last step's: a sequence per step would settle the whole matrix
+    every time, so by the sizes the form is not taken; from eight steps in order on it is."""
+    from flyvec_amd import synthetic
+    to = oracle_lib
+    V, K, w, B, n_steps, eps = 12000, 210, 5, 200, 60, 2e-4
+    tokens, offsets = small_corpus(60000, V, seed=2)
+    starts, invf = to.window_starts(offsets, w), to.inverse_frequency(tokens, V)
+    W0 = synthetic.synapses(K, V, seed=3, sigma=0.02)
+    t, perm = _trainer(tokens, offsets, V, K, w, B, W0, mode=0)
+    N = len(starts) // B
+    run = {"six and a jump": 6, "twelve and a jump": 12}.get(order, 1)
+    at = [(s % N if order == "short" else 3 * s % N if order == "strided" else 4 if order == "again" else
+           (s // run * 31 + s % run) % (N - 1)) * B for s in range(n_steps)]
+    n = B - 7 if order == "short" else B
+    Wo = W0.copy()
+    for s in range(12):
+        t.step(s * B, B, eps)
+        to.train_steps(Wo, tokens, starts, perm, s * B, B, 1, w, invf, eps)
+    t.sync()
+    before = t.row_update_steps
+    for first in at:
+        t.step(first, n, eps)
+        to.train_step(Wo, to.inflate(tokens, starts, perm, first, n, w, V), invf, eps)
+    taken = t.row_update_steps - before
+    assert np.array_equal(t.get_weights().view(np.uint32), Wo.view(np.uint32))
+    assert taken >= n_steps - 12 if run == 12 else taken == 0
+    t.close()
+
+
 @pytest.mark.parametrize("entries", [1, 3])
 def test_more_sentinels_than_a_wave_notes(gpu, oracle_lib, entries):
     from flyvec_amd import synthetic

@@ -202,9 +202,12 @@ static int fv_trainer_reserve_windows(fv_trainer *t, uint64_t n_windows) {
   return FV_OK;
 }
 
+// Single dense launches whose answer has been heard (of those counted in `verdicts`).
+static uint32_t fv_rows_heard(const fv_trainer *t) { return (uint32_t)(*(volatile unsigned long long *)t->rows_verdict >> 32); }
+
 // The matrix or the corpus is another: what the launches have said so far says nothing of it.
 static void fv_rows_forget_verdicts(fv_trainer *t) {
-  t->verdicts = t->verdicts_base = (uint32_t)(*(volatile unsigned long long *)t->rows_verdict >> 32);
+  t->verdicts = t->verdicts_base = fv_rows_heard(t);
   t->verdicts_asked = false;
   t->rows_clear = FV_ROWS_CLEAR;
 }
@@ -311,6 +314,7 @@ static hipError_t fv_trainer_drain(fv_trainer *t) {
   hipError_t e = fv_trainer_settle(t);
   if (e == hipSuccess) e = hipStreamSynchronize(t->stream);
   if (e == hipSuccess) fv_trainer_leaves_flight(t);
+  if (e == hipSuccess && t->rows_verdict) t->verdicts = fv_rows_heard(t);  // (launches that were counted and never made)
   t->in_a_row = 0;
   return e;
 }
@@ -901,7 +905,7 @@ static bool fv_groups_in_sparse(const fv_trainer *t) {
 
 // Waits until the device has done `launches` of the trainer's single dense launches, or everything it was given.
 static void fv_rows_wait_for(fv_trainer *t, uint32_t launches) {
-  while ((int32_t)((uint32_t)(*(volatile unsigned long long *)t->rows_verdict >> 32) - launches) < 0) {
+  while ((int32_t)(fv_rows_heard(t) - launches) < 0) {
     if (hipStreamQuery(t->stream) != hipErrorNotReady) break;
     std::this_thread::yield();
   }
@@ -924,13 +928,18 @@ static bool fv_rows_take(fv_trainer *t, float eps, bool alone, bool follows) {
   // (the larger the synapses, the more often the dense elements decide).
   const uint32_t clear = (uint32_t)*(volatile unsigned long long *)t->rows_verdict;
   const bool sequence = t->to_come + t->in_a_row >= FV_ROWS_SEQUENCE;
+  // A call that waits for its steps itself keeps the host near the device (fv_enqueue_step); steps that are only enqueued
+  // wait for nothing: no more of them go unheard than have been found clear in a row before (what an unclear one among them
+  // costs is no more than those have gained).
+  const uint32_t unheard = t->verdicts - fv_rows_heard(t), most_unheard = clear > 2 * FV_ROWS_REFRESH ? clear : 2 * FV_ROWS_REFRESH;
+  if (!t->caller_waits && unheard > most_unheard) return false;
   if (t->rows_behind) {
     if (clear != 0) return follows || sequence;
     if (t->rows_clear < FV_ROWS_CLEAR_MOST) t->rows_clear *= 2;
     return false;
   }
   if (!t->top2_valid || !sequence) return false;
-  if (!t->verdicts_asked && t->to_come >= FV_ROWS_SEQUENCE && t->verdicts - t->verdicts_base >= FV_ROWS_CLEAR + 2) {
+  if (!t->verdicts_asked && t->caller_waits && t->to_come >= FV_ROWS_SEQUENCE && t->verdicts - t->verdicts_base >= FV_ROWS_CLEAR + 2) {
     // the first steps of an epoch on a new matrix: their answers are worth a short wait, the device has a step left to do
     fv_rows_wait_for(t, t->verdicts - 1);
     t->verdicts_asked = true;
@@ -964,7 +973,7 @@ static int fv_enqueue_step(fv_trainer *t, uint64_t first, uint32_t n, float eps,
   const bool rows_go_on = rows && sampled_ahead && t->ahead_marked;
   const bool refresh = t->rows_since >= FV_ROWS_REFRESH || (t->rows_mode == 0 && t->rows_drift >= FV_ROWS_DRIFT);
   if (whole && t->rows_behind && (!rows || !rows_go_on || refresh)) FV_HIP(fv_trainer_settle(t));
-  if (rows && refresh) {
+  if (rows && refresh && t->caller_waits) {
     // no further ahead of the device than to the refresh before the last: what its launches find has to be heard of
     fv_rows_wait_for(t, t->rows_mark_before);
     t->rows_mark_before = t->rows_mark;
@@ -1422,6 +1431,7 @@ extern "C" int fv_trainer_run_epoch(fv_trainer *t, uint64_t epoch_id, uint64_t n
       t->step_tag = (uint32_t)(k / t->B) + 1u;
       const uint64_t behind = (t->n_windows - k - n + t->B - 1) / t->B;
       t->to_come = behind < FV_ROWS_SEQUENCE ? (uint32_t)behind : FV_ROWS_SEQUENCE;
+      t->caller_waits = true;
       if (n < t->B && k > 0 && t->stale_tail)
         // flyvec/src/cuda_funcs.cu:1679 against :1700-1732: only the sampler sees the remainder, the other
         // kernels run on all Num rows, those behind the remainder being the previous minibatch's
@@ -1431,6 +1441,7 @@ extern "C" int fv_trainer_run_epoch(fv_trainer *t, uint64_t epoch_id, uint64_t n
     }
     t->step_tag = 0;
     t->to_come = 0;
+    t->caller_waits = false;
     FV_TRY(rc);
     FV_HIP(fv_trainer_drain(t));
     uint32_t tag = 0;
@@ -1617,9 +1628,11 @@ extern "C" int fv_trainer_time_steps(fv_trainer *t, uint64_t first_window, uint3
   FV_HIP(hipEventRecord(e0, t->stream));
   for (uint32_t s = 0; s < n_steps && rc == FV_OK; ++s) {
     t->to_come = n_steps - 1 - s;
+    t->caller_waits = true;
     rc = fv_enqueue_step(t, first_window + (uint64_t)s * t->B, t->B, eps, 0.0f, nullptr);
   }
   t->to_come = 0;
+  t->caller_waits = false;
   FV_HIP(fv_trainer_settle(t));  // (part of what the steps take)
   FV_HIP(hipEventRecord(e1, t->stream));
   FV_HIP(fv_trainer_drain(t));

@@ -161,6 +161,7 @@ struct fv_trainer {
   int32_t *idx_ahead2;      // the minibatch after the next, sampled by such a step (room for it in the same allocation)
   bool ahead_marked;        // idx_ahead and idx_ahead2 hold the next two minibatches, and row_need knows them
   uint32_t to_come;         // steps the caller is going to enqueue behind the present one without looking at the matrix
+  bool caller_waits;        // and waits for them before it returns
   bool capturing;           // steps are being captured into a graph
   uint32_t in_a_row;        // steps enqueued since somebody waited for the stream, each on the windows behind the last one's
   float *xx_last;           // xx of the last step

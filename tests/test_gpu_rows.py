@@ -197,6 +197,30 @@ def test_steps_that_do_not_follow_each_other(gpu, oracle_lib, order):
     t.close()
 
 
+@pytest.mark.parametrize("mode", [0, 2])
+def test_steps_are_enqueued_without_waiting_for_the_device(gpu, mode):
+    """2000 steps of 20 to 40 us: the host is done with them long before the device is (8 to 10 us a step)."""
+    import time
+    from flyvec_amd import synthetic
+    V, K, w, B, n_steps = 20000, 400, 5, 2000, 2000
+    tokens, offsets = small_corpus(400000, V, seed=2)
+    t, _ = _trainer(tokens, offsets, V, K, w, B, synthetic.synapses(K, V, seed=3, sigma=0.02), mode=mode)
+    N = t.num_windows // B
+    t.step(0, B, 2e-4)
+    t.sync()
+    before, ratios = t.row_update_steps, []
+    for _ in range(3):
+        t0 = time.perf_counter()
+        for s in range(n_steps):
+            t.step(s % N * B, B, 2e-4)
+        t1 = time.perf_counter()
+        t.sync()
+        ratios.append((t1 - t0) / (time.perf_counter() - t0))
+    assert t.row_update_steps - before > n_steps / 4
+    assert min(ratios) < 0.7, ratios
+    t.close()
+
+
 @pytest.mark.parametrize("entries", [1, 3])
 def test_more_sentinels_than_a_wave_notes(gpu, oracle_lib, entries):
     from flyvec_amd import synthetic

@@ -381,7 +381,7 @@ extern "C" int fv_trainer_destroy(fv_trainer *t) {
 
 // Whether the dense launch of a step should visit only the rows somebody needs, going by the sizes.
 static bool fv_rows_worth_it(const fv_trainer *t) {
-  return t->rows_ok && t->ldk >= FV_ROWS_LEAST_LDK && (uint64_t)t->B * t->w <= FV_ROWS_MOST_POSITIONS * t->N && (uint64_t)t->total4 * 16 >= FV_ROWS_LEAST_BYTES;
+  return t->rows_ok && fv_rows_pay(t->N, t->ldk, (uint64_t)t->B * t->w);
 }
 
 // Entries of an index matrix: a row per window of a minibatch, and the padding behind them.
@@ -935,7 +935,7 @@ static bool fv_rows_take(fv_trainer *t, float eps, bool alone, bool follows) {
   if (!t->caller_waits && unheard > most_unheard) return false;
   if (t->rows_behind) {
     if (clear != 0) return follows || sequence;
-    if (t->rows_clear < FV_ROWS_CLEAR_MOST) t->rows_clear *= 2;
+    t->rows_clear = fv_rows_clear_after(t->rows_clear);
     return false;
   }
   if (!t->top2_valid || !sequence) return false;

@@ -3,15 +3,15 @@
 // Row i of the token-major matrix is read by a step only if token i stands in one of its windows. The dense update
 // of any other row (W += s * (-xx[h] * W), element by element) can wait: applied later, one step's update after
 // the other, the same fp32 operations run in the same order on the same values, so the matrix comes out the
-// same bit for bit. What has to be kept of a step is xx (ldk floats) and s, for FV_ROWS_AGE steps. A dense
+// same bit for bit. What has to be kept of a step is xx (ldk floats) and s, for 16 steps, or 8 of the widest rows (fv_rows_age). A dense
 // launch then visits
 //   - the rows its own step has touched (they hold the sentinels of its sparse elements),
 //   - the rows the next step reads,
-//   - the rows that lack FV_ROWS_AGE steps' updates,
+//   - the rows that lack as many steps' updates as are kept,
 // and brings them all up to date; the others it neither reads nor writes. At K = 400, V = 20000, w = 11, B = 10000 and
 // Zipf-distributed tokens that is half the rows, at K = 1000, V = 50000, w = 15, B = 50000 0.69 of them.
 // Measured, every row against rows as needed: the dense launch 21.7 and 17.2 us, 148 and 112; a step of an epoch 52.7 and
-// 45.0, 441 and 400; 27.7 and 26.5 at K = 209, V = 7919, w = 7, B = 3001 (FV_ROWS_MOST_POSITIONS has more).
+// 45.0, 441 and 400; 27.7 and 26.5 at K = 209, V = 7919, w = 7, B = 3001 (fv_rows_pay has more).
 //
 // What bounds the launch at K = 400 (clock from its first wave; 17.2 us in the trace): arguments, then the list, then the
 // first groups of W, one trip behind the other (4.1 us until the block's barrier), 3.7 us for the rows that lack one
@@ -31,6 +31,7 @@
 // with an exchange between its blocks, and updates every row.
 #pragma once
 
+#include "fv_rows_plan.h"
 #include "fv_train_dense.h"
 #include "fv_train_row_list.h"
 
@@ -46,24 +47,6 @@
 #define FV_ROWS_REFRESH 128u
 #define FV_ROWS_DRIFT 0.02  // or when |W| may have grown by this much, which takes at least FV_ROWS_DRIFT_STEPS steps
 #define FV_ROWS_DRIFT_STEPS 32
-// Launches in a row that have to find the sparse elements' maximum twice the dense bound before a sequence begins: at
-// first, and at most (twice as many each time a sequence ended because one of its launches did not). A launch that cannot
-// tell max|ds| goes over the matrix twice (at K = 400 on a corpus of 10 M tokens with larger synapses, where the dense elements
-// decide in half of the steps, a step took 61 us so and 54 with every row updated). With the rule, synapses of 1 to 40 times the usual
-// size (the bound grows with their square) at K = 400: 44.5 us up to 2.7 times, 49.6 at 2.9, 50.9 to 51.8 from 3.1 on, every row 51.9.
-#define FV_ROWS_CLEAR 3u
-#define FV_ROWS_CLEAR_MOST 1024u
-// Where visiting rows pays: at most so many window positions per row of the matrix, at least so many bytes of matrix.
-// Measured per step, every row / rows as needed (us; Zipf tokens unless "uniform"): 0.4 MB 24.3 / 23.0, 0.5 MB 22.0 / 22.4,
-// 4 MB 24.6 / 22.1, 8 MB and 0.1 positions a row 26.1 / 22.2, 9.6 MB and 7.5 positions 36.2 / 36.3,
-// 16 MB and 2.75 positions 28.7 / 29.1, 30 positions 67.3 / 68.1,
-// 64 MB and 2.75 positions 52.7 / 45.0 (uniform 69.7 / 67.1), 11 positions 97.1 / 94.1, 80 MB and 0.2 positions 50.6 / 34.3,
-// 22 positions 183.3 / 178.2, 400 MB and 7.5 positions 441 / 400 (uniform 690 / 677).
-#define FV_ROWS_MOST_POSITIONS 24ull
-#define FV_ROWS_LEAST_BYTES (4ull << 20)
-#define FV_ROWS_LEAST_LDK 32u  // (the lists take 16 bytes per row: an eighth of a matrix this narrow)
-// Steps whose xx is kept (a power of two): what fits the dense launch's LDS beside its lists.
-static inline uint32_t fv_rows_age(uint32_t ldk) { return ldk <= 1024 ? 16u : 8u; }
 
 struct fv_rows_args {
   fv_rows_list_args list;

@@ -148,21 +148,54 @@ def test_dense_launches_chosen_behind_a_launch_that_gave_up(gpu, oracle_lib, lau
     t.close()
 
 
-def test_left_alone_where_the_maximum_keeps_failing(gpu, oracle_lib):
-    """Chosen by the sizes, the form is not taken, or left again, where the launches have to make the pass for max|ds|."""
+@pytest.mark.parametrize("synapses", ["small", "middling", "planted"])
+def test_chosen_by_the_sizes_and_by_what_the_launches_find(gpu, oracle_lib, synapses):
+    """Three epochs of 253 steps, the form chosen as by default. The largest |ds| of the sparse elements is 40 to 115 times
+    the dense ones' bound (small: the form is taken but for the first steps on a new matrix, through several refreshes of
+    the bound), 1.4 to 3.8 times (middling: it is entered and left, as a launch that finds less than twice ends it), or just the
+    largest of all (planted: no launch finds it clear and the form is never taken)."""
+    from flyvec_amd import synthetic
     to = oracle_lib
     V, K, w, B = 12000, 100, 5, 200
     tokens, offsets = small_corpus(60000, V, seed=2)
     starts, invf = to.window_starts(offsets, w), to.inverse_frequency(tokens, V)
-    W0 = _planted(tokens, V, K)
-    t, perm = _trainer(tokens, offsets, V, K, w, B, W0, mode=0)
+    W0 = _planted(tokens, V, K) if synapses == "planted" else synthetic.synapses(K, V, seed=3, sigma=0.02 if synapses == "small" else 0.11)
+    t, perm = _trainer(tokens, offsets, V, K, w, B, W0, lr0=5e-4, mode=0)
     Wo = W0.copy()
     n_steps = (len(starts) + B - 1) // B
     for ep in (3, 4, 5):
         t.run_epoch(ep, 15)
-        to.train_steps(Wo, tokens, starts, perm, 0, B, n_steps, w, invf, to.epoch_eps(1e-3, ep, 15))
+        to.train_steps(Wo, tokens, starts, perm, 0, B, n_steps, w, invf, to.epoch_eps(5e-4, ep, 15))
         assert np.array_equal(t.get_weights().view(np.uint32), Wo.view(np.uint32)), ep
-    assert n_steps > 100 and t.row_update_steps < 3 * n_steps - 30
+    taken, known = t.row_update_steps, t.dense_path_counts[0]
+    assert n_steps == 254 and sum(t.dense_path_counts) == 3 * n_steps
+    if synapses == "small":
+        assert taken >= 3 * n_steps - 10 and known >= 3 * n_steps - 1
+    elif synapses == "middling":
+        assert 0 < taken < 3 * n_steps - 100
+    else:
+        assert taken == 0
+    t.close()
+
+
+@pytest.mark.parametrize("eps,taken", [(6.2e-4, True), (6.3e-4, False)])
+def test_left_alone_beyond_the_largest_learning_rate(gpu, oracle_lib, eps, taken):
+    """The bound of |W| grows by |eps| a step: by the sizes the form asks for 32 steps between two refreshes of it."""
+    from flyvec_amd import synthetic
+    to = oracle_lib
+    V, K, w, B, n_steps = 12000, 100, 5, 200, 40
+    tokens, offsets = small_corpus(60000, V, seed=2)
+    starts, invf = to.window_starts(offsets, w), to.inverse_frequency(tokens, V)
+    W0 = synthetic.synapses(K, V, seed=3, sigma=0.02)
+    t, perm = _trainer(tokens, offsets, V, K, w, B, W0, mode=0)
+    for rep in range(2):  # (the first steps' answers are in hand)
+        for s in range(rep * n_steps, (rep + 1) * n_steps):
+            t.step(s * B, B, eps)
+        t.sync()
+    Wo = W0.copy()
+    to.train_steps(Wo, tokens, starts, perm, 0, B, 2 * n_steps, w, invf, np.float32(eps))
+    assert np.array_equal(t.get_weights().view(np.uint32), Wo.view(np.uint32))
+    assert t.row_update_steps >= n_steps - 9 if taken else t.row_update_steps == 0
     t.close()
 
 

@@ -11,9 +11,13 @@
 // additions; if all three results share a binade and the two differences are equal, the state
 // is steady and the remaining additions inside the binade are one integer multiply-add on the
 // bit pattern (stopping short of the binade's ends); binade crossings, including the passage
-// through zero, are taken with real additions.  Fewer than FV_REPEAT_JUMP additions are simply made, eight to a turn:
-// a turn that looks for the steady state costs as much as sixty additions (the division), and the sums of an ordinary
-// minibatch have a few dozen.  Compiles for the host too, where the tests check it against the plain loop.
+// through zero, are taken with real additions.  Fewer than FV_REPEAT_JUMP additions are simply made, eight to a turn: a
+// turn that looks for the steady state divides, and the sums of an ordinary minibatch have a few additions to a few dozen.
+// Where the line lies, in us of a whole step with 4 (as good as always looking), 32, 48, 64, 96, 256: K = 400, V = 20000,
+// B = 10000 51.9 51.6 51.6 51.6 51.6 51.7, with the anti-Hebbian term 68.7 68.3 68.4 68.5 68.5 68.5; K = 209, V = 7919, B =
+// 3001 26.8 26.5 26.4 26.4 26.4 26.5; K = 100, V = 2000, B = 10000 38.5 38.5 38.6 38.7 38.9 39.1; K = 60, V = 1000, B =
+// 16000 42.0 42.2 42.2 42.3 42.7 -; K = 1000, V = 50000, B = 50000 406.8 404.8 404.6 404.7 404.8 -. (Replays of the launch by itself
+// say otherwise: the elements it then finds are sentinels.)  Compiles for the host too, where the tests check it against the plain loop.
 #pragma once
 
 #include <stdint.h>
@@ -48,7 +52,7 @@ FV_HD float fv_add1(float a, float b) {
 }
 
 #ifndef FV_REPEAT_JUMP
-#define FV_REPEAT_JUMP 96u
+#define FV_REPEAT_JUMP 48u
 #endif
 
 FV_HD float fv_add_repeat(float v, float f, uint32_t n) {

@@ -438,7 +438,8 @@ __device__ __forceinline__ void fv_sparse_block(const fv_sparse_args &a) {
     // The launch lasts as long as its few heaviest blocks: their waves go first wherever they share a
     // SIMD with the waves of light blocks.
     if (c_h > FV_SP_HEAVY) __builtin_amdgcn_s_setprio(3);
-    // the window ids of the usual neuron go to LDS while the activations travel (the counting pass starts behind a barrier)
+    // the window ids of the usual neuron go to LDS while the activations travel (the counting pass starts behind a barrier):
+    // a whole step with the ids behind xx and so 51.6 and 51.5 us, 26.5 and 26.3, 39.2 and 39.0 (sizes as at the scan below)
     if (!DELTA && c_h <= stage_cap) stage_ids(0);
     // xx[h]: the thread's group first, in row order onto +0 (what was fetched, then, for a thread with more matches
     // than that, the rest one by one), then the tree over the threads
@@ -622,9 +623,9 @@ __device__ __forceinline__ void fv_sparse_block(const fv_sparse_args &a) {
         // Bits 8 i .. 8 i + 7 of `mine`: the non-zero counters of the thread's i-th group of four words. narrow: the low
         // halves of the words, then the high ones (a packed minimum with 1 leaves a word's two answers 16 bits apart: three
         // instructions a word where there were eight). All blocks of a compute unit come through here at about the same
-        // time and the vector units are what they wait for: 1.6 to 1.9 us of every block's 7 to 12. With the plain
-        // additions of fv_add_repeat and the window ids staged while the activations travel, K = 400, V = 20000,
-        // B = 10000: 15.1 -> 14.2 us, with the anti-Hebbian term 31.0 -> 28.9, K = 209, V = 7919, B = 3001 11.2 -> 10.1.
+        // time and the vector units are what they wait for: 1.6 to 1.9 us of every block's 7 to 12. A whole step with two
+        // comparisons a word and so: K = 400, V = 20000, B = 10000 51.9 and 51.5 us, K = 209, V = 7919, B = 3001 26.6 and
+        // 26.3, K = 100, V = 2000, B = 10000 39.1 and 39.0.
         constexpr int n_groups = (CW / 4 + T - 1) / T;
         static_assert(n_groups <= 8, "a 64-bit mask holds eight groups");
         uint64_t mine = 0;

@@ -91,10 +91,11 @@ def kernel_bytes(K, N, w, B, single_dense_launch=False):
     once each way. The sparse term is 16 bytes per window position in the byte model (token id, 1/f look-up,
     read and write of the element): as six launches half of it falls to the sparse launch and half to the slot
     update; with the single dense launch the sparse launch is held to all 16 (it reads the ids and 1/f, reads the
-    elements and writes the sentinels) and the dense launch's share is the records it reads back."""
+    elements and writes the sentinels) and the dense launch's share is the records it reads back. The grouping launch
+    reads a 16-bit winner and an activation per window and writes the window's place in the order."""
     return {
         "gather_winner": 4 * B * w * K,
-        "group_xx": 8 * B,
+        "group_xx": 10 * B,
         "sparse_owners": (16 if single_dense_launch else 8) * B * w,
         "absmax_ds": 4 * K * N,
         "update": 8 * K * N,

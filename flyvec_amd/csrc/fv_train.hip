@@ -10,11 +10,12 @@
 //                      neurons spread over lanes (:248-263, double accumulators, one rounding),
 //                      argmax by a wave reduction (:488-561) and the winner's frequency-scaled
 //                      activation (:289-305; it is only ever read at the winner, :731).
-//   2. group + xx      one block per neuron h: the ordered list of the windows h won and xx[h], the
+//   2. group + xx      the ordered list of the windows a neuron h won and xx[h], the
 //                      sum of their scaled activations (:722-744 -- the reference's atomic order
 //                      is undefined, this one is fixed, so a step is reproducible bit for bit).
-//                      A launch of its own only for batches beyond 16384 windows and for steps
-//                      with the anti-Hebbian term: otherwise the blocks of launch 3 do it
+//                      A launch of its own, a block per one to four neurons, for batches beyond
+//                      16384 windows (with the anti-Hebbian term also where the blocks of launch 3
+//                      have no slot regions of their own): otherwise the blocks of launch 3 do it
 //                      themselves, from the bit rows launch 1 leaves.
 //   3. sparse owners   four blocks per neuron, one per column class: the sparse Hebbian term of
 //                      row h (:657-672). A block alone owns its elements (h, column), so it counts

@@ -257,7 +257,7 @@ __device__ __forceinline__ uint32_t fv_nonzero_halves(uint32_t word) {
 }
 
 // DELTA: the neuron's elements are counted over two lists of windows, those it won and those in
-// which it came second, into two counter arrays; a record carries both counts.
+// which it came second, into two counter arrays; ds is formed from both, and the record carries it.
 // GROUPING: no grouping launch has run. Every class block takes its neuron's windows from the bit row
 // the winner kernel has filled (a thread's two words are one group of 64 windows: the step has no more than
 // 64 * FV_SP_THREADS), stages the window ids in LDS by rank, and adds the neuron's scaled activations in the

@@ -200,8 +200,8 @@ class Trainer:
 
     def set_row_updates(self, mode):
         """1: the single dense launch updates every row of the matrix in every step; 2: the rows the step has touched
-        or the next one reads, each with all the steps it lacks, where it can; 0 (the default): by the sizes.
-        Same results."""
+        or the next one reads, each with all the steps it lacks, where it can; 0 (the default): by the sizes, in steps
+        that follow each other, at |eps| up to 6.25e-4, and by what the launches before have found. Same results."""
         check(self.lib.fv_trainer_set_row_updates(self.handle, int(mode)))
 
     @property

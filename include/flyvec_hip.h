@@ -187,7 +187,7 @@ int fv_trainer_set_permutation(fv_trainer *t, const uint64_t *perm, uint64_t n);
 int fv_trainer_get_permutation(fv_trainer *t, uint64_t *out_perm, uint64_t capacity);
 
 /* One pass of the minibatch loop body, flyvec/src/cuda_funcs.cu:1662-1803, on windows
- * perm[first_window .. first_window + n_windows) with n_windows <= batch. Asynchronous. */
+ * perm[first_window .. first_window + n_windows) with n_windows <= batch. Asynchronous: it waits for nothing. */
 int fv_trainer_step(fv_trainer *t, uint64_t first_window, uint32_t n_windows, float eps);
 
 /* The same step with the anti-Hebbian term of strength `delta` (flyvec/src/cuda_funcs.cu:495-548,
@@ -250,9 +250,9 @@ int fv_trainer_get_dense_forms(fv_trainer *t, uint64_t *out_one, uint64_t *out_t
  * register or its streaming form, as the matrix size and that call decide), 2 = separate launches. */
 int fv_trainer_get_dense_launches(fv_trainer *t, uint32_t *out_launches);
 /* Grouping the windows of a step by winner (what flyvec/src/cuda_funcs.cu:1719-1721 leaves in
- * max_IDs and xx) runs inside the sparse-element launch when the trainer's batch is at most 16384
- * windows and the step has no anti-Hebbian term, as a launch of its own otherwise. separate = 1 forces the launch of its
- * own, 0 returns to that rule. Results are bit-identical either way. */
+ * max_IDs and xx) runs inside the sparse-element launch when the trainer's batch is at most 16384 windows (with the
+ * anti-Hebbian term: and that launch's blocks have records of their own, below), as a launch of its own otherwise.
+ * separate = 1 forces the launch of its own, 0 returns to that rule. Results are bit-identical either way. */
 int fv_trainer_set_grouping_launch(fv_trainer *t, uint32_t separate);
 int fv_trainer_get_grouping_launch(fv_trainer *t, uint32_t *out_separate); /* the form a step without the anti-Hebbian term takes */
 /* Where the sparse-element launch that groups for itself keeps a step's records of sparse elements (the
@@ -272,9 +272,12 @@ int fv_trainer_set_light_blocks(fv_trainer *t, uint32_t on);
 /* How the single dense launch takes the rows of W (a row holds the weights of one token). mode 1: it updates every row
  * in every step. mode 2: where it can (no other trainer in flight, no duplicate pruning) it visits the rows that this
  * step has touched or the next one reads, and brings each up to date with all the steps it lacks; nothing is
- * left undone when a call that waits for the trainer returns. mode 0, the default: by the sizes, where at least eight
- * steps follow each other without such a call in between. Results are bit-identical. get: steps so far whose dense
- * launch visited rows. No counterpart in the reference. */
+ * left undone when fv_trainer_sync or a call that returns something of the matrix or of a step returns. mode 0, the
+ * default: at the sizes where that was measured to be faster, where at least eight steps follow each other, each on the
+ * windows behind the last one's, without such a call in between, where |eps| <= 6.25e-4 (at a learning rate of 0.002 over
+ * 15 epochs: from the twelfth epoch on) and where the launches before have found max|ds| to be a sparse element's by a
+ * factor of two. Results are bit-identical. get: steps so far whose dense launch visited rows. No counterpart in the
+ * reference. */
 int fv_trainer_set_row_updates(fv_trainer *t, uint32_t mode);
 int fv_trainer_get_row_updates(fv_trainer *t, uint64_t *out_steps);
 /* Test hook. The single dense launch notes the sparse elements it meets (their sentinels) in LDS lists, one of

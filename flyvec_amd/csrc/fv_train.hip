@@ -309,8 +309,9 @@ static hipError_t fv_trainer_settle(fv_trainer *t) {
   return hipGetLastError();
 }
 
-// Waits for the trainer's stream, every row of the matrix up to date. Every wait of this file goes through here, so that a trainer whose steps have been
-// waited for by whatever call is out of the count.
+// Waits for the trainer's stream, every row of the matrix up to date. Every wait of this file goes through here, but
+// for the copies of get_window_starts, get_permutation and set_weights, which wait for the stream themselves and say so:
+// a trainer whose steps have been waited for by whatever call is out of the count.
 static hipError_t fv_trainer_drain(fv_trainer *t) {
   hipError_t e = fv_trainer_settle(t);
   if (e == hipSuccess) e = hipStreamSynchronize(t->stream);

@@ -232,11 +232,11 @@ def test_steps_that_do_not_follow_each_other(gpu, oracle_lib, order):
 
 @pytest.mark.parametrize("mode", [0, 2])
 def test_steps_are_enqueued_without_waiting_for_the_device(gpu, mode):
-    """2000 steps of 20 to 40 us: the host is done with them long before the device is (8 to 10 us a step)."""
+    """2000 steps of 30 to 40 us: the host is done with them long before the device is (8 to 10 us a step)."""
     import time
     from flyvec_amd import synthetic
-    V, K, w, B, n_steps = 20000, 400, 5, 2000, 2000
-    tokens, offsets = small_corpus(400000, V, seed=2)
+    V, K, w, B, n_steps = 20000, 400, 11, 4000, 2000
+    tokens, offsets = small_corpus(1500000, V, seed=2)
     t, _ = _trainer(tokens, offsets, V, K, w, B, synthetic.synapses(K, V, seed=3, sigma=0.02), mode=mode)
     N = t.num_windows // B
     t.step(0, B, 2e-4)
@@ -250,7 +250,7 @@ def test_steps_are_enqueued_without_waiting_for_the_device(gpu, mode):
         t.sync()
         ratios.append((t1 - t0) / (time.perf_counter() - t0))
     assert t.row_update_steps - before > n_steps / 4
-    assert min(ratios) < 0.7, ratios
+    assert min(ratios) < 0.6, ratios
     t.close()
 
 
